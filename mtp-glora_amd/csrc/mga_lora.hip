@@ -293,12 +293,11 @@ __global__ __launch_bounds__(256) void lora_down_ring_kernel(LoraDownArgs a) {
     // flight, so with the dropout output written here the wait is a full one.
     if (c >= RING - 1 && !WRITE_H) __builtin_amdgcn_s_waitcnt(vmcnt_imm(3 * kOps + 4));
     else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-    // every wave's part of chunk c is in; chunk c - 1's buffer is free. A bare
-    // barrier between compiler fences: __syncthreads' memory fence would make
-    // the compiler wait for every load in flight, the ring's included.
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
+    // every wave's part of chunk c is in; chunk c - 1's buffer is free.
+    // __syncthreads' memory fence would make the compiler wait for every load
+    // in flight, the ring's included; the barrier waits for this wave's LDS
+    // reads of chunk c - 1, whose products the compiler may place after it.
+    lds_barrier();
     issue(c + RING - 1);
     // the operands of chunk c (issued before the two loads just above)
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(2));
@@ -857,17 +856,18 @@ __device__ __forceinline__ void lora_skinny_body(const LoraSkinnyArgs &a) {
   };
 
   // chunk c: its loads landed (the next two chunks' loads may still be in
-  // flight), a bare barrier (every wave's part is in, and the buffer of chunk
-  // c - 1 is free), then the loads of chunk c + 3 and the products of chunk c
+  // flight), a barrier behind this wave's LDS reads (every wave's part is in,
+  // and the buffer of chunk c - 1 is free: the compiler sinks chunk c - 1's
+  // products, and with them the wait for their operand reads, past a bare
+  // s_barrier, and the loads of chunk c + 3 then overwrite operands not yet
+  // read), then the loads of chunk c + 3 and the products of chunk c
   // (every iteration runs all four chunks, those past the share without
   // products, so the loads in flight at the loop head are the same on every
   // path and the compiler adds no wait of its own)
   auto chunk = [&](auto bsel, int c) {
     constexpr int B = decltype(bsel)::value;
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * NL));
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
+    lds_barrier();
     issue(c + 3, B == 0 ? sY3 : (B == 1 ? sY0 : (B == 2 ? sY1 : sY2)),
           B == 0 ? sM3 : (B == 1 ? sM0 : (B == 2 ? sM1 : sM2)));
     if (c < nch)
