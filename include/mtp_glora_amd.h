@@ -167,6 +167,50 @@ int mga_attn_bwd(const void *q, int64_t q_sh, int64_t q_ss,
                  int32_t head_dim, int32_t dtype, float scale, int32_t passes, void *stream);
 
 /*
+ * mga_attn_fwd and mga_attn_bwd with a workspace for partial results, which
+ * lets a launch whose work items would leave part of the GPU idle (a short
+ * chunk against a long prefix, or the last round of any chunk) split its last
+ * items over their keys: the parts' fp32 results are combined in a fixed
+ * order, so calls stay bit-for-bit repeatable. Results agree with the calls
+ * without a workspace up to the order of fp32 sums.
+ * workspace: mga_attn_workspace_bytes(...) bytes (backward 0 or 1) of device
+ *   memory, 16-byte aligned, used by this call only; NULL (or a shape that
+ *   needs none): the call is mga_attn_fwd / mga_attn_bwd. A non-NULL workspace
+ *   smaller than needed is MGA_ERR_INVALID.
+ * mga_attn_workspace_bytes depends on the current device's number of compute
+ * units; 0 for a shape that is not split (or invalid sizes).
+ */
+int64_t mga_attn_workspace_bytes(int32_t S, int32_t L, int32_t Hq, int32_t Hkv, int32_t head_dim, int32_t dtype,
+                                 int32_t backward);
+int mga_attn_fwd_ws(const void *q, int64_t q_sh, int64_t q_ss,
+                    const void *k, int64_t k_sh, int64_t k_ss,
+                    const void *v, int64_t v_sh, int64_t v_ss,
+                    void *o, int64_t o_sh, int64_t o_ss,
+                    float *lse, const int32_t *code,
+                    const int32_t *kv_num, const int32_t *kv_idx,
+                    const int32_t *full_kv_num, const int32_t *full_kv_idx,
+                    int32_t S, int32_t L, int32_t P, int32_t Hq, int32_t Hkv,
+                    int32_t head_dim, int32_t dtype, float scale,
+                    void *workspace, int64_t workspace_bytes, void *stream);
+int mga_attn_bwd_ws(const void *q, int64_t q_sh, int64_t q_ss,
+                    const void *k, int64_t k_sh, int64_t k_ss,
+                    const void *v, int64_t v_sh, int64_t v_ss,
+                    const void *o, int64_t o_sh, int64_t o_ss,
+                    const void *dout, int64_t do_sh, int64_t do_ss,
+                    const float *lse, float *delta,
+                    void *dq, int64_t dq_sh, int64_t dq_ss,
+                    void *dk, int64_t dk_sh, int64_t dk_ss,
+                    void *dv, int64_t dv_sh, int64_t dv_ss,
+                    int32_t grad_start, const int32_t *code,
+                    const int32_t *kv_num, const int32_t *kv_idx,
+                    const int32_t *full_kv_num, const int32_t *full_kv_idx,
+                    const int32_t *q_num, const int32_t *q_idx,
+                    const int32_t *full_q_num, const int32_t *full_q_idx,
+                    int32_t S, int32_t L, int32_t P, int32_t Hq, int32_t Hkv,
+                    int32_t head_dim, int32_t dtype, float scale, int32_t passes,
+                    void *workspace, int64_t workspace_bytes, void *stream);
+
+/*
  * mga_attn_bwd without the delta workspace argument, for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc). No counterpart in the reference. delta

@@ -47,6 +47,15 @@ SIGNATURES = {
                      _P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64,
                      _I32, _P, _P, _P, _P, _P, _P, _P, _P, _P,
                      _I32, _I32, _I32, _I32, _I32, _I32, _I32, _F32, _I32, _P],
+    "mga_attn_workspace_bytes": [_I32, _I32, _I32, _I32, _I32, _I32, _I32],
+    "mga_attn_fwd_ws": [_P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64,
+                        _P, _P, _P, _P, _P, _P,
+                        _I32, _I32, _I32, _I32, _I32, _I32, _I32, _F32, _P, _I64, _P],
+    "mga_attn_bwd_ws": [_P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64,
+                        _P, _P,
+                        _P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64,
+                        _I32, _P, _P, _P, _P, _P, _P, _P, _P, _P,
+                        _I32, _I32, _I32, _I32, _I32, _I32, _I32, _F32, _I32, _P, _I64, _P],
     "mga_attn_bwd_noalloc": [_P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64,
                              _P,
                              _P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64,
@@ -70,7 +79,7 @@ SIGNATURES = {
     "mga_soft_ce_bwd": [_P, _I64, _P, _I64, _I32, _I32, _I32, _P, _P, _P, _I64, _P],
 }
 _RESTYPES = {"mga_last_error": ctypes.c_char_p, "mga_soft_ce_workspace_floats": ctypes.c_int64,
-             "mga_gated_lora_workspace_bytes": ctypes.c_int64}
+             "mga_gated_lora_workspace_bytes": ctypes.c_int64, "mga_attn_workspace_bytes": ctypes.c_int64}
 
 
 class MGAError(RuntimeError):

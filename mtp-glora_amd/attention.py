@@ -54,7 +54,7 @@ class _MTPAttention(torch.autograd.Function):
         passes = _lib.BWD_DQ | (_lib.BWD_DKDV if need_kv else 0)
         dq, dk, dv = ops.attn_bwd(q, k_full, v_full, o, lse, do, mask.mtp_code,
                                   mask.kernel_tensors(), mask.prefix_len, ctx.scale, grad_start,
-                                  passes=passes)
+                                  passes=passes, key_split=True)
         dq = dq if ctx.needs_input_grad[0] else None
         dk = dk if ctx.needs_input_grad[1] else None
         dv = dv if ctx.needs_input_grad[2] else None

@@ -7,8 +7,14 @@
 //   waves per SIMD), two 32-row blocks per head; each staged K/V tile feeds
 //   all 8 waves, half the tile loads and LDS writes per MFMA of two 4-wave
 //   workgroups sharing the CU.
-// * kDqSplit: the last round of kDqPair items when it would fill at most half
-//   of the CUs: each half of an item (one 32-row block per head) runs as an
+// With a workspace (mga_attn_bwd_ws) the items of a last round that would leave
+// slots idle run as parts of their tile lists in the same launch (KeySplit),
+// whose fp32 sums attn_bwd_dq_merge_kernel adds: [508 rows x 32 heads] against
+// 20 491 prefix keys 442 -> 244 + 8 us, 2 529 rows against 4 093 (fp16) 405 ->
+// 326 + 8 us.
+// * kDqSplit (calls without a workspace): the last round of kDqPair items when
+//   it would fill at most half of the CUs: each half of an item (one 32-row
+//   block per head) runs as an
 //   8-wave workgroup whose two 4-wave groups take alternate tiles of the list;
 //   group 1 hands its dQ partial sums to group 0 through LDS at the end, added
 //   in a fixed order.
@@ -31,6 +37,7 @@
 
 #include "mga_common.hpp"
 #include "mga_internal.hpp"
+#include "mga_key_split.hpp"
 
 namespace mga {
 
@@ -43,6 +50,10 @@ constexpr int kSubKeys = 32;   // keys per compute block (the accumulators hold 
 __host__ __device__ __forceinline__ int heads_per_wg_dq(int G) { return (G % 4 == 0) ? 4 : (G % 2 == 0 ? 2 : 1); }
 
 enum { kDq4 = 0, kDqPair = 1, kDqSplit = 2 };
+
+// A part's fixed cost (about 7 us against 5.2 us a tile) and the merge launch's
+// (8 us), in key tiles (for key_split_plan).
+constexpr float kDqPartTiles = 1.5f, kDqMergeTiles = 2.f;
 
 // Sum over this lane's half of the row (dims ks*16 + hi*8 .. +8) of o * d.
 template <int HD, typename T>
@@ -62,7 +73,8 @@ __device__ __forceinline__ float half_row_dot(const T *o, const T *d, int hi) {
 }  // namespace
 
 template <int HD, typename T, int MODE>
-__global__ __launch_bounds__(MODE == kDq4 ? 256 : 512, 2) void attn_bwd_dq_kernel(AttnArgs a, int k1, int kn) {
+__global__ __launch_bounds__(MODE == kDq4 ? 256 : 512, 2) void attn_bwd_dq_kernel(AttnArgs a, int k1, int kn,
+                                                                                    KeySplit sp) {
   constexpr int NG = MODE == kDqSplit ? 2 : 1;    // groups splitting the tile list
   constexpr int NWD = MODE == kDqPair ? 8 : 4;    // waves sharing each staged tile
   typedef typename MfmaElem<T>::type E;
@@ -86,21 +98,20 @@ __global__ __launch_bounds__(MODE == kDq4 ? 256 : 512, 2) void attn_bwd_dq_kerne
   const int HPW = heads_per_wg_dq(G);
   const int QR4 = 32 * (4 / HPW);   // rows of 4 waves: 32, 64 or 128
   const int nslice = G / HPW;
-  int li, nqb, qr_item;
-  if constexpr (MODE == kDq4) {
-    qr_item = QR4;
-    nqb = (a.S + QR4 - 1) / QR4;
-    li = xcd_swizzle(blockIdx.x, a.Hkv * nslice * nqb);
+  const int qr_item = MODE == kDq4 ? QR4 : 2 * QR4;
+  const int nqb = (a.S + qr_item - 1) / qr_item;
+  const int n_items = a.Hkv * nslice * nqb;
+  const int xcd = blockIdx.x & 7;
+  const int t = (int)(blockIdx.x >> 3);
+  int o, part = -1;   // part: the share of the tile list, -1 = all of it
+  if constexpr (MODE == kDqSplit) {
+    o = k1 + (t >> 1);
   } else {
-    qr_item = 2 * QR4;
-    nqb = (a.S + qr_item - 1) / qr_item;
-    const int n_items = a.Hkv * nslice * nqb;
-    const int xcd = blockIdx.x & 7;
-    const int o = k1 + (int)(MODE == kDqSplit ? blockIdx.x >> 4 : blockIdx.x >> 3);
-    const int n_x = n_items / 8 + (xcd < n_items % 8 ? 1 : 0);
-    if (o >= n_x || o >= k1 + kn) return;
-    li = xcd * (n_items / 8) + min(xcd, n_items % 8) + o;
+    sp.locate(t, o, part);
   }
+  const int n_x = n_items / 8 + (xcd < n_items % 8 ? 1 : 0);
+  if (o >= n_x || o >= k1 + kn) return;
+  const int li = xcd * (n_items / 8) + min(xcd, n_items % 8) + o;
   const int g = li / (nslice * nqb);
   const int rem = li % (nslice * nqb);
   const int qb = nqb - 1 - rem / nslice;
@@ -140,7 +151,7 @@ __global__ __launch_bounds__(MODE == kDq4 ? 256 : 512, 2) void attn_bwd_dq_kerne
   // (0 for a row that sees no key), -delta, and the row's mask threshold
   // (0: sees no key; 1: regular row, sees the regular keys; 2^31 - 1 - c: mask
   // row of code c, sees the mask keys of codes >= c). A row past S reads as 0.
-  if (in && hi == 0 && grp == 0) {
+  if (in && hi == 0 && grp == 0 && part <= 0) {
     const int64_t plane = (int64_t)a.Hq * a.S, at = (int64_t)h * a.S + row;
     a.delta[at] = none ? 0.f : -lse * (1.f / a.scale);
     a.delta[plane + at] = -del;
@@ -153,11 +164,17 @@ __global__ __launch_bounds__(MODE == kDq4 ? 256 : 512, 2) void attn_bwd_dq_kerne
 
   TileList tiles = tile_list(a.kv_num, a.kv_idx, a.fkv_num, a.fkv_idx, qt, a.nKV);
   const int npart = tiles.npart;
-  const int ntot = tiles.ntot;
+  // the workgroup's share of the list (all of it unless the item is split),
+  // entries t0 .. t0 + nt - 1
+  int t0 = 0, nt = tiles.ntot;
+  if (MODE != kDqSplit && part >= 0) {
+    t0 = sp.begin(part, tiles.ntot);
+    nt = sp.begin(part + 1, tiles.ntot) - t0;
+  }
   constexpr int kSub = kBlock / kStep;      // steps per 128-key tile
-  const int nstep = kSub * ((ntot - grp + NG - 1) / NG);   // this group's steps
-  const int nloop = kSub * ((ntot + NG - 1) / NG);        // group 0's (>= group 1's)
-  auto tile_of = [&](int j) { return NG * (j / kSub) + grp; };
+  const int nstep = kSub * ((nt - grp + NG - 1) / NG);   // this group's steps
+  const int nloop = kSub * ((nt + NG - 1) / NG);        // group 0's (>= group 1's)
+  auto tile_of = [&](int j) { return t0 + NG * (j / kSub) + grp; };
   auto step_base = [&](int j) { return tiles.at(tile_of(j)) * kBlock + (j % kSub) * kStep; };
 
   // K / V / dO operand of k-step ks: row l32, granule (2 ks + hi) ^ swz(l32),
@@ -317,6 +334,20 @@ __global__ __launch_bounds__(MODE == kDq4 ? 256 : 512, 2) void attn_bwd_dq_kerne
       for (int r = 0; r < 16; ++r) dqacc[db][r] += x[(db * 16 + r) * 64 + lane];
   }
 
+  if constexpr (MODE != kDqSplit) {
+    if (part >= 0) {   // a part's dQ^T sums: attn_bwd_dq_merge_kernel adds them
+      float *po = sp.ws + (sp.slot(o, part, xcd) * (blockDim.x / 64) + wave) * (HD * 32);
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const f32x4 v = {dqacc[db][4 * q], dqacc[db][4 * q + 1], dqacc[db][4 * q + 2], dqacc[db][4 * q + 3]};
+          *reinterpret_cast<f32x4 *>(po + ((db * 4 + q) * 64 + lane) * 4) = v;
+        }
+      return;
+    }
+  }
+
   if (in) {
     T *row_out = reinterpret_cast<T *>(a.dq) + h * a.dq_sh + (int64_t)row * a.dq_ss;
 #pragma unroll
@@ -328,6 +359,45 @@ __global__ __launch_bounds__(MODE == kDq4 ? 256 : 512, 2) void attn_bwd_dq_kerne
                c[4 * i + 2] * a.scale, c[4 * i + 3] * a.scale);
       }
   }
+}
+
+// dQ = scale * the parts' sums of the split items, added in the order of the
+// parts (bit-for-bit repeatable). Workgroup (item u of the XCD's split items,
+// 32-dim block db), threads as in the item's workgroups.
+template <int HD, typename T, int NW>
+__global__ __launch_bounds__(64 * NW) void attn_bwd_dq_merge_kernel(AttnArgs a, KeySplit sp) {
+  constexpr int DB = HD / 32;
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int l32 = lane & 31, hi = lane >> 5;
+  const int G = a.Hq / a.Hkv;
+  const int HPW = heads_per_wg_dq(G);
+  const int qr_item = (NW / 4) * 32 * (4 / HPW);
+  const int nslice = G / HPW;
+  const int nqb = (a.S + qr_item - 1) / qr_item;
+  const int n_items = a.Hkv * nslice * nqb;
+  const int xcd = blockIdx.x & 7, u = (int)(blockIdx.x >> 3) / DB, db = (int)(blockIdx.x >> 3) % DB;
+  const int o = sp.k + u;
+  if (o >= n_items / 8 + (xcd < n_items % 8 ? 1 : 0)) return;
+  const int li = xcd * (n_items / 8) + min(xcd, n_items % 8) + o;
+  const int g = li / (nslice * nqb), rem = li % (nslice * nqb);
+  const int h = g * G + (rem % nslice) * HPW + wave % HPW;
+  const int row = (nqb - 1 - rem / nslice) * qr_item + (wave / HPW) * 32 + l32;
+  const float *p0 = sp.ws + (sp.slot(o, 0, xcd) * NW + wave) * (HD * 32);
+  const int64_t step = (int64_t)8 * NW * (HD * 32);   // to the next part
+  f32x16 acc = zero16();
+  for (int p = 0; p < sp.ns; ++p)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const f32x4 v = *reinterpret_cast<const f32x4 *>(p0 + p * step + ((db * 4 + q) * 64 + lane) * 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[4 * q + e] += v[e];
+    }
+  if (row >= a.S) return;
+  T *row_out = reinterpret_cast<T *>(a.dq) + h * a.dq_sh + (int64_t)row * a.dq_ss;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    store4(row_out + db * 32 + 8 * i + 4 * hi, acc[4 * i] * a.scale, acc[4 * i + 1] * a.scale,
+           acc[4 * i + 2] * a.scale, acc[4 * i + 3] * a.scale);
 }
 
 // kDqPair items per XCD (the rest run as kDqSplit): each XCD takes a
@@ -344,24 +414,66 @@ int dq_split_point(int items, int L, int cus) {
   return (nmax > m && r > 0 && r <= m / 2) ? nmax - r : nmax;
 }
 
-template <int HD, typename T>
-void dq_launch(const AttnArgs &a, hipStream_t st) {
+namespace {
+
+// waves of a workgroup, rows of an item, head slices of a kv head, items,
+// items per XCD at most, workgroup slots per XCD
+struct DqGrid {
+  int nw, rows, nslice, items, nmax, slots;
+};
+
+DqGrid dq_grid(const AttnArgs &a) {
   const int G = a.Hq / a.Hkv;
   const int HPW = heads_per_wg_dq(G);
-  const int QR4 = 32 * (4 / HPW);
-  if (HPW == 1) {
-    const int nqb = (a.S + QR4 - 1) / QR4;
-    hipLaunchKernelGGL((attn_bwd_dq_kernel<HD, T, kDq4>), dim3(a.Hkv * G * nqb), dim3(256), 0, st, a, 0, 0);
-    return;
+  DqGrid f;
+  f.nw = HPW == 1 ? 4 : 8;
+  f.rows = (f.nw / 4) * 32 * (4 / HPW);
+  f.nslice = G / HPW;
+  f.items = a.Hkv * f.nslice * ((a.S + f.rows - 1) / f.rows);
+  f.nmax = (f.items + 7) / 8;
+  f.slots = std::max(1, (f.nw == 8 ? 1 : 2) * (device_cu_count() / 8));
+  return f;
+}
+
+KeySplit dq_split(const AttnArgs &a) {
+  const DqGrid f = dq_grid(a);
+  return key_split_plan(f.nmax, f.slots, last_round_tiles(a.S, a.P, a.Hkv, f.nslice, f.rows, f.nmax % f.slots),
+                        kDqPartTiles, kDqMergeTiles);
+}
+
+}  // namespace
+
+int64_t attn_bwd_ws_floats(const AttnArgs &a, int head_dim, int dtype) {
+  if (dtype == kDtF32) return 0;   // the fp32 kernels do not split
+  const KeySplit sp = dq_split(a);
+  const DqGrid f = dq_grid(a);
+  return sp.ns > 1 ? (int64_t)8 * sp.r * sp.ns * f.nw * head_dim * 32 : 0;
+}
+
+template <int HD, typename T>
+void dq_launch(const AttnArgs &a, hipStream_t st) {
+  const DqGrid f = dq_grid(a);
+  KeySplit sp = a.ws ? dq_split(a) : no_split(f.nmax);
+  int k1 = f.nmax, grid;
+  if (sp.ns > 1) {
+    sp.ws = a.ws;
+    grid = 8 * sp.groups();
+  } else {
+    if (f.nw == 8) k1 = dq_split_point(f.items, a.L, device_cu_count());
+    grid = 8 * k1;
   }
-  const int nqb = (a.S + 2 * QR4 - 1) / (2 * QR4);
-  const int items = a.Hkv * (G / HPW) * nqb;
-  const int nmax = (items + 7) / 8;
-  const int k1 = dq_split_point(items, a.L, device_cu_count());
-  if (k1 > 0) hipLaunchKernelGGL((attn_bwd_dq_kernel<HD, T, kDqPair>), dim3(8 * k1), dim3(512), 0, st, a, 0, k1);
-  if (k1 < nmax)
-    hipLaunchKernelGGL((attn_bwd_dq_kernel<HD, T, kDqSplit>), dim3(16 * (nmax - k1)), dim3(512), 0, st, a, k1,
-                       nmax - k1);
+  if (grid > 0) {
+    if (f.nw == 8) hipLaunchKernelGGL((attn_bwd_dq_kernel<HD, T, kDqPair>), dim3(grid), dim3(512), 0, st, a, 0, k1, sp);
+    else hipLaunchKernelGGL((attn_bwd_dq_kernel<HD, T, kDq4>), dim3(grid), dim3(256), 0, st, a, 0, k1, sp);
+  }
+  if (sp.ns > 1) {
+    const dim3 mg(8 * sp.r * (HD / 32));
+    if (f.nw == 8) hipLaunchKernelGGL((attn_bwd_dq_merge_kernel<HD, T, 8>), mg, dim3(512), 0, st, a, sp);
+    else hipLaunchKernelGGL((attn_bwd_dq_merge_kernel<HD, T, 4>), mg, dim3(256), 0, st, a, sp);
+  } else if (k1 < f.nmax) {
+    hipLaunchKernelGGL((attn_bwd_dq_kernel<HD, T, kDqSplit>), dim3(16 * (f.nmax - k1)), dim3(512), 0, st, a, k1,
+                       f.nmax - k1, sp);
+  }
 }
 
 template void dq_launch<128, bf16_t>(const AttnArgs &, hipStream_t);

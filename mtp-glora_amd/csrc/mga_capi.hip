@@ -85,6 +85,17 @@ int check_attn_common(int32_t S, int32_t L, int32_t P, int32_t Hq, int32_t Hkv, 
   return MGA_OK;
 }
 
+// The workspace of a key-split pass: none (null) runs the pass unsplit.
+int check_attn_ws(const char *fn, void *ws, int64_t bytes, int64_t need, float **out) {
+  *out = nullptr;
+  if (!ws || need == 0) return MGA_OK;
+  if (bytes < need)
+    return fail(MGA_ERR_INVALID, "%s: workspace of %lld bytes, %lld needed", fn, (long long)bytes, (long long)need);
+  if (!aligned16(ws)) return fail(MGA_ERR_INVALID, "%s: workspace not 16-byte aligned", fn);
+  *out = static_cast<float *>(ws);
+  return MGA_OK;
+}
+
 // Workspace of mga_attn_bwd_noalloc (the backward's row data: three words per
 // query head and row): a device array of 3 * kNoAllocRows floats, one copy on
 // every GPU the library runs on, held until the process ends. Host code
@@ -181,12 +192,32 @@ int mga_mtp_block_mask(const int64_t *gate, int64_t gate_stride, int32_t S, int6
   return check_launch("mga_mtp_block_mask");
 }
 
+int64_t mga_attn_workspace_bytes(int32_t S, int32_t L, int32_t Hq, int32_t Hkv, int32_t head_dim, int32_t dtype,
+                                 int32_t backward) {
+  if (check_attn_common(S, L, L - S, Hq, Hkv, head_dim, dtype, 1.f) != MGA_OK) return 0;
+  mga::AttnArgs a = {};
+  a.S = S; a.L = L; a.P = L - S; a.Hq = Hq; a.Hkv = Hkv;
+  a.nQ = (S + MGA_BLOCK - 1) / MGA_BLOCK;
+  a.nKV = (L + MGA_BLOCK - 1) / MGA_BLOCK;
+  return 4 * (backward ? mga::attn_bwd_ws_floats(a, head_dim, dtype) : mga::attn_fwd_ws_floats(a, head_dim, dtype));
+}
+
 int mga_attn_fwd(const void *q, int64_t q_sh, int64_t q_ss, const void *k, int64_t k_sh,
                  int64_t k_ss, const void *v, int64_t v_sh, int64_t v_ss, void *o, int64_t o_sh,
                  int64_t o_ss, float *lse, const int32_t *code, const int32_t *kv_num,
                  const int32_t *kv_idx, const int32_t *full_kv_num, const int32_t *full_kv_idx,
                  int32_t S, int32_t L, int32_t P, int32_t Hq, int32_t Hkv, int32_t head_dim,
                  int32_t dtype, float scale, void *stream) {
+  return mga_attn_fwd_ws(q, q_sh, q_ss, k, k_sh, k_ss, v, v_sh, v_ss, o, o_sh, o_ss, lse, code, kv_num, kv_idx,
+                         full_kv_num, full_kv_idx, S, L, P, Hq, Hkv, head_dim, dtype, scale, nullptr, 0, stream);
+}
+
+int mga_attn_fwd_ws(const void *q, int64_t q_sh, int64_t q_ss, const void *k, int64_t k_sh,
+                    int64_t k_ss, const void *v, int64_t v_sh, int64_t v_ss, void *o, int64_t o_sh,
+                    int64_t o_ss, float *lse, const int32_t *code, const int32_t *kv_num,
+                    const int32_t *kv_idx, const int32_t *full_kv_num, const int32_t *full_kv_idx,
+                    int32_t S, int32_t L, int32_t P, int32_t Hq, int32_t Hkv, int32_t head_dim,
+                    int32_t dtype, float scale, void *workspace, int64_t workspace_bytes, void *stream) {
   int rc;
   if ((rc = check_attn_common(S, L, P, Hq, Hkv, head_dim, dtype, scale))) return rc;
   const int eb = elem_bytes(dtype);
@@ -208,6 +239,9 @@ int mga_attn_fwd(const void *q, int64_t q_sh, int64_t q_ss, const void *k, int64
   a.nKV = (L + MGA_BLOCK - 1) / MGA_BLOCK;
   a.scale = scale;
   a.scale_log2 = scale * mga::kLog2e;
+  if ((rc = check_attn_ws("mga_attn_fwd_ws", workspace, workspace_bytes,
+                          4 * mga::attn_fwd_ws_floats(a, head_dim, dtype), &a.ws)))
+    return rc;
   mga::launch_attn_fwd(a, head_dim, dtype, (hipStream_t)stream);
   return check_launch("mga_attn_fwd");
 }
@@ -223,6 +257,23 @@ int mga_attn_bwd(const void *q, int64_t q_sh, int64_t q_ss, const void *k, int64
                  const int32_t *full_q_idx, int32_t S, int32_t L, int32_t P, int32_t Hq,
                  int32_t Hkv, int32_t head_dim, int32_t dtype, float scale, int32_t passes,
                  void *stream) {
+  return mga_attn_bwd_ws(q, q_sh, q_ss, k, k_sh, k_ss, v, v_sh, v_ss, o, o_sh, o_ss, dout, do_sh, do_ss, lse, delta,
+                         dq, dq_sh, dq_ss, dk, dk_sh, dk_ss, dv, dv_sh, dv_ss, grad_start, code, kv_num, kv_idx,
+                         full_kv_num, full_kv_idx, q_num, q_idx, full_q_num, full_q_idx, S, L, P, Hq, Hkv, head_dim,
+                         dtype, scale, passes, nullptr, 0, stream);
+}
+
+int mga_attn_bwd_ws(const void *q, int64_t q_sh, int64_t q_ss, const void *k, int64_t k_sh,
+                    int64_t k_ss, const void *v, int64_t v_sh, int64_t v_ss, const void *o,
+                    int64_t o_sh, int64_t o_ss, const void *dout, int64_t do_sh, int64_t do_ss,
+                    const float *lse, float *delta, void *dq, int64_t dq_sh, int64_t dq_ss, void *dk,
+                    int64_t dk_sh, int64_t dk_ss, void *dv, int64_t dv_sh, int64_t dv_ss,
+                    int32_t grad_start, const int32_t *code, const int32_t *kv_num,
+                    const int32_t *kv_idx, const int32_t *full_kv_num, const int32_t *full_kv_idx,
+                    const int32_t *q_num, const int32_t *q_idx, const int32_t *full_q_num,
+                    const int32_t *full_q_idx, int32_t S, int32_t L, int32_t P, int32_t Hq,
+                    int32_t Hkv, int32_t head_dim, int32_t dtype, float scale, int32_t passes,
+                    void *workspace, int64_t workspace_bytes, void *stream) {
   int rc;
   if ((rc = check_attn_common(S, L, P, Hq, Hkv, head_dim, dtype, scale))) return rc;
   if (passes <= 0 || (passes & ~(MGA_BWD_DQ | MGA_BWD_DKDV)))
@@ -266,6 +317,9 @@ int mga_attn_bwd(const void *q, int64_t q_sh, int64_t q_ss, const void *k, int64
   a.nKV = (L + MGA_BLOCK - 1) / MGA_BLOCK;
   a.scale = scale;
   a.scale_log2 = scale * mga::kLog2e;
+  if ((rc = check_attn_ws("mga_attn_bwd_ws", workspace, workspace_bytes,
+                          4 * mga::attn_bwd_ws_floats(a, head_dim, dtype), &a.ws)))
+    return rc;
   mga::launch_attn_bwd(a, head_dim, dtype, passes, (hipStream_t)stream);
   return check_launch("mga_attn_bwd");
 }

@@ -20,9 +20,15 @@
 //   scores of step j + 1 are computed while the softmax of step j runs, in
 //   one scheduling region whose MFMAs and VALU instructions are interleaved,
 //   then O^T takes step j's probabilities (one barrier per step).
-// * split: a last round of items that would leave half of an XCD's workgroup
-//   slots empty runs each row block as an 8-wave workgroup whose two 4-wave
-//   groups split the tile list (as in the 4-wave form) and merge through LDS.
+// With a workspace (mga_attn_fwd_ws) the items of a last round that would
+// leave slots idle run as parts of their tile lists in the same launch
+// (KeySplit), whose fp32 (O, offset, row sum) attn_fwd_merge_kernel combines:
+// [508 rows x 32 heads] against 20 491 prefix keys 412 -> 213 + 9 us, 2 529 rows
+// against 4 093 (fp16) 345 -> 265 + 9 us.
+// * split (calls without a workspace): a last round of items that would leave
+//   half of an XCD's workgroup slots empty runs each row block as an 8-wave
+//   workgroup whose two 4-wave groups split the tile list (as in the 4-wave
+//   form) and merge through LDS.
 // K runs one step ahead of V: while the K tile of step j + 1 and the V tile of
 // step j are read, the K tile of step j + 2 and the V tile of step j + 1 load
 // straight into the two other named buffers.
@@ -45,6 +51,7 @@
 
 #include "mga_common.hpp"
 #include "mga_internal.hpp"
+#include "mga_key_split.hpp"
 
 namespace mga {
 
@@ -74,6 +81,11 @@ __host__ __device__ __forceinline__ int units_per_item(int HPW) { return HPW >= 
 
 enum { kFwd4 = 0, kFwdPair = 1, kFwdSplit = 2 };
 
+// A part's fixed cost (Q and first tiles' latency, the partial results' write:
+// about 6 us against 3.8 us a tile) and the merge launch's (9 us), in key tiles
+// (for key_split_plan).
+constexpr float kFwdPartTiles = 1.5f, kFwdMergeTiles = 2.5f;
+
 }  // namespace
 
 // An item is (kv head, slice of HPW query heads, U consecutive blocks of
@@ -95,7 +107,8 @@ enum { kFwd4 = 0, kFwdPair = 1, kFwdSplit = 2 };
 //   the GPU idle).
 // The launch runs items [k1, k1 + kn) of each XCD's share.
 template <int HD, typename T, int MODE>
-__global__ __launch_bounds__(MODE == kFwd4 ? 256 : 512, 2) void attn_fwd_kernel(AttnArgs a, int k1, int kn) {
+__global__ __launch_bounds__(MODE == kFwd4 ? 256 : 512, 2) void attn_fwd_kernel(AttnArgs a, int k1, int kn,
+                                                                                  KeySplit sp) {
   constexpr int NG = MODE == kFwdSplit ? 2 : 1;    // groups splitting the tile list
   constexpr int NWD = 4;                           // waves loading each staged tile
   typedef typename MfmaElem<T>::type E;
@@ -129,7 +142,12 @@ __global__ __launch_bounds__(MODE == kFwd4 ? 256 : 512, 2) void attn_fwd_kernel(
   const int n_items = a.Hkv * nslice * nqb;
   const int xcd = blockIdx.x & 7;
   const int t = (int)(blockIdx.x >> 3);
-  const int o = k1 + (MODE == kFwdSplit ? t / U : t);
+  int o, part = -1;   // part: the share of the tile list, -1 = all of it
+  if constexpr (MODE == kFwdSplit) {
+    o = k1 + t / U;
+  } else {
+    sp.locate(t, o, part);
+  }
   const int n_x = n_items / 8 + (xcd < n_items % 8 ? 1 : 0);
   if (o >= n_x || o >= k1 + kn) return;
   const int li = xcd * (n_items / 8) + min(xcd, n_items % 8) + o;
@@ -161,9 +179,16 @@ __global__ __launch_bounds__(MODE == kFwd4 ? 256 : 512, 2) void attn_fwd_kernel(
 
   TileList tiles = tile_list(a.kv_num, a.kv_idx, a.fkv_num, a.fkv_idx, qt, a.nKV);
   const int npart = tiles.npart;
-  const int nstep = kStepsPerTile * ((tiles.ntot - grp + NG - 1) / NG);   // this group's steps
-  const int nloop = kStepsPerTile * ((tiles.ntot + NG - 1) / NG);        // group 0's (>= group 1's)
-  auto tile_of = [&](int j) { return NG * (j / kStepsPerTile) + grp; };
+  // the workgroup's share of the list (all of it unless the item is split),
+  // entries t0 .. t0 + nt - 1
+  int t0 = 0, nt = tiles.ntot;
+  if (MODE != kFwdSplit && part >= 0) {
+    t0 = sp.begin(part, tiles.ntot);
+    nt = sp.begin(part + 1, tiles.ntot) - t0;
+  }
+  const int nstep = kStepsPerTile * ((nt - grp + NG - 1) / NG);   // this group's steps
+  const int nloop = kStepsPerTile * ((nt + NG - 1) / NG);        // group 0's (>= group 1's)
+  auto tile_of = [&](int j) { return t0 + NG * (j / kStepsPerTile) + grp; };
   auto step_base = [&](int j) { return tiles.at(tile_of(j)) * kBlock + (j % kStepsPerTile) * kStepKeys; };
 
   // per-lane LDS offsets: K rows (A operand of QK^T) and the V^T transpose reads
@@ -526,6 +551,22 @@ __global__ __launch_bounds__(MODE == kFwd4 ? 256 : 512, 2) void attn_fwd_kernel(
     m_run = mm;
   }
 
+  if constexpr (MODE != kFwdSplit) {
+    if (part >= 0) {   // a part's raw (O^T, offset, row sum): attn_fwd_merge_kernel combines them
+      float *po = sp.ws + (sp.slot(o, part, xcd) * (blockDim.x / 64) + wave) * kPartFloats<HD>;
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const f32x4 v = {oacc[db][4 * q], oacc[db][4 * q + 1], oacc[db][4 * q + 2], oacc[db][4 * q + 3]};
+          *reinterpret_cast<f32x4 *>(po + ((db * 4 + q) * 64 + lane) * 4) = v;
+        }
+      po[HD * 32 + lane] = m_run;
+      po[HD * 32 + 64 + lane] = l_run;
+      return;
+    }
+  }
+
   // ---- epilogue: normalise, write O [S, Hq, D] and the natural-log LSE -------
   const float lt = l_run + xor32(l_run);
   if (row < a.S) {
@@ -544,12 +585,67 @@ __global__ __launch_bounds__(MODE == kFwd4 ? 256 : 512, 2) void attn_fwd_kernel(
   }
 }
 
+// Combines the parts of the split items: O = sum of the parts' O scaled to the
+// largest offset, over the sum of their row sums scaled alike, in the order of
+// the parts (bit-for-bit repeatable). Workgroup (item u of the XCD's split
+// items, 32-dim block db); the threads hold the elements that the item's
+// workgroups held. Bound by the reads of the parts (L2 or the memory-side
+// cache, which they were just written to).
+template <int HD, typename T, int NW>
+__global__ __launch_bounds__(64 * NW) void attn_fwd_merge_kernel(AttnArgs a, KeySplit sp) {
+  constexpr int DB = HD / 32;
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int l32 = lane & 31, hi = lane >> 5;
+  const int G = a.Hq / a.Hkv;
+  const int HPW = heads_per_wg(G);
+  const int QU = units_per_item(HPW) * 32 * (4 / HPW);
+  const int nslice = G / HPW;
+  const int nqb = (a.S + QU - 1) / QU;
+  const int n_items = a.Hkv * nslice * nqb;
+  const int xcd = blockIdx.x & 7, u = (int)(blockIdx.x >> 3) / DB, db = (int)(blockIdx.x >> 3) % DB;
+  const int o = sp.k + u;
+  if (o >= n_items / 8 + (xcd < n_items % 8 ? 1 : 0)) return;
+  const int li = xcd * (n_items / 8) + min(xcd, n_items % 8) + o;
+  const int g = li / (nslice * nqb), rem = li % (nslice * nqb);
+  const int h = g * G + (rem % nslice) * HPW + wave % HPW;
+  const int row = (nqb - 1 - rem / nslice) * QU + (wave / HPW) * 32 + l32;
+  const float *p0 = sp.ws + (sp.slot(o, 0, xcd) * NW + wave) * kPartFloats<HD>;
+  const int64_t step = (int64_t)8 * kPartFloats<HD> * NW;   // to the next part
+  float mm = kNegInfF;
+  for (int p = 0; p < sp.ns; ++p) mm = fmaxf(mm, p0[p * step + HD * 32 + lane]);
+  const float mu = mm == kNegInfF ? 0.f : mm;   // no part saw an unmasked key: every weight is 0
+  float l = 0.f;
+  f32x16 acc = zero16();
+  for (int p = 0; p < sp.ns; ++p) {
+    const float *pp = p0 + p * step;
+    const float w = exp2f_(pp[HD * 32 + lane] - mu);
+    l += pp[HD * 32 + 64 + lane] * w;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const f32x4 v = *reinterpret_cast<const f32x4 *>(pp + ((db * 4 + q) * 64 + lane) * 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[4 * q + e] += v[e] * w;
+    }
+  }
+  const float lt = l + xor32(l);
+  if (row >= a.S) return;
+  const float inv = lt > 0.f ? 1.f / lt : 0.f;
+  if (hi == 0 && db == 0) a.lse[(int64_t)h * a.S + row] = lt > 0.f ? (mm + __log2f(lt)) * kLn2 : kNegInfF;
+  T *orow = reinterpret_cast<T *>(const_cast<void *>(a.o)) + h * a.o_sh + (int64_t)row * a.o_ss;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    store4(orow + db * 32 + 8 * i + 4 * hi, acc[4 * i] * inv, acc[4 * i + 1] * inv, acc[4 * i + 2] * inv,
+           acc[4 * i + 3] * inv);
+}
+
 // explicit instantiations: clang otherwise drops some host launch stubs of
 // this template (the bf16 ones), leaving undefined symbols
-#define MGA_FWD_INST(HD, T)                                                     \
-  template __global__ void attn_fwd_kernel<HD, T, kFwd4>(AttnArgs, int, int);    \
-  template __global__ void attn_fwd_kernel<HD, T, kFwdPair>(AttnArgs, int, int); \
-  template __global__ void attn_fwd_kernel<HD, T, kFwdSplit>(AttnArgs, int, int);
+#define MGA_FWD_INST(HD, T)                                                               \
+  template __global__ void attn_fwd_kernel<HD, T, kFwd4>(AttnArgs, int, int, KeySplit);    \
+  template __global__ void attn_fwd_kernel<HD, T, kFwdPair>(AttnArgs, int, int, KeySplit); \
+  template __global__ void attn_fwd_kernel<HD, T, kFwdSplit>(AttnArgs, int, int, KeySplit); \
+  template __global__ void attn_fwd_merge_kernel<HD, T, 4>(AttnArgs, KeySplit);            \
+  template __global__ void attn_fwd_merge_kernel<HD, T, 8>(AttnArgs, KeySplit);
 MGA_FWD_INST(128, bf16_t)
 MGA_FWD_INST(64, bf16_t)
 MGA_FWD_INST(128, f16_t)
@@ -572,24 +668,68 @@ int fwd_split_point(int items, int L, int m) {
   return (nmax > m && r > 0 && r <= m / 2) ? nmax - r : nmax;
 }
 
-template <int HD, typename T>
-static void fwd_launch(const AttnArgs &a, hipStream_t st) {
+namespace {
+
+// waves of a workgroup, rows of an item, head slices of a kv head, items,
+// items per XCD at most, workgroup slots per XCD
+struct FwdGrid {
+  int U, nw, rows, nslice, items, nmax, slots;
+};
+
+FwdGrid fwd_grid(const AttnArgs &a) {
   const int G = a.Hq / a.Hkv;
   const int HPW = heads_per_wg(G);
-  const int U = units_per_item(HPW);
-  const int QU = U * 32 * (4 / HPW);
-  const int nqb = (a.S + QU - 1) / QU;
-  const int items = a.Hkv * (G / HPW) * nqb;
-  const int nmax = (items + 7) / 8;
-  const int cx = device_cu_count() / 8;   // CUs per XCD
-  const int k1 = fwd_split_point(items, a.L, U == 2 ? cx : 2 * cx);
-  if (k1 > 0) {
-    if (U == 2) hipLaunchKernelGGL((attn_fwd_kernel<HD, T, kFwdPair>), dim3(8 * k1), dim3(512), 0, st, a, 0, k1);
-    else hipLaunchKernelGGL((attn_fwd_kernel<HD, T, kFwd4>), dim3(8 * k1), dim3(256), 0, st, a, 0, k1);
+  FwdGrid f;
+  f.U = units_per_item(HPW);
+  f.rows = f.U * 32 * (4 / HPW);
+  f.nslice = G / HPW;
+  f.items = a.Hkv * f.nslice * ((a.S + f.rows - 1) / f.rows);
+  f.nmax = (f.items + 7) / 8;
+  f.nw = 4 * f.U;
+  f.slots = std::max(1, (f.U == 2 ? 1 : 2) * (device_cu_count() / 8));
+  return f;
+}
+
+}  // namespace
+
+// The split of the last items over their keys, ns = 1 for none.
+static KeySplit fwd_split(const AttnArgs &a) {
+  const FwdGrid f = fwd_grid(a);
+  return key_split_plan(f.nmax, f.slots, last_round_tiles(a.S, a.P, a.Hkv, f.nslice, f.rows, f.nmax % f.slots),
+                        kFwdPartTiles, kFwdMergeTiles);
+}
+
+int64_t attn_fwd_ws_floats(const AttnArgs &a, int head_dim, int dtype) {
+  if (dtype == kDtF32) return 0;   // the fp32 kernels do not split
+  const KeySplit sp = fwd_split(a);
+  const FwdGrid f = fwd_grid(a);
+  return sp.ns > 1 ? (int64_t)8 * sp.r * sp.ns * f.nw * part_floats(head_dim) : 0;
+}
+
+template <int HD, typename T>
+static void fwd_launch(const AttnArgs &a, hipStream_t st) {
+  const FwdGrid f = fwd_grid(a);
+  KeySplit sp = a.ws ? fwd_split(a) : no_split(f.nmax);
+  int k1 = f.nmax, grid = 8 * f.nmax;
+  if (sp.ns > 1) {
+    sp.ws = a.ws;
+    grid = 8 * sp.groups();
+  } else {
+    k1 = fwd_split_point(f.items, a.L, f.slots);
+    grid = 8 * k1;
   }
-  if (k1 < nmax)
-    hipLaunchKernelGGL((attn_fwd_kernel<HD, T, kFwdSplit>), dim3(8 * U * (nmax - k1)), dim3(512), 0, st, a, k1,
-                       nmax - k1);
+  if (grid > 0) {
+    if (f.U == 2) hipLaunchKernelGGL((attn_fwd_kernel<HD, T, kFwdPair>), dim3(grid), dim3(512), 0, st, a, 0, k1, sp);
+    else hipLaunchKernelGGL((attn_fwd_kernel<HD, T, kFwd4>), dim3(grid), dim3(256), 0, st, a, 0, k1, sp);
+  }
+  if (sp.ns > 1) {
+    const dim3 mg(8 * sp.r * (HD / 32));
+    if (f.U == 2) hipLaunchKernelGGL((attn_fwd_merge_kernel<HD, T, 8>), mg, dim3(512), 0, st, a, sp);
+    else hipLaunchKernelGGL((attn_fwd_merge_kernel<HD, T, 4>), mg, dim3(256), 0, st, a, sp);
+  } else if (k1 < f.nmax) {
+    hipLaunchKernelGGL((attn_fwd_kernel<HD, T, kFwdSplit>), dim3(8 * f.U * (f.nmax - k1)), dim3(512), 0, st, a, k1,
+                       f.nmax - k1, sp);
+  }
 }
 
 template <int HD>

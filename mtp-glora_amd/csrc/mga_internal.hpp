@@ -23,6 +23,7 @@ struct AttnArgs {
   const int32_t *q_num, *q_idx, *fq_num, *fq_idx;
   int32_t S, L, P, Hq, Hkv, nQ, nKV;
   float scale, scale_log2;
+  float *ws;                                // partial results of key-split items, or null (no key split)
 };
 
 void launch_kv_copy_rows(const void *src_k, const void *src_v, int64_t src_sh_b, int64_t src_ss_b,
@@ -46,6 +47,10 @@ constexpr int kDtF16 = 2;
 
 // head_dim in {64, 128}; dtype one of kDt*.
 void launch_attn_fwd(const AttnArgs &a, int head_dim, int dtype, hipStream_t stream);
+// fp32 words of AttnArgs::ws that the forward / the dQ pass of this shape use
+// (S, L, nKV, Hq and Hkv set), 0 where they do not split their items.
+int64_t attn_fwd_ws_floats(const AttnArgs &a, int head_dim, int dtype);
+int64_t attn_bwd_ws_floats(const AttnArgs &a, int head_dim, int dtype);
 // passes: kBwdDq (delta + dQ) and/or kBwdDkDv (dK/dV; reads the delta the dQ pass wrote).
 constexpr int kBwdDq = 1;
 constexpr int kBwdDkDv = 2;

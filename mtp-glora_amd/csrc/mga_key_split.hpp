@@ -1,0 +1,115 @@
+// Splitting the last work items of an attention launch over their keys.
+//
+// The forward and dQ launches hand each XCD a contiguous share of the items,
+// one workgroup per slot (a CU, or half of one); an item walks its whole tile
+// list. When the items of a share are not a multiple of the slots, the last
+// round leaves slots idle for as long as a full walk: 8 items on 32 slots (a
+// 512-row chunk) use a quarter of the GPU. The r items of that round are
+// therefore split into parts of their tile lists; a part is a workgroup of its
+// own and writes fp32 partial results, which a small kernel combines in the
+// order of the parts.
+#pragma once
+
+#include <algorithm>
+#include <cmath>
+
+#include "mga_common.hpp"
+
+namespace mga {
+
+// Items 0 .. k - 1 of each XCD's share run whole, the other r in ns parts:
+// part 0 takes first / 1024 of an item's tile list, the later ones equal
+// shares of the rest. Workgroup t of an XCD: the whole items, then every
+// item's part 0, then the other parts.
+struct KeySplit {
+  int k;
+  int r;
+  int ns;
+  int first;
+  float *ws;   // parts, [item * ns + part][XCD][wave][part_floats]
+
+  // number of workgroups per XCD
+  __host__ __device__ int groups() const { return k + r * ns; }
+  // workgroup t: its item (within the share) and part, -1 = the whole list
+  __device__ __forceinline__ void locate(int t, int &item, int &part) const {
+    item = t;
+    part = -1;
+    if (t < k) return;
+    const int u = t - k;
+    if (u < r) {
+      part = 0;
+    } else {
+      const int v = u - r;
+      item = k + v / (ns - 1);
+      part = 1 + v % (ns - 1);
+    }
+  }
+  // first entry of a part's share of n tile-list entries (part ns: n)
+  __device__ __forceinline__ int begin(int part, int n) const {
+    if (part == 0) return 0;
+    const int f = (n * first + 512) >> 10;
+    return f + (n - f) * (part - 1) / (ns - 1);
+  }
+  // a part's index among the parts in ws
+  __device__ __forceinline__ int64_t slot(int item, int part, int xcd) const {
+    return ((int64_t)(item - k) * ns + part) * 8 + xcd;
+  }
+};
+
+// fp32 words of one wave's part of the forward: O^T, offset and row sum per lane.
+template <int HD>
+constexpr int kPartFloats = HD * 32 + 128;
+inline int part_floats(int head_dim) { return head_dim * 32 + 128; }
+
+inline KeySplit no_split(int nmax) { return KeySplit{nmax, 0, 1, 1024, nullptr}; }
+
+// Key tiles of the longest item of the last round: an XCD whose share lies in
+// whole kv heads (longest items first) ends with the items of a head's first
+// rows.
+inline int last_round_tiles(int S, int P, int Hkv, int nslice, int rows, int r) {
+  const int last = Hkv % 8 == 0 ? rows * ((r + nslice - 1) / nslice) : S;
+  return (P + std::min(S, last) + kBlock - 1) / kBlock;
+}
+
+// nmax: items of the largest share; slots: workgroups an XCD runs at once;
+// ntile: key tiles of the longest item of the last round; part_cost, merge_cost: what a part
+// costs beyond its tiles and what the combining launch costs, in tiles. Of
+// two shapes per ns the plan takes the one with the least time to the end:
+// * equal parts, run in rounds of the slots;
+// * r < slots: a long first part for r of the slots, short ones in rounds on
+//   the other slots - r, so long that both end together (24 items on 32
+//   slots: 3/4 of each item in one piece, the rest three to a free slot).
+// A part keeps at least kMinPartTiles tiles; kMaxPartRounds bounds the
+// workspace (133 KB a part at head_dim 128).
+constexpr int kMinPartTiles = 4, kMaxParts = 16, kMaxPartRounds = 4;
+inline KeySplit key_split_plan(int nmax, int slots, int ntile, float part_cost, float merge_cost) {
+  KeySplit best = no_split(nmax);
+  slots = std::max(slots, 1);
+  const int r = nmax % slots;
+  if (r == 0) return best;
+  const float T = (float)ntile;
+  float best_cost = T;   // the last round unsplit
+  for (int ns = 2; ns <= kMaxParts && r * ns <= kMaxPartRounds * slots; ++ns) {
+    if (ntile >= kMinPartTiles * ns) {
+      const int rounds = (r * ns + slots - 1) / slots;
+      const float cost = rounds * ((float)((ntile + ns - 1) / ns) + part_cost) + merge_cost;
+      if (cost < best_cost) {
+        best_cost = cost;
+        best = KeySplit{nmax - r, r, ns, 1024 / ns, nullptr};
+      }
+    }
+    const int rounds = (r * (ns - 1) + slots - r - 1) / (slots - r);   // of the short parts
+    const float per = (float)rounds / (ns - 1);
+    const float big = (per * T + (rounds - 1) * part_cost) / (1.f + per);   // big + part_cost = short parts' end
+    if (big < T && (T - big) / (ns - 1) >= kMinPartTiles) {
+      const float cost = std::ceil(big) + part_cost + merge_cost;
+      if (cost < best_cost) {
+        best_cost = cost;
+        best = KeySplit{nmax - r, r, ns, (int)(1024.f * big / T), nullptr};
+      }
+    }
+  }
+  return best;
+}
+
+}  // namespace mga

@@ -6,6 +6,7 @@ error, never a reason to compute elsewhere.
 """
 from __future__ import annotations
 
+import functools
 import math
 
 import torch
@@ -155,6 +156,23 @@ def mtp_block_mask_tensors(gate: torch.Tensor, P: int) -> dict:
 # Attention
 # ----------------------------------------------------------------------------
 
+@functools.lru_cache(maxsize=1024)
+def _attn_ws_bytes(S: int, L: int, Hq: int, Hkv: int, D: int, dtype: int, backward: int, device: int) -> int:
+    with torch.cuda.device(device):
+        return int(_lib.load().mga_attn_workspace_bytes(S, L, Hq, Hkv, D, dtype, backward))
+
+
+def _attn_workspace(S, L, Hq, Hkv, D, dtype: int, backward: int, dev):
+    """(pointer, bytes, tensor) of the workspace in which a pass that would
+    leave part of the GPU idle keeps its parts' results; (None, 0, None) where
+    the shape needs none."""
+    n = _attn_ws_bytes(S, L, Hq, Hkv, D, dtype, backward, dev.index)
+    if n == 0:
+        return None, 0, None
+    ws = torch.empty(n, dtype=torch.uint8, device=dev)
+    return ws.data_ptr(), n, ws
+
+
 def attn_fwd(q, k, v, code, bm: dict, P: int, scale: float):
     """q [1, Hq, S, D]; k/v [1, Hkv, L, D] with L = P + S.
     Returns o [1, S, Hq, D] (contiguous) and lse [1, Hq, S] fp32 (natural log)."""
@@ -171,11 +189,13 @@ def attn_fwd(q, k, v, code, bm: dict, P: int, scale: float):
         raise TypeError("query, key and value must share one dtype")
     o = torch.empty(1, S, Hq, D, dtype=qq.dtype, device=qq.device)
     lse = torch.empty(1, Hq, S, dtype=torch.float32, device=qq.device)
-    _lib.call("mga_attn_fwd", qq.data_ptr(), q_sh, q_ss, kk.data_ptr(), k_sh, k_ss,
+    dt = dtype_code(qq.dtype)
+    wp, wn, ws = _attn_workspace(S, L, Hq, Hkv, D, dt, 0, qq.device)
+    _lib.call("mga_attn_fwd_ws", qq.data_ptr(), q_sh, q_ss, kk.data_ptr(), k_sh, k_ss,
               vv.data_ptr(), v_sh, v_ss, o.data_ptr(), D, Hq * D, lse.data_ptr(), code.data_ptr(),
               bm["kv_num_blocks"].data_ptr(), bm["kv_indices"].data_ptr(),
               bm["full_kv_num_blocks"].data_ptr(), bm["full_kv_indices"].data_ptr(),
-              S, L, P, Hq, Hkv, D, dtype_code(qq.dtype), float(scale), _stream(qq))
+              S, L, P, Hq, Hkv, D, dt, float(scale), wp, wn, _stream(qq))
     return o, lse
 
 
@@ -196,7 +216,7 @@ def bwd_buffers(q, k, grad_start: int) -> dict:
 
 def attn_bwd(q, k, v, o, lse, dout, code, bm: dict, P: int, scale: float, grad_start: int,
              passes: int = _lib.BWD_DQ | _lib.BWD_DKDV, buffers: dict | None = None,
-             no_alloc: bool = False):
+             no_alloc: bool = False, key_split: bool = False):
     """Gradients of ``attn_fwd``. Returns dq [1, Hq, S, D] (a transposed view of
     an [1, S, Hq, D] buffer), and dk, dv [1, Hkv, L - grad_start, D] (views of
     [1, L - grad_start, Hkv, D] buffers) or None when grad_start == L.
@@ -206,7 +226,13 @@ def attn_bwd(q, k, v, o, lse, dout, code, bm: dict, P: int, scale: float, grad_s
     same ``buffers`` (from ``bwd_buffers``) to both, the dQ pass first.
 
     ``no_alloc`` calls ``mga_attn_bwd_noalloc``: delta lives in the library's
-    fixed per-GPU workspace instead of ``buffers["delta"]``."""
+    fixed per-GPU workspace instead of ``buffers["delta"]``.
+
+    ``key_split`` gives the dQ pass a workspace (``mga_attn_bwd_ws``), so that
+    it may split its last work items over their keys; dQ then differs from the
+    unsplit call's in the order of its fp32 sums."""
+    if key_split and no_alloc:
+        raise ValueError("key_split needs a workspace, which no_alloc forbids")
     qq, q_sh, q_ss = _rows("query", q)
     kk, k_sh, k_ss = _rows("key", k)
     vv, v_sh, v_ss = _rows("value", v)
@@ -229,20 +255,21 @@ def attn_bwd(q, k, v, o, lse, dout, code, bm: dict, P: int, scale: float, grad_s
     dk_ptr = dk.data_ptr() if dk is not None else None
     dv_ptr = dv.data_ptr() if dv is not None else None
     # o3 is [S, Hq, D]: element (h, s, d) at h * D + s * Hq * D + d
-    head = (["mga_attn_bwd_noalloc", qq.data_ptr(), q_sh, q_ss, kk.data_ptr(), k_sh, k_ss,
-             vv.data_ptr(), v_sh, v_ss, o3.data_ptr(), o3.stride(1), o3.stride(0),
-             d3.data_ptr(), d3.stride(1), d3.stride(0), lse.data_ptr()] if no_alloc else
-            ["mga_attn_bwd", qq.data_ptr(), q_sh, q_ss, kk.data_ptr(), k_sh, k_ss,
-             vv.data_ptr(), v_sh, v_ss, o3.data_ptr(), o3.stride(1), o3.stride(0),
-             d3.data_ptr(), d3.stride(1), d3.stride(0), lse.data_ptr(), delta.data_ptr()])
-    _lib.call(*head,
-              dq.data_ptr(), D, Hq * D, dk_ptr, D, Hkv * D, dv_ptr, D, Hkv * D,
-              int(grad_start), code.data_ptr(),
-              bm["kv_num_blocks"].data_ptr(), bm["kv_indices"].data_ptr(),
-              bm["full_kv_num_blocks"].data_ptr(), bm["full_kv_indices"].data_ptr(),
-              bm["q_num_blocks"].data_ptr(), bm["q_indices"].data_ptr(),
-              bm["full_q_num_blocks"].data_ptr(), bm["full_q_indices"].data_ptr(),
-              S, L, P, Hq, Hkv, D, dtype_code(qq.dtype), float(scale), int(passes), _stream(qq))
+    dt = dtype_code(qq.dtype)
+    operands = [qq.data_ptr(), q_sh, q_ss, kk.data_ptr(), k_sh, k_ss, vv.data_ptr(), v_sh, v_ss,
+                o3.data_ptr(), o3.stride(1), o3.stride(0), d3.data_ptr(), d3.stride(1), d3.stride(0),
+                lse.data_ptr()]
+    rest = [dq.data_ptr(), D, Hq * D, dk_ptr, D, Hkv * D, dv_ptr, D, Hkv * D, int(grad_start), code.data_ptr(),
+            bm["kv_num_blocks"].data_ptr(), bm["kv_indices"].data_ptr(),
+            bm["full_kv_num_blocks"].data_ptr(), bm["full_kv_indices"].data_ptr(),
+            bm["q_num_blocks"].data_ptr(), bm["q_indices"].data_ptr(),
+            bm["full_q_num_blocks"].data_ptr(), bm["full_q_indices"].data_ptr(),
+            S, L, P, Hq, Hkv, D, dt, float(scale), int(passes)]
+    if no_alloc:
+        _lib.call("mga_attn_bwd_noalloc", *operands, *rest, _stream(qq))
+    else:
+        wp, wn, ws = (_attn_workspace(S, L, Hq, Hkv, D, dt, 1, qq.device) if key_split else (None, 0, None))
+        _lib.call("mga_attn_bwd_ws", *operands, delta.data_ptr(), *rest, wp, wn, _stream(qq))
     dq_t = dq.transpose(1, 2)
     if dk is None:
         return dq_t, None, None

@@ -1,0 +1,92 @@
+"""Attention launches whose last work items are split over their keys
+(mga_attn_fwd_ws / mga_attn_bwd_ws with a workspace) against the same calls
+without one, at chunk sizes around the plan's edges: fewer items than slots,
+one item past a round, rows and keys past the last tile, an item whose tile
+list is shorter than its parts.
+
+Bounds, u the operand type's unit roundoff (2^-8 bf16, 2^-11 fp16: half a
+unit in the last place of a value at the bottom of its binade, so two
+roundings of nearly the same value lie up to 2 u apart):
+* o: the parts round their probabilities at another running offset, so each
+  of the two outputs is off by at most u sum p |v| <= u max|v| before its own
+  rounding: |o - o'| <= 2 u (max|v| + |o|);
+* lse: fp32 sums in another order, |lse - lse'| <= 1e-5;
+* dQ: dS is formed from the same lse, so only the fp32 sum's order (bounded by
+  1e-5 max|dq|) and the output's rounding differ:
+  |dq - dq'| <= 2 u |dq| + 1e-5 max|dq|.
+Repeated calls are equal bit for bit."""
+import pytest
+import torch
+
+from gpu_helpers import chunk_layout, qkv
+
+UNIT = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
+
+CASES = [
+    dict(n_reg=371, n_anchor=33, P=4491, Hq=32, Hkv=8, D=128, pad=5),     # 8 items an XCD
+    dict(n_reg=2049, n_anchor=8, P=1500, Hq=32, Hkv=8, D=128, pad=0),     # one 64-row item past a round
+    dict(n_reg=1201, n_anchor=75, P=4099, Hq=32, Hkv=8, D=128, pad=35),   # 24 items: a long and a short part each
+    dict(n_reg=129, n_anchor=3, P=8197, Hq=28, Hkv=4, D=128, pad=1),      # G = 7: 4-wave workgroups
+    dict(n_reg=65, n_anchor=5, P=2500, Hq=8, Hkv=8, D=64, pad=0),         # G = 1
+    dict(n_reg=500, n_anchor=40, P=1500, Hq=12, Hkv=2, D=64, pad=70),     # G = 6, 16 items on 8 XCDs, pad tiles
+    dict(n_reg=1500, n_anchor=75, P=0, Hq=16, Hkv=8, D=128, pad=0),      # no prefix: lists shorter than the longest
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("c", CASES)
+def test_split_equals_unsplit(mga, dev, c, dtype):
+    print(f"case {c} {dtype}", flush=True)
+    ops, lib = mga.ops, mga._lib
+    P, D, scale, u = c["P"], c["D"], c["D"] ** -0.5, UNIT[dtype]
+    seq = chunk_layout(c["n_reg"], c["n_anchor"], 4, P, seed=5, pad=c["pad"])
+    S = len(seq.gate)
+    q, k, v, kp, vp, do = qkv(S, P, c["Hq"], c["Hkv"], D, dtype, dev, seed=5, std=1.0)
+    kf, vf = torch.cat([kp, k], 2), torch.cat([vp, v], 2)
+    mask = mga.build_mtp_block_mask(torch.tensor(seq.gate, device=dev)[None], P)
+    bm, code = mask.kernel_tensors(), mask.mtp_code
+    size = (S, P + S, c["Hq"], c["Hkv"], D, ops.dtype_code(dtype))
+    assert lib.load().mga_attn_workspace_bytes(*size, 0) > 0 and lib.load().mga_attn_workspace_bytes(*size, 1) > 0
+
+    o, lse = ops.attn_fwd(q, kf, vf, code, bm, P, scale)
+    o1, lse1 = torch.empty_like(o), torch.empty_like(lse)
+    lib.call("mga_attn_fwd", q.data_ptr(), q.stride(1), q.stride(2), kf.data_ptr(), kf.stride(1), kf.stride(2),
+             vf.data_ptr(), vf.stride(1), vf.stride(2), o1.data_ptr(), D, c["Hq"] * D, lse1.data_ptr(),
+             code.data_ptr(), bm["kv_num_blocks"].data_ptr(), bm["kv_indices"].data_ptr(),
+             bm["full_kv_num_blocks"].data_ptr(), bm["full_kv_indices"].data_ptr(),
+             S, P + S, P, c["Hq"], c["Hkv"], D, ops.dtype_code(dtype), scale,
+             torch.cuda.current_stream().cuda_stream)
+    assert torch.equal(torch.isneginf(lse), torch.isneginf(lse1))
+    seen = torch.isfinite(lse1)
+    assert float((lse - lse1)[seen].abs().max()) <= 1e-5
+    d = (o.float() - o1.float()).abs()
+    assert bool((d <= 2 * u * (float(vf.abs().max()) + o1.float().abs())).all())
+
+    args = (q, kf, vf, o1, lse1, do, code, bm, P, scale, P)
+    dq, dk, dv = ops.attn_bwd(*args, key_split=True)
+    dq1, dk1, dv1 = ops.attn_bwd(*args)
+    assert torch.equal(dk, dk1) and torch.equal(dv, dv1)
+    d = (dq.float() - dq1.float()).abs()
+    assert bool((d <= 2 * u * dq1.float().abs() + 1e-5 * float(dq1.float().abs().max())).all())
+
+    again, _ = ops.attn_fwd(q, kf, vf, code, bm, P, scale)
+    assert torch.equal(o, again) and torch.equal(dq, ops.attn_bwd(*args, key_split=True)[0])
+
+
+def test_workspace_plan(mga):
+    """Whole rounds and short key lists need no workspace; the split ones stay
+    below 600 MB at the largest sizes; a smaller workspace is refused before
+    any device work."""
+    lib = mga.load_library()
+    assert lib.mga_attn_workspace_bytes(2048, 30720, 32, 8, 128, 0, 0) == 0     # 32 items an XCD
+    assert lib.mga_attn_workspace_bytes(320, 320, 32, 8, 128, 0, 0) == 0        # three tiles of keys
+    assert lib.mga_attn_workspace_bytes(508, 20999, 32, 8, 96, 0, 0) == 0       # not a supported head_dim
+    for S in range(33, 6200, 97):
+        for P in (0, 1000, 30000, 131072):
+            for back in (0, 1):
+                assert 0 <= lib.mga_attn_workspace_bytes(S, P + S, 32, 8, 128, 0, back) < 600 << 20
+    p = 16
+    base = [p, 128, 4096, p, 128 * 64, 128, p, 128 * 64, 128, p, 128, 4096, p, p, p, p, p, p]
+    rc = lib.mga_attn_fwd_ws(*base, 508, 20999, 20491, 32, 8, 128, 0, 0.1, p, 64, None)
+    assert rc == mga._lib.MGA_ERR_INVALID and b"workspace" in lib.mga_last_error()
