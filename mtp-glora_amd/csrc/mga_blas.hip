@@ -106,16 +106,23 @@ int gemm(int dtype, bool ta, bool tb, int64_t M, int64_t N, int64_t K, const voi
     uint64_t max_ws = ws_bytes;
     hipblasLtMatmulPreferenceCreate(&pref);
     hipblasLtMatmulPreferenceSetAttribute(pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &max_ws, sizeof(max_ws));
-    hipblasLtMatmulHeuristicResult_t res[1];
-    int found = 0;
+    // the heuristic's first choice that fits the workspace: for some long
+    // reductions (K = 24 576) it ranks algorithms first that need more than the
+    // preference's limit
+    constexpr int kMostAlgos = 16;
+    hipblasLtMatmulHeuristicResult_t res[kMostAlgos];
+    int found = 0, pick = 0;
     st = hipblasLtMatmulAlgoGetHeuristic(h->second, p.desc, p.la, p.lb, p.ld, p.ld, pref, 1, res, &found);
+    if (st == HIPBLAS_STATUS_SUCCESS && found > 0 && res[0].workspaceSize > ws_bytes)
+      st = hipblasLtMatmulAlgoGetHeuristic(h->second, p.desc, p.la, p.lb, p.ld, p.ld, pref, kMostAlgos, res, &found);
     hipblasLtMatmulPreferenceDestroy(pref);
-    if (st != HIPBLAS_STATUS_SUCCESS || found == 0) {
+    while (pick < found && res[pick].workspaceSize > ws_bytes) ++pick;
+    if (st != HIPBLAS_STATUS_SUCCESS || found == 0 || pick == found) {
       *err = st != HIPBLAS_STATUS_SUCCESS ? status_name(st) : "no hipBLASLt algorithm for this GEMM";
       return -1;
     }
-    p.algo = res[0].algo;
-    p.ws = res[0].workspaceSize;
+    p.algo = res[pick].algo;
+    p.ws = res[pick].workspaceSize;
     it = g_plans.emplace(key, p).first;
   }
   const Plan &p = it->second;

@@ -265,3 +265,28 @@ def test_repeated_calls_equal_bit_for_bit(dev):
         else:
             for name, a, b in zip(("t", "grad_A", "grad_B"), first, out):
                 assert torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("S,K,N,r", [(1303, 4096, 24576, 64), (97, 4096, 24576, 32), (2500, 12288, 4096, 16)])
+def test_long_reductions(dev, S, K, N, r):
+    """Qwen3-8B gate_up- and down-projections: dX sums over up to 24 576
+    columns, where the GEMM library's first choice of algorithm can need more
+    workspace than the layer has. Against float64 on the GPU, with the bf16
+    unit roundoff 2^-8 for each rounding: y rounds t (carried by |t| |B|^T), the
+    LoRA term and the sum; dX rounds d_a (by |d_a| |A|), d_a A and the sum."""
+    lm = lora_mod()
+    x, W, A, B, gt = make(S, K, N, r, dev, seed=S)
+    dy = torch.randn(S, N, generator=torch.Generator(device=dev).manual_seed(S + 7), device=dev).bfloat16()
+    y, t, h = lm.gated_lora_forward(x, W, A, B, gt, 2.0, 0.0, 0)
+    gx, _, _ = lm.gated_lora_backward(dy, x, h, t, W, A, B, gt, 2.0, 0.0, 0, True, False, False)
+    X, Wd, Ad, Bd, DY, G = (v.double() for v in (x, W, A, B, dy, gt[:, None]))
+    lora = 2.0 * G * ((X @ Ad.t()) @ Bd.t())
+    ref = X @ Wd.t() + lora
+    lora_abs = 2.0 * G * ((X @ Ad.t()).abs() @ Bd.abs().t())
+    bound = U * (ref.abs() + lora.abs() + lora_abs) + 1e-5 * ref.abs().max()
+    assert bool(((y.double() - ref).abs() <= bound).all())
+    d_a = 2.0 * G * (DY @ Bd)
+    base = DY @ Wd
+    ref = base + d_a @ Ad
+    bound = U * (ref.abs() + (ref - base).abs() + d_a.abs() @ Ad.abs()) + 1e-5 * ref.abs().max()
+    assert bool(((gx.double() - ref).abs() <= bound).all())
