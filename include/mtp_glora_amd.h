@@ -173,15 +173,15 @@ int mga_attn_bwd(const void *q, int64_t q_sh, int64_t q_ss,
  * items over their keys: the parts' fp32 results are combined in a fixed
  * order, so calls stay bit-for-bit repeatable. Results agree with the calls
  * without a workspace up to the order of fp32 sums.
- * workspace: mga_attn_workspace_bytes(...) bytes (backward 0 or 1) of device
- *   memory, 16-byte aligned, used by this call only; NULL (or a shape that
+ * workspace: mga_attn_workspace_bytes(...) bytes (backward 0 or 1; grad_start
+ *   as in mga_attn_bwd, 0 for the forward) of device memory, 16-byte aligned, used by this call only; NULL (or a shape that
  *   needs none): the call is mga_attn_fwd / mga_attn_bwd. A non-NULL workspace
  *   smaller than needed is MGA_ERR_INVALID.
  * mga_attn_workspace_bytes depends on the current device's number of compute
  * units; 0 for a shape that is not split (or invalid sizes).
  */
 int64_t mga_attn_workspace_bytes(int32_t S, int32_t L, int32_t Hq, int32_t Hkv, int32_t head_dim, int32_t dtype,
-                                 int32_t backward);
+                                 int32_t backward, int32_t grad_start);
 int mga_attn_fwd_ws(const void *q, int64_t q_sh, int64_t q_ss,
                     const void *k, int64_t k_sh, int64_t k_ss,
                     const void *v, int64_t v_sh, int64_t v_ss,

@@ -47,7 +47,7 @@ SIGNATURES = {
                      _P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64,
                      _I32, _P, _P, _P, _P, _P, _P, _P, _P, _P,
                      _I32, _I32, _I32, _I32, _I32, _I32, _I32, _F32, _I32, _P],
-    "mga_attn_workspace_bytes": [_I32, _I32, _I32, _I32, _I32, _I32, _I32],
+    "mga_attn_workspace_bytes": [_I32, _I32, _I32, _I32, _I32, _I32, _I32, _I32],
     "mga_attn_fwd_ws": [_P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64,
                         _P, _P, _P, _P, _P, _P,
                         _I32, _I32, _I32, _I32, _I32, _I32, _I32, _F32, _P, _I64, _P],

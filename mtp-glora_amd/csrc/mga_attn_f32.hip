@@ -30,8 +30,15 @@
 //             the transposed block mask x the G query heads:
 //             S = Q K^T, dP = dO V^T, dS = P (dP - delta),
 //             dV^T += dO^T P, dK^T += Q^T dS.
+// Each is bound by the serial walk over its steps (about 3 us each, one wave
+// per SIMD keeping the matrix core about 60 % busy), so with a workspace the
+// items of a last round that would leave CUs idle run in parts (KeySplit, down
+// to two steps) and small kernels combine them: at [323 rows, 4 / 2 heads of
+// 64, 768 prefix keys], 12 and 6 items on 256 CUs, forward 100 -> 15 + 10 us,
+// dQ 126 -> 20 + 6 us, dK/dV 111 -> 16 + 6 us.
 #include "mga_common.hpp"
 #include "mga_internal.hpp"
+#include "mga_key_split.hpp"
 
 namespace mga {
 
@@ -90,27 +97,49 @@ struct Stage32 {
 __host__ __device__ __forceinline__ int heads_per_wg_f32(int G) { return (G % 4 == 0) ? 4 : (G % 2 == 0 ? 2 : 1); }
 
 // Query-side work item of the forward and dQ kernels: 4 waves = HPW heads of
-// one kv head x (4 / HPW) blocks of 32 rows.
+// one kv head x (4 / HPW) blocks of 32 rows. XCD x runs a contiguous share of
+// the items; its workgroup t an item of the share, or a part of one.
 struct QItem {
   int g, h, row, qt;
 };
 
-__device__ __forceinline__ QItem q_item(const AttnArgs &a) {
+// false: past the share
+__device__ __forceinline__ bool q_item(const AttnArgs &a, int xcd, int o, QItem &it) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int G = a.Hq / a.Hkv;
   const int HPW = heads_per_wg_f32(G);
   const int QR = kR * (4 / HPW);
   const int nslice = G / HPW;
   const int nqb = (a.S + QR - 1) / QR;
-  const int li = xcd_swizzle(blockIdx.x, a.Hkv * nslice * nqb);
-  QItem it;
+  const int n = a.Hkv * nslice * nqb;
+  if (o >= n / 8 + (xcd < n % 8 ? 1 : 0)) return false;
+  const int li = xcd * (n / 8) + min(xcd, n % 8) + o;
   it.g = li / (nslice * nqb);
   const int rem = li % (nslice * nqb);
   const int qb = nqb - 1 - rem / nslice;
   it.h = it.g * G + (rem % nslice) * HPW + wave % HPW;
   it.row = qb * QR + (wave / HPW) * kR + (lane & 31);
   it.qt = (qb * QR) / kBlock;
-  return it;
+  return true;
+}
+
+// A part's 16 accumulators per lane and 32-dim block, in 16-byte runs.
+__device__ __forceinline__ void part_store(float *p, int db, const f32x16 &v) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    *reinterpret_cast<f32x4 *>(p + ((db * 4 + q) * 64 + lane) * 4) =
+        f32x4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+}
+// acc += w * the part's
+__device__ __forceinline__ void part_add(const float *p, int db, float w, f32x16 &acc) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const f32x4 v = *reinterpret_cast<const f32x4 *>(p + ((db * 4 + q) * 64 + lane) * 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[4 * q + e] += v[e] * w;
+  }
 }
 
 }  // namespace
@@ -119,7 +148,7 @@ __device__ __forceinline__ QItem q_item(const AttnArgs &a) {
 // Forward
 // ---------------------------------------------------------------------------
 template <int HD>
-__global__ __launch_bounds__(256, 2) void attn_fwd_f32_kernel(AttnArgs a) {
+__global__ __launch_bounds__(256, 2) void attn_fwd_f32_kernel(AttnArgs a, KeySplit sp) {
   constexpr int KH = HD / 2;   // MFMA steps over head_dim
   constexpr int DB = HD / 32;  // 32-dim blocks of O^T
   constexpr int TILE = kR * kStride<HD>;
@@ -127,7 +156,11 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_f32_kernel(AttnArgs a) {
   __shared__ int sW0[kR], sW1[kR];
 
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
-  const QItem it = q_item(a);
+  const int xcd = blockIdx.x & 7;
+  QItem it;
+  int o, part;
+  sp.locate((int)(blockIdx.x >> 3), o, part);
+  if (!q_item(a, xcd, o, it)) return;
   const int row = it.row, qr = min(row, a.S - 1);
   const float *qp = reinterpret_cast<const float *>(a.q) + it.h * a.q_sh + (int64_t)qr * a.q_ss + KH * hi;
   const float *kp = reinterpret_cast<const float *>(a.k) + it.g * a.k_sh;
@@ -145,8 +178,10 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_f32_kernel(AttnArgs a) {
 
   TileList tiles = tile_list(a.kv_num, a.kv_idx, a.fkv_num, a.fkv_idx, it.qt, a.nKV);
   constexpr int kSub = kBlock / kR;
-  const int nstep = kSub * tiles.ntot;
-  auto step_base = [&](int j) { return tiles.at(j / kSub) * kBlock + (j % kSub) * kR; };
+  // the workgroup's steps of the list: all, or the part's
+  const int j0 = part < 0 ? 0 : sp.begin(part, kSub * tiles.ntot);
+  const int nstep = (part < 0 ? kSub * tiles.ntot : sp.begin(part + 1, kSub * tiles.ntot)) - j0;
+  auto step_base = [&](int j) { return tiles.at((j0 + j) / kSub) * kBlock + ((j0 + j) % kSub) * kR; };
 
   Stage32<HD> stK, stV;
   KeyCode wkey;
@@ -249,6 +284,14 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_f32_kernel(AttnArgs a) {
     }
   }
 
+  if (part >= 0) {   // raw (O^T, offset, row sum): attn_fwd_f32_merge_kernel combines the parts
+    float *po = sp.ws + (sp.slot(o, part, xcd) * 4 + (tid >> 6)) * kPartFloats<HD>;
+#pragma unroll
+    for (int db = 0; db < DB; ++db) part_store(po, db, oacc[db]);
+    po[HD * 32 + lane] = m_run;
+    po[HD * 32 + 64 + lane] = l_run;
+    return;
+  }
   const float lt = l_run + xor32(l_run);
   if (row < a.S) {
     const float inv = lt > 0.f ? 1.f / lt : 0.f;
@@ -267,7 +310,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_f32_kernel(AttnArgs a) {
 // Backward, dQ pass (also writes delta)
 // ---------------------------------------------------------------------------
 template <int HD>
-__global__ __launch_bounds__(256, 1) void attn_bwd_dq_f32_kernel(AttnArgs a) {
+__global__ __launch_bounds__(256, 1) void attn_bwd_dq_f32_kernel(AttnArgs a, KeySplit sp) {
   constexpr int KH = HD / 2;
   constexpr int DB = HD / 32;
   constexpr int TILE = kR * kStride<HD>;
@@ -275,7 +318,11 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_f32_kernel(AttnArgs a) {
   __shared__ int sW0[kR], sW1[kR];
 
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
-  const QItem it = q_item(a);
+  const int xcd = blockIdx.x & 7;
+  QItem it;
+  int o, part;
+  sp.locate((int)(blockIdx.x >> 3), o, part);
+  if (!q_item(a, xcd, o, it)) return;
   const int row = it.row, qr = min(row, a.S - 1);
   const bool in = row < a.S;
   const float *qp = reinterpret_cast<const float *>(a.q) + it.h * a.q_sh + (int64_t)qr * a.q_ss + KH * hi;
@@ -300,7 +347,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_f32_kernel(AttnArgs a) {
   }
   del += xor32(del);
   if (!in) del = 0.f;
-  if (in && hi == 0) a.delta[(int64_t)it.h * a.S + row] = del;
+  if (in && hi == 0 && part <= 0) a.delta[(int64_t)it.h * a.S + row] = del;
   const float lse = in ? a.lse[(int64_t)it.h * a.S + row] : kNegInfF32;
   const float lse2 = lse == kNegInfF32 ? 0.f : lse * kLog2e;
   const int qcode = in ? a.code[row] : kCodePad;
@@ -309,8 +356,10 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_f32_kernel(AttnArgs a) {
 
   TileList tiles = tile_list(a.kv_num, a.kv_idx, a.fkv_num, a.fkv_idx, it.qt, a.nKV);
   constexpr int kSub = kBlock / kR;
-  const int nstep = kSub * tiles.ntot;
-  auto step_base = [&](int j) { return tiles.at(j / kSub) * kBlock + (j % kSub) * kR; };
+  // the workgroup's steps of the list: all, or the part's
+  const int j0 = part < 0 ? 0 : sp.begin(part, kSub * tiles.ntot);
+  const int nstep = (part < 0 ? kSub * tiles.ntot : sp.begin(part + 1, kSub * tiles.ntot)) - j0;
+  auto step_base = [&](int j) { return tiles.at((j0 + j) / kSub) * kBlock + ((j0 + j) % kSub) * kR; };
 
   Stage32<HD> stK, stV;
   KeyCode wkey;
@@ -403,6 +452,12 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_f32_kernel(AttnArgs a) {
     }
   }
 
+  if (part >= 0) {   // the part's sums: attn_bwd_dq_f32_merge_kernel adds them
+    float *po = sp.ws + (sp.slot(o, part, xcd) * 4 + (tid >> 6)) * (HD * 32);
+#pragma unroll
+    for (int db = 0; db < DB; ++db) part_store(po, db, dqacc[db]);
+    return;
+  }
   if (in) {
     float *out = reinterpret_cast<float *>(a.dq) + it.h * a.dq_sh + (int64_t)row * a.dq_ss;
 #pragma unroll
@@ -418,7 +473,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_f32_kernel(AttnArgs a) {
 // Backward, dK/dV pass (reads the delta of the dQ pass)
 // ---------------------------------------------------------------------------
 template <int HD>
-__global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_f32_kernel(AttnArgs a, int kt0) {
+__global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_f32_kernel(AttnArgs a, int kt0, KeySplit sp) {
   constexpr int KH = HD / 2;
   constexpr int DB = HD / 32;
   constexpr int TILE = kR * kStride<HD>;
@@ -431,7 +486,12 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_f32_kernel(AttnArgs a, i
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hi = lane >> 5, wave = tid >> 6;
   const int G = a.Hq / a.Hkv;
   const int nkt = a.nKV - kt0;
-  const int li = xcd_swizzle(blockIdx.x, a.Hkv * nkt);
+  const int n_items = a.Hkv * nkt;
+  const int xcd = blockIdx.x & 7;
+  int o, part;
+  sp.locate((int)(blockIdx.x >> 3), o, part);
+  if (o >= n_items / 8 + (xcd < n_items % 8 ? 1 : 0)) return;
+  const int li = xcd * (n_items / 8) + min(xcd, n_items % 8) + o;
   const int g = li / nkt;
   const int kt = kt0 + li % nkt;
   const int key = kt * kBlock + kR * wave + l32;
@@ -458,10 +518,14 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_f32_kernel(AttnArgs a, i
   TileList tiles = tile_list(a.q_num, a.q_idx, a.fq_num, a.fq_idx, kt, a.nQ);
   constexpr int kSub = kBlock / kR;
   const int per_tile = kSub * G;
-  const int nstep = per_tile * tiles.ntot;
-  // step j: query tile j / per_tile, 32-row block, head of the kv group
-  auto step_q0 = [&](int j) { return tiles.at(j / per_tile) * kBlock + ((j % per_tile) / G) * kR; };
-  auto step_h = [&](int j) { return g * G + (j % per_tile) % G; };
+  const int j0 = part < 0 ? 0 : sp.begin(part, per_tile * tiles.ntot);
+  const int nstep = (part < 0 ? per_tile * tiles.ntot : sp.begin(part + 1, per_tile * tiles.ntot)) - j0;
+  // step j of the whole list: query tile j / per_tile, 32-row block, head of the kv group
+  auto step_q0 = [&](int j) {
+    j += j0;
+    return tiles.at(j / per_tile) * kBlock + ((j % per_tile) / G) * kR;
+  };
+  auto step_h = [&](int j) { return g * G + ((j0 + j) % per_tile) % G; };
 
   Stage32<HD> stQ, stD;
   float rl = 0.f, re = 0.f;
@@ -599,6 +663,15 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_f32_kernel(AttnArgs a, i
     }
   }
 
+  if (part >= 0) {   // the part's sums, dK^T then dV^T: attn_bwd_dkdv_f32_merge_kernel adds them
+    float *po = sp.ws + (sp.slot(o, part, xcd) * 4 + wave) * (2 * HD * 32);
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+      part_store(po, db, dk[db]);
+      part_store(po, DB + db, dv[db]);
+    }
+    return;
+  }
   // lane = key, registers = dims 32 db + 8 (r / 4) + 4 hi + r % 4
   if (key >= a.grad_start && key < a.L) {
     const int64_t r = key - a.grad_start;
@@ -616,14 +689,106 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_f32_kernel(AttnArgs a, i
   }
 }
 
-template __global__ void attn_fwd_f32_kernel<128>(AttnArgs);
-template __global__ void attn_fwd_f32_kernel<64>(AttnArgs);
-template __global__ void attn_bwd_dq_f32_kernel<128>(AttnArgs);
-template __global__ void attn_bwd_dq_f32_kernel<64>(AttnArgs);
-template __global__ void attn_bwd_dkdv_f32_kernel<128>(AttnArgs, int);
-template __global__ void attn_bwd_dkdv_f32_kernel<64>(AttnArgs, int);
+// ---------------------------------------------------------------------------
+// Combining the parts of split items, in the order of the parts. Workgroup
+// (item u of the XCD's split items, 32-dim block db), threads as in the item's
+// workgroups.
+// ---------------------------------------------------------------------------
+template <int HD>
+__global__ __launch_bounds__(256) void attn_fwd_f32_merge_kernel(AttnArgs a, KeySplit sp) {
+  constexpr int DB = HD / 32;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, hi = lane >> 5;
+  const int xcd = blockIdx.x & 7, o = sp.k + (int)(blockIdx.x >> 3) / DB, db = (int)(blockIdx.x >> 3) % DB;
+  QItem it;
+  if (!q_item(a, xcd, o, it)) return;
+  const float *p0 = sp.ws + (sp.slot(o, 0, xcd) * 4 + wave) * kPartFloats<HD>;
+  const int64_t step = (int64_t)8 * 4 * kPartFloats<HD>;
+  float m = kNegInfF32;
+#pragma unroll 4
+  for (int p = 0; p < sp.ns; ++p) m = fmaxf(m, p0[p * step + HD * 32 + lane]);
+  const float mu = m == kNegInfF32 ? 0.f : m;   // no part saw an unmasked key: every weight is 0
+  float l = 0.f;
+  f32x16 acc = zero16();
+#pragma unroll 4
+  for (int p = 0; p < sp.ns; ++p) {
+    const float *pp = p0 + p * step;
+    const float w = __builtin_amdgcn_exp2f(pp[HD * 32 + lane] - mu);
+    l += pp[HD * 32 + 64 + lane] * w;
+    part_add(pp, db, w, acc);
+  }
+  const float lt = l + xor32(l);
+  if (it.row >= a.S) return;
+  const float inv = lt > 0.f ? 1.f / lt : 0.f;
+  if (hi == 0 && db == 0) a.lse[(int64_t)it.h * a.S + it.row] = lt > 0.f ? (m + __log2f(lt)) * kLn2 : kNegInfF32;
+  float *orow = reinterpret_cast<float *>(const_cast<void *>(a.o)) + it.h * a.o_sh + (int64_t)it.row * a.o_ss;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    store4(orow + db * 32 + 8 * i + 4 * hi, acc[4 * i] * inv, acc[4 * i + 1] * inv, acc[4 * i + 2] * inv,
+           acc[4 * i + 3] * inv);
+}
+
+template <int HD>
+__global__ __launch_bounds__(256) void attn_bwd_dq_f32_merge_kernel(AttnArgs a, KeySplit sp) {
+  constexpr int DB = HD / 32;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, hi = lane >> 5;
+  const int xcd = blockIdx.x & 7, o = sp.k + (int)(blockIdx.x >> 3) / DB, db = (int)(blockIdx.x >> 3) % DB;
+  QItem it;
+  if (!q_item(a, xcd, o, it) || it.row >= a.S) return;
+  const float *p0 = sp.ws + (sp.slot(o, 0, xcd) * 4 + wave) * (HD * 32);
+  f32x16 acc = zero16();
+#pragma unroll 4
+  for (int p = 0; p < sp.ns; ++p) part_add(p0 + p * (int64_t)(8 * 4 * HD * 32), db, 1.f, acc);
+  float *out = reinterpret_cast<float *>(a.dq) + it.h * a.dq_sh + (int64_t)it.row * a.dq_ss;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    store4(out + db * 32 + 8 * i + 4 * hi, acc[4 * i] * a.scale, acc[4 * i + 1] * a.scale, acc[4 * i + 2] * a.scale,
+           acc[4 * i + 3] * a.scale);
+}
+
+// db: 32-dim blocks of dK, then of dV
+template <int HD>
+__global__ __launch_bounds__(256) void attn_bwd_dkdv_f32_merge_kernel(AttnArgs a, int kt0, KeySplit sp) {
+  constexpr int DB = HD / 32;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, hi = lane >> 5;
+  const int xcd = blockIdx.x & 7, o = sp.k + (int)(blockIdx.x >> 3) / (2 * DB), db = (int)(blockIdx.x >> 3) % (2 * DB);
+  const int nkt = a.nKV - kt0;
+  const int n_items = a.Hkv * nkt;
+  if (o >= n_items / 8 + (xcd < n_items % 8 ? 1 : 0)) return;
+  const int li = xcd * (n_items / 8) + min(xcd, n_items % 8) + o;
+  const int g = li / nkt;
+  const int key = (kt0 + li % nkt) * kBlock + kR * wave + (lane & 31);
+  if (key < a.grad_start || key >= a.L) return;
+  const float *p0 = sp.ws + (sp.slot(o, 0, xcd) * 4 + wave) * (2 * HD * 32);
+  f32x16 acc = zero16();
+#pragma unroll 4
+  for (int p = 0; p < sp.ns; ++p) part_add(p0 + p * (int64_t)(8 * 4 * 2 * HD * 32), db, 1.f, acc);
+  const int64_t r = key - a.grad_start;
+  const bool isk = db < DB;
+  const float f = isk ? a.scale : 1.f;
+  float *out = isk ? reinterpret_cast<float *>(a.dk) + g * a.dk_sh + r * a.dk_ss
+                   : reinterpret_cast<float *>(a.dv) + g * a.dv_sh + r * a.dv_ss;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    store4(out + (isk ? db : db - DB) * 32 + 8 * i + 4 * hi, acc[4 * i] * f, acc[4 * i + 1] * f, acc[4 * i + 2] * f,
+           acc[4 * i + 3] * f);
+}
+
+#define MGA_F32_INST(HD)                                                            \
+  template __global__ void attn_fwd_f32_kernel<HD>(AttnArgs, KeySplit);             \
+  template __global__ void attn_bwd_dq_f32_kernel<HD>(AttnArgs, KeySplit);          \
+  template __global__ void attn_bwd_dkdv_f32_kernel<HD>(AttnArgs, int, KeySplit);   \
+  template __global__ void attn_fwd_f32_merge_kernel<HD>(AttnArgs, KeySplit);       \
+  template __global__ void attn_bwd_dq_f32_merge_kernel<HD>(AttnArgs, KeySplit);    \
+  template __global__ void attn_bwd_dkdv_f32_merge_kernel<HD>(AttnArgs, int, KeySplit);
+MGA_F32_INST(128)
+MGA_F32_INST(64)
+#undef MGA_F32_INST
 
 namespace {
+
+// A part's fixed cost and the combining launch's, in 32-key (32-row) steps of
+// about 3 us.
+constexpr float kPartSteps = 1.f, kMergeSteps = 2.f;
 
 int q_items(const AttnArgs &a) {
   const int G = a.Hq / a.Hkv;
@@ -632,25 +797,66 @@ int q_items(const AttnArgs &a) {
   return a.Hkv * (G / HPW) * ((a.S + QR - 1) / QR);
 }
 
+// One workgroup per CU counts as a slot: a wave's fp32 MFMAs nearly fill its SIMD.
+KeySplit plan(int items, int nstep) {
+  return key_split_plan((items + 7) / 8, device_cu_count() / 8, nstep, kPartSteps, kMergeSteps, 2);
+}
+
+KeySplit q_split(const AttnArgs &a) { return plan(q_items(a), kBlock / kR * a.nKV); }
+
+KeySplit k_split(const AttnArgs &a, int kt0) {
+  return plan(a.Hkv * (a.nKV - kt0), kBlock / kR * a.nQ * (a.Hq / a.Hkv));
+}
+
+int64_t parts(const KeySplit &sp) { return sp.ns > 1 ? (int64_t)8 * 4 * sp.r * sp.ns : 0; }   // waves
+
+template <int HD>
+void fwd_f32(const AttnArgs &a, hipStream_t st) {
+  KeySplit sp = a.ws ? q_split(a) : no_split((q_items(a) + 7) / 8);
+  sp.ws = a.ws;
+  hipLaunchKernelGGL((attn_fwd_f32_kernel<HD>), dim3(8 * sp.groups()), dim3(256), 0, st, a, sp);
+  if (sp.ns > 1)
+    hipLaunchKernelGGL((attn_fwd_f32_merge_kernel<HD>), dim3(8 * sp.r * (HD / 32)), dim3(256), 0, st, a, sp);
+}
+
 template <int HD>
 void bwd_f32(const AttnArgs &a, int passes, hipStream_t st) {
-  if (passes & kBwdDq) hipLaunchKernelGGL((attn_bwd_dq_f32_kernel<HD>), dim3(q_items(a)), dim3(256), 0, st, a);
+  if (passes & kBwdDq) {
+    KeySplit sp = a.ws ? q_split(a) : no_split((q_items(a) + 7) / 8);
+    sp.ws = a.ws;
+    hipLaunchKernelGGL((attn_bwd_dq_f32_kernel<HD>), dim3(8 * sp.groups()), dim3(256), 0, st, a, sp);
+    if (sp.ns > 1)
+      hipLaunchKernelGGL((attn_bwd_dq_f32_merge_kernel<HD>), dim3(8 * sp.r * (HD / 32)), dim3(256), 0, st, a, sp);
+  }
   if ((passes & kBwdDkDv) && a.grad_start < a.L) {
     const int kt0 = a.grad_start / kBlock;
-    hipLaunchKernelGGL((attn_bwd_dkdv_f32_kernel<HD>), dim3(a.Hkv * (a.nKV - kt0)), dim3(256), 0, st, a, kt0);
+    KeySplit sp = a.ws ? k_split(a, kt0) : no_split((a.Hkv * (a.nKV - kt0) + 7) / 8);
+    sp.ws = a.ws;
+    hipLaunchKernelGGL((attn_bwd_dkdv_f32_kernel<HD>), dim3(8 * sp.groups()), dim3(256), 0, st, a, kt0, sp);
+    if (sp.ns > 1)
+      hipLaunchKernelGGL((attn_bwd_dkdv_f32_merge_kernel<HD>), dim3(8 * sp.r * (HD / 16)), dim3(256), 0, st, a, kt0,
+                         sp);
   }
 }
 
 }  // namespace
 
 void launch_attn_fwd_f32(const AttnArgs &a, int head_dim, hipStream_t st) {
-  if (head_dim == 128) hipLaunchKernelGGL((attn_fwd_f32_kernel<128>), dim3(q_items(a)), dim3(256), 0, st, a);
-  else hipLaunchKernelGGL((attn_fwd_f32_kernel<64>), dim3(q_items(a)), dim3(256), 0, st, a);
+  if (head_dim == 128) fwd_f32<128>(a, st);
+  else fwd_f32<64>(a, st);
 }
 
 void launch_attn_bwd_f32(const AttnArgs &a, int head_dim, int passes, hipStream_t st) {
   if (head_dim == 128) bwd_f32<128>(a, passes, st);
   else bwd_f32<64>(a, passes, st);
+}
+
+int64_t attn_fwd_f32_ws_floats(const AttnArgs &a, int head_dim) { return parts(q_split(a)) * part_floats(head_dim); }
+
+int64_t attn_bwd_f32_ws_floats(const AttnArgs &a, int head_dim) {
+  const int64_t q = parts(q_split(a)) * head_dim * 32;
+  const int kt0 = a.grad_start / kBlock;
+  return a.grad_start < a.L ? std::max(q, parts(k_split(a, kt0)) * 2 * head_dim * 32) : q;
 }
 
 }  // namespace mga

@@ -385,6 +385,7 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_merge_kernel(AttnArgs a, 
   const float *p0 = sp.ws + (sp.slot(o, 0, xcd) * NW + wave) * (HD * 32);
   const int64_t step = (int64_t)8 * NW * (HD * 32);   // to the next part
   f32x16 acc = zero16();
+#pragma unroll 4
   for (int p = 0; p < sp.ns; ++p)
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -438,13 +439,13 @@ DqGrid dq_grid(const AttnArgs &a) {
 KeySplit dq_split(const AttnArgs &a) {
   const DqGrid f = dq_grid(a);
   return key_split_plan(f.nmax, f.slots, last_round_tiles(a.S, a.P, a.Hkv, f.nslice, f.rows, f.nmax % f.slots),
-                        kDqPartTiles, kDqMergeTiles);
+                        kDqPartTiles, kDqMergeTiles, 4);
 }
 
 }  // namespace
 
 int64_t attn_bwd_ws_floats(const AttnArgs &a, int head_dim, int dtype) {
-  if (dtype == kDtF32) return 0;   // the fp32 kernels do not split
+  if (dtype == kDtF32) return attn_bwd_f32_ws_floats(a, head_dim);
   const KeySplit sp = dq_split(a);
   const DqGrid f = dq_grid(a);
   return sp.ns > 1 ? (int64_t)8 * sp.r * sp.ns * f.nw * head_dim * 32 : 0;

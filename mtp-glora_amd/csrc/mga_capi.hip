@@ -193,10 +193,12 @@ int mga_mtp_block_mask(const int64_t *gate, int64_t gate_stride, int32_t S, int6
 }
 
 int64_t mga_attn_workspace_bytes(int32_t S, int32_t L, int32_t Hq, int32_t Hkv, int32_t head_dim, int32_t dtype,
-                                 int32_t backward) {
-  if (check_attn_common(S, L, L - S, Hq, Hkv, head_dim, dtype, 1.f) != MGA_OK) return 0;
+                                 int32_t backward, int32_t grad_start) {
+  if (check_attn_common(S, L, L - S, Hq, Hkv, head_dim, dtype, 1.f) != MGA_OK || grad_start < 0 || grad_start > L)
+    return 0;
   mga::AttnArgs a = {};
   a.S = S; a.L = L; a.P = L - S; a.Hq = Hq; a.Hkv = Hkv;
+  a.grad_start = grad_start;
   a.nQ = (S + MGA_BLOCK - 1) / MGA_BLOCK;
   a.nKV = (L + MGA_BLOCK - 1) / MGA_BLOCK;
   return 4 * (backward ? mga::attn_bwd_ws_floats(a, head_dim, dtype) : mga::attn_fwd_ws_floats(a, head_dim, dtype));

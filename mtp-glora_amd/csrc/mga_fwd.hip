@@ -612,10 +612,12 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_merge_kernel(AttnArgs a, Key
   const float *p0 = sp.ws + (sp.slot(o, 0, xcd) * NW + wave) * kPartFloats<HD>;
   const int64_t step = (int64_t)8 * kPartFloats<HD> * NW;   // to the next part
   float mm = kNegInfF;
+#pragma unroll 4
   for (int p = 0; p < sp.ns; ++p) mm = fmaxf(mm, p0[p * step + HD * 32 + lane]);
   const float mu = mm == kNegInfF ? 0.f : mm;   // no part saw an unmasked key: every weight is 0
   float l = 0.f;
   f32x16 acc = zero16();
+#pragma unroll 4
   for (int p = 0; p < sp.ns; ++p) {
     const float *pp = p0 + p * step;
     const float w = exp2f_(pp[HD * 32 + lane] - mu);
@@ -696,11 +698,11 @@ FwdGrid fwd_grid(const AttnArgs &a) {
 static KeySplit fwd_split(const AttnArgs &a) {
   const FwdGrid f = fwd_grid(a);
   return key_split_plan(f.nmax, f.slots, last_round_tiles(a.S, a.P, a.Hkv, f.nslice, f.rows, f.nmax % f.slots),
-                        kFwdPartTiles, kFwdMergeTiles);
+                        kFwdPartTiles, kFwdMergeTiles, 4);
 }
 
 int64_t attn_fwd_ws_floats(const AttnArgs &a, int head_dim, int dtype) {
-  if (dtype == kDtF32) return 0;   // the fp32 kernels do not split
+  if (dtype == kDtF32) return attn_fwd_f32_ws_floats(a, head_dim);
   const KeySplit sp = fwd_split(a);
   const FwdGrid f = fwd_grid(a);
   return sp.ns > 1 ? (int64_t)8 * sp.r * sp.ns * f.nw * part_floats(head_dim) : 0;

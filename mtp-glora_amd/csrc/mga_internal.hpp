@@ -48,7 +48,8 @@ constexpr int kDtF16 = 2;
 // head_dim in {64, 128}; dtype one of kDt*.
 void launch_attn_fwd(const AttnArgs &a, int head_dim, int dtype, hipStream_t stream);
 // fp32 words of AttnArgs::ws that the forward / the dQ pass of this shape use
-// (S, L, nKV, Hq and Hkv set), 0 where they do not split their items.
+// (S, L, P, nQ, nKV, Hq, Hkv and, for the backward, grad_start set), 0 where
+// they do not split their items.
 int64_t attn_fwd_ws_floats(const AttnArgs &a, int head_dim, int dtype);
 int64_t attn_bwd_ws_floats(const AttnArgs &a, int head_dim, int dtype);
 // passes: kBwdDq (delta + dQ) and/or kBwdDkDv (dK/dV; reads the delta the dQ pass wrote).
@@ -58,6 +59,8 @@ void launch_attn_bwd(const AttnArgs &a, int head_dim, int dtype, int passes, hip
 // fp32 operands (mga_attn_f32.hip): fp32 MFMAs throughout; same contract.
 void launch_attn_fwd_f32(const AttnArgs &a, int head_dim, hipStream_t stream);
 void launch_attn_bwd_f32(const AttnArgs &a, int head_dim, int passes, hipStream_t stream);
+int64_t attn_fwd_f32_ws_floats(const AttnArgs &a, int head_dim);
+int64_t attn_bwd_f32_ws_floats(const AttnArgs &a, int head_dim);
 
 // Fused Qwen3 q/k RMSNorm + rotary embedding (mga_qk_rope.hip). Operands are
 // [S, heads, D] addressed with (token stride, head stride) in elements; cos

@@ -79,10 +79,10 @@ inline int last_round_tiles(int S, int P, int Hkv, int nslice, int rows, int r) 
 // * r < slots: a long first part for r of the slots, short ones in rounds on
 //   the other slots - r, so long that both end together (24 items on 32
 //   slots: 3/4 of each item in one piece, the rest three to a free slot).
-// A part keeps at least kMinPartTiles tiles; kMaxPartRounds bounds the
+// A part keeps at least min_part tiles; kMaxPartRounds bounds the
 // workspace (133 KB a part at head_dim 128).
-constexpr int kMinPartTiles = 4, kMaxParts = 16, kMaxPartRounds = 4;
-inline KeySplit key_split_plan(int nmax, int slots, int ntile, float part_cost, float merge_cost) {
+constexpr int kMaxParts = 16, kMaxPartRounds = 4;
+inline KeySplit key_split_plan(int nmax, int slots, int ntile, float part_cost, float merge_cost, int min_part) {
   KeySplit best = no_split(nmax);
   slots = std::max(slots, 1);
   const int r = nmax % slots;
@@ -90,7 +90,7 @@ inline KeySplit key_split_plan(int nmax, int slots, int ntile, float part_cost, 
   const float T = (float)ntile;
   float best_cost = T;   // the last round unsplit
   for (int ns = 2; ns <= kMaxParts && r * ns <= kMaxPartRounds * slots; ++ns) {
-    if (ntile >= kMinPartTiles * ns) {
+    if (ntile >= min_part * ns) {
       const int rounds = (r * ns + slots - 1) / slots;
       const float cost = rounds * ((float)((ntile + ns - 1) / ns) + part_cost) + merge_cost;
       if (cost < best_cost) {
@@ -101,7 +101,7 @@ inline KeySplit key_split_plan(int nmax, int slots, int ntile, float part_cost, 
     const int rounds = (r * (ns - 1) + slots - r - 1) / (slots - r);   // of the short parts
     const float per = (float)rounds / (ns - 1);
     const float big = (per * T + (rounds - 1) * part_cost) / (1.f + per);   // big + part_cost = short parts' end
-    if (big < T && (T - big) / (ns - 1) >= kMinPartTiles) {
+    if (big < T && (T - big) / (ns - 1) >= min_part) {
       const float cost = std::ceil(big) + part_cost + merge_cost;
       if (cost < best_cost) {
         best_cost = cost;

@@ -157,16 +157,17 @@ def mtp_block_mask_tensors(gate: torch.Tensor, P: int) -> dict:
 # ----------------------------------------------------------------------------
 
 @functools.lru_cache(maxsize=1024)
-def _attn_ws_bytes(S: int, L: int, Hq: int, Hkv: int, D: int, dtype: int, backward: int, device: int) -> int:
+def _attn_ws_bytes(S: int, L: int, Hq: int, Hkv: int, D: int, dtype: int, backward: int, grad_start: int,
+                   device: int) -> int:
     with torch.cuda.device(device):
-        return int(_lib.load().mga_attn_workspace_bytes(S, L, Hq, Hkv, D, dtype, backward))
+        return int(_lib.load().mga_attn_workspace_bytes(S, L, Hq, Hkv, D, dtype, backward, grad_start))
 
 
-def _attn_workspace(S, L, Hq, Hkv, D, dtype: int, backward: int, dev):
+def _attn_workspace(S, L, Hq, Hkv, D, dtype: int, backward: int, grad_start: int, dev):
     """(pointer, bytes, tensor) of the workspace in which a pass that would
     leave part of the GPU idle keeps its parts' results; (None, 0, None) where
     the shape needs none."""
-    n = _attn_ws_bytes(S, L, Hq, Hkv, D, dtype, backward, dev.index)
+    n = _attn_ws_bytes(S, L, Hq, Hkv, D, dtype, backward, grad_start, dev.index)
     if n == 0:
         return None, 0, None
     ws = torch.empty(n, dtype=torch.uint8, device=dev)
@@ -190,7 +191,7 @@ def attn_fwd(q, k, v, code, bm: dict, P: int, scale: float):
     o = torch.empty(1, S, Hq, D, dtype=qq.dtype, device=qq.device)
     lse = torch.empty(1, Hq, S, dtype=torch.float32, device=qq.device)
     dt = dtype_code(qq.dtype)
-    wp, wn, ws = _attn_workspace(S, L, Hq, Hkv, D, dt, 0, qq.device)
+    wp, wn, ws = _attn_workspace(S, L, Hq, Hkv, D, dt, 0, 0, qq.device)
     _lib.call("mga_attn_fwd_ws", qq.data_ptr(), q_sh, q_ss, kk.data_ptr(), k_sh, k_ss,
               vv.data_ptr(), v_sh, v_ss, o.data_ptr(), D, Hq * D, lse.data_ptr(), code.data_ptr(),
               bm["kv_num_blocks"].data_ptr(), bm["kv_indices"].data_ptr(),
@@ -228,9 +229,9 @@ def attn_bwd(q, k, v, o, lse, dout, code, bm: dict, P: int, scale: float, grad_s
     ``no_alloc`` calls ``mga_attn_bwd_noalloc``: delta lives in the library's
     fixed per-GPU workspace instead of ``buffers["delta"]``.
 
-    ``key_split`` gives the dQ pass a workspace (``mga_attn_bwd_ws``), so that
-    it may split its last work items over their keys; dQ then differs from the
-    unsplit call's in the order of its fp32 sums."""
+    ``key_split`` gives the call a workspace (``mga_attn_bwd_ws``), so that a
+    pass may split its last work items over their tile lists; the gradients then
+    differ from the unsplit call's in the order of their fp32 sums."""
     if key_split and no_alloc:
         raise ValueError("key_split needs a workspace, which no_alloc forbids")
     qq, q_sh, q_ss = _rows("query", q)
@@ -268,7 +269,8 @@ def attn_bwd(q, k, v, o, lse, dout, code, bm: dict, P: int, scale: float, grad_s
     if no_alloc:
         _lib.call("mga_attn_bwd_noalloc", *operands, *rest, _stream(qq))
     else:
-        wp, wn, ws = (_attn_workspace(S, L, Hq, Hkv, D, dt, 1, qq.device) if key_split else (None, 0, None))
+        wp, wn, ws = (_attn_workspace(S, L, Hq, Hkv, D, dt, 1, int(grad_start), qq.device) if key_split
+                      else (None, 0, None))
         _lib.call("mga_attn_bwd_ws", *operands, delta.data_ptr(), *rest, wp, wn, _stream(qq))
     dq_t = dq.transpose(1, 2)
     if dk is None:
