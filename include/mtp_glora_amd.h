@@ -390,6 +390,13 @@ int mga_soft_ce_fwd(const void *student, int64_t student_row_stride,
                     int32_t n_rows, int32_t n_cols, int32_t dtype,
                     float *row_loss, float *stats, float *workspace, void *stream);
 
+/* mga_soft_ce_fwd that also writes the sum of the row losses (fp32, added in a
+ * fixed order) to loss_sum: the value the autograd function returns
+ * (loss.py:294). */
+int mga_soft_ce_loss(const void *student, int64_t student_row_stride, const void *teacher,
+                     int64_t teacher_row_stride, int32_t n_rows, int32_t n_cols, int32_t dtype,
+                     float *row_loss, float *stats, float *loss_sum, float *workspace, void *stream);
+
 /*
  * Backward of mga_soft_ce_fwd for the student (the teacher gets none):
  *   grad[r, j] = grad_output * (e^{x - mx} / dx - e^{t - mt} / dt)

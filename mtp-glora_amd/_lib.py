@@ -76,6 +76,7 @@ SIGNATURES = {
                            _F64, _U64, _I32, _I32, _I32, _I32, _P, _I64, _P, _I64, _P, _I64, _P, _I64, _I32, _P],
     "mga_soft_ce_workspace_floats": [_I32, _I32],
     "mga_soft_ce_fwd": [_P, _I64, _P, _I64, _I32, _I32, _I32, _P, _P, _P, _P],
+    "mga_soft_ce_loss": [_P, _I64, _P, _I64, _I32, _I32, _I32, _P, _P, _P, _P, _P],
     "mga_soft_ce_bwd": [_P, _I64, _P, _I64, _I32, _I32, _I32, _P, _P, _P, _I64, _P],
 }
 _RESTYPES = {"mga_last_error": ctypes.c_char_p, "mga_soft_ce_workspace_floats": ctypes.c_int64,

@@ -780,19 +780,34 @@ int check_soft_ce(const char *fn, const void *x, int64_t xs, const void *t, int6
   return rc;
 }
 
+int soft_ce_fwd(const char *fn, const void *student, int64_t student_row_stride, const void *teacher,
+                int64_t teacher_row_stride, int32_t n_rows, int32_t n_cols, int32_t dtype, float *row_loss,
+                float *stats, float *loss_sum, float *workspace, void *stream) {
+  bool vec = true;
+  int rc = check_soft_ce(fn, student, student_row_stride, teacher, teacher_row_stride, n_rows, n_cols,
+                         dtype, &vec);
+  if (rc != MGA_OK) return rc;
+  if (!row_loss || !stats || !workspace) return fail(MGA_ERR_INVALID, "%s: null output or workspace", fn);
+  mga::launch_soft_ce_fwd(student, student_row_stride, teacher, teacher_row_stride, n_rows, n_cols,
+                          dtype, vec, row_loss, stats, loss_sum, workspace, (hipStream_t)stream);
+  return check_launch(fn);
+}
+
 }  // namespace
 
 int mga_soft_ce_fwd(const void *student, int64_t student_row_stride, const void *teacher,
                     int64_t teacher_row_stride, int32_t n_rows, int32_t n_cols, int32_t dtype, float *row_loss,
                     float *stats, float *workspace, void *stream) {
-  bool vec = true;
-  int rc = check_soft_ce("mga_soft_ce_fwd", student, student_row_stride, teacher, teacher_row_stride, n_rows, n_cols,
-                         dtype, &vec);
-  if (rc != MGA_OK) return rc;
-  if (!row_loss || !stats || !workspace) return fail(MGA_ERR_INVALID, "mga_soft_ce_fwd: null output or workspace");
-  mga::launch_soft_ce_fwd(student, student_row_stride, teacher, teacher_row_stride, n_rows, n_cols,
-                          dtype, vec, row_loss, stats, workspace, (hipStream_t)stream);
-  return check_launch("mga_soft_ce_fwd");
+  return soft_ce_fwd("mga_soft_ce_fwd", student, student_row_stride, teacher, teacher_row_stride, n_rows, n_cols,
+                     dtype, row_loss, stats, nullptr, workspace, stream);
+}
+
+int mga_soft_ce_loss(const void *student, int64_t student_row_stride, const void *teacher,
+                     int64_t teacher_row_stride, int32_t n_rows, int32_t n_cols, int32_t dtype, float *row_loss,
+                     float *stats, float *loss_sum, float *workspace, void *stream) {
+  if (!loss_sum) return fail(MGA_ERR_INVALID, "mga_soft_ce_loss: null loss_sum");
+  return soft_ce_fwd("mga_soft_ce_loss", student, student_row_stride, teacher, teacher_row_stride, n_rows, n_cols,
+                     dtype, row_loss, stats, loss_sum, workspace, stream);
 }
 
 int mga_soft_ce_bwd(const void *student, int64_t student_row_stride, const void *teacher,

@@ -168,7 +168,7 @@ void launch_lora_gen_dx_mask(int dtype, void *dx, int64_t dx_rs, int32_t S, int3
 // in elements; vec: 16-byte vector loads (every row start 16-byte aligned).
 int64_t soft_ce_workspace_floats(int32_t n_rows, int32_t n_cols);
 void launch_soft_ce_fwd(const void *x, int64_t xs, const void *t, int64_t ts, int32_t N, int32_t V, int dtype,
-                        bool vec, float *loss, float *stats, float *ws, hipStream_t stream);
+                        bool vec, float *loss, float *stats, float *sum, float *ws, hipStream_t stream);
 void launch_soft_ce_bwd(const void *x, int64_t xs, const void *t, int64_t ts, int32_t N, int32_t V, int dtype,
                         bool vec, const float *grad_out, const float *stats, void *g, int64_t gs,
                         hipStream_t stream);

@@ -7,8 +7,9 @@
 //       range of x and t keeps the online statistics of both rows at once,
 //       (mx, dx) of x and (mt, dt, S = sum e^{t - mt} x) of t, and writes
 //       them per split;
-//   soft_ce_combine_kernel  - one thread per row merges the splits in a fixed
-//       order and writes ce = -S / dt + mx + log dx and (mx, dx, mt, dt).
+//   soft_ce_combine_kernel  - one workgroup merges the splits of each row in
+//       a fixed order, writes ce = -S / dt + mx + log dx and (mx, dx, mt, dt),
+//       and sums the row losses.
 // The reference reads x twice (an x pass, then a fused t + x pass,
 // mtp_glora/core/loss.py:63-124); here both rows are read once.
 // Backward: grad_x = go * (e^{x - mx} / dx - e^{t - mt} / dt), written in the
@@ -53,7 +54,8 @@ struct Stats {
       s *= sc;
       mt = gt;
     }
-    const float mxl = mx * kL2E, mtl = mt * kL2E;
+    // nothing but -inf so far: exponents of -inf, not of -inf + inf
+    const float mxl = mx == kNegInf ? 0.f : mx * kL2E, mtl = mt == kNegInf ? 0.f : mt * kL2E;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       dx += ex2(__builtin_fmaf(x[i], kL2E, -mxl));
@@ -93,10 +95,13 @@ struct Stats {
 template <typename T>
 struct Vec {   // bf16 and fp16
   static constexpr int W = 8;
-  __device__ __forceinline__ static void load(const T *p, float (&v)[W]) {
-    const auto a = __builtin_bit_cast(typename Elem<T>::v8, load8(p));
+  __device__ __forceinline__ static void unpack(const i32x4 &r, float *v) {
+    const auto a = __builtin_bit_cast(typename Elem<T>::v8, r);
 #pragma unroll
     for (int i = 0; i < W; ++i) v[i] = (float)a[i];
+  }
+  __device__ __forceinline__ static void load(const T *p, float (&v)[W]) {
+    unpack(*reinterpret_cast<const i32x4 *>(p), v);
   }
   __device__ __forceinline__ static void store(T *p, const float (&v)[W]) {
     typename Elem<T>::v8 a;
@@ -108,10 +113,13 @@ struct Vec {   // bf16 and fp16
 template <>
 struct Vec<float> {
   static constexpr int W = 4;
-  __device__ __forceinline__ static void load(const float *p, float (&v)[W]) {
-    const f32x4 a = *reinterpret_cast<const f32x4 *>(p);
+  __device__ __forceinline__ static void unpack(const i32x4 &r, float *v) {
+    const f32x4 a = __builtin_bit_cast(f32x4, r);
 #pragma unroll
     for (int i = 0; i < W; ++i) v[i] = a[i];
+  }
+  __device__ __forceinline__ static void load(const float *p, float (&v)[W]) {
+    unpack(*reinterpret_cast<const i32x4 *>(p), v);
   }
   __device__ __forceinline__ static void store(float *p, const float (&v)[W]) {
     f32x4 a = {v[0], v[1], v[2], v[3]};
@@ -135,12 +143,34 @@ __global__ __launch_bounds__(kThreads) void soft_ce_partial_kernel(const T *__re
   Stats st;
   int cs = c0;   // first column left for the element loop
   if constexpr (VEC) {
+    // two vectors of x and of t per turn, the next turn's loads issued before
+    // this turn's arithmetic (about 75 cycles of VALU work per wave and pair
+    // against the streams' 100): [52, 151936] 11.0 -> 9.4 us, level at 1 024
+    // rows, where the streams alone bound it (5.4 TB/s by itself, 4.5 TB/s
+    // behind a backward whose gradient is still being written back)
     constexpr int W = Vec<T>::W;
     const int nvec = (c1 - c0) / W;
-    for (int i = tid; i < nvec; i += kThreads) {
+    const int nturn = nvec / (2 * kThreads);
+    const i32x4 *xp = reinterpret_cast<const i32x4 *>(xr + c0) + tid;
+    const i32x4 *tp = reinterpret_cast<const i32x4 *>(tr + c0) + tid;
+    if (nturn > 0) {
+      i32x4 xa = xp[0], ta = tp[0], xb = xp[kThreads], tb = tp[kThreads];
+      for (int i = 1; i <= nturn; ++i) {
+        const int n = min(i, nturn - 1) * 2 * kThreads;   // the last turn reads its own vectors again
+        const i32x4 xc = xp[n], tc = tp[n], xd = xp[n + kThreads], td = tp[n + kThreads];
+        float xv[2 * W], tv[2 * W];
+        Vec<T>::unpack(xa, xv);
+        Vec<T>::unpack(ta, tv);
+        Vec<T>::unpack(xb, xv + W);
+        Vec<T>::unpack(tb, tv + W);
+        st.add(xv, tv);
+        xa = xc; ta = tc; xb = xd; tb = td;
+      }
+    }
+    for (int i = nturn * 2 * kThreads + tid; i < nvec; i += kThreads) {
       float xv[W], tv[W];
-      Vec<T>::load(xr + c0 + i * W, xv);
-      Vec<T>::load(tr + c0 + i * W, tv);
+      Vec<T>::unpack(xp[i - tid], xv);
+      Vec<T>::unpack(tp[i - tid], tv);
       st.add(xv, tv);
     }
     cs = c0 + nvec * W;
@@ -183,28 +213,53 @@ __global__ __launch_bounds__(kThreads) void soft_ce_partial_kernel(const T *__re
   }
 }
 
-__global__ __launch_bounds__(kThreads) void soft_ce_combine_kernel(const float *__restrict__ part, int32_t N,
-                                                                 int32_t nsplit, float *__restrict__ loss,
-                                                                 float *__restrict__ stats) {
-  const int row = blockIdx.x * kThreads + threadIdx.x;
-  if (row >= N) return;
-  Stats acc;
-  for (int sp = 0; sp < nsplit; ++sp) {
-    const float *p = part + ((int64_t)row * nsplit + sp) * 5;
-    Stats o;
-    o.mx = p[0];
-    o.dx = p[1];
-    o.mt = p[2];
-    o.dt = p[3];
-    o.s = p[4];
-    acc.merge(o);
+// One workgroup: tpr (a power of two) neighbouring lanes take a row's splits and
+// merge them in a fixed order, then the row losses are summed, in a fixed
+// order, into *sum (unless null). Latency-bound (at most a few hundred KB): the
+// splits' loads of a row run side by side, 10.8 us for one thread a row at 52
+// rows of 19 splits against 5.2 us, and the separate sum's launch is gone.
+__global__ __launch_bounds__(1024) void soft_ce_combine_kernel(const float *__restrict__ part, int32_t N,
+                                                               int32_t nsplit, int32_t tpr,
+                                                               float *__restrict__ loss, float *__restrict__ stats,
+                                                               float *__restrict__ sum) {
+  const int tid = threadIdx.x, j = tid & (tpr - 1);
+  float total = 0.f;
+  for (int r0 = 0; r0 < N; r0 += 1024 / tpr) {
+    const int row = r0 + tid / tpr;
+    Stats acc;
+    if (row < N)
+      for (int sp = j; sp < nsplit; sp += tpr) {
+        const float *p = part + ((int64_t)row * nsplit + sp) * 5;
+        Stats o;
+        o.mx = p[0];
+        o.dx = p[1];
+        o.mt = p[2];
+        o.dt = p[3];
+        o.s = p[4];
+        acc.merge(o);
+      }
+    for (int m = tpr >> 1; m >= 1; m >>= 1) acc.merge(acc.shfl_xor(m));
+    if (row < N && j == 0) {
+      const float dx = fmaxf(acc.dx, kClamp), dt = fmaxf(acc.dt, kClamp);
+      const float ce = -(acc.s / dt) + acc.mx + logf(dx);
+      total += ce;
+      loss[row] = ce;
+      stats[row] = acc.mx;
+      stats[N + row] = dx;
+      stats[2 * N + row] = acc.mt;
+      stats[3 * N + row] = dt;
+    }
   }
-  const float dx = fmaxf(acc.dx, kClamp), dt = fmaxf(acc.dt, kClamp);
-  loss[row] = -(acc.s / dt) + acc.mx + logf(dx);
-  stats[row] = acc.mx;
-  stats[N + row] = dx;
-  stats[2 * N + row] = acc.mt;
-  stats[3 * N + row] = dt;
+  if (!sum) return;
+  for (int m = 32; m >= 1; m >>= 1) total += __shfl_xor(total, m, 64);
+  __shared__ float wsum[16];
+  if ((tid & 63) == 0) wsum[tid >> 6] = total;
+  __syncthreads();
+  if (tid < 64) {
+    float v = tid < 16 ? wsum[tid] : 0.f;
+    for (int m = 8; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
+    if (tid == 0) *sum = v;
+  }
 }
 
 template <typename T, bool VEC>
@@ -266,7 +321,7 @@ int64_t soft_ce_workspace_floats(int32_t N, int32_t V) {
 
 template <typename T>
 static void fwd_typed(const void *x, int64_t xs, const void *t, int64_t ts, int32_t N, int32_t V, bool vec,
-                      float *loss, float *stats, float *ws, hipStream_t st) {
+                      float *loss, float *stats, float *sum, float *ws, hipStream_t st) {
   int32_t ns, ch;
   soft_ce_plan(N, V, &ns, &ch);
   const dim3 grid((unsigned)((int64_t)N * ns));
@@ -276,8 +331,9 @@ static void fwd_typed(const void *x, int64_t xs, const void *t, int64_t ts, int3
   else
     hipLaunchKernelGGL((soft_ce_partial_kernel<T, false>), grid, dim3(kThreads), 0, st, (const T *)x, xs,
                        (const T *)t, ts, V, ch, ns, ws);
-  hipLaunchKernelGGL(soft_ce_combine_kernel, dim3((N + kThreads - 1) / kThreads), dim3(kThreads), 0, st, ws, N,
-                     ns, loss, stats);
+  int tpr = 1;
+  while (tpr < ns && tpr < 64) tpr *= 2;
+  hipLaunchKernelGGL(soft_ce_combine_kernel, dim3(1), dim3(1024), 0, st, ws, N, ns, tpr, loss, stats, sum);
 }
 
 template <typename T>
@@ -295,10 +351,10 @@ static void bwd_typed(const void *x, int64_t xs, const void *t, int64_t ts, int3
 }
 
 void launch_soft_ce_fwd(const void *x, int64_t xs, const void *t, int64_t ts, int32_t N, int32_t V, int dtype,
-                        bool vec, float *loss, float *stats, float *ws, hipStream_t st) {
-  if (dtype == kDtF32) fwd_typed<float>(x, xs, t, ts, N, V, vec, loss, stats, ws, st);
-  else if (dtype == kDtF16) fwd_typed<f16_t>(x, xs, t, ts, N, V, vec, loss, stats, ws, st);
-  else fwd_typed<bf16_t>(x, xs, t, ts, N, V, vec, loss, stats, ws, st);
+                        bool vec, float *loss, float *stats, float *sum, float *ws, hipStream_t st) {
+  if (dtype == kDtF32) fwd_typed<float>(x, xs, t, ts, N, V, vec, loss, stats, sum, ws, st);
+  else if (dtype == kDtF16) fwd_typed<f16_t>(x, xs, t, ts, N, V, vec, loss, stats, sum, ws, st);
+  else fwd_typed<bf16_t>(x, xs, t, ts, N, V, vec, loss, stats, sum, ws, st);
 }
 
 void launch_soft_ce_bwd(const void *x, int64_t xs, const void *t, int64_t ts, int32_t N, int32_t V, int dtype,

@@ -35,8 +35,8 @@ def _row_view(name: str, t: torch.Tensor, rows: int, cols: int):
     return v
 
 
-def soft_ce_forward(student: torch.Tensor, teacher: torch.Tensor):
-    """Row losses [B*T] and the saved statistics [4, B*T] (mx, dx, mt, dt)."""
+def _forward(student: torch.Tensor, teacher: torch.Tensor):
+    """Row losses [B*T], their sum and the saved statistics [4, B*T]."""
     if student.shape != teacher.shape:
         raise ValueError(f"student {tuple(student.shape)} and teacher {tuple(teacher.shape)} differ")
     if student.dtype != teacher.dtype:
@@ -49,8 +49,15 @@ def soft_ce_forward(student: torch.Tensor, teacher: torch.Tensor):
     loss = torch.empty(N, device=dev, dtype=torch.float32)
     stats = torch.empty(4, N, device=dev, dtype=torch.float32)
     ws = torch.empty(int(_lib.load().mga_soft_ce_workspace_floats(N, V)), device=dev, dtype=torch.float32)
-    _lib.call("mga_soft_ce_fwd", x.data_ptr(), x.stride(0), t.data_ptr(), t.stride(0), N, V,
-              dtype_code(x.dtype), loss.data_ptr(), stats.data_ptr(), ws.data_ptr(), _stream(x))
+    total = torch.empty((), device=dev, dtype=torch.float32)
+    _lib.call("mga_soft_ce_loss", x.data_ptr(), x.stride(0), t.data_ptr(), t.stride(0), N, V,
+              dtype_code(x.dtype), loss.data_ptr(), stats.data_ptr(), total.data_ptr(), ws.data_ptr(), _stream(x))
+    return loss, total, stats
+
+
+def soft_ce_forward(student: torch.Tensor, teacher: torch.Tensor):
+    """Row losses [B*T] and the saved statistics [4, B*T] (mx, dx, mt, dt)."""
+    loss, _, stats = _forward(student, teacher)
     return loss, stats
 
 
@@ -75,9 +82,9 @@ class StableSoftCrossEntropy(torch.autograd.Function):
     def forward(ctx, student_logits: torch.Tensor, teacher_logits: torch.Tensor):
         if student_logits.ndim != 3 or teacher_logits.ndim != 3:
             raise ValueError("student and teacher logits must be [B, T, V]")
-        loss, stats = soft_ce_forward(student_logits.detach(), teacher_logits.detach())
+        _, total, stats = _forward(student_logits.detach(), teacher_logits.detach())
         ctx.save_for_backward(student_logits.detach(), teacher_logits.detach(), stats)
-        return loss.sum()
+        return total
 
     @staticmethod
     def backward(ctx, grad_output):

@@ -122,3 +122,24 @@ def test_argument_errors(mga, dev):
         mga.StableSoftCrossEntropy.apply(x, x.bfloat16())
     with pytest.raises(RuntimeError):
         mga.StableSoftCrossEntropy.apply(x.cpu(), x.cpu())
+
+
+@pytest.mark.parametrize("rows,V,dtype", [(1, 600008, torch.bfloat16),    # more splits than lanes of a wave
+                                          (52, 151936, torch.bfloat16), (3, 8191, torch.float32),
+                                          (1025, 4104, torch.float16),    # a row past the workgroup's first pass
+                                          (7, 2049, torch.bfloat16)])
+def test_splits_and_row_sum(mga, dev, rows, V, dtype):
+    """Row splits and the row sum at the edges of their loops, against float64
+    on the GPU: fp32 sums of V terms, so 1e-5 relative; a leading run of
+    masked (-inf) student logits longer than a thread's first vectors."""
+    from importlib import import_module
+    lossmod = import_module("mtp-glora_amd.loss")
+    g = torch.Generator(device=dev).manual_seed(V)
+    x = (torch.randn(1, rows, V, generator=g, device=dev) * 3).to(dtype)
+    t = (torch.randn(1, rows, V, generator=g, device=dev) * 3).to(dtype)
+    t[:, :, :2000] = float("-inf")
+    want = -(torch.softmax(t.double(), -1) * torch.log_softmax(x.double(), -1)).sum(-1)[0]
+    loss, _ = lossmod.soft_ce_forward(x, t)
+    assert bool(((loss.double() - want).abs() <= 1e-5 * want.abs()).all())
+    total = mga.StableSoftCrossEntropy.apply(x, t)
+    assert total.shape == () and abs(float(total) - float(want.sum())) <= 1e-5 * float(want.sum())
