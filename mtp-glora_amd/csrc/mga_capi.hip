@@ -464,13 +464,13 @@ struct LoraWs {
 //  (bf16) | split-K partial sums of the down-projection: 8 x S x 96 fp32 |
 //  lora_A in MFMA-operand order, up to 96 ranks at a time: K / 16 x 3 KB |
 //  split partial sums of grad_A: 16 x rpad x K fp32 | split partial sums of
-//  lora_B's backward products: 8 x max(S, N) x rpad fp32]
+//  lora_B's backward products]
 int64_t lora_ws_bytes(int32_t S, int32_t K, int32_t N, int32_t rank) {
   const int64_t rp = lora_rpad(rank);
   return kBlasWorkspace + 2 * align256((int64_t)S * rp * 4) + align256((int64_t)K * rp * 2) +
          align256((int64_t)8 * S * 96 * 4) + align256((int64_t)K / 16 * 3 * 1024) +
          align256((int64_t)mga::kDaMaxSplit * rp * K * 4) +
-         align256((int64_t)mga::kSkinnyMaxSplit * std::max(S, N) * rp * 4);
+         align256(mga::lora_skinny_part_floats(S, N, (int32_t)rp) * 4);
 }
 
 LoraWs lora_ws(void *ws, int32_t S, int32_t K, int32_t rank) {
@@ -704,26 +704,23 @@ int mga_gated_lora_bwd(const void *grad_y, int64_t gy_rs, const void *x, int64_t
   // u = dY B, d_a = T(T(T(u) gate) s) (the gradient at lora_A's output), and
   // dB = dY^T t: one streaming pass over dY each (ranks up to 128, 16-byte
   // rows), else hipBLASLt
+  constexpr int64_t kMaxStride = int64_t(1) << 23;   // 32-bit lane offsets over 64 rows
   const bool skinny = rank <= 128 && N % 8 == 0 && aligned16(grad_y) && gy_rs % 8 == 0 && aligned16(lora_b) &&
-                      b_rs % 8 == 0 && aligned16(t) && t_rs % 8 == 0;
-  mga::LoraSkinnyArgs sk = {};
-  sk.dy = grad_y; sk.dy_rs = gy_rs; sk.part = w.skpart; sk.S = S; sk.N = N; sk.rank = rank; sk.rp = (int32_t)rp;
+                      b_rs % 8 == 0 && aligned16(t) && t_rs % 8 == 0 && gy_rs < kMaxStride && b_rs < kMaxStride &&
+                      t_rs < kMaxStride;
   if (skinny) {
-    sk.sm = lora_b; sk.sm_rs = b_rs;
-    mga::launch_lora_grad_u(sk, gate, scaling, w.da, rp, st);
+    mga::LoraSkinnyArgs sk = {};
+    sk.dy = grad_y; sk.dy_rs = gy_rs; sk.t = t; sk.t_rs = t_rs; sk.b = lora_b; sk.b_rs = b_rs;
+    sk.S = S; sk.N = N; sk.rank = rank; sk.rp = (int32_t)rp;
+    mga::launch_lora_grad_ub(sk, w.skpart, gate, scaling, w.da, rp, grad_b, gb_rs, st);
     if ((rc = check_launch(fn)) != MGA_OK) return rc;
   } else {
     if ((rc = blas(fn, false, false, S, rank, N, grad_y, gy_rs, lora_b, b_rs, false, w.u, rp, w, st)) != MGA_OK)
       return rc;
     mga::launch_lora_scale_rows(w.u, rp, gate, scaling, S, rank, (int32_t)rp, w.da, rp, st);
     if ((rc = check_launch(fn)) != MGA_OK) return rc;
-  }
-  if (grad_b && skinny) {
-    sk.sm = t; sk.sm_rs = t_rs;
-    mga::launch_lora_grad_b(sk, grad_b, gb_rs, st);
-    if ((rc = check_launch(fn)) != MGA_OK) return rc;
-  } else if (grad_b && (rc = blas(fn, true, false, N, rank, S, grad_y, gy_rs, t, t_rs, false, grad_b, gb_rs, w, st))) {
-    return rc;
+    if (grad_b && (rc = blas(fn, true, false, N, rank, S, grad_y, gy_rs, t, t_rs, false, grad_b, gb_rs, w, st)))
+      return rc;
   }
   if (grad_x) {
     // the LoRA path's gradient first (through dropout when it is on), then

@@ -131,18 +131,20 @@ struct LoraDaArgs {
 };
 constexpr int kDaMaxSplit = 16;
 // lora_B's backward products over the streamed dY (mga_lora.hip): dB = dY^T t
-// (small = t [S, >= rank]) and u = dY B (small = lora_B [N, rank]); rank <= 128,
-// rows 16-byte aligned with strides a multiple of 8, N a multiple of 8.
+// and d_a = T(T(T(dY B) * gate) * scaling); rank <= 128, rows 16-byte aligned
+// with strides a multiple of 8 below 2^23, N a multiple of 8.
 struct LoraSkinnyArgs {
   const void *dy; int64_t dy_rs;       // [S, N] bf16
-  const void *sm; int64_t sm_rs;       // t or lora_B
-  float *part;                         // split partial sums [nsplit, lines, rp] fp32
-  int32_t S, N, rank, rp;
+  const void *t; int64_t t_rs;         // [S, >= rank] bf16
+  const void *b; int64_t b_rs;         // lora_B [N, rank] bf16
+  float *part_u, *part_b;              // split partial sums [nsu, S, rp] and [nsb, N, rp] fp32
+  int32_t S, N, rank, rp, nsu, nsb;
 };
-constexpr int kSkinnyMaxSplit = 8;
-void launch_lora_grad_b(const LoraSkinnyArgs &a, void *db, int64_t db_rs, hipStream_t stream);
-void launch_lora_grad_u(const LoraSkinnyArgs &a, const float *gate, float scaling, void *da, int64_t da_rs,
-                        hipStream_t stream);
+constexpr int kSkinnyMaxSplit = 16;
+int64_t lora_skinny_part_floats(int32_t S, int32_t N, int32_t rp);
+// db null: d_a only
+void launch_lora_grad_ub(LoraSkinnyArgs a, float *part, const float *gate, float scaling, void *da, int64_t da_rs,
+                         void *db, int64_t db_rs, hipStream_t stream);
 void launch_lora_down(const LoraDownArgs &a, hipStream_t stream);
 void launch_lora_da(const LoraDaArgs &a, hipStream_t stream);
 void launch_lora_dx(const LoraDxArgs &a, hipStream_t stream);

@@ -35,9 +35,9 @@
 //   8-byte-aligned rows: one row per lane, the output's columns along the
 //   lane's registers.
 // * lora_skinny_kernel: lora_B's backward products u = dY B and dB = dY^T t,
-//   each one streaming pass over dY (the rank-r side staged beside it), fp32
-//   split sums added in a fixed order by lora_u_finish_kernel (which also
-//   forms d_a = T(T(T(u) * gate) * s)) and lora_db_finish_kernel.
+//   each one streaming pass over dY (the rank-r side staged beside it) in one
+//   launch, fp32 split sums added in a fixed order by
+//   lora_skinny_finish_kernel (which also forms d_a = T(T(T(u) * gate) * s)).
 // * lora_scale_rows_kernel: d_a = T(T(u * gate) * s), u = dY B, when u comes
 //   from hipBLASLt (ranks above 128, unaligned rows).
 // * lora_transpose_kernel: A^T padded to a multiple of 32 ranks (the dX
@@ -699,103 +699,93 @@ __global__ __launch_bounds__(256) void lora_transpose_kernel(const bf16_t *A, in
 // ---- lora_B's backward: the two skinny products over the streamed dY -------
 // MODE 0: dB^T partials   part[split][n][r] = sum over the split's rows s of dY[s][n] t[s][r]
 // MODE 1: u^T partials    part[split][s][r] = sum over the split's columns n of dY[s][n] B[n][r]
-// HBM-bound on dY (each element read once per product). A workgroup of 4
-// waves owns 64 output lines (columns n for MODE 0, rows s for MODE 1) and a
-// share of the 64-wide chunks of the reduced dimension. Each chunk stages a
-// 64 x 64 dY tile (rows s, columns n, swizzled) and the chunk's 64 rows of the
-// small matrix (t for MODE 0, B for MODE 1) as compact rows of RP = 32 RB
-// elements, in a ring of four named buffers (three chunks ahead) filled with
-// direct loads. Every wave issues the same loads per chunk, and every load in
-// flight is a direct load, so the waits name exact counts. Wave w takes
-// k-step w (16 of the 64) of every chunk for all (rank block, line block)
-// outputs:
+// One launch runs both (the u workgroups first). A workgroup of 8 waves owns
+// 128 output lines (columns n for MODE 0, rows s for MODE 1) and a share of
+// the 64-wide chunks of the reduced dimension. Each chunk stages two 64 x 64
+// dY tiles (rows s, columns n, swizzled), one per 64 lines, and the chunk's 64
+// rows of the small matrix (t for MODE 0, B for MODE 1) as compact rows of
+// RP = 32 RB elements, in a ring of four stages filled up to four chunks ahead
+// by direct loads. Wave w takes k-step w % 4 (16 of the 64) of every chunk for
+// its 64 lines (half w / 4) and all ranks:
 //   MODE 0: dB^T[r][n] += t^T[r][s] dY[s][n]      A: t^T, B: dY  (transposed LDS reads)
 //   MODE 1: u^T[r][s]  += B^T[r][n] dY^T[n][s]    A: B^T (transposed read), B: dY rows (8-byte reads)
 // so a lane holds one output line and 16 ranks of each rank block, written
 // as 16-byte runs. The waves' sums are added in a fixed order at the end.
-// Rank columns past the rank and lines past the end hold junk that no
-// finishing kernel reads; reduced-dimension entries past the end are zeroed
-// in an operand. CLAMP (S or N not a multiple of 64) clamps each lane's rows
-// and columns at the edges; without it every address is a wave-uniform base
-// plus a loop-invariant lane offset, which also keeps the compiler from
-// waiting on loads in flight whose address registers a later read would reuse.
-template <int MODE, int RB, bool CLAMP>
-__device__ __forceinline__ void lora_skinny_body(const LoraSkinnyArgs &a) {
+// Bound by the workgroup's start and end (about 6 us: first loads, final sums)
+// and 0.45 us a chunk, 0.65 us once all CUs stream (dY from HBM, the small
+// matrix from L2), so the splits give every CU one long workgroup where they
+// can. 128 lines a workgroup bring 1.75 bytes into LDS per byte of dY at rank
+// 96 (64 lines: 2.5). At [5120, 6144] x rank 96 38 us, and 5.4 us to finish both
+// (one launch per product with 64 lines: 28.7 + 5.4 and 25.6 + 6.2 us); at
+// [1387, 4096] x rank 32 8.2 + 4.7 us (6.7 + 4.8 and 6.6 + 4.8 us).
+// The loads are inline asm through buffer resources (the caller of the wait
+// counts them: 2 dY loads a wave and chunk, and the small matrix's 4 RB loads
+// dealt to the 8 waves); rows past the end arrive as zeros, dY columns past N as
+// other elements of dY, which are zeroed in the operand where they are reduced
+// over and stay in lines that nothing reads otherwise. Rank columns past the
+// rank hold junk that the finishing kernel does not read.
+template <int MODE, int RB>
+__device__ __forceinline__ void lora_skinny_body(const LoraSkinnyArgs &a, int blk, int split, int nsplit, bf16_t *lds) {
   constexpr int RP = 32 * RB;                 // compact small-tile row (elements)
-  constexpr int YT = 64 * 64, MT = 64 * RP;
+  constexpr int YT = 64 * 64, MT = 64 * RP, STAGE = 2 * YT + MT;
   constexpr int MG = RP / 8;                  // granules per small-tile row
-  constexpr int MI = 64 * MG / 256;           // small-tile loads per thread (1 .. 4)
-  constexpr int NL = 2 + MI;                  // loads per thread per chunk
-  __shared__ __attribute__((aligned(16))) bf16_t sY0[YT], sY1[YT], sY2[YT], sY3[YT];
-  __shared__ __attribute__((aligned(16))) bf16_t sM0[MT], sM1[MT], sM2[MT], sM3[MT];
-  const int w = wave_id(), tid = threadIdx.x, lane = tid & 63;
+  constexpr int MIA = (RB + 1) / 2, MIB = RB / 2;   // small-tile loads of waves 0-3, of waves 4-7
+  const int w = wave_id(), lane = threadIdx.x & 63;
+  const int kq = w & 3, half = w >> 2;
   const int l32 = lane & 31, hi = lane >> 5;
-  const int line0 = blockIdx.x * 64;
+  const int line0 = blk * 128 + 64 * half;    // the wave's first line
   const int nlines = MODE == 0 ? a.N : a.S;   // output lines
   const int kdim = MODE == 0 ? a.S : a.N;     // reduced dimension
   const int nall = (kdim + 63) / 64;
-  const int c0 = (int)((int64_t)nall * blockIdx.y / gridDim.y);
-  const int nch = (int)((int64_t)nall * (blockIdx.y + 1) / gridDim.y) - c0;
+  const int c0 = (int)((int64_t)nall * split / nsplit);
+  const int nch = (int)((int64_t)nall * (split + 1) / nsplit) - c0;
   const bf16_t *dy = reinterpret_cast<const bf16_t *>(a.dy);
-  const bf16_t *sm = reinterpret_cast<const bf16_t *>(a.sm);
-  // granules of a small-matrix row that hold rank columns (a slot past them
-  // reads the last one again: its columns are never used)
-  const int mg_last = (a.rank + 7) / 8 - 1;
+  const bf16_t *sm = reinterpret_cast<const bf16_t *>(MODE == 0 ? a.t : a.b);
+  const int64_t sm_rs = MODE == 0 ? a.t_rs : a.b_rs;
+  const int mcols = (a.rank + 7) / 8 * 8;
 
-  // Per-lane sources. dY tile: 8 granules per row, 8 rows per load, wave w
-  // loads rows 16 w .. 16 w + 15 (two loads). Small tile: MG granules per row,
-  // load i of thread t fills slot 256 i + t (row slot / MG, granule slot % MG).
-  const int yp = lane & 7, yr = lane >> 3;
-  int mrow[MI], mgr[MI];
-#pragma unroll
-  for (int i = 0; i < MI; ++i) {
-    const int slot = 256 * i + tid;
-    mrow[i] = slot / MG;
-    mgr[i] = min(slot % MG, mg_last);
-  }
-  // full chunks: a wave-uniform base plus these 32-bit lane offsets (bytes)
-  uint32_t yo[2], mo[MI];
+  // Per-lane byte offsets. dY tile: 8 granules per row, 8 rows per load, wave
+  // kq of the half loads rows 16 kq .. 16 kq + 15 (two loads). Small tile: load
+  // i of wave w fills slots 64 (w + 8 i) + lane (row slot / MG, granule slot %
+  // MG; a granule past the rank reads the last one again).
+  uint32_t yo[2], mo[MIA];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const int r = 16 * w + 8 * i + yr;
-    yo[i] = opaque_u32((uint32_t)((r * a.dy_rs + 8 * (yp ^ swz<64>(r))) * 2));
+    const int r = 16 * kq + 8 * i + (lane >> 3);
+    yo[i] = opaque_u32((uint32_t)(r * a.dy_rs * 2) + (uint32_t)(16 * ((lane & 7) ^ swz<64>(r))));
   }
 #pragma unroll
-  for (int i = 0; i < MI; ++i) mo[i] = opaque_u32((uint32_t)((mrow[i] * a.sm_rs + 8 * mgr[i]) * 2));
+  for (int i = 0; i < MIA; ++i) {
+    const int slot = 64 * (w + 8 * i) + lane;
+    mo[i] = opaque_u32((uint32_t)((slot / MG) * sm_rs * 2) + (uint32_t)(16 * min(slot % MG, mcols / 8 - 1)));
+  }
   // Workgroups start their share at different chunks (rotated by the line
-  // block), so that the many workgroups streaming the same share at the same
-  // time do not all read the same rows of the small matrix at once.
-  const int rot = blockIdx.x % nch;
+  // block), so that those streaming the same share at the same time do not all
+  // read the same rows of the small matrix at once.
+  const int rot = blk % max(nch, 1);
   auto chunk_of = [&](int c) { const int r = c + rot; return c0 + (r >= nch ? r - nch : r); };
-  auto issue = [&](int c, bf16_t *tY, bf16_t *tM) {
-    const int cc = chunk_of(min(c, nch - 1));   // past the share: the share's last chunk again
-    const int k0 = cc * 64;
-    const int yrow0 = MODE == 0 ? k0 : line0, ycol0 = MODE == 0 ? line0 : k0;
-    bf16_t *dY = tY + 16 * w * 64;
-    if (!CLAMP || (yrow0 + 64 <= a.S && ycol0 + 64 <= a.N)) {
-      const char *b = reinterpret_cast<const char *>(dy + (int64_t)yrow0 * a.dy_rs + ycol0);
+  auto issue = [&](int c, bf16_t *st) {
+    const int k0 = chunk_of(min(c, nch - 1)) * 64;   // past the share: its last chunk again
+    const int r0 = MODE == 0 ? k0 : line0, n0 = MODE == 0 ? line0 : k0;
+    // resource ranges end with the last element of the tile's last existing row
+    const int64_t yb = (int64_t)(min(64, a.S - r0) - 1) * a.dy_rs + a.N - n0;
+    const i32x4 ry = buf_rsrc(dy + (r0 < a.S ? (int64_t)r0 * a.dy_rs + n0 : 0), r0 < a.S && yb > 0 ? (uint32_t)(yb * 2) : 0u);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) __builtin_amdgcn_global_load_lds(b + yo[i], (lds_void *)(dY + 8 * i * 64), 16, 0, 0);
-    } else {   // rows past S repeat the last row, columns past N the last granule
+    for (int i = 0; i < 2; ++i) bdma16(ry, yo[i], st + half * YT + (16 * kq + 8 * i) * 64);
+    const int64_t mb = (int64_t)(min(64, kdim - k0) - 1) * sm_rs + mcols;
+    const i32x4 rm = buf_rsrc(sm + (int64_t)k0 * sm_rs, (uint32_t)(mb * 2));
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int r = 16 * w + 8 * i + yr;
-        const int g = yp ^ swz<64>(r);
-        const int srow = min(yrow0 + r, a.S - 1), ncol = min(ycol0 + 8 * g, a.N - 8);
-        __builtin_amdgcn_global_load_lds(dy + (int64_t)srow * a.dy_rs + ncol, (lds_void *)(dY + 8 * i * 64), 16, 0, 0);
-      }
-    }
-    if (!CLAMP || k0 + 64 <= kdim) {
-      const char *b = reinterpret_cast<const char *>(sm + (int64_t)k0 * a.sm_rs);
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-        __builtin_amdgcn_global_load_lds(b + mo[i], (lds_void *)(tM + 2048 * i + 512 * w), 16, 0, 0);
-    } else {
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-        __builtin_amdgcn_global_load_lds(sm + (int64_t)min(k0 + mrow[i], kdim - 1) * a.sm_rs + 8 * mgr[i],
-                                         (lds_void *)(tM + 2048 * i + 512 * w), 16, 0, 0);
-    }
+    for (int i = 0; i < MIA; ++i)
+      if (i < MIB || w < 4) bdma16(rm, mo[i], st + 2 * YT + 512 * (w + 8 * i));
+  };
+  // the loads of the three (two) newest chunks stay in flight
+  auto wait3 = [&]() {
+    if (MIA == MIB || w < 4) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * (2 + MIA)) : "memory");
+    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * (2 + MIB)) : "memory");
+  };
+  auto wait2 = [&]() {
+    if (MIA == MIB || w < 4) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (2 + MIA)) : "memory");
+    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (2 + MIB)) : "memory");
   };
 
   // A operand from a compact k-major tile (rows k, RP columns): lane (l32, hi)
@@ -803,12 +793,12 @@ __device__ __forceinline__ void lora_skinny_body(const LoraSkinnyArgs &a) {
   // (the k order of TrLane), by two transposed reads
   const int ti = lane & 15;
   const uint32_t mro[2] = {
-      opaque_u32((uint32_t)(((4 * hi + (ti >> 2)) * RP + 16 * ((lane >> 4) & 1) + 4 * (ti & 3)) * 2)),
-      opaque_u32((uint32_t)(((8 + 4 * hi + (ti >> 2)) * RP + 16 * ((lane >> 4) & 1) + 4 * (ti & 3)) * 2))};
-  auto m_operand = [&](const bf16_t *tM, int k0, int rb) {
-    const char *b = reinterpret_cast<const char *>(tM) + (k0 * RP + 32 * rb) * 2;
-    return join8(lds_tr4(reinterpret_cast<const bf16_t *>(b + mro[0])),
-                 lds_tr4(reinterpret_cast<const bf16_t *>(b + mro[1])));
+      opaque_u32((uint32_t)(((16 * kq + 4 * hi + (ti >> 2)) * RP + 16 * ((lane >> 4) & 1) + 4 * (ti & 3)) * 2)),
+      opaque_u32((uint32_t)(((16 * kq + 8 + 4 * hi + (ti >> 2)) * RP + 16 * ((lane >> 4) & 1) + 4 * (ti & 3)) * 2))};
+  auto m_operand = [&](const bf16_t *tM, int rb) {
+    const char *p = reinterpret_cast<const char *>(tM) + 64 * rb;
+    return join8(lds_tr4(reinterpret_cast<const bf16_t *>(p + mro[0])),
+                 lds_tr4(reinterpret_cast<const bf16_t *>(p + mro[1])));
   };
   TrOffsets<64> try_;
   try_.init(lane);
@@ -816,142 +806,137 @@ __device__ __forceinline__ void lora_skinny_body(const LoraSkinnyArgs &a) {
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) acc[rb][0] = acc[rb][1] = zero16();
 
-  auto compute = [&](int c, const bf16_t *tY, const bf16_t *tM) {
-    const int kb = chunk_of(c) * 64 + 16 * w;        // first reduced index of this wave's k-step
-    const bool tail = CLAMP && kb + 16 > kdim;
-    bf16x8 av[RB], bv[2];
+  auto operands = [&](int c, const bf16_t *st, bf16x8 (&av)[RB], bf16x8 (&bv)[2]) {
+    const bf16_t *tY = st + half * YT, *tM = st + 2 * YT;
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) av[rb] = m_operand(tM, 16 * w, rb);
+    for (int rb = 0; rb < RB; ++rb) av[rb] = m_operand(tM, rb);
     if (MODE == 0) {
 #pragma unroll
-      for (int nb = 0; nb < 2; ++nb) bv[nb] = try_.operand(tY, 16 * w, nb);
+      for (int nb = 0; nb < 2; ++nb) bv[nb] = try_.operand(tY, 16 * kq, nb);
     } else {
-      // dY row 32 sb + l32, columns 16 w + 4 hi + 0..3 and 16 w + 8 + 4 hi + 0..3
+      // dY row 32 sb + l32, columns 16 kq + 4 hi + 0..3 and 16 kq + 8 + 4 hi + 0..3
 #pragma unroll
       for (int sb = 0; sb < 2; ++sb) {
         const int r = 32 * sb + l32;
-        const i32x2 x = *reinterpret_cast<const i32x2 *>(tY + tile_off<64>(r, 2 * w) + 4 * hi);
-        const i32x2 y = *reinterpret_cast<const i32x2 *>(tY + tile_off<64>(r, 2 * w + 1) + 4 * hi);
-        const i32x4 v = {x[0], x[1], y[0], y[1]};
-        bv[sb] = __builtin_bit_cast(bf16x8, v);
+        bv[sb] = lds_read4x2(tY + tile_off<64>(r, 2 * kq) + 4 * hi, tY + tile_off<64>(r, 2 * kq + 1) + 4 * hi);
       }
-    }
-    if (tail) {   // reduced entries kb + 4 hi + e and kb + 8 + 4 hi + e past the end are zeroed
+      const int kb = chunk_of(c) * 64 + 16 * kq;
+      if (kb + 16 > kdim) {   // columns kb + 4 hi + e and kb + 8 + 4 hi + e past N
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const bool out = kb + 4 * hi + (e & 3) + 8 * (e >> 2) >= kdim;
-        if (MODE == 0) {
-#pragma unroll
-          for (int rb = 0; rb < RB; ++rb) av[rb][e] = out ? (bf16_t)0.f : av[rb][e];
-        } else {
+        for (int e = 0; e < 8; ++e) {
+          const bool out = kb + 4 * hi + (e & 3) + 8 * (e >> 2) >= kdim;
 #pragma unroll
           for (int sb = 0; sb < 2; ++sb) bv[sb][e] = out ? (bf16_t)0.f : bv[sb][e];
         }
       }
     }
+  };
+
+  // chunk c: its operands were read in the turn before, so its stage is free
+  // behind a barrier. This wave's loads of chunk c + 1 landed, then a barrier
+  // behind this wave's LDS reads (every wave's part of c + 1 is in, and every
+  // wave has read c), the loads of chunk c + 4 into c's stage, the operand reads
+  // of c + 1, and the products of c under them.
+  bf16x8 av[2][RB], bv[2][2];
+  if (nch > 0) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) issue(q, lds + q * STAGE);
+    wait3();
+    lds_barrier();
+    operands(0, lds, av[0], bv[0]);
+    for (int cb = 0; cb < nch; cb += 4)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (cb + q < nch) {
+          if (cb + q + 1 < nch) {
+            wait2();
+            lds_barrier();
+            issue(cb + q + 4, lds + q * STAGE);
+            operands(cb + q + 1, lds + ((q + 1) & 3) * STAGE, av[(q + 1) & 1], bv[(q + 1) & 1]);
+          }
+#pragma unroll
+          for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int lb = 0; lb < 2; ++lb) acc[rb][lb] = mfma32<bf16_t>(av[q & 1][rb], bv[q & 1][lb], acc[rb][lb]);
+        }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the ring's trailing loads
+  __syncthreads();
+
+  // fixed-order sum of the four k-step waves of each half through LDS, 32 lines
+  // at a time: every wave parks its accumulators, then wave kq adds the four
+  // waves' registers 4 kq .. 4 kq + 3 and writes them as this split's partial:
+  // lane = line 32 lb + l32, ranks 32 rb + 8 kq + 4 hi + 0..3
+  f32x4 *park = reinterpret_cast<f32x4 *>(lds) + half * (4 * RB * 4 * 64);
+  float *part = MODE == 0 ? a.part_b : a.part_u;
+#pragma unroll
+  for (int lb = 0; lb < 2; ++lb) {
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-      for (int lb = 0; lb < 2; ++lb) acc[rb][lb] = mfma32<bf16_t>(av[rb], bv[lb], acc[rb][lb]);
-  };
-
-  // chunk c: its loads landed (the next two chunks' loads may still be in
-  // flight), a barrier behind this wave's LDS reads (every wave's part is in,
-  // and the buffer of chunk c - 1 is free: the compiler sinks chunk c - 1's
-  // products, and with them the wait for their operand reads, past a bare
-  // s_barrier, and the loads of chunk c + 3 then overwrite operands not yet
-  // read), then the loads of chunk c + 3 and the products of chunk c
-  // (every iteration runs all four chunks, those past the share without
-  // products, so the loads in flight at the loop head are the same on every
-  // path and the compiler adds no wait of its own)
-  auto chunk = [&](auto bsel, int c) {
-    constexpr int B = decltype(bsel)::value;
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * NL));
-    lds_barrier();
-    issue(c + 3, B == 0 ? sY3 : (B == 1 ? sY0 : (B == 2 ? sY1 : sY2)),
-          B == 0 ? sM3 : (B == 1 ? sM0 : (B == 2 ? sM1 : sM2)));
-    if (c < nch)
-      compute(c, B == 0 ? sY0 : (B == 1 ? sY1 : (B == 2 ? sY2 : sY3)),
-              B == 0 ? sM0 : (B == 1 ? sM1 : (B == 2 ? sM2 : sM3)));
-  };
-  issue(0, sY0, sM0);
-  issue(1, sY1, sM1);
-  issue(2, sY2, sM2);
-  for (int c = 0; c < nch; c += 4) {
-    chunk(std::integral_constant<int, 0>{}, c);
-    chunk(std::integral_constant<int, 1>{}, c + 1);
-    chunk(std::integral_constant<int, 2>{}, c + 2);
-    chunk(std::integral_constant<int, 3>{}, c + 3);
-  }
-  __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));   // the ring's trailing loads
-  __syncthreads();
-
-  // fixed-order sum of the waves' accumulators through LDS (the ring's dY
-  // buffers, 3 x 16 x 64 floats), then this split's partial: lane = line
-  // 32 lb + l32, registers = ranks 32 rb + 8 (q / 4) + 4 hi + q % 4
-  float *park = reinterpret_cast<float *>(sY0);
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-    for (int lb = 0; lb < 2; ++lb) {
-      if (w > 0)
-#pragma unroll
-        for (int q = 0; q < 16; ++q) park[((w - 1) * 16 + q) * 64 + lane] = acc[rb][lb][q];
-      __syncthreads();
-      if (w == 0) {
-#pragma unroll
-        for (int v = 0; v < 3; ++v)
-#pragma unroll
-          for (int q = 0; q < 16; ++q) acc[rb][lb][q] += park[(v * 16 + q) * 64 + lane];
-        const int line = line0 + 32 * lb + l32;
-        if (line < nlines) {
-          float *out = a.part + ((int64_t)blockIdx.y * nlines + line) * a.rp + 32 * rb + 4 * hi;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const f32x4 v = {acc[rb][lb][4 * i], acc[rb][lb][4 * i + 1], acc[rb][lb][4 * i + 2],
-                             acc[rb][lb][4 * i + 3]};
-            *reinterpret_cast<f32x4 *>(out + 8 * i) = v;
-          }
-        }
+      for (int q = 0; q < 4; ++q) {
+        const f32x16 &c = acc[rb][lb];
+        park[((kq * RB + rb) * 4 + q) * 64 + lane] = f32x4{c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3]};
       }
-      __syncthreads();
+    __syncthreads();
+    const int line = line0 + 32 * lb + l32;
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+      f32x4 v = park[(rb * 4 + kq) * 64 + lane];
+#pragma unroll
+      for (int k = 1; k < 4; ++k) {
+        const f32x4 x = park[((k * RB + rb) * 4 + kq) * 64 + lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] += x[e];
+      }
+      if (line < nlines)
+        *reinterpret_cast<f32x4 *>(part + ((int64_t)split * nlines + line) * a.rp + 32 * rb + 8 * kq + 4 * hi) = v;
     }
+    __syncthreads();
+  }
 }
 
-template <int MODE, int RB>
-__global__ __launch_bounds__(256, 2) void lora_skinny_kernel(LoraSkinnyArgs a) {
-  lora_skinny_body<MODE, RB, false>(a);
-}
-template <int MODE, int RB>
-__global__ __launch_bounds__(256, 2) void lora_skinny_clamp_kernel(LoraSkinnyArgs a) {
-  lora_skinny_body<MODE, RB, true>(a);
-}
-
-// dB[n][r] = T(sum over the splits, in order), r < rank.
-__global__ __launch_bounds__(256) void lora_db_finish_kernel(LoraSkinnyArgs a, int nsplit, bf16_t *db, int64_t db_rs) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (int64_t)a.N * a.rank) return;
-  const int n = (int)(i / a.rank), r = (int)(i - (int64_t)n * a.rank);
-  float v = 0.f;
-  for (int y = 0; y < nsplit; ++y) v += a.part[((int64_t)y * a.N + n) * a.rp + r];
-  db[(int64_t)n * db_rs + r] = (bf16_t)v;
+template <int RB>
+__global__ __launch_bounds__(512, 1) void lora_skinny_kernel(LoraSkinnyArgs a) {
+  __shared__ __attribute__((aligned(16))) bf16_t lds[4 * (2 * 64 * 64 + 64 * 32 * RB)];
+  const int nbu = (a.S + 127) / 128, nbb = (a.N + 127) / 128;
+  const int i = blockIdx.x;
+  if (i < nbu * a.nsu) lora_skinny_body<1, RB>(a, i % nbu, i / nbu, a.nsu, lds);
+  else lora_skinny_body<0, RB>(a, (i - nbu * a.nsu) % nbb, (i - nbu * a.nsu) / nbb, a.nsb, lds);
 }
 
 // d_a[s][r] = T(T(T(u) * gate[s]) * scaling), u = the sum over the splits in
-// order; 0 for rank <= r < rpad. The roundings of the chain dY B (bf16), then
-// lora_scale_rows.
-__global__ __launch_bounds__(256) void lora_u_finish_kernel(LoraSkinnyArgs a, int nsplit, const float *gate,
-                                                            float scaling, bf16_t *da, int64_t da_rs) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (int64_t)a.S * a.rp) return;
-  const int s = (int)(i / a.rp), r = (int)(i - (int64_t)s * a.rp);
-  float v = 0.f;
-  if (r < a.rank) {
-    for (int y = 0; y < nsplit; ++y) v += a.part[((int64_t)y * a.S + s) * a.rp + r];
-    const float g = gate ? gate[s] : 1.f;
-    v = rnd(rnd(rnd(v) * g) * scaling);
+// order; 0 for rank <= r < rp (the roundings of the chain dY B (bf16), then
+// lora_scale_rows); dB[n][r] = T(sum over the splits, in order), r < rank
+// (nsb > 0). Four ranks a thread.
+__global__ __launch_bounds__(256) void lora_skinny_finish_kernel(LoraSkinnyArgs a, const float *gate, float scaling,
+                                                                 bf16_t *da, int64_t da_rs, bf16_t *db,
+                                                                 int64_t db_rs) {
+  const int64_t nu = (int64_t)a.S * (a.rp / 4), nb = a.nsb > 0 ? (int64_t)a.N * (a.rp / 4) : 0;
+  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const bool isb = i >= nu;
+  if (isb) i -= nu;
+  if (isb && i >= nb) return;
+  const int line = (int)(i / (a.rp / 4)), r = 4 * (int)(i - (int64_t)line * (a.rp / 4));
+  const int nlines = isb ? a.N : a.S, ns = isb ? a.nsb : a.nsu;
+  const float *p = (isb ? a.part_b : a.part_u) + (int64_t)line * a.rp + r;
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int y = 0; y < ns; ++y) {
+    const f32x4 x = *reinterpret_cast<const f32x4 *>(p + (int64_t)y * nlines * a.rp);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] += x[e];
   }
-  da[(int64_t)s * da_rs + r] = (bf16_t)v;
+  if (isb) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (r + e < a.rank) db[(int64_t)line * db_rs + r + e] = (bf16_t)v[e];
+    return;
+  }
+  const float g = gate ? gate[line] : 1.f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = r + e < a.rank ? rnd(rnd(rnd(v[e]) * g) * scaling) : 0.f;
+  store4(da + (int64_t)line * da_rs + r, v[0], v[1], v[2], v[3]);
 }
 
 namespace {
@@ -1140,54 +1125,53 @@ void launch_lora_gen_scale_rows(int dtype, const void *u, int64_t u_rs, const fl
                        u_rs, gate, scaling, (int32_t)gate_first, S, rank, rpad, reinterpret_cast<f16_t *>(out), out_rs);
 }
 
-namespace {
-
-// splits of the reduced dimension: about two workgroups per CU, at most
-// kSkinnyMaxSplit, at least one 64-wide chunk each
-int skinny_splits(int lines, int kdim) {
-  const int nblk = (lines + 63) / 64, nch = (kdim + 63) / 64;
-  const int want = (2 * 256 + nblk - 1) / nblk;
-  return std::max(1, std::min({want, kSkinnyMaxSplit, nch}));
-}
-
-template <int MODE>
-void launch_skinny(const LoraSkinnyArgs &a, int nsplit, hipStream_t st) {
-  const int lines = MODE == 0 ? a.N : a.S;
-  const dim3 grid((unsigned)((lines + 63) / 64), (unsigned)nsplit), blk(256);
-  if (a.S % 64 == 0 && a.N % 64 == 0) {
-    switch (a.rp / 32) {
-      case 1: hipLaunchKernelGGL((lora_skinny_kernel<MODE, 1>), grid, blk, 0, st, a); break;
-      case 2: hipLaunchKernelGGL((lora_skinny_kernel<MODE, 2>), grid, blk, 0, st, a); break;
-      case 3: hipLaunchKernelGGL((lora_skinny_kernel<MODE, 3>), grid, blk, 0, st, a); break;
-      default: hipLaunchKernelGGL((lora_skinny_kernel<MODE, 4>), grid, blk, 0, st, a); break;
-    }
-  } else {
-    switch (a.rp / 32) {
-      case 1: hipLaunchKernelGGL((lora_skinny_clamp_kernel<MODE, 1>), grid, blk, 0, st, a); break;
-      case 2: hipLaunchKernelGGL((lora_skinny_clamp_kernel<MODE, 2>), grid, blk, 0, st, a); break;
-      case 3: hipLaunchKernelGGL((lora_skinny_clamp_kernel<MODE, 3>), grid, blk, 0, st, a); break;
-      default: hipLaunchKernelGGL((lora_skinny_clamp_kernel<MODE, 4>), grid, blk, 0, st, a); break;
+// Splits of the reduced dimensions: rounds of one workgroup per CU with the
+// smallest number of chunks from the first to the last, kSkinnyStart chunks'
+// time going into a workgroup's first loads and final sums (7 to 14 measure
+// level).
+void lora_skinny_plan(int32_t S, int32_t N, bool with_b, int32_t *nsu, int32_t *nsb) {
+  constexpr int kSkinnyStart = 8;
+  const int cus = device_cu_count();
+  const int64_t nbu = (S + 127) / 128, nbb = (N + 127) / 128;
+  const int cu = (N + 63) / 64, cb = (S + 63) / 64;   // chunks of a whole u, of a whole dB line block
+  const int longest = with_b ? std::max(cu, cb) : cu;
+  int64_t best = INT64_MAX;
+  for (int len = 1; len <= longest; ++len) {
+    const int u = (cu + len - 1) / len, b = with_b ? (cb + len - 1) / len : 0;
+    if (u > kSkinnyMaxSplit || b > kSkinnyMaxSplit) continue;
+    const int64_t wgs = nbu * u + nbb * b;
+    const int64_t cost = ((wgs + cus - 1) / cus) * (len + kSkinnyStart);
+    if (cost < best) {
+      best = cost;
+      *nsu = u;
+      *nsb = b;
     }
   }
 }
 
-}  // namespace
-
-void launch_lora_grad_b(const LoraSkinnyArgs &a, void *db, int64_t db_rs, hipStream_t st) {
-  const int ns = skinny_splits(a.N, a.S);
-  launch_skinny<0>(a, ns, st);
-  const int64_t n = (int64_t)a.N * a.rank;
-  hipLaunchKernelGGL(lora_db_finish_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, ns,
-                     reinterpret_cast<bf16_t *>(db), db_rs);
+int64_t lora_skinny_part_floats(int32_t S, int32_t N, int32_t rp) {
+  int32_t nsu = 1, nsb = 1;
+  lora_skinny_plan(S, N, true, &nsu, &nsb);
+  int32_t nsu1 = 1, nsb1 = 0;
+  lora_skinny_plan(S, N, false, &nsu1, &nsb1);
+  return std::max((int64_t)nsu * S + (int64_t)nsb * N, (int64_t)nsu1 * S) * rp;
 }
 
-void launch_lora_grad_u(const LoraSkinnyArgs &a, const float *gate, float scaling, void *da, int64_t da_rs,
-                        hipStream_t st) {
-  const int ns = skinny_splits(a.S, a.N);
-  launch_skinny<1>(a, ns, st);
-  const int64_t n = (int64_t)a.S * a.rp;
-  hipLaunchKernelGGL(lora_u_finish_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, ns, gate, scaling,
-                     reinterpret_cast<bf16_t *>(da), da_rs);
+void launch_lora_grad_ub(LoraSkinnyArgs a, float *part, const float *gate, float scaling, void *da, int64_t da_rs,
+                         void *db, int64_t db_rs, hipStream_t st) {
+  lora_skinny_plan(a.S, a.N, db != nullptr, &a.nsu, &a.nsb);
+  a.part_u = part;
+  a.part_b = part + (int64_t)a.nsu * a.S * a.rp;
+  const unsigned nwg = (unsigned)((a.S + 127) / 128 * a.nsu + (a.N + 127) / 128 * a.nsb);
+  switch (a.rp / 32) {
+    case 1: hipLaunchKernelGGL(lora_skinny_kernel<1>, dim3(nwg), dim3(512), 0, st, a); break;
+    case 2: hipLaunchKernelGGL(lora_skinny_kernel<2>, dim3(nwg), dim3(512), 0, st, a); break;
+    case 3: hipLaunchKernelGGL(lora_skinny_kernel<3>, dim3(nwg), dim3(512), 0, st, a); break;
+    default: hipLaunchKernelGGL(lora_skinny_kernel<4>, dim3(nwg), dim3(512), 0, st, a); break;
+  }
+  const int64_t n = ((int64_t)a.S + (a.nsb > 0 ? a.N : 0)) * (a.rp / 4);
+  hipLaunchKernelGGL(lora_skinny_finish_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, gate, scaling,
+                     reinterpret_cast<bf16_t *>(da), da_rs, reinterpret_cast<bf16_t *>(db), db_rs);
 }
 
 }  // namespace mga
