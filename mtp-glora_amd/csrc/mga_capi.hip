@@ -447,6 +447,8 @@ int mga_qk_norm_rope_bwd(const void *q, int64_t q_ss, int64_t q_hs, const void *
 
 namespace {
 
+// the streaming kernels' 32-bit lane offsets over 64 rows (128 of lora_A)
+constexpr int64_t kMaxStreamStride = int64_t(1) << 23;
 constexpr int64_t kBlasWorkspace = int64_t(32) << 20;   // hipBLASLt workspace per call
 
 int64_t align256(int64_t b) { return (b + 255) & ~int64_t(255); }
@@ -455,22 +457,14 @@ int64_t lora_rpad(int32_t rank) { return (rank + 31) / 32 * 32; }
 struct LoraWs {
   void *blas, *u, *da, *at;
   float *part;
-  void *packed;
-  float *dapart;
-  float *skpart;
 };
 
 // [hipBLASLt workspace | u = dY B : S x rpad | d_a : S x rpad | A^T : K x rpad
-//  (bf16) | split-K partial sums of the down-projection: 8 x S x 96 fp32 |
-//  lora_A in MFMA-operand order, up to 96 ranks at a time: K / 16 x 3 KB |
-//  split partial sums of grad_A: 16 x rpad x K fp32 | split partial sums of
-//  lora_B's backward products]
+//  (bf16) | fp32 partial sums of the streaming products, one at a time]
 int64_t lora_ws_bytes(int32_t S, int32_t K, int32_t N, int32_t rank) {
   const int64_t rp = lora_rpad(rank);
   return kBlasWorkspace + 2 * align256((int64_t)S * rp * 4) + align256((int64_t)K * rp * 2) +
-         align256((int64_t)8 * S * 96 * 4) + align256((int64_t)K / 16 * 3 * 1024) +
-         align256((int64_t)mga::kDaMaxSplit * rp * K * 4) +
-         align256(mga::lora_skinny_part_floats(S, N, (int32_t)rp) * 4);
+         align256(mga::lora_part_floats(S, K, N, rank) * 4);
 }
 
 LoraWs lora_ws(void *ws, int32_t S, int32_t K, int32_t rank) {
@@ -482,10 +476,6 @@ LoraWs lora_ws(void *ws, int32_t S, int32_t K, int32_t rank) {
   w.da = static_cast<char *>(w.u) + align256((int64_t)S * rp * 4);
   w.at = static_cast<char *>(w.da) + align256((int64_t)S * rp * 4);
   w.part = reinterpret_cast<float *>(static_cast<char *>(w.at) + align256((int64_t)K * rp * 2));
-  w.packed = reinterpret_cast<char *>(w.part) + align256((int64_t)8 * S * 96 * 4);
-  w.dapart = reinterpret_cast<float *>(static_cast<char *>(w.packed) + align256((int64_t)K / 16 * 3 * 1024));
-  w.skpart = reinterpret_cast<float *>(reinterpret_cast<char *>(w.dapart) +
-                                       align256((int64_t)mga::kDaMaxSplit * rp * K * 4));
   return w;
 }
 
@@ -503,6 +493,8 @@ int check_vec_rows(const char *fn, const char *name, const void *ptr, int64_t rs
   if (!aligned16(ptr)) return fail(MGA_ERR_INVALID, "%s: %s is not 16-byte aligned", fn, name);
   if (rs < cols || rs % 8) return fail(MGA_ERR_INVALID, "%s: %s row stride %lld must be >= %lld and a multiple of 8",
                                        fn, name, (long long)rs, (long long)cols);
+  if (rs >= kMaxStreamStride)
+    return fail(MGA_ERR_INVALID, "%s: %s row stride %lld is too large (limit 2^23)", fn, name, (long long)rs);
   return MGA_OK;
 }
 
@@ -512,6 +504,9 @@ int check_rows_ld(const char *fn, const char *name, const void *ptr, int64_t rs,
                              (long long)cols);
   return MGA_OK;
 }
+
+// rows that 16-byte vectors can read or write
+bool rows16(const void *p, int64_t rs) { return aligned16(p) && rs % 8 == 0; }
 
 uint32_t drop_threshold(double p) { return (uint32_t)llround(p * 65536.0); }
 float keep_scale(double p) { return (float)(1.0 / (1.0 - p)); }
@@ -634,14 +629,21 @@ int mga_gated_lora_fwd(const void *x, int64_t x_rs, const void *weight, int64_t 
   mga::LoraDownArgs a = {};
   a.x = x; a.x_rs = x_rs; a.A = lora_a; a.a_rs = a_rs; a.gate = gate; a.scaling = scaling;
   a.keep_scale = keep_scale(dropout_p); a.thr = thr; a.seed = seed; a.h = thr && h ? h : nullptr; a.h_rs = h_rs;
-  a.t = t; a.t_rs = t_rs; a.part = w.part; a.packed = w.packed; a.S = S; a.K = K; a.rank = rank;
+  a.t = t; a.t_rs = t_rs; a.part = w.part; a.S = S; a.K = K; a.rank = rank;
   mga::launch_lora_down(a, st);
   if ((rc = check_launch(fn)) != MGA_OK) return rc;
   // y = T(t B^T), then y = T(x W^T + y): the base GEMM reads the LoRA term in
   // its epilogue (free in a compute-bound GEMM) instead of a second pass over y
-  if ((rc = blas(fn, false, true, S, N, rank, t, t_rs, lora_b, b_rs, false, y, y_rs, w, st)) != MGA_OK) return rc;
-  if ((rc = blas(fn, false, true, S, N, K, x, x_rs, weight, w_rs, true, y, y_rs, w, st)) != MGA_OK) return rc;
-  return MGA_OK;
+  if (rank <= 128 && N % 8 == 0 && rows16(y, y_rs) && rows16(t, t_rs) && rows16(lora_b, b_rs)) {
+    mga::LoraOuter o = {};
+    o.d = t; o.d_rs = t_rs; o.w = lora_b; o.w_rs = b_rs; o.out = y; o.out_rs = y_rs;
+    o.rows = S; o.cols = N; o.rank = rank;
+    mga::launch_lora_outer(o, true, st);
+    if ((rc = check_launch(fn)) != MGA_OK) return rc;
+  } else if ((rc = blas(fn, false, true, S, N, rank, t, t_rs, lora_b, b_rs, false, y, y_rs, w, st)) != MGA_OK) {
+    return rc;
+  }
+  return blas(fn, false, true, S, N, K, x, x_rs, weight, w_rs, true, y, y_rs, w, st);
 }
 
 int mga_gated_lora_bwd(const void *grad_y, int64_t gy_rs, const void *x, int64_t x_rs, const void *h, int64_t h_rs,
@@ -704,15 +706,13 @@ int mga_gated_lora_bwd(const void *grad_y, int64_t gy_rs, const void *x, int64_t
   // u = dY B, d_a = T(T(T(u) gate) s) (the gradient at lora_A's output), and
   // dB = dY^T t: one streaming pass over dY each (ranks up to 128, 16-byte
   // rows), else hipBLASLt
-  constexpr int64_t kMaxStride = int64_t(1) << 23;   // 32-bit lane offsets over 64 rows
-  const bool skinny = rank <= 128 && N % 8 == 0 && aligned16(grad_y) && gy_rs % 8 == 0 && aligned16(lora_b) &&
-                      b_rs % 8 == 0 && aligned16(t) && t_rs % 8 == 0 && gy_rs < kMaxStride && b_rs < kMaxStride &&
-                      t_rs < kMaxStride;
+  const bool skinny = rank <= 128 && N % 8 == 0 && rows16(grad_y, gy_rs) && rows16(lora_b, b_rs) && rows16(t, t_rs) &&
+                      gy_rs < kMaxStreamStride && b_rs < kMaxStreamStride && t_rs < kMaxStreamStride;
   if (skinny) {
     mga::LoraSkinnyArgs sk = {};
     sk.dy = grad_y; sk.dy_rs = gy_rs; sk.t = t; sk.t_rs = t_rs; sk.b = lora_b; sk.b_rs = b_rs;
-    sk.S = S; sk.N = N; sk.rank = rank; sk.rp = (int32_t)rp;
-    mga::launch_lora_grad_ub(sk, w.skpart, gate, scaling, w.da, rp, grad_b, gb_rs, st);
+    sk.S = S; sk.N = N; sk.rank = rank;
+    mga::launch_lora_grad_ub(sk, w.part, gate, scaling, w.da, rp, grad_b, gb_rs, st);
     if ((rc = check_launch(fn)) != MGA_OK) return rc;
   } else {
     if ((rc = blas(fn, false, false, S, rank, N, grad_y, gy_rs, lora_b, b_rs, false, w.u, rp, w, st)) != MGA_OK)
@@ -725,12 +725,18 @@ int mga_gated_lora_bwd(const void *grad_y, int64_t gy_rs, const void *x, int64_t
   if (grad_x) {
     // the LoRA path's gradient first (through dropout when it is on), then
     // dX = T(dY W + that): the base GEMM accumulates onto it in its epilogue
-    if (thr) {
+    if (rank <= 128 && rows16(grad_x, gx_rs) && rows16(lora_a, a_rs)) {
+      mga::LoraOuter o = {};
+      o.d = w.da; o.d_rs = rp; o.w = lora_a; o.w_rs = a_rs; o.out = grad_x; o.out_rs = gx_rs;
+      o.keep_scale = keep_scale(dropout_p); o.thr = thr; o.seed = seed; o.rows = S; o.cols = K; o.rank = rank;
+      mga::launch_lora_outer(o, false, st);
+      if ((rc = check_launch(fn)) != MGA_OK) return rc;
+    } else if (thr) {
       mga::launch_lora_transpose(lora_a, a_rs, rank, K, (int32_t)rp, w.at, rp, st);
       mga::LoraDxArgs d = {};
       d.da = w.da; d.da_rs = rp; d.At = w.at; d.at_rs = rp; d.dx = grad_x; d.dx_rs = gx_rs;
       d.keep_scale = keep_scale(dropout_p); d.thr = thr; d.seed = seed; d.S = S; d.K = K; d.rank = rank;
-      mga::launch_lora_dx(d, st);
+      mga::launch_lora_dx_rows(d, st);
       if ((rc = check_launch(fn)) != MGA_OK) return rc;
     } else if ((rc = blas(fn, false, false, S, K, rank, w.da, rp, lora_a, a_rs, false, grad_x, gx_rs, w, st))) {
       return rc;
@@ -741,7 +747,7 @@ int mga_gated_lora_bwd(const void *grad_y, int64_t gy_rs, const void *x, int64_t
   // dA = d_a^T dropout(x)
   if (da_from_x) {
     mga::LoraDaArgs d = {};
-    d.x = x; d.x_rs = x_rs; d.da = w.da; d.da_rs = rp; d.dA = grad_a; d.dA_rs = ga_rs; d.part = w.dapart;
+    d.x = x; d.x_rs = x_rs; d.da = w.da; d.da_rs = rp; d.dA = grad_a; d.dA_rs = ga_rs; d.part = w.part;
     d.keep_scale = keep_scale(dropout_p); d.thr = thr; d.seed = seed; d.S = S; d.K = K; d.rank = rank;
     mga::launch_lora_da(d, st);
     if ((rc = check_launch(fn)) != MGA_OK) return rc;

@@ -98,16 +98,15 @@ int gemm_bf16(bool ta, bool tb, int64_t M, int64_t N, int64_t K, const void *A, 
 
 // Gated LoRA kernels (mga_lora.hip).
 struct LoraDownArgs {
-  const void *x; int64_t x_rs;         // [S, K] bf16
+  const void *x; int64_t x_rs;         // [S, K] bf16, K a multiple of 16
   const void *A; int64_t a_rs;         // lora_A weight [rank, K]
   const float *gate;                   // [S] or null (= 1)
   float scaling, keep_scale;           // alpha / rank; 1 / (1 - p)
   uint32_t thr;                        // 16-bit drop threshold, 0 = no dropout
   uint64_t seed;
-  void *h; int64_t h_rs;               // dropout output [S, K] (thr > 0)
+  void *h; int64_t h_rs;               // dropout output [S, K] (thr > 0), or null
   void *t; int64_t t_rs;               // [S, rpad] bf16 out
-  float *part;                         // split-K partial sums: 8 x S x 96 fp32, or null (no split)
-  void *packed;                        // lora_A in MFMA-operand order: K / 16 x 3 blocks of 1 KB
+  float *part;                         // partial sums, lora_part_floats
   int32_t S, K, rank;
 };
 struct LoraDxArgs {
@@ -123,31 +122,55 @@ struct LoraDaArgs {
   const void *x; int64_t x_rs;         // [S, K] bf16, the layer input
   const void *da; int64_t da_rs;       // [S, rpad] bf16 gradient at lora_A's output (zero past the rank)
   void *dA; int64_t dA_rs;             // [rank, K] bf16 out
-  float *part;                         // split partial sums [nsplit, 32 ceil(rank / 32), K] fp32
+  float *part;                         // partial sums, lora_part_floats
   float keep_scale;
   uint32_t thr;                        // 16-bit drop threshold (> 0)
   uint64_t seed;
   int32_t S, K, rank;
 };
-constexpr int kDaMaxSplit = 16;
-// lora_B's backward products over the streamed dY (mga_lora.hip): dB = dY^T t
-// and d_a = T(T(T(dY B) * gate) * scaling); rank <= 128, rows 16-byte aligned
-// with strides a multiple of 8 below 2^23, N a multiple of 8.
+// lora_B's backward products over the streamed dY: dB = dY^T t and d_a =
+// T(T(T(dY B) * gate) * scaling); rank <= 128, N a multiple of 8.
 struct LoraSkinnyArgs {
   const void *dy; int64_t dy_rs;       // [S, N] bf16
   const void *t; int64_t t_rs;         // [S, >= rank] bf16
   const void *b; int64_t b_rs;         // lora_B [N, rank] bf16
-  float *part_u, *part_b;              // split partial sums [nsu, S, rp] and [nsb, N, rp] fp32
-  int32_t S, N, rank, rp, nsu, nsb;
+  int32_t S, N, rank;
 };
-constexpr int kSkinnyMaxSplit = 16;
-int64_t lora_skinny_part_floats(int32_t S, int32_t N, int32_t rp);
+// One rank-r product that streams a wide operand (see lora_stream_body). Rows
+// 16-byte aligned, strides a multiple of 8 elements below 2^23 (32-bit lane
+// offsets over 64 rows; lora_A's over 128 ranks).
+struct LoraStream {
+  const void *x; int64_t x_rs;         // [rows, cols] bf16
+  const void *sm; int64_t sm_rs;       // the small matrix, bf16
+  float *part;                         // partial sums of the ns splits, fp32
+  void *h; int64_t h_rs;               // dropout output, or null
+  float keep_scale;
+  uint32_t thr;
+  uint64_t seed;
+  int32_t rows, cols, rank, ns;
+};
+// fp32 words for the partial sums of any streaming product of a layer
+int64_t lora_part_floats(int32_t S, int32_t K, int32_t N, int32_t rank);
 // db null: d_a only
-void launch_lora_grad_ub(LoraSkinnyArgs a, float *part, const float *gate, float scaling, void *da, int64_t da_rs,
-                         void *db, int64_t db_rs, hipStream_t stream);
+void launch_lora_grad_ub(const LoraSkinnyArgs &a, float *part, const float *gate, float scaling, void *da,
+                         int64_t da_rs, void *db, int64_t db_rs, hipStream_t stream);
 void launch_lora_down(const LoraDownArgs &a, hipStream_t stream);
 void launch_lora_da(const LoraDaArgs &a, hipStream_t stream);
-void launch_lora_dx(const LoraDxArgs &a, hipStream_t stream);
+void launch_lora_dx_rows(const LoraDxArgs &a, hipStream_t stream);
+// out = T(d W), W = w^T (colmaj: w [cols, rank]) or w ([rank, cols]), with the
+// dropout's backward where thr > 0 (w [rank, cols] only). rank <= 128; d rows
+// zero-padded to a multiple of 32 ranks and 16-byte aligned; cols a multiple of
+// 8; w and out rows 16-byte aligned.
+struct LoraOuter {
+  const void *d; int64_t d_rs;         // [rows, rpad] bf16
+  const void *w; int64_t w_rs;
+  void *out; int64_t out_rs;           // [rows, cols] bf16
+  float keep_scale;
+  uint32_t thr;
+  uint64_t seed;
+  int32_t rows, cols, rank;
+};
+void launch_lora_outer(const LoraOuter &a, bool colmaj, hipStream_t stream);
 void launch_lora_scale_rows(const void *u, int64_t u_rs, const float *gate, float scaling, int32_t S,
                             int32_t rank, int32_t rpad, void *da, int64_t da_rs, hipStream_t stream);
 void launch_lora_transpose(const void *A, int64_t a_rs, int32_t rank, int32_t K, int32_t rpad, void *At,

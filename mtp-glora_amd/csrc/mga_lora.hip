@@ -3,45 +3,28 @@
 //
 //   out = base(x) + s * B(A(dropout(x))) * gate
 //
-// The plain GEMMs (x W^T, the rank-r up-projection accumulated into the
-// output, dY W, and d_a^T h when the forward kept h) go to hipBLASLt
+// The plain GEMMs (x W^T and dY W, accumulated onto the rank-r term, and d_a^T h
+// when the forward kept h) go to hipBLASLt
 // (mga_blas.hip). The kernels here fuse what a library GEMM cannot, or stream
 // what it runs far from the HBM bound:
 //
-// * the down-projection t = T(T(s * T(h A^T)) * gate) for every row, h =
-//   dropout(x) drawn on the fly (written out only on request: the backward's
-//   lora_da_kernel draws the same mask again from x).
-//   HBM-bound on x; v_mfma_f32_32x32x16_bf16 with 32 rows per workgroup.
-//   lora_down_ring_kernel (K a multiple of 128) streams 128-wide chunks of
-//   the x rows through a ring of four LDS buffers with direct loads (1 KB per
-//   instruction, three chunks ahead) and reads A's operands from a copy in
-//   MFMA-operand order (lora_pack_a_kernel: one contiguous 1 KB read per
-//   operand); it splits K over up to 8 workgroups per row block, whose fp32
-//   partial sums lora_down_finish_kernel adds in a fixed order.
-//   lora_down_kernel (other K) reads its operands straight from global
-//   memory, K split over 8 waves. Operand loads that give each lane its own
-//   row touch 32 cache lines per instruction; staging x through LDS and
-//   packing A is what makes the first kernel faster.
-// * lora_dx_kernel (dropout on): the LoRA path's input gradient
-//   L = T(mask * T(scale * T(d_a A))), written to dX; the base gradient dY W
-//   is then accumulated on top by hipBLASLt (beta = 1), so dX is written once
-//   here and read once inside that compute-bound GEMM. The rank-r product
-//   runs on MFMA. A workgroup covers 128 columns x 128 rows: the A^T tile of
-//   its columns is shared through LDS, d_a goes straight into MFMA operands,
-//   and each wave transposes its rounded 32 x 32 result blocks through a
-//   small LDS tile so that a lane owns 8 consecutive columns of a row: dX is
-//   written in 16-byte runs with one hash per element pair.
-//   lora_dx_rows_kernel serves K not a multiple of 128, ranks above 128 and
-//   8-byte-aligned rows: one row per lane, the output's columns along the
-//   lane's registers.
-// * lora_skinny_kernel: lora_B's backward products u = dY B and dB = dY^T t,
-//   each one streaming pass over dY (the rank-r side staged beside it) in one
-//   launch, fp32 split sums added in a fixed order by
-//   lora_skinny_finish_kernel (which also forms d_a = T(T(T(u) * gate) * s)).
+// * the products that stream a wide operand once (lora_stream_body): the
+//   down-projection t = T(T(s * T(h A^T)) * gate), h = dropout(x) drawn on the
+//   fly (written out only on request); lora_B's u = dY B and dB = dY^T t; and
+//   lora_A's dA = d_a^T h, which draws the same mask again from x. fp32 split
+//   sums are added in a fixed order by finishing kernels, which also form t and
+//   d_a = T(T(T(u) * gate) * s).
+// * lora_outer_kernel: the rank-r products that write a wide result once, the
+//   up-projection T(t B^T) and the LoRA path's input gradient
+//   L = T(mask * T(scale * T(d_a A))); the base product x W^T or dY W is then
+//   accumulated on top by hipBLASLt (beta = 1), so the result is written once
+//   here and read once inside that compute-bound GEMM. lora_dx_rows_kernel
+//   serves the gradient at ranks above 128, columns not a multiple of 8 and
+//   8-byte-aligned rows, one row per lane, from a transposed lora_A.
 // * lora_scale_rows_kernel: d_a = T(T(u * gate) * s), u = dY B, when u comes
 //   from hipBLASLt (ranks above 128, unaligned rows).
-// * lora_transpose_kernel: A^T padded to a multiple of 32 ranks (the dX
-//   kernel's MFMA operand wants rank-contiguous rows).
+// * lora_transpose_kernel: A^T padded to a multiple of 32 ranks (for
+//   lora_dx_rows_kernel, whose operand wants rank-contiguous rows).
 //
 // T rounds to bf16. With the scaling a power of two and gate values 0 / 1 (the
 // reference's alpha = 2 * rank and clamped gate mask), applying s and the gate
@@ -78,6 +61,27 @@ __device__ __forceinline__ uint32_t pair_bits(uint64_t seed, uint64_t pair) {
   return fmix32(fmix32((uint32_t)pair ^ (uint32_t)seed) ^ (uint32_t)(pair >> 32) ^ (uint32_t)(seed >> 32));
 }
 
+// Dropout of 8 consecutive elements, pair pj (a multiple of 4) the first:
+// kept elements times keep_scale, rounded to bf16, the others 0. thr > 0; the
+// compares are bits > thr - 1, on the low 16 bits and on the whole word, and
+// the four pairs share the upper word of pj: about 140 cycles of VALU work a
+// pair and wave, 64 of them the four quarter-rate multiplies.
+__device__ __forceinline__ bf16x8 drop8(bf16x8 v, uint64_t pj, uint64_t seed, uint32_t thr, float keep_scale) {
+  const uint32_t lo = (uint32_t)pj ^ (uint32_t)seed, hi = (uint32_t)(pj >> 32) ^ (uint32_t)(seed >> 32);
+  const uint16_t t_lo = (uint16_t)(thr - 1);
+  const uint32_t t_hi = ((thr - 1) << 16) | 0xffffu;
+  i32x4 r;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const uint32_t bits = fmix32(fmix32(lo ^ (uint32_t)e) ^ hi);
+    const float a = (uint16_t)bits > t_lo ? (float)v[2 * e] * keep_scale : 0.f;
+    const float b = bits > t_hi ? (float)v[2 * e + 1] * keep_scale : 0.f;
+    // asm: the compiler splits the pair into two conversions and a permute
+    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r[e]) : "v"(a), "v"(b));
+  }
+  return __builtin_bit_cast(bf16x8, r);
+}
+
 __device__ __forceinline__ float rnd(float v) { return (float)(bf16_t)v; }
 
 __device__ __forceinline__ bf16x8 zero8() {
@@ -87,394 +91,115 @@ __device__ __forceinline__ bf16x8 zero8() {
   return z;
 }
 
-// s_waitcnt immediate waiting for vmcnt <= n only (gfx9 encoding: vmcnt[3:0]
-// in bits 3:0, vmcnt[5:4] in bits 15:14; expcnt and lgkmcnt at their maxima)
-constexpr int vmcnt_imm(int n) { return (n & 0xf) | (0x7 << 4) | (0xf << 8) | ((n >> 4) << 14); }
-
-constexpr int kDownWaves = 8;
-constexpr int kDownMaxSplit = 8;   // split-K parts of the LDS down-projection (partials: 8 x S x 96 fp32)
-
 }  // namespace
 
-// Grid: ceil(S / 32) workgroups of 8 waves. Wave w takes the 16-wide k steps
-// w, w + 8, ... of the workgroup's 32 rows; NB = ranks / 32 accumulator blocks.
-// Loads are unconditional (rows past S and ranks past the rank read a clamped,
-// valid address; their sums land only in outputs that are dropped or zeroed)
-// and issued kU steps ahead of the MFMAs that use them.
-template <int NB, bool DROP>
-__global__ __launch_bounds__(kDownWaves * 64) void lora_down_kernel(LoraDownArgs a) {
-  constexpr int kU = NB >= 3 ? 4 : 8;
-  const int w = wave_id(), lane = threadIdx.x & 63;
-  const int s0 = blockIdx.x * 32;
-  const int row = s0 + (lane & 31);
-  const bool row_ok = row < a.S;
-  const int rowc = row_ok ? row : a.S - 1;
-  const int kq = 8 * (lane >> 5);
-  const bf16_t *xr = reinterpret_cast<const bf16_t *>(a.x) + (int64_t)rowc * a.x_rs + kq;
-  bf16_t *hr = (DROP && a.h) ? reinterpret_cast<bf16_t *>(a.h) + (int64_t)rowc * a.h_rs + kq : nullptr;
-  const bf16_t *ar[NB];
-#pragma unroll
-  for (int nb = 0; nb < NB; ++nb) {
-    const int r = nb * 32 + (lane & 31);
-    ar[nb] = reinterpret_cast<const bf16_t *>(a.A) + (int64_t)(r < a.rank ? r : a.rank - 1) * a.a_rs + kq;
-  }
-  f32x16 acc[NB];
-#pragma unroll
-  for (int nb = 0; nb < NB; ++nb) acc[nb] = zero16();
-  const uint64_t pair0 = ((uint64_t)rowc * (uint64_t)a.K + (uint64_t)kq) >> 1;
-  const int nsteps = (a.K / 16 - w + kDownWaves - 1) / kDownWaves;   // wave-uniform
-
-  // one k step: dropout on the x operand (h written out), then the MFMAs
-  auto consume = [&](bf16x8 &xv, const bf16x8 (&av)[NB], int step) {
-    if constexpr (DROP) {
-      const int k0 = 16 * (w + kDownWaves * step);
-      const uint64_t pj = pair0 + ((uint64_t)k0 >> 1);
-#pragma unroll
-      for (int e = 0; e < 8; e += 2) {
-        const uint32_t bits = pair_bits(a.seed, pj + (e >> 1));
-        const bool k_lo = (bits & 0xffffu) >= a.thr, k_hi = (bits >> 16) >= a.thr;
-        xv[e] = k_lo ? (bf16_t)((float)xv[e] * a.keep_scale) : (bf16_t)0.f;
-        xv[e + 1] = k_hi ? (bf16_t)((float)xv[e + 1] * a.keep_scale) : (bf16_t)0.f;
-      }
-      if (row_ok && hr) *reinterpret_cast<i32x4 *>(hr + k0) = __builtin_bit_cast(i32x4, xv);
-    }
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) acc[nb] = mfma32<bf16_t>(xv, av[nb], acc[nb]);
-  };
-  auto load_step = [&](bf16x8 &xv, bf16x8 (&av)[NB], int step) {
-    const int k0 = 16 * (w + kDownWaves * step);
-    xv = load8(xr + k0);
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) av[nb] = load8(ar[nb] + k0);
-  };
-
-  // full groups of kU steps: all loads of a group issued before its MFMAs,
-  // with no branch in between
-  const int nfull = nsteps / kU * kU;
-  for (int i = 0; i < nfull; i += kU) {
-    bf16x8 xv[kU], av[kU][NB];
-#pragma unroll
-    for (int u = 0; u < kU; ++u) load_step(xv[u], av[u], i + u);
-#pragma unroll
-    for (int u = 0; u < kU; ++u) consume(xv[u], av[u], i + u);
-  }
-  for (int i = nfull; i < nsteps; ++i) {
-    bf16x8 xv, av[NB];
-    load_step(xv, av, i);
-    consume(xv, av, i);
-  }
-
-  // fixed-order reduction of the 8 waves' partial sums: 4..7 into 0..3, then 1..3 into 0
-  __shared__ float red[4][NB][16][64];
-  if (w >= 4) {
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-      for (int q = 0; q < 16; ++q) red[w - 4][nb][q][lane] = acc[nb][q];
-  }
-  __syncthreads();
-  if (w < 4) {
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-      for (int q = 0; q < 16; ++q) acc[nb][q] += red[w][nb][q][lane];
-  }
-  __syncthreads();
-  if (w >= 1 && w < 4) {
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-      for (int q = 0; q < 16; ++q) red[w - 1][nb][q][lane] = acc[nb][q];
-  }
-  __syncthreads();
-  if (w != 0) return;
-#pragma unroll
-  for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-    for (int q = 0; q < 16; ++q) acc[nb][q] += red[0][nb][q][lane] + red[1][nb][q][lane] + red[2][nb][q][lane];
-
-  bf16_t *t = reinterpret_cast<bf16_t *>(a.t);
-#pragma unroll
-  for (int q = 0; q < 16; ++q) {
-    const int s = s0 + 8 * (q >> 2) + 4 * (lane >> 5) + (q & 3);
-    if (s >= a.S) continue;
-    const float g = a.gate ? a.gate[s] : 1.f;
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-      const int r = nb * 32 + (lane & 31);
-      // lora_A output in bf16, then the scaling and the gate, each rounded
-      const float v = r < a.rank ? rnd(rnd(acc[nb][q]) * a.scaling) * g : 0.f;
-      t[(int64_t)s * a.t_rs + r] = (bf16_t)v;
-    }
-  }
-}
-
-// lora_A in MFMA-operand order: 1 KB block (kstep, nb) = K/16 k-steps x NB
-// rank blocks, lane (l32, hi) holding A[32 nb + l32][16 kstep + 8 hi .. + 8]
-// (zero past the rank), so every operand load of the down-projection below is
-// one contiguous 1 KB wave read. One thread per 16-byte granule.
-__global__ __launch_bounds__(256) void lora_pack_a_kernel(const bf16_t *A, int64_t a_rs, int32_t rank, int32_t K,
-                                                          int32_t nb_n, i32x4 *pk) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (int64_t)(K / 16) * nb_n * 64) return;
-  const int lane = (int)(i & 63);
-  const int64_t blk = i >> 6;
-  const int nb = (int)(blk % nb_n);
-  const int64_t kstep = blk / nb_n;
-  const int r = nb * 32 + (lane & 31);
-  const int64_t k = kstep * 16 + 8 * (lane >> 5);
-  i32x4 v = {0, 0, 0, 0};
-  if (r < rank) v = *reinterpret_cast<const i32x4 *>(A + (int64_t)r * a_rs + k);
-  pk[i] = v;
-}
-
-// Down-projection for K a multiple of 128 with the x rows streamed through a
-// ring of four LDS buffers (direct loads, three 128-column chunks ahead) and
-// lora_A's operands read straight from the packed copy (L2-resident, one 1 KB
-// read per operand). Grid (ceil(S / 32), nsplit): a workgroup of 4 waves owns
-// 32 rows and a contiguous share of the chunks; wave w takes k-steps 2w, 2w+1
-// of every chunk, and the waves' sums are added in a fixed order at the end.
-// Every wave issues the same memory instructions in every iteration (a chunk
-// past the share reloads the share's last chunk into its free buffer; the
-// operand loads of a chunk past the share read the last one), so the waits
-// can name exact counts: the chunk's own loads, and its operands. vmcnt
-// retires loads in issue order but stores out of order with them, so when
-// the kernel also writes the dropout output it waits for everything instead.
-template <int NB, bool DROP, bool WRITE_H>
-__global__ __launch_bounds__(256) void lora_down_ring_kernel(LoraDownArgs a) {
-  constexpr int HD = 128, NRA = 32 * NB, RING = 4, TILE = 32 * HD;
-  // per-iteration vector-memory loads of a wave after its chunk loads: the
-  // next chunk's operands (2 NB)
-  constexpr int kOps = 2 * NB;
-  __shared__ __attribute__((aligned(16))) bf16_t sX[RING * TILE];
-  const int w = wave_id(), lane = threadIdx.x & 63;
-  const int l32 = lane & 31, hi = lane >> 5;
-  const int s0 = blockIdx.x * 32;
-  const int row = s0 + l32;
-  const bool row_ok = row < a.S;
-  const int nrows = a.S - s0 < 32 ? a.S - s0 : 32;
-  const bf16_t *xb = reinterpret_cast<const bf16_t *>(a.x) + (int64_t)s0 * a.x_rs;
-  const i32x4 *pk = reinterpret_cast<const i32x4 *>(a.packed);
-  DmaLane<HD, 32> dx;
-  dx.init();
-  const uint32_t lrx = dx.lane_row(a.x_rs);
-  const auto rowsx = dx.rows(a.x_rs);
-  const uint32_t orow = opaque_u32((uint32_t)(l32 * HD + (((uint32_t)hi ^ swz<HD>(l32)) << 3)) * 2u);
-  bf16_t *hr = WRITE_H ? reinterpret_cast<bf16_t *>(a.h) + (int64_t)(row_ok ? row : 0) * a.h_rs : nullptr;
-  const uint64_t prow = (uint64_t)(row_ok ? row : 0) * (uint64_t)a.K;
-  const int nall = a.K / HD;
-  const int cbeg = (int)((int64_t)nall * blockIdx.y / gridDim.y);
-  const int nchunks = (int)((int64_t)nall * (blockIdx.y + 1) / gridDim.y) - cbeg;
-
-  auto issue = [&](int c) {   // chunk c of the share into buffer c % RING (past the share: its last chunk)
-    const int col = (cbeg + min(c, nchunks - 1)) * HD;
-    bf16_t *tx = sX + (c % RING) * TILE;
-    if (nrows == 32) dx.issue(tx, xb + col, rowsx, lrx);
-    else dx.issue_clamped(tx, xb + col, a.x_rs, nrows);
-  };
-  auto load_ops = [&](int c, bf16x8 (&op)[2][NB]) {
-    const int64_t kstep0 = (int64_t)(cbeg + min(c, nchunks - 1)) * (HD / 16) + 2 * w;
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb)
-        op[j][nb] = __builtin_bit_cast(bf16x8, pk[((kstep0 + j) * NB + nb) * 64 + lane]);
-  };
-
-  f32x16 acc[NB];
-#pragma unroll
-  for (int nb = 0; nb < NB; ++nb) acc[nb] = zero16();
-  // operands of the current / next chunk in two named register sets that
-  // swap roles each iteration (the loop runs two chunks per trip)
-  bf16x8 opa[2][NB], opb[2][NB];
-  auto chunk = [&](int c, bf16x8 (&opc)[2][NB], bf16x8 (&opn)[2][NB]) {
-    // this wave's loads of chunk c have landed (the first iterations wait for
-    // everything). vmcnt counts in issue order only while no store is in
-    // flight, so with the dropout output written here the wait is a full one.
-    if (c >= RING - 1 && !WRITE_H) __builtin_amdgcn_s_waitcnt(vmcnt_imm(3 * kOps + 4));
-    else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-    // every wave's part of chunk c is in; chunk c - 1's buffer is free.
-    // __syncthreads' memory fence would make the compiler wait for every load
-    // in flight, the ring's included; the barrier waits for this wave's LDS
-    // reads of chunk c - 1, whose products the compiler may place after it.
-    lds_barrier();
-    issue(c + RING - 1);
-    // the operands of chunk c (issued before the two loads just above)
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(2));
-    const uint32_t ob = orow + (uint32_t)((c % RING) * TILE * 2);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int ks = 2 * w + j;
-      bf16x8 xv = lds_read8(reinterpret_cast<const bf16_t *>(lds_at(sX, ob ^ (uint32_t)(ks << 5))));
-      if constexpr (DROP) {
-        const int k0 = (cbeg + c) * HD + ks * 16 + 8 * hi;
-        const uint64_t pj = (prow + (uint64_t)k0) >> 1;
-#pragma unroll
-        for (int e = 0; e < 8; e += 2) {
-          const uint32_t bits = pair_bits(a.seed, pj + (e >> 1));
-          const bool k_lo = (bits & 0xffffu) >= a.thr, k_hi = (bits >> 16) >= a.thr;
-          xv[e] = k_lo ? (bf16_t)((float)xv[e] * a.keep_scale) : (bf16_t)0.f;
-          xv[e + 1] = k_hi ? (bf16_t)((float)xv[e + 1] * a.keep_scale) : (bf16_t)0.f;
-        }
-        // one store instruction per k-step (lanes of rows past S masked off;
-        // a wave always has a row below S, so the store is never skipped)
-        if constexpr (WRITE_H)
-          if (row_ok) *reinterpret_cast<i32x4 *>(hr + k0) = __builtin_bit_cast(i32x4, xv);
-      }
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb) acc[nb] = mfma32<bf16_t>(xv, opc[j][nb], acc[nb]);
-    }
-    load_ops(c + 1, opn);
-  };
-
-  issue(0);
-  issue(1);
-  issue(2);
-  load_ops(0, opa);
-  for (int c = 0; c < nchunks; c += 2) {
-    chunk(c, opa, opb);
-    if (c + 1 < nchunks) chunk(c + 1, opb, opa);
-  }
-  __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));   // the ring's trailing loads
-  __syncthreads();
-
-  // fixed-order reduction through the ring, one rank block at a time
-  float *park = reinterpret_cast<float *>(sX);
-#pragma unroll
-  for (int nb = 0; nb < NB; ++nb) {
-    if (w > 0)
-#pragma unroll
-      for (int q = 0; q < 16; ++q) park[((w - 1) * 16 + q) * 64 + lane] = acc[nb][q];
-    __syncthreads();
-    if (w == 0)
-#pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        const int o = q * 64 + lane;
-        acc[nb][q] += park[o] + park[16 * 64 + o] + park[32 * 64 + o];
-      }
-    __syncthreads();
-  }
-  if (w != 0) return;
-  if (gridDim.y > 1) {   // fp32 partial sums [split][S][32 NB]; lora_down_finish_kernel adds them
-    float *part = a.part + (int64_t)blockIdx.y * a.S * NRA;
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int s = s0 + 8 * (q >> 2) + 4 * hi + (q & 3);
-      if (s >= a.S) continue;
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb) part[(int64_t)s * NRA + nb * 32 + l32] = acc[nb][q];
-    }
-    return;
-  }
-  bf16_t *t = reinterpret_cast<bf16_t *>(a.t);
-#pragma unroll
-  for (int q = 0; q < 16; ++q) {
-    const int s = s0 + 8 * (q >> 2) + 4 * hi + (q & 3);
-    if (s >= a.S) continue;
-    const float g = a.gate ? a.gate[s] : 1.f;
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-      const int r = nb * 32 + l32;
-      const float v = r < a.rank ? rnd(rnd(acc[nb][q]) * a.scaling) * g : 0.f;
-      t[(int64_t)s * a.t_rs + r] = (bf16_t)v;
-    }
-  }
-}
-
-// t[s][r] = T(T(s * T(sum over the splits, in order)) * gate) from the partial
-// sums of the split-K down-projection (ranks nr = 32 NB of this launch).
-__global__ __launch_bounds__(256) void lora_down_finish_kernel(LoraDownArgs a, int nsplit, int nr) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (int64_t)a.S * nr) return;
-  const int s = (int)(i / nr), r = (int)(i - (int64_t)s * nr);
-  float v = 0.f;
-  for (int k = 0; k < nsplit; ++k) v += a.part[(int64_t)k * a.S * nr + i];
-  const float g = a.gate ? a.gate[s] : 1.f;
-  const float out = r < a.rank ? rnd(rnd(v) * a.scaling) * g : 0.f;
-  reinterpret_cast<bf16_t *>(a.t)[(int64_t)s * a.t_rs + r] = (bf16_t)out;
-}
-
-// Grid: (K / 128, ceil(S / 128)), 4 waves. The workgroup's 128 columns of
-// A^T (rank-padded rows) are copied once into LDS and shared; wave w computes
-// rows 32 w .. 32 w + 31 of the 128-row block, one 32 x 32 block at a time:
-// D[s][k] = sum_r d_a[s][r] A^T[k][r] (A operand: the lane's d_a row from
-// global memory; B operand: the A^T row of the lane's column, from LDS). The
-// rounded block T(D) goes through a per-wave LDS tile so that each lane then
-// owns 8 consecutive columns of one row: dX is written with 16-byte stores
-// and each dropout hash serves its element pair. NK = 16-rank steps of the
+// out[s][c] = T(sum_r d[s][r] W(r, c)) of the rank-padded rows d (t or d_a) and
+// a small weight, written once: the up-projection t B^T (W = lora_B [cols,
+// rank]: COLMAJ) and the LoRA term d_a A of dX (W = lora_A [rank, cols]), there
+// with the dropout's backward T(mask * T(.) / (1 - p)) applied (DROP). The base
+// product is accumulated on top by the compute-bound base GEMM.
+// Bound by the writes of out (and the hashes, 140 cycles a pair). A workgroup
+// of up to 10 waves takes 128 columns, its W tile shared through LDS (COLMAJ:
+// 128 rows of RP ranks, padded; else RP rows of 128 columns, swizzled, read
+// transposed, so no transposed copy of lora_A is needed), and 32 rows a wave,
+// two 32 x 32 blocks at a time; the rounded blocks go through a per-wave LDS
+// tile so that each lane then owns 8 consecutive columns of one row: 16-byte
+// stores (whole lines a wave), and each hash serves its element pair. The number of waves is chosen
+// so that the workgroups fill whole rounds of the CUs (outer_waves). In the
+// layer, at [5120, 6144] x rank 96, t B^T takes 17.7 us (hipBLASLt 25.6 us; a
+// plain write of as much 10.7 us), and the dropped d_a A of 4 096 columns 23 us
+// (20.4 + 5.1 us with a transposed copy of lora_A).
+// cols a multiple of 8, out rows 16-byte aligned, NK = 16-rank steps of the
 // padded rank (even).
-template <int NK>
-__global__ __launch_bounds__(256) void lora_dx_kernel(LoraDxArgs a) {
+constexpr int kOuterTs = 72;   // row stride of a wave's 32 x 64 result tile (144 bytes)
+constexpr int kOuterWaves = 10;
+template <int NK, bool COLMAJ>
+constexpr int kOuterTile = COLMAJ ? 128 * (NK * 16 + 8) : 128 * NK * 16;   // elements of the W tile
+
+template <int NK, bool COLMAJ, bool DROP>
+__global__ __launch_bounds__(64 * kOuterWaves) void lora_outer_kernel(LoraOuter a) {
   constexpr int RP = NK * 16;          // padded rank
-  constexpr int LS = RP + 8;           // LDS row stride of A^T (elements)
-  constexpr int TS = 40;               // row stride of a wave's 32 x 32 result tile (80 bytes)
-  __shared__ __attribute__((aligned(16))) bf16_t sAt[128 * LS];
-  __shared__ __attribute__((aligned(16))) bf16_t sT[4][32 * TS];
-  const int w = wave_id(), lane = threadIdx.x & 63, tid = threadIdx.x;
+  constexpr int LS = RP + 8;           // COLMAJ: LDS row stride of the W tile (elements)
+  extern __shared__ __attribute__((aligned(16))) bf16_t outer_lds[];
+  bf16_t *sW = outer_lds;
+  const int w = wave_id(), lane = threadIdx.x & 63, tid = threadIdx.x, nt = blockDim.x;
+  bf16_t *tile = outer_lds + kOuterTile<NK, COLMAJ> + w * 32 * kOuterTs;
   const int l32 = lane & 31, hi = lane >> 5;
-  const int kb0 = blockIdx.x * 128;
-  const int s0 = blockIdx.y * 128 + w * 32;
-  {
-    // every granule load issued before the first LDS write (one memory wait)
-    constexpr int kGran = RP / 8;      // 16-byte granules per row
-    constexpr int kPer = 128 * kGran / 256;
-    const bf16_t *src = reinterpret_cast<const bf16_t *>(a.At) + (int64_t)kb0 * a.at_rs;
-    i32x4 g16[kPer];
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-      const int i = tid + 256 * j, r = i / kGran, g = i - r * kGran;
-      g16[j] = *reinterpret_cast<const i32x4 *>(src + (int64_t)r * a.at_rs + g * 8);
-    }
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-      const int i = tid + 256 * j, r = i / kGran, g = i - r * kGran;
-      *reinterpret_cast<i32x4 *>(sAt + r * LS + g * 8) = g16[j];
-    }
-  }
-  const int srow = s0 + l32 < a.S ? s0 + l32 : a.S - 1;   // rows past S: computed, never stored
-  const bf16_t *dar = reinterpret_cast<const bf16_t *>(a.da) + (int64_t)srow * a.da_rs + 8 * hi;
+  const int c0 = blockIdx.x * 128;
+  const int s0 = (blockIdx.y * (nt >> 6) + w) * 32;
+  const bf16_t *wp = reinterpret_cast<const bf16_t *>(a.w);
+  const int srow = min(s0 + l32, a.rows - 1);   // rows past the end: computed, never stored
+  const bf16_t *dr = reinterpret_cast<const bf16_t *>(a.d) + (int64_t)srow * a.d_rs;
   bf16x8 dv[NK];
 #pragma unroll
-  for (int j = 0; j < NK; ++j) dv[j] = load8(dar + 16 * j);
-  // epilogue ownership: lane -> row er (+16 for the second half), columns ec .. ec + 7
-  const int er = lane >> 2, ec = (lane & 3) * 8;
-  bf16_t *dx = reinterpret_cast<bf16_t *>(a.dx);
-  bf16_t *tile = sT[w];
-  auto dx_at = [&](int r, int blk) {
-    const int s = s0 + r;
-    return dx + (int64_t)(s < a.S ? s : a.S - 1) * a.dx_rs + kb0 + blk * 32 + ec;
-  };
+  for (int j = 0; j < NK; ++j) {
+    if constexpr (COLMAJ) {
+      dv[j] = load8(dr + 16 * j + 8 * hi);
+    } else {   // the k order of the transposed reads
+      const i32x2 x = *reinterpret_cast<const i32x2 *>(dr + 16 * j + 4 * hi);
+      const i32x2 y = *reinterpret_cast<const i32x2 *>(dr + 16 * j + 8 + 4 * hi);
+      dv[j] = __builtin_bit_cast(bf16x8, i32x4{x[0], x[1], y[0], y[1]});
+    }
+  }
+  // the W tile, four granules a thread in flight: each batch's loads are issued
+  // before its first LDS write
+  constexpr int kGran = 16 * RP, kPerRow = COLMAJ ? RP / 8 : 16;   // granules, granules of a tile row
+  for (int i0 = 0; i0 < kGran; i0 += 4 * nt) {
+    bf16x8 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int i = i0 + u * nt + tid, r = i / kPerRow, g = i % kPerRow;
+      v[u] = zero8();
+      if (COLMAJ ? (i < kGran && c0 + r < a.cols && 8 * g < a.rank) : (r < a.rank && c0 + 8 * g < a.cols))
+        v[u] = load8(wp + (COLMAJ ? (int64_t)(c0 + r) * a.w_rs + 8 * g : (int64_t)r * a.w_rs + c0 + 8 * g));
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int i = i0 + u * nt + tid, r = i / kPerRow, g = i % kPerRow;
+      if (COLMAJ && 8 * g + 8 > a.rank)   // the elements past the rank belong to the next row
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (8 * g + e >= a.rank) v[u][e] = (bf16_t)0.f;
+      if (i < kGran)
+        *reinterpret_cast<i32x4 *>(sW + (COLMAJ ? r * LS + 8 * g : tile_off<128>(r, g))) = __builtin_bit_cast(i32x4, v[u]);
+    }
+  }
+  TrOffsets<128> tro;
+  if constexpr (!COLMAJ) tro.init(lane);
+  // epilogue ownership: lane -> rows er + 8 h, columns ec .. ec + 7 of a block
+  // pair: eight lanes write a row's whole 128-byte line
+  const int er = lane >> 3, ec = (lane & 7) * 8;
+  bf16_t *out = reinterpret_cast<bf16_t *>(a.out);
   __syncthreads();
+  if (s0 >= a.rows) return;
 #pragma unroll
-  for (int blk = 0; blk < 4; ++blk) {
-    f32x16 acc = zero16();
-    const bf16_t *brow = sAt + (blk * 32 + l32) * LS + 8 * hi;
+  for (int bp = 0; bp < 2; ++bp) {
 #pragma unroll
-    for (int j = 0; j < NK; ++j) acc = mfma32<bf16_t>(dv[j], lds_read8(brow + 16 * j), acc);
-    // d(dropout(x)) = T(d_a A): lane holds column l32 of rows 8 (q / 4) + 4 hi + q % 4
+    for (int bi = 0; bi < 2; ++bi) {
+      const int blk = 2 * bp + bi;
+      f32x16 acc = zero16();
 #pragma unroll
-    for (int q = 0; q < 16; ++q) tile[(8 * (q >> 2) + 4 * hi + (q & 3)) * TS + l32] = (bf16_t)acc[q];
+      for (int j = 0; j < NK; ++j) {
+        const bf16x8 wv = COLMAJ ? lds_read8(sW + (blk * 32 + l32) * LS + 16 * j + 8 * hi) : tro.operand(sW, 16 * j, blk);
+        acc = mfma32<bf16_t>(dv[j], wv, acc);
+      }
+      // lane holds column l32 of rows 8 (q / 4) + 4 hi + q % 4
+#pragma unroll
+      for (int q = 0; q < 16; ++q)
+        tile[(8 * (q >> 2) + 4 * hi + (q & 3)) * kOuterTs + 32 * bi + l32] = (bf16_t)acc[q];
+    }
     __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): this wave's tile writes done
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int r = er + 16 * h, s = s0 + r;
-      const bf16x8 dh = lds_read8(tile + r * TS + ec);
-      if (s < a.S) {
-        const int k = kb0 + blk * 32 + ec;
-        const uint64_t pj = ((uint64_t)s * (uint64_t)a.K + (uint64_t)k) >> 1;
-        bf16x8 o;
-#pragma unroll
-        for (int e = 0; e < 8; e += 2) {
-          const uint32_t bits = pair_bits(a.seed, pj + (e >> 1));
-          const bool k_lo = (bits & 0xffffu) >= a.thr, k_hi = (bits >> 16) >= a.thr;
-          o[e] = (bf16_t)(k_lo ? (float)dh[e] * a.keep_scale : 0.f);           // dropout backward
-          o[e + 1] = (bf16_t)(k_hi ? (float)dh[e + 1] * a.keep_scale : 0.f);
-        }
-        *reinterpret_cast<i32x4 *>(dx_at(r, blk)) = __builtin_bit_cast(i32x4, o);
+    for (int h = 0; h < 4; ++h) {
+      const int r = er + 8 * h, s = s0 + r, c = c0 + bp * 64 + ec;
+      bf16x8 v = lds_read8(tile + r * kOuterTs + ec);
+      if (s < a.rows && c < a.cols) {
+        if (DROP) v = drop8(v, ((uint64_t)s * (uint64_t)a.cols + (uint64_t)c) >> 1, a.seed, a.thr, a.keep_scale);
+        *reinterpret_cast<i32x4 *>(out + (int64_t)s * a.out_rs + c) = __builtin_bit_cast(i32x4, v);
       }
     }
-    __builtin_amdgcn_wave_barrier();   // the tile is rewritten by the next block
+    __builtin_amdgcn_wave_barrier();   // the tile is rewritten by the next pair
   }
 }
 
@@ -543,126 +268,6 @@ __global__ __launch_bounds__(256) void lora_dx_rows_kernel(LoraDxArgs a) {
   }
 }
 
-// grad_A = d_a^T dropout(x) with the dropout drawn again from x (so the
-// forward need not keep its dropout output): K a multiple of 128, ranks in
-// launches of up to 128. Grid (K / 128, nsplit): a workgroup owns 128
-// columns and a share of the rows, 32 at a time. Each step stages the rows'
-// dropout(x) (one hash per element pair, as in the forward) and their d_a
-// through registers into LDS (double-buffered), and wave w accumulates
-// D[r][k] = sum_s d_a[s][r] h[s][k] for its 32 columns and every rank block,
-// both MFMA operands read with the transposed LDS read (lane = r or k,
-// 8 consecutive rows s). Split partial sums go to fp32 [split][r][k] and
-// lora_da_finish_kernel adds them in a fixed order.
-template <int NB>
-__global__ __launch_bounds__(256) void lora_da_kernel(LoraDaArgs a, int r0) {
-  constexpr int HD = 128, TILE = 32 * HD;
-  __shared__ __attribute__((aligned(16))) bf16_t sX0[TILE], sX1[TILE], sD0[TILE], sD1[TILE];
-  const int w = wave_id(), tid = threadIdx.x, lane = tid & 63;
-  const int l32 = lane & 31, hi = lane >> 5;
-  const int kc0 = blockIdx.x * HD;
-  const int nst = (a.S + 31) / 32;
-  const int st0 = (int)((int64_t)nst * blockIdx.y / gridDim.y);
-  const int st1 = (int)((int64_t)nst * (blockIdx.y + 1) / gridDim.y);
-  const int rc = min(a.rank - r0, 32 * NB);   // ranks of this launch
-  const bf16_t *xb = reinterpret_cast<const bf16_t *>(a.x);
-  const bf16_t *db = reinterpret_cast<const bf16_t *>(a.da) + r0;
-  TrOffsets<HD> tro;
-  tro.init(lane);
-  // staged granules of one step: x 2 per thread, d_a NB / 2 per thread (rounded up)
-  constexpr int kDG = (32 * NB * 4 + 255) / 256;
-  i32x4 gx[2], gd[kDG];
-  auto load = [&](int st) {
-    const int s0 = st * 32;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int gi = tid + 256 * i, r = gi >> 4, g = gi & 15;
-      const int s = s0 + r;
-      const i32x4 v = *reinterpret_cast<const i32x4 *>(xb + (int64_t)min(s, a.S - 1) * a.x_rs + kc0 + 8 * g);
-      bf16x8 h = __builtin_bit_cast(bf16x8, v);
-      const uint64_t pj = ((uint64_t)min(s, a.S - 1) * (uint64_t)a.K + (uint64_t)(kc0 + 8 * g)) >> 1;
-#pragma unroll
-      for (int e = 0; e < 8; e += 2) {
-        const uint32_t bits = pair_bits(a.seed, pj + (e >> 1));
-        const bool k_lo = s < a.S && (bits & 0xffffu) >= a.thr, k_hi = s < a.S && (bits >> 16) >= a.thr;
-        h[e] = k_lo ? (bf16_t)((float)h[e] * a.keep_scale) : (bf16_t)0.f;
-        h[e + 1] = k_hi ? (bf16_t)((float)h[e + 1] * a.keep_scale) : (bf16_t)0.f;
-      }
-      gx[i] = __builtin_bit_cast(i32x4, h);
-    }
-#pragma unroll
-    for (int i = 0; i < kDG; ++i) {
-      const int gi = tid + 256 * i, r = gi / (4 * NB), g = gi % (4 * NB);
-      const int s = s0 + r;
-      i32x4 v = {0, 0, 0, 0};
-      if (gi < 32 * 4 * NB && s < a.S) v = *reinterpret_cast<const i32x4 *>(db + (int64_t)s * a.da_rs + 8 * g);
-      gd[i] = v;
-    }
-  };
-  auto store = [&](bf16_t *tx, bf16_t *td) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int gi = tid + 256 * i;
-      *reinterpret_cast<i32x4 *>(tx + tile_off<HD>(gi >> 4, gi & 15)) = gx[i];
-    }
-#pragma unroll
-    for (int i = 0; i < kDG; ++i) {
-      const int gi = tid + 256 * i;
-      if (gi < 32 * 4 * NB) *reinterpret_cast<i32x4 *>(td + tile_off<HD>(gi / (4 * NB), gi % (4 * NB))) = gd[i];
-    }
-  };
-  f32x16 acc[NB];
-#pragma unroll
-  for (int rb = 0; rb < NB; ++rb) acc[rb] = zero16();
-  auto step = [&](auto bsel, int st) {
-    constexpr int B = decltype(bsel)::value;
-    const bf16_t *tx = B ? sX1 : sX0;
-    const bf16_t *td = B ? sD1 : sD0;
-    if (st + 1 < st1) load(st + 1);
-#pragma unroll
-    for (int ss = 0; ss < 2; ++ss) {
-      const bf16x8 hb = tro.operand(tx, 16 * ss, w);
-#pragma unroll
-      for (int rb = 0; rb < NB; ++rb) acc[rb] = mfma32<bf16_t>(tro.operand(td, 16 * ss, rb), hb, acc[rb]);
-    }
-    if (st + 1 < st1) store(B ? sX0 : sX1, B ? sD0 : sD1);
-    __syncthreads();
-  };
-  if (st0 < st1) {
-    load(st0);
-    store(sX0, sD0);
-  }
-  __syncthreads();
-  for (int st = st0; st < st1; st += 2) {
-    step(std::integral_constant<int, 0>{}, st);
-    if (st + 1 < st1) step(std::integral_constant<int, 1>{}, st + 1);
-  }
-  // lane holds column kc0 + 32 w + l32 of rows 8 (q / 4) + 4 hi + q % 4 of each rank block
-  const int k = kc0 + 32 * w + l32;
-  const int rp = (a.rank + 31) / 32 * 32;
-#pragma unroll
-  for (int rb = 0; rb < NB; ++rb)
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int r = 32 * rb + 8 * (q >> 2) + 4 * hi + (q & 3);
-      if (r >= rc) continue;
-      if (gridDim.y > 1)
-        a.part[((int64_t)blockIdx.y * rp + r0 + r) * a.K + k] = acc[rb][q];
-      else
-        reinterpret_cast<bf16_t *>(a.dA)[(int64_t)(r0 + r) * a.dA_rs + k] = (bf16_t)acc[rb][q];
-    }
-}
-
-// grad_A[r][k] = T(sum over the splits, in order) of lora_da_kernel's partials.
-__global__ __launch_bounds__(256) void lora_da_finish_kernel(LoraDaArgs a, int nsplit) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (int64_t)a.rank * a.K) return;
-  const int r = (int)(i / a.K), k = (int)(i - (int64_t)r * a.K);
-  const int rp = (a.rank + 31) / 32 * 32;
-  float v = 0.f;
-  for (int y = 0; y < nsplit; ++y) v += a.part[((int64_t)y * rp + r) * a.K + k];
-  reinterpret_cast<bf16_t *>(a.dA)[(int64_t)r * a.dA_rs + k] = (bf16_t)v;
-}
-
 // d_a[s][r] = T(T(u[s][r] * gate[s]) * s) for r < rank, 0 up to rpad.
 __global__ __launch_bounds__(256) void lora_scale_rows_kernel(const bf16_t *u, int64_t u_rs, const float *gate,
                                                               float scaling, int32_t S, int32_t rank, int32_t rpad,
@@ -696,68 +301,92 @@ __global__ __launch_bounds__(256) void lora_transpose_kernel(const bf16_t *A, in
 }
 
 
-// ---- lora_B's backward: the two skinny products over the streamed dY -------
-// MODE 0: dB^T partials   part[split][n][r] = sum over the split's rows s of dY[s][n] t[s][r]
-// MODE 1: u^T partials    part[split][s][r] = sum over the split's columns n of dY[s][n] B[n][r]
-// One launch runs both (the u workgroups first). A workgroup of 8 waves owns
-// 128 output lines (columns n for MODE 0, rows s for MODE 1) and a share of
-// the 64-wide chunks of the reduced dimension. Each chunk stages two 64 x 64
-// dY tiles (rows s, columns n, swizzled), one per 64 lines, and the chunk's 64
-// rows of the small matrix (t for MODE 0, B for MODE 1) as compact rows of
-// RP = 32 RB elements, in a ring of four stages filled up to four chunks ahead
-// by direct loads. Wave w takes k-step w % 4 (16 of the 64) of every chunk for
-// its 64 lines (half w / 4) and all ranks:
-//   MODE 0: dB^T[r][n] += t^T[r][s] dY[s][n]      A: t^T, B: dY  (transposed LDS reads)
-//   MODE 1: u^T[r][s]  += B^T[r][n] dY^T[n][s]    A: B^T (transposed read), B: dY rows (8-byte reads)
-// so a lane holds one output line and 16 ranks of each rank block, written
-// as 16-byte runs. The waves' sums are added in a fixed order at the end.
+// ---- the rank-r products that stream a wide operand -------------------------
+// X [rows, cols] (dY or the layer input x) is read once; the small matrix has
+// one line of ranks per reduced entry (t, d_a, lora_B) or per rank (lora_A):
+//   kDb:   part[split][n][r] = sum over the split's rows s of dY[s][n] t[s][r]
+//   kU:    part[split][s][r] = sum over the split's columns n of dY[s][n] B[n][r]
+//   kDa:   part[split][r][k] = sum over the split's rows s of d_a[s][r] h[s][k]
+//   kDown: part[split][s][r] = sum over the split's columns k of h[s][k] A[r][k]
+// with h = dropout(x) drawn on the fly (one hash per element pair). A workgroup
+// of 8 waves owns 128 output lines (columns of X for kDb and kDa, rows for kU
+// and kDown) and a share of the 64-wide chunks of the reduced dimension. Each
+// chunk stages two 64 x 64 X tiles (rows, columns, swizzled), one per 64
+// lines, and the chunk's part of the small matrix (64 compact rows of RP =
+// 32 RB ranks; for kDown RP rows of 64 columns, swizzled), in a ring of four
+// stages filled up to four chunks ahead by direct loads. Wave w takes k-step
+// w % 4 (16 of the 64) of every chunk for its 64 lines (half w / 4) and all
+// ranks:
+//   kDb:   dB^T[r][n] += t^T[r][s] dY[s][n]      A: t^T, B: dY  (transposed LDS reads)
+//   kU:    u^T[r][s]  += B^T[r][n] dY^T[n][s]    A: B^T (transposed read), B: dY rows (8-byte reads)
+//   kDa:   dA^T[k][r] += h^T[k][s] d_a[s][r]     the operands of kDb exchanged
+//   kDown: t^T[r][s]  += A[r][k] h^T[k][s]       A: lora_A rows, B: x rows (16-byte reads)
+// kDown applies the dropout to the operand it read, whose 8 columns are 4
+// pairs; kDa, whose operand holds one column of 8 rows, applies it in place to
+// the 16-byte granules that the wave itself loaded, before the barrier that
+// publishes them. A lane holds one output line and 16 ranks of each rank block
+// (kDa: one rank and 16 columns), written as 16-byte runs. The waves' sums are
+// added in a fixed order at the end.
 // Bound by the workgroup's start and end (about 6 us: first loads, final sums)
-// and 0.45 us a chunk, 0.65 us once all CUs stream (dY from HBM, the small
-// matrix from L2), so the splits give every CU one long workgroup where they
-// can. 128 lines a workgroup bring 1.75 bytes into LDS per byte of dY at rank
-// 96 (64 lines: 2.5). At [5120, 6144] x rank 96 38 us, and 5.4 us to finish both
-// (one launch per product with 64 lines: 28.7 + 5.4 and 25.6 + 6.2 us); at
+// and 0.45 us a chunk, 0.65 us once all CUs stream (X from HBM, the small
+// matrix from L2; the hashes of a chunk are 0.8 us of VALU work), so the splits
+// give every CU one long workgroup where they can. 128 lines a workgroup bring
+// 1.75 bytes into LDS per byte of X at rank 96 (64 lines: 2.5).
+// kDb and kU at [5120, 6144] x rank 96 38 us, and 5.4 us to finish both (one
+// launch per product with 64 lines: 28.7 + 5.4 and 25.6 + 6.2 us); at
 // [1387, 4096] x rank 32 8.2 + 4.7 us (6.7 + 4.8 and 6.6 + 4.8 us).
+// The hashes bound kDown and kDa there (1.2 us a chunk): [5120, 4096] x rank 96
+// with dropout 26.3 + 5.3 and 26.5 + 5.0 us with the finishing launches (an
+// earlier kernel with a packed copy of lora_A 5.1 + 26.5 + 5.4, staging through
+// registers for dA 30.2 + 7.6 us).
 // The loads are inline asm through buffer resources (the caller of the wait
-// counts them: 2 dY loads a wave and chunk, and the small matrix's 4 RB loads
-// dealt to the 8 waves); rows past the end arrive as zeros, dY columns past N as
-// other elements of dY, which are zeroed in the operand where they are reduced
-// over and stay in lines that nothing reads otherwise. Rank columns past the
-// rank hold junk that the finishing kernel does not read.
-template <int MODE, int RB>
-__device__ __forceinline__ void lora_skinny_body(const LoraSkinnyArgs &a, int blk, int split, int nsplit, bf16_t *lds) {
-  constexpr int RP = 32 * RB;                 // compact small-tile row (elements)
+// counts them: 2 X loads a wave and chunk, and the small matrix's 4 RB loads
+// dealt to the 8 waves); rows past the end arrive as zeros, columns past the
+// end as other elements of X, which are zeroed in the operand where they are
+// reduced over and stay in lines that nothing reads otherwise. Rank columns
+// past the rank hold junk that the finishing kernels do not read.
+enum { kDb = 0, kU = 1, kDa = 2, kDown = 3 };
+
+template <int KIND, int RB, bool DROP, bool WRITE_H>
+__device__ __forceinline__ void lora_stream_body(const LoraStream &a, int blk, int split, bf16_t *lds) {
+  constexpr bool kCols = KIND == kDb || KIND == kDa;   // lines are columns of X, rows are reduced
+  constexpr int RP = 32 * RB;                 // ranks of a small tile
   constexpr int YT = 64 * 64, MT = 64 * RP, STAGE = 2 * YT + MT;
-  constexpr int MG = RP / 8;                  // granules per small-tile row
+  constexpr int MG = RP / 8;                  // granules per compact small-tile row
   constexpr int MIA = (RB + 1) / 2, MIB = RB / 2;   // small-tile loads of waves 0-3, of waves 4-7
   const int w = wave_id(), lane = threadIdx.x & 63;
   const int kq = w & 3, half = w >> 2;
   const int l32 = lane & 31, hi = lane >> 5;
   const int line0 = blk * 128 + 64 * half;    // the wave's first line
-  const int nlines = MODE == 0 ? a.N : a.S;   // output lines
-  const int kdim = MODE == 0 ? a.S : a.N;     // reduced dimension
+  const int nlines = kCols ? a.cols : a.rows;   // output lines
+  const int kdim = kCols ? a.rows : a.cols;     // reduced dimension
   const int nall = (kdim + 63) / 64;
-  const int c0 = (int)((int64_t)nall * split / nsplit);
-  const int nch = (int)((int64_t)nall * (split + 1) / nsplit) - c0;
-  const bf16_t *dy = reinterpret_cast<const bf16_t *>(a.dy);
-  const bf16_t *sm = reinterpret_cast<const bf16_t *>(MODE == 0 ? a.t : a.b);
-  const int64_t sm_rs = MODE == 0 ? a.t_rs : a.b_rs;
+  const int c0 = (int)((int64_t)nall * split / a.ns);
+  const int nch = (int)((int64_t)nall * (split + 1) / a.ns) - c0;
+  const bf16_t *x = reinterpret_cast<const bf16_t *>(a.x);
+  const bf16_t *sm = reinterpret_cast<const bf16_t *>(a.sm);
   const int mcols = (a.rank + 7) / 8 * 8;
 
-  // Per-lane byte offsets. dY tile: 8 granules per row, 8 rows per load, wave
-  // kq of the half loads rows 16 kq .. 16 kq + 15 (two loads). Small tile: load
-  // i of wave w fills slots 64 (w + 8 i) + lane (row slot / MG, granule slot %
-  // MG; a granule past the rank reads the last one again).
+  // Per-lane byte offsets. X tile: 8 granules per row, 8 rows per load, wave kq
+  // of the half loads rows 16 kq .. 16 kq + 15 (two loads). Small tile, load i
+  // of wave w: compact rows, slots 64 (w + 8 i) + lane (row slot / MG, granule
+  // slot % MG; a granule past the rank reads the last one again); kDown, ranks
+  // 8 (w + 8 i) + lane / 8.
   uint32_t yo[2], mo[MIA];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int r = 16 * kq + 8 * i + (lane >> 3);
-    yo[i] = opaque_u32((uint32_t)(r * a.dy_rs * 2) + (uint32_t)(16 * ((lane & 7) ^ swz<64>(r))));
+    yo[i] = opaque_u32((uint32_t)(r * a.x_rs * 2) + (uint32_t)(16 * ((lane & 7) ^ swz<64>(r))));
   }
 #pragma unroll
   for (int i = 0; i < MIA; ++i) {
-    const int slot = 64 * (w + 8 * i) + lane;
-    mo[i] = opaque_u32((uint32_t)((slot / MG) * sm_rs * 2) + (uint32_t)(16 * min(slot % MG, mcols / 8 - 1)));
+    if constexpr (KIND == kDown) {
+      const int r = 8 * (w + 8 * i) + (lane >> 3);
+      mo[i] = opaque_u32((uint32_t)(r * a.sm_rs * 2) + (uint32_t)(16 * ((lane & 7) ^ swz<64>(r))));
+    } else {
+      const int slot = 64 * (w + 8 * i) + lane;
+      mo[i] = opaque_u32((uint32_t)((slot / MG) * a.sm_rs * 2) + (uint32_t)(16 * min(slot % MG, mcols / 8 - 1)));
+    }
   }
   // Workgroups start their share at different chunks (rotated by the line
   // block), so that those streaming the same share at the same time do not all
@@ -766,42 +395,65 @@ __device__ __forceinline__ void lora_skinny_body(const LoraSkinnyArgs &a, int bl
   auto chunk_of = [&](int c) { const int r = c + rot; return c0 + (r >= nch ? r - nch : r); };
   auto issue = [&](int c, bf16_t *st) {
     const int k0 = chunk_of(min(c, nch - 1)) * 64;   // past the share: its last chunk again
-    const int r0 = MODE == 0 ? k0 : line0, n0 = MODE == 0 ? line0 : k0;
+    const int r0 = kCols ? k0 : line0, n0 = kCols ? line0 : k0;
     // resource ranges end with the last element of the tile's last existing row
-    const int64_t yb = (int64_t)(min(64, a.S - r0) - 1) * a.dy_rs + a.N - n0;
-    const i32x4 ry = buf_rsrc(dy + (r0 < a.S ? (int64_t)r0 * a.dy_rs + n0 : 0), r0 < a.S && yb > 0 ? (uint32_t)(yb * 2) : 0u);
+    const int64_t yb = (int64_t)(min(64, a.rows - r0) - 1) * a.x_rs + a.cols - n0;
+    const i32x4 ry =
+        buf_rsrc(x + (r0 < a.rows ? (int64_t)r0 * a.x_rs + n0 : 0), r0 < a.rows && yb > 0 ? (uint32_t)(yb * 2) : 0u);
 #pragma unroll
     for (int i = 0; i < 2; ++i) bdma16(ry, yo[i], st + half * YT + (16 * kq + 8 * i) * 64);
-    const int64_t mb = (int64_t)(min(64, kdim - k0) - 1) * sm_rs + mcols;
-    const i32x4 rm = buf_rsrc(sm + (int64_t)k0 * sm_rs, (uint32_t)(mb * 2));
+    i32x4 rm;
+    if constexpr (KIND == kDown)
+      rm = buf_rsrc(sm + k0, (uint32_t)(((int64_t)(min(a.rank, RP) - 1) * a.sm_rs + a.cols - k0) * 2));
+    else
+      rm = buf_rsrc(sm + (int64_t)k0 * a.sm_rs, (uint32_t)(((int64_t)(min(64, kdim - k0) - 1) * a.sm_rs + mcols) * 2));
 #pragma unroll
     for (int i = 0; i < MIA; ++i)
       if (i < MIB || w < 4) bdma16(rm, mo[i], st + 2 * YT + 512 * (w + 8 * i));
   };
-  // the loads of the three (two) newest chunks stay in flight
+  // the loads of the three (two) newest chunks stay in flight; with the
+  // dropout output's stores among them, which may retire out of order, none
   auto wait3 = [&]() {
     if (MIA == MIB || w < 4) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * (2 + MIA)) : "memory");
     else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * (2 + MIB)) : "memory");
   };
   auto wait2 = [&]() {
-    if (MIA == MIB || w < 4) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (2 + MIA)) : "memory");
+    if (WRITE_H) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    else if (MIA == MIB || w < 4) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (2 + MIA)) : "memory");
     else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (2 + MIB)) : "memory");
   };
+  // dropout of the 8 elements of row s from column k on (columns a multiple of 16)
+  auto drop = [&](const bf16x8 &v, int s, int k) {
+    return drop8(v, ((uint64_t)s * (uint64_t)a.cols + (uint64_t)k) >> 1, a.seed, a.thr, a.keep_scale);
+  };
+  // kDa: dropout, in place, of the granules of chunk c that this wave loaded
+  auto drop_own = [&](int c, bf16_t *st) {
+    if constexpr (KIND == kDa && DROP) {
+      const int k0 = chunk_of(c) * 64;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int r = 16 * kq + 8 * i + (lane >> 3), g = (lane & 7) ^ swz<64>(r);
+        bf16_t *p = st + half * YT + (16 * kq + 8 * i) * 64 + lane * 8;
+        *reinterpret_cast<i32x4 *>(p) = __builtin_bit_cast(i32x4, drop(lds_read8(p), k0 + r, line0 + 8 * g));
+      }
+    }
+  };
 
-  // A operand from a compact k-major tile (rows k, RP columns): lane (l32, hi)
-  // takes column 32 rb + l32 at rows k0 + 4 hi + 0..3 and k0 + 8 + 4 hi + 0..3
-  // (the k order of TrLane), by two transposed reads
+  // small operand from a compact k-major tile (rows k, RP columns): lane (l32,
+  // hi) takes column 32 rb + l32 at rows k0 + 4 hi + 0..3 and k0 + 8 + 4 hi +
+  // 0..3 (the k order of TrLane), by two transposed reads
   const int ti = lane & 15;
   const uint32_t mro[2] = {
       opaque_u32((uint32_t)(((16 * kq + 4 * hi + (ti >> 2)) * RP + 16 * ((lane >> 4) & 1) + 4 * (ti & 3)) * 2)),
       opaque_u32((uint32_t)(((16 * kq + 8 + 4 * hi + (ti >> 2)) * RP + 16 * ((lane >> 4) & 1) + 4 * (ti & 3)) * 2))};
   auto m_operand = [&](const bf16_t *tM, int rb) {
+    if constexpr (KIND == kDown) return lds_read8(tM + tile_off<64>(32 * rb + l32, 2 * kq + hi));
     const char *p = reinterpret_cast<const char *>(tM) + 64 * rb;
     return join8(lds_tr4(reinterpret_cast<const bf16_t *>(p + mro[0])),
                  lds_tr4(reinterpret_cast<const bf16_t *>(p + mro[1])));
   };
   TrOffsets<64> try_;
-  try_.init(lane);
+  if constexpr (kCols) try_.init(lane);
   f32x16 acc[RB][2];
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) acc[rb][0] = acc[rb][1] = zero16();
@@ -810,25 +462,34 @@ __device__ __forceinline__ void lora_skinny_body(const LoraSkinnyArgs &a, int bl
     const bf16_t *tY = st + half * YT, *tM = st + 2 * YT;
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) av[rb] = m_operand(tM, rb);
-    if (MODE == 0) {
+    if constexpr (kCols) {
 #pragma unroll
       for (int nb = 0; nb < 2; ++nb) bv[nb] = try_.operand(tY, 16 * kq, nb);
     } else {
-      // dY row 32 sb + l32, columns 16 kq + 4 hi + 0..3 and 16 kq + 8 + 4 hi + 0..3
+      const int kb = chunk_of(c) * 64 + 16 * kq;
 #pragma unroll
       for (int sb = 0; sb < 2; ++sb) {
         const int r = 32 * sb + l32;
-        bv[sb] = lds_read4x2(tY + tile_off<64>(r, 2 * kq) + 4 * hi, tY + tile_off<64>(r, 2 * kq + 1) + 4 * hi);
-      }
-      const int kb = chunk_of(c) * 64 + 16 * kq;
-      if (kb + 16 > kdim) {   // columns kb + 4 hi + e and kb + 8 + 4 hi + e past N
+        if constexpr (KIND == kU) {
+          // dY columns kb + 4 hi + 0..3 and kb + 8 + 4 hi + 0..3 of row r
+          bv[sb] = lds_read4x2(tY + tile_off<64>(r, 2 * kq) + 4 * hi, tY + tile_off<64>(r, 2 * kq + 1) + 4 * hi);
+          if (kb + 16 > kdim)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const bool out = kb + 4 * hi + (e & 3) + 8 * (e >> 2) >= kdim;
-#pragma unroll
-          for (int sb = 0; sb < 2; ++sb) bv[sb][e] = out ? (bf16_t)0.f : bv[sb][e];
+            for (int e = 0; e < 8; ++e)
+              if (kb + 4 * hi + (e & 3) + 8 * (e >> 2) >= kdim) bv[sb][e] = (bf16_t)0.f;
+        } else {
+          // x columns kb + 8 hi + 0..7 of row r (the columns are a multiple of 16)
+          bv[sb] = lds_read8(tY + tile_off<64>(r, 2 * kq + hi));
+          if (DROP) bv[sb] = drop(bv[sb], line0 + r, kb + 8 * hi);
+          if (kb >= kdim) bv[sb] = zero8();
+          if (WRITE_H && DROP && kb < kdim && line0 + r < a.rows)
+            *reinterpret_cast<i32x4 *>(reinterpret_cast<bf16_t *>(a.h) + (int64_t)(line0 + r) * a.h_rs + kb + 8 * hi) =
+                __builtin_bit_cast(i32x4, bv[sb]);
         }
       }
+      if (KIND == kDown && kb >= kdim)   // lora_A's elements there belong to the next rank
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) av[rb] = zero8();
     }
   };
 
@@ -842,6 +503,7 @@ __device__ __forceinline__ void lora_skinny_body(const LoraSkinnyArgs &a, int bl
 #pragma unroll
     for (int q = 0; q < 4; ++q) issue(q, lds + q * STAGE);
     wait3();
+    drop_own(0, lds);
     lds_barrier();
     operands(0, lds, av[0], bv[0]);
     for (int cb = 0; cb < nch; cb += 4)
@@ -850,6 +512,7 @@ __device__ __forceinline__ void lora_skinny_body(const LoraSkinnyArgs &a, int bl
         if (cb + q < nch) {
           if (cb + q + 1 < nch) {
             wait2();
+            drop_own(cb + q + 1, lds + ((q + 1) & 3) * STAGE);
             lds_barrier();
             issue(cb + q + 4, lds + q * STAGE);
             operands(cb + q + 1, lds + ((q + 1) & 3) * STAGE, av[(q + 1) & 1], bv[(q + 1) & 1]);
@@ -857,7 +520,9 @@ __device__ __forceinline__ void lora_skinny_body(const LoraSkinnyArgs &a, int bl
 #pragma unroll
           for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-            for (int lb = 0; lb < 2; ++lb) acc[rb][lb] = mfma32<bf16_t>(av[q & 1][rb], bv[q & 1][lb], acc[rb][lb]);
+            for (int lb = 0; lb < 2; ++lb)
+              acc[rb][lb] = KIND == kDa ? mfma32<bf16_t>(bv[q & 1][lb], av[q & 1][rb], acc[rb][lb])
+                                        : mfma32<bf16_t>(av[q & 1][rb], bv[q & 1][lb], acc[rb][lb]);
         }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the ring's trailing loads
@@ -866,9 +531,9 @@ __device__ __forceinline__ void lora_skinny_body(const LoraSkinnyArgs &a, int bl
   // fixed-order sum of the four k-step waves of each half through LDS, 32 lines
   // at a time: every wave parks its accumulators, then wave kq adds the four
   // waves' registers 4 kq .. 4 kq + 3 and writes them as this split's partial:
-  // lane = line 32 lb + l32, ranks 32 rb + 8 kq + 4 hi + 0..3
+  // lane = line 32 lb + l32, ranks 32 rb + 8 kq + 4 hi + 0..3 (kDa: rank
+  // 32 rb + l32, lines 32 lb + 8 kq + 4 hi + 0..3)
   f32x4 *park = reinterpret_cast<f32x4 *>(lds) + half * (4 * RB * 4 * 64);
-  float *part = MODE == 0 ? a.part_b : a.part_u;
 #pragma unroll
   for (int lb = 0; lb < 2; ++lb) {
 #pragma unroll
@@ -879,156 +544,193 @@ __device__ __forceinline__ void lora_skinny_body(const LoraSkinnyArgs &a, int bl
         park[((kq * RB + rb) * 4 + q) * 64 + lane] = f32x4{c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3]};
       }
     __syncthreads();
-    const int line = line0 + 32 * lb + l32;
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
       f32x4 v = park[(rb * 4 + kq) * 64 + lane];
 #pragma unroll
       for (int k = 1; k < 4; ++k) {
-        const f32x4 x = park[((k * RB + rb) * 4 + kq) * 64 + lane];
+        const f32x4 y = park[((k * RB + rb) * 4 + kq) * 64 + lane];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] += x[e];
+        for (int e = 0; e < 4; ++e) v[e] += y[e];
       }
-      if (line < nlines)
-        *reinterpret_cast<f32x4 *>(part + ((int64_t)split * nlines + line) * a.rp + 32 * rb + 8 * kq + 4 * hi) = v;
+      if constexpr (KIND == kDa) {
+        const int line = line0 + 32 * lb + 8 * kq + 4 * hi;   // the columns are a multiple of 16
+        if (line < nlines)
+          *reinterpret_cast<f32x4 *>(a.part + ((int64_t)split * RP + 32 * rb + l32) * nlines + line) = v;
+      } else {
+        const int line = line0 + 32 * lb + l32;
+        if (line < nlines)
+          *reinterpret_cast<f32x4 *>(a.part + ((int64_t)split * nlines + line) * RP + 32 * rb + 8 * kq + 4 * hi) = v;
+      }
     }
     __syncthreads();
   }
 }
 
 template <int RB>
-__global__ __launch_bounds__(512, 1) void lora_skinny_kernel(LoraSkinnyArgs a) {
-  __shared__ __attribute__((aligned(16))) bf16_t lds[4 * (2 * 64 * 64 + 64 * 32 * RB)];
-  const int nbu = (a.S + 127) / 128, nbb = (a.N + 127) / 128;
+constexpr int kStreamLds = 4 * (2 * 64 * 64 + 64 * 32 * RB);   // elements
+
+// kU over u, kDb over b (ns = 0: not wanted)
+template <int RB>
+__global__ __launch_bounds__(512, 1) void lora_skinny_kernel(LoraStream u, LoraStream b) {
+  __shared__ __attribute__((aligned(16))) bf16_t lds[kStreamLds<RB>];
+  const int nbu = (u.rows + 127) / 128, nbb = (b.cols + 127) / 128;
   const int i = blockIdx.x;
-  if (i < nbu * a.nsu) lora_skinny_body<1, RB>(a, i % nbu, i / nbu, a.nsu, lds);
-  else lora_skinny_body<0, RB>(a, (i - nbu * a.nsu) % nbb, (i - nbu * a.nsu) / nbb, a.nsb, lds);
+  if (i < nbu * u.ns) lora_stream_body<kU, RB, false, false>(u, i % nbu, i / nbu, lds);
+  else lora_stream_body<kDb, RB, false, false>(b, (i - nbu * u.ns) % nbb, (i - nbu * u.ns) / nbb, lds);
+}
+
+template <int RB>
+__global__ __launch_bounds__(512, 1) void lora_da_kernel(LoraStream a) {
+  __shared__ __attribute__((aligned(16))) bf16_t lds[kStreamLds<RB>];
+  const int nb = (a.cols + 127) / 128;
+  lora_stream_body<kDa, RB, true, false>(a, blockIdx.x % nb, blockIdx.x / nb, lds);
+}
+
+template <int RB, bool DROP, bool WRITE_H>
+__global__ __launch_bounds__(512, 1) void lora_down_kernel(LoraStream a) {
+  __shared__ __attribute__((aligned(16))) bf16_t lds[kStreamLds<RB>];
+  const int nb = (a.rows + 127) / 128;
+  lora_stream_body<kDown, RB, DROP, WRITE_H>(a, blockIdx.x % nb, blockIdx.x / nb, lds);
+}
+
+// t[s][r] = T(T(s * T(sum over the splits, in order)) * gate), 0 for rank <= r
+// < 32 RB. Four ranks a thread.
+__global__ __launch_bounds__(256) void lora_down_finish_kernel(LoraStream a, int rp, const float *gate, float scaling,
+                                                               bf16_t *t, int64_t t_rs) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= (int64_t)a.rows * (rp / 4)) return;
+  const int s = (int)(i / (rp / 4)), r = 4 * (int)(i - (int64_t)s * (rp / 4));
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int y = 0; y < a.ns; ++y) {
+    const f32x4 x = *reinterpret_cast<const f32x4 *>(a.part + ((int64_t)y * a.rows + s) * rp + r);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] += x[e];
+  }
+  const float g = gate ? gate[s] : 1.f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = r + e < a.rank ? rnd(rnd(v[e]) * scaling) * g : 0.f;
+  bf16_t *out = t + (int64_t)s * t_rs + r;
+  if ((t_rs & 3) == 0 && ((uintptr_t)t & 7) == 0) store4(out, v[0], v[1], v[2], v[3]);
+  else
+#pragma unroll
+    for (int e = 0; e < 4; ++e) out[e] = (bf16_t)v[e];
+}
+
+// dA[r][k] = T(sum over the splits, in order) for r < rank. Four columns a thread.
+__global__ __launch_bounds__(256) void lora_da_finish_kernel(LoraStream a, int rp, bf16_t *dA, int64_t dA_rs) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= (int64_t)a.rank * (a.cols / 4)) return;
+  const int r = (int)(i / (a.cols / 4)), k = 4 * (int)(i - (int64_t)r * (a.cols / 4));
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int y = 0; y < a.ns; ++y) {
+    const f32x4 x = *reinterpret_cast<const f32x4 *>(a.part + ((int64_t)y * rp + r) * a.cols + k);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] += x[e];
+  }
+  bf16_t *out = dA + (int64_t)r * dA_rs + k;
+  if ((dA_rs & 3) == 0 && ((uintptr_t)dA & 7) == 0) store4(out, v[0], v[1], v[2], v[3]);
+  else
+#pragma unroll
+    for (int e = 0; e < 4; ++e) out[e] = (bf16_t)v[e];
 }
 
 // d_a[s][r] = T(T(T(u) * gate[s]) * scaling), u = the sum over the splits in
 // order; 0 for rank <= r < rp (the roundings of the chain dY B (bf16), then
 // lora_scale_rows); dB[n][r] = T(sum over the splits, in order), r < rank
 // (nsb > 0). Four ranks a thread.
-__global__ __launch_bounds__(256) void lora_skinny_finish_kernel(LoraSkinnyArgs a, const float *gate, float scaling,
-                                                                 bf16_t *da, int64_t da_rs, bf16_t *db,
+__global__ __launch_bounds__(256) void lora_skinny_finish_kernel(LoraStream u, LoraStream b, int rp, const float *gate,
+                                                                 float scaling, bf16_t *da, int64_t da_rs, bf16_t *db,
                                                                  int64_t db_rs) {
-  const int64_t nu = (int64_t)a.S * (a.rp / 4), nb = a.nsb > 0 ? (int64_t)a.N * (a.rp / 4) : 0;
+  const int64_t nu = (int64_t)u.rows * (rp / 4), nb = b.ns > 0 ? (int64_t)b.cols * (rp / 4) : 0;
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const bool isb = i >= nu;
   if (isb) i -= nu;
   if (isb && i >= nb) return;
-  const int line = (int)(i / (a.rp / 4)), r = 4 * (int)(i - (int64_t)line * (a.rp / 4));
-  const int nlines = isb ? a.N : a.S, ns = isb ? a.nsb : a.nsu;
-  const float *p = (isb ? a.part_b : a.part_u) + (int64_t)line * a.rp + r;
+  const int line = (int)(i / (rp / 4)), r = 4 * (int)(i - (int64_t)line * (rp / 4));
+  const int nlines = isb ? b.cols : u.rows, ns = isb ? b.ns : u.ns;
+  const float *p = (isb ? b.part : u.part) + (int64_t)line * rp + r;
   f32x4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
   for (int y = 0; y < ns; ++y) {
-    const f32x4 x = *reinterpret_cast<const f32x4 *>(p + (int64_t)y * nlines * a.rp);
+    const f32x4 x = *reinterpret_cast<const f32x4 *>(p + (int64_t)y * nlines * rp);
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] += x[e];
   }
   if (isb) {
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      if (r + e < a.rank) db[(int64_t)line * db_rs + r + e] = (bf16_t)v[e];
+      if (r + e < b.rank) db[(int64_t)line * db_rs + r + e] = (bf16_t)v[e];
     return;
   }
   const float g = gate ? gate[line] : 1.f;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) v[e] = r + e < a.rank ? rnd(rnd(rnd(v[e]) * g) * scaling) : 0.f;
+  for (int e = 0; e < 4; ++e) v[e] = r + e < u.rank ? rnd(rnd(rnd(v[e]) * g) * scaling) : 0.f;
   store4(da + (int64_t)line * da_rs + r, v[0], v[1], v[2], v[3]);
+}
+
+// The general form of the LoRA term of dX (ranks above 128, columns a multiple
+// of 16 only, 8-byte aligned rows), from a transposed copy of lora_A.
+void launch_lora_dx_rows(const LoraDxArgs &a, hipStream_t st) {
+  const dim3 grid((unsigned)((a.K + 511) / 512), (unsigned)((a.S + 31) / 32)), block(256);
+  switch ((a.rank + 31) / 32) {
+    case 1: hipLaunchKernelGGL((lora_dx_rows_kernel<2>), grid, block, 0, st, a); break;
+    case 2: hipLaunchKernelGGL((lora_dx_rows_kernel<4>), grid, block, 0, st, a); break;
+    case 3: hipLaunchKernelGGL((lora_dx_rows_kernel<6>), grid, block, 0, st, a); break;
+    case 4: hipLaunchKernelGGL((lora_dx_rows_kernel<8>), grid, block, 0, st, a); break;
+    default: hipLaunchKernelGGL((lora_dx_rows_kernel<2>), grid, block, 0, st, a); break;   // 2-step chunks
+  }
 }
 
 namespace {
 
-template <int NB>
-void launch_down_nb(const LoraDownArgs &a, hipStream_t st) {
-  const dim3 grid((unsigned)((a.S + 31) / 32));
-  if (a.K % 128 == 0 && a.packed) {
-    // lora_A into operand order, then the ring kernel; split K until every CU
-    // has about two workgroups, each keeping at least four chunks
-    const int64_t ng = (int64_t)(a.K / 16) * NB * 64;
-    hipLaunchKernelGGL(lora_pack_a_kernel, dim3((unsigned)((ng + 255) / 256)), dim3(256), 0, st,
-                       reinterpret_cast<const bf16_t *>(a.A), a.a_rs, a.rank, a.K, NB,
-                       reinterpret_cast<i32x4 *>(a.packed));
-    const int nrb = (a.S + 31) / 32, nch = a.K / 128;
-    int nsplit = 1;
-    if (a.part)
-      while (nsplit < kDownMaxSplit && nrb * nsplit < 512 && nch / (2 * nsplit) >= 4) nsplit *= 2;
-    const dim3 g2((unsigned)nrb, (unsigned)nsplit);
-    if (a.thr > 0 && a.h) hipLaunchKernelGGL((lora_down_ring_kernel<NB, true, true>), g2, dim3(256), 0, st, a);
-    else if (a.thr > 0) hipLaunchKernelGGL((lora_down_ring_kernel<NB, true, false>), g2, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((lora_down_ring_kernel<NB, false, false>), g2, dim3(256), 0, st, a);
-    if (nsplit > 1) {
-      const int64_t n = (int64_t)a.S * 32 * NB;
-      hipLaunchKernelGGL(lora_down_finish_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, nsplit,
-                         32 * NB);
+// Waves of an outer-product workgroup, 6 to 10: the count that leaves the CUs
+// the least uneven number of waves (workgroups per CU, rounded up, times
+// waves), the larger of equals. Each workgroup copies the W tile: [3000, 24576]
+// x rank 64 takes 64 us with 1 wave, 39 with 2, 27 with 4 to 10; [5120, 6144] x
+// rank 96 takes 49, 26, 19 (4), 17.8 (6) and 15.5 us (10).
+int outer_waves(int row_blocks, int col_blocks) {
+  const int cus = device_cu_count();
+  int best = 1;
+  int64_t best_cost = INT64_MAX;
+  for (int w = std::min(row_blocks, 6); w <= std::min(row_blocks, kOuterWaves); ++w) {
+    const int64_t wgs = (int64_t)((row_blocks + w - 1) / w) * col_blocks;
+    const int64_t cost = (wgs + cus - 1) / cus * w;
+    if (cost <= best_cost) {
+      best_cost = cost;
+      best = w;
     }
-    return;
   }
-  if (a.thr > 0) hipLaunchKernelGGL((lora_down_kernel<NB, true>), grid, dim3(kDownWaves * 64), 0, st, a);
-  else hipLaunchKernelGGL((lora_down_kernel<NB, false>), grid, dim3(kDownWaves * 64), 0, st, a);
+  return best;
+}
+
+template <int NK, bool COLMAJ, bool DROP>
+void outer_launch(const LoraOuter &a, hipStream_t st) {
+  const int rb = (a.rows + 31) / 32, cb = (a.cols + 127) / 128;
+  const int w = outer_waves(rb, cb);
+  const size_t lds = 2 * ((size_t)kOuterTile<NK, COLMAJ> + (size_t)w * 32 * kOuterTs);
+  hipLaunchKernelGGL((lora_outer_kernel<NK, COLMAJ, DROP>), dim3((unsigned)cb, (unsigned)((rb + w - 1) / w)),
+                     dim3(64 * w), lds, st, a);
+}
+
+template <bool COLMAJ, bool DROP>
+void outer_rank(const LoraOuter &a, hipStream_t st) {
+  switch ((a.rank + 31) / 32) {
+    case 1: outer_launch<2, COLMAJ, DROP>(a, st); break;
+    case 2: outer_launch<4, COLMAJ, DROP>(a, st); break;
+    case 3: outer_launch<6, COLMAJ, DROP>(a, st); break;
+    default: outer_launch<8, COLMAJ, DROP>(a, st); break;
+  }
 }
 
 }  // namespace
 
-// Ranks in chunks of up to 96 (three accumulator blocks per wave); the
-// dropout output is written by the first chunk only (every chunk draws the
-// same bits).
-void launch_lora_down(const LoraDownArgs &a, hipStream_t st) {
-  for (int r0 = 0; r0 < a.rank; r0 += 96) {
-    LoraDownArgs c = a;
-    c.rank = a.rank - r0 < 96 ? a.rank - r0 : 96;
-    c.A = reinterpret_cast<const bf16_t *>(a.A) + (int64_t)r0 * a.a_rs;
-    c.t = reinterpret_cast<bf16_t *>(a.t) + r0;
-    if (r0 > 0) c.h = nullptr;
-    switch ((c.rank + 31) / 32) {
-      case 1: launch_down_nb<1>(c, st); break;
-      case 2: launch_down_nb<2>(c, st); break;
-      default: launch_down_nb<3>(c, st); break;
-    }
-  }
-}
-
-void launch_lora_dx(const LoraDxArgs &a, hipStream_t st) {
-  // the LDS-staged kernel moves dX in 16-byte runs: rows must start 16-byte aligned
-  if (a.K % 128 || a.rank > 128 || a.dx_rs % 8) {
-    const dim3 grid((unsigned)((a.K + 511) / 512), (unsigned)((a.S + 31) / 32)), block(256);
-    switch ((a.rank + 31) / 32) {
-      case 1: hipLaunchKernelGGL((lora_dx_rows_kernel<2>), grid, block, 0, st, a); break;
-      case 2: hipLaunchKernelGGL((lora_dx_rows_kernel<4>), grid, block, 0, st, a); break;
-      case 3: hipLaunchKernelGGL((lora_dx_rows_kernel<6>), grid, block, 0, st, a); break;
-      case 4: hipLaunchKernelGGL((lora_dx_rows_kernel<8>), grid, block, 0, st, a); break;
-      default: hipLaunchKernelGGL((lora_dx_rows_kernel<2>), grid, block, 0, st, a); break;   // 2-step chunks
-    }
-    return;
-  }
-  const dim3 grid((unsigned)(a.K / 128), (unsigned)((a.S + 127) / 128)), block(256);
-  switch ((a.rank + 31) / 32) {
-    case 1: hipLaunchKernelGGL((lora_dx_kernel<2>), grid, block, 0, st, a); break;
-    case 2: hipLaunchKernelGGL((lora_dx_kernel<4>), grid, block, 0, st, a); break;
-    case 3: hipLaunchKernelGGL((lora_dx_kernel<6>), grid, block, 0, st, a); break;
-    default: hipLaunchKernelGGL((lora_dx_kernel<8>), grid, block, 0, st, a); break;
-  }
-}
-
-void launch_lora_da(const LoraDaArgs &a, hipStream_t st) {
-  const int nkb = a.K / 128, nst = (a.S + 31) / 32;
-  int nsplit = 1;
-  while (nsplit < kDaMaxSplit && nkb * nsplit < 512 && nst / (2 * nsplit) >= 4) nsplit *= 2;
-  const dim3 grid((unsigned)nkb, (unsigned)nsplit), block(256);
-  for (int r0 = 0; r0 < a.rank; r0 += 128) {
-    switch ((min(a.rank - r0, 128) + 31) / 32) {
-      case 1: hipLaunchKernelGGL((lora_da_kernel<1>), grid, block, 0, st, a, r0); break;
-      case 2: hipLaunchKernelGGL((lora_da_kernel<2>), grid, block, 0, st, a, r0); break;
-      case 3: hipLaunchKernelGGL((lora_da_kernel<3>), grid, block, 0, st, a, r0); break;
-      default: hipLaunchKernelGGL((lora_da_kernel<4>), grid, block, 0, st, a, r0); break;
-    }
-  }
-  if (nsplit > 1) {
-    const int64_t n = (int64_t)a.rank * a.K;
-    hipLaunchKernelGGL(lora_da_finish_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, nsplit);
-  }
+void launch_lora_outer(const LoraOuter &a, bool colmaj, hipStream_t st) {
+  if (colmaj) outer_rank<true, false>(a, st);
+  else if (a.thr > 0) outer_rank<false, true>(a, st);
+  else outer_rank<false, false>(a, st);
 }
 
 void launch_lora_scale_rows(const void *u, int64_t u_rs, const float *gate, float scaling, int32_t S, int32_t rank,
@@ -1125,53 +827,125 @@ void launch_lora_gen_scale_rows(int dtype, const void *u, int64_t u_rs, const fl
                        u_rs, gate, scaling, (int32_t)gate_first, S, rank, rpad, reinterpret_cast<f16_t *>(out), out_rs);
 }
 
-// Splits of the reduced dimensions: rounds of one workgroup per CU with the
-// smallest number of chunks from the first to the last, kSkinnyStart chunks'
-// time going into a workgroup's first loads and final sums (7 to 14 measure
-// level).
-void lora_skinny_plan(int32_t S, int32_t N, bool with_b, int32_t *nsu, int32_t *nsb) {
-  constexpr int kSkinnyStart = 8;
+namespace {
+
+// Splits of the reduced dimensions of one or two streaming products (line
+// blocks, chunks): rounds of one workgroup per CU with the smallest number of
+// chunks from the first to the last, kStreamStart chunks' time going into a
+// workgroup's first loads and final sums (7 to 14 measure level).
+void stream_plan(int64_t nb0, int ch0, int32_t *ns0, int64_t nb1, int ch1, int32_t *ns1) {
+  constexpr int kStreamStart = 8, kMaxSplit = 16;
   const int cus = device_cu_count();
-  const int64_t nbu = (S + 127) / 128, nbb = (N + 127) / 128;
-  const int cu = (N + 63) / 64, cb = (S + 63) / 64;   // chunks of a whole u, of a whole dB line block
-  const int longest = with_b ? std::max(cu, cb) : cu;
   int64_t best = INT64_MAX;
-  for (int len = 1; len <= longest; ++len) {
-    const int u = (cu + len - 1) / len, b = with_b ? (cb + len - 1) / len : 0;
-    if (u > kSkinnyMaxSplit || b > kSkinnyMaxSplit) continue;
-    const int64_t wgs = nbu * u + nbb * b;
-    const int64_t cost = ((wgs + cus - 1) / cus) * (len + kSkinnyStart);
+  for (int len = 1; len <= std::max(ch0, ch1); ++len) {
+    const int a = (ch0 + len - 1) / len, b = (ch1 + len - 1) / len;
+    if (a > kMaxSplit || b > kMaxSplit) continue;
+    const int64_t wgs = nb0 * a + nb1 * b;
+    const int64_t cost = ((wgs + cus - 1) / cus) * (len + kStreamStart);
     if (cost < best) {
       best = cost;
-      *nsu = u;
-      *nsb = b;
+      *ns0 = a;
+      *ns1 = b;
     }
   }
 }
 
-int64_t lora_skinny_part_floats(int32_t S, int32_t N, int32_t rp) {
-  int32_t nsu = 1, nsb = 1;
-  lora_skinny_plan(S, N, true, &nsu, &nsb);
-  int32_t nsu1 = 1, nsb1 = 0;
-  lora_skinny_plan(S, N, false, &nsu1, &nsb1);
-  return std::max((int64_t)nsu * S + (int64_t)nsb * N, (int64_t)nsu1 * S) * rp;
+int blocks128(int n) { return (n + 127) / 128; }
+int chunks64(int n) { return (n + 63) / 64; }
+int32_t stream_split(int lines, int kdim) {
+  int32_t ns = 1, none = 0;
+  stream_plan(blocks128(lines), chunks64(kdim), &ns, 0, 0, &none);
+  return ns;
+}
+void skinny_plan(int32_t S, int32_t N, bool with_b, int32_t *nsu, int32_t *nsb) {
+  stream_plan(blocks128(S), chunks64(N), nsu, with_b ? blocks128(N) : 0, with_b ? chunks64(S) : 0, nsb);
 }
 
-void launch_lora_grad_ub(LoraSkinnyArgs a, float *part, const float *gate, float scaling, void *da, int64_t da_rs,
-                         void *db, int64_t db_rs, hipStream_t st) {
-  lora_skinny_plan(a.S, a.N, db != nullptr, &a.nsu, &a.nsb);
-  a.part_u = part;
-  a.part_b = part + (int64_t)a.nsu * a.S * a.rp;
-  const unsigned nwg = (unsigned)((a.S + 127) / 128 * a.nsu + (a.N + 127) / 128 * a.nsb);
-  switch (a.rp / 32) {
-    case 1: hipLaunchKernelGGL(lora_skinny_kernel<1>, dim3(nwg), dim3(512), 0, st, a); break;
-    case 2: hipLaunchKernelGGL(lora_skinny_kernel<2>, dim3(nwg), dim3(512), 0, st, a); break;
-    case 3: hipLaunchKernelGGL(lora_skinny_kernel<3>, dim3(nwg), dim3(512), 0, st, a); break;
-    default: hipLaunchKernelGGL(lora_skinny_kernel<4>, dim3(nwg), dim3(512), 0, st, a); break;
+template <int RB>
+void down_rb(const LoraStream &a, bool drop, hipStream_t st) {
+  const dim3 grid((unsigned)(blocks128(a.rows) * a.ns)), blk(512);
+  if (drop && a.h) hipLaunchKernelGGL((lora_down_kernel<RB, true, true>), grid, blk, 0, st, a);
+  else if (drop) hipLaunchKernelGGL((lora_down_kernel<RB, true, false>), grid, blk, 0, st, a);
+  else hipLaunchKernelGGL((lora_down_kernel<RB, false, false>), grid, blk, 0, st, a);
+}
+
+}  // namespace
+
+// Partial sums of every streaming product of a layer (one at a time, but for u
+// and dB): ranks up to 128 at a time.
+int64_t lora_part_floats(int32_t S, int32_t K, int32_t N, int32_t rank) {
+  const int64_t rp = (std::min(rank, 128) + 31) / 32 * 32;
+  int32_t nsu = 1, nsb = 1, nsu1 = 1, none = 0;
+  skinny_plan(S, N, true, &nsu, &nsb);
+  skinny_plan(S, N, false, &nsu1, &none);
+  return rp * std::max({(int64_t)nsu * S + (int64_t)nsb * N, (int64_t)nsu1 * S, (int64_t)stream_split(S, K) * S,
+                        (int64_t)stream_split(K, S) * K});
+}
+
+// Ranks in launches of up to 128; the dropout output is written by the first
+// (every launch draws the same bits).
+void launch_lora_down(const LoraDownArgs &d, hipStream_t st) {
+  for (int r0 = 0; r0 < d.rank; r0 += 128) {
+    LoraStream a = {};
+    a.x = d.x; a.x_rs = d.x_rs; a.rows = d.S; a.cols = d.K;
+    a.sm = reinterpret_cast<const bf16_t *>(d.A) + (int64_t)r0 * d.a_rs; a.sm_rs = d.a_rs;
+    a.part = d.part; a.rank = std::min(d.rank - r0, 128); a.ns = stream_split(d.S, d.K);
+    a.keep_scale = d.keep_scale; a.thr = d.thr; a.seed = d.seed;
+    a.h = r0 == 0 ? d.h : nullptr; a.h_rs = d.h_rs;
+    const int rb = (a.rank + 31) / 32;
+    switch (rb) {
+      case 1: down_rb<1>(a, d.thr > 0, st); break;
+      case 2: down_rb<2>(a, d.thr > 0, st); break;
+      case 3: down_rb<3>(a, d.thr > 0, st); break;
+      default: down_rb<4>(a, d.thr > 0, st); break;
+    }
+    const int64_t n = (int64_t)d.S * (8 * rb);
+    hipLaunchKernelGGL(lora_down_finish_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, 32 * rb,
+                       d.gate, d.scaling, reinterpret_cast<bf16_t *>(d.t) + r0, d.t_rs);
   }
-  const int64_t n = ((int64_t)a.S + (a.nsb > 0 ? a.N : 0)) * (a.rp / 4);
-  hipLaunchKernelGGL(lora_skinny_finish_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, gate, scaling,
-                     reinterpret_cast<bf16_t *>(da), da_rs, reinterpret_cast<bf16_t *>(db), db_rs);
+}
+
+void launch_lora_da(const LoraDaArgs &d, hipStream_t st) {
+  for (int r0 = 0; r0 < d.rank; r0 += 128) {
+    LoraStream a = {};
+    a.x = d.x; a.x_rs = d.x_rs; a.rows = d.S; a.cols = d.K;
+    a.sm = reinterpret_cast<const bf16_t *>(d.da) + r0; a.sm_rs = d.da_rs;
+    a.part = d.part; a.rank = std::min(d.rank - r0, 128); a.ns = stream_split(d.K, d.S);
+    a.keep_scale = d.keep_scale; a.thr = d.thr; a.seed = d.seed;
+    const int rb = (a.rank + 31) / 32;
+    const dim3 grid((unsigned)(blocks128(d.K) * a.ns)), blk(512);
+    switch (rb) {
+      case 1: hipLaunchKernelGGL((lora_da_kernel<1>), grid, blk, 0, st, a); break;
+      case 2: hipLaunchKernelGGL((lora_da_kernel<2>), grid, blk, 0, st, a); break;
+      case 3: hipLaunchKernelGGL((lora_da_kernel<3>), grid, blk, 0, st, a); break;
+      default: hipLaunchKernelGGL((lora_da_kernel<4>), grid, blk, 0, st, a); break;
+    }
+    const int64_t n = (int64_t)a.rank * (d.K / 4);
+    hipLaunchKernelGGL(lora_da_finish_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, 32 * rb,
+                       reinterpret_cast<bf16_t *>(d.dA) + (int64_t)r0 * d.dA_rs, d.dA_rs);
+  }
+}
+
+void launch_lora_grad_ub(const LoraSkinnyArgs &d, float *part, const float *gate, float scaling, void *da,
+                         int64_t da_rs, void *db, int64_t db_rs, hipStream_t st) {
+  LoraStream u = {}, b = {};
+  u.x = b.x = d.dy; u.x_rs = b.x_rs = d.dy_rs; u.rows = b.rows = d.S; u.cols = b.cols = d.N;
+  u.rank = b.rank = d.rank;
+  u.sm = d.b; u.sm_rs = d.b_rs; b.sm = d.t; b.sm_rs = d.t_rs;
+  skinny_plan(d.S, d.N, db != nullptr, &u.ns, &b.ns);
+  const int rb = (d.rank + 31) / 32;
+  u.part = part;
+  b.part = part + (int64_t)u.ns * d.S * (32 * rb);
+  const dim3 grid((unsigned)(blocks128(d.S) * u.ns + blocks128(d.N) * b.ns)), blk(512);
+  switch (rb) {
+    case 1: hipLaunchKernelGGL(lora_skinny_kernel<1>, grid, blk, 0, st, u, b); break;
+    case 2: hipLaunchKernelGGL(lora_skinny_kernel<2>, grid, blk, 0, st, u, b); break;
+    case 3: hipLaunchKernelGGL(lora_skinny_kernel<3>, grid, blk, 0, st, u, b); break;
+    default: hipLaunchKernelGGL(lora_skinny_kernel<4>, grid, blk, 0, st, u, b); break;
+  }
+  const int64_t n = ((int64_t)d.S + (b.ns > 0 ? d.N : 0)) * (8 * rb);
+  hipLaunchKernelGGL(lora_skinny_finish_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, u, b, 32 * rb,
+                     gate, scaling, reinterpret_cast<bf16_t *>(da), da_rs, reinterpret_cast<bf16_t *>(db), db_rs);
 }
 
 }  // namespace mga

@@ -290,3 +290,22 @@ def test_long_reductions(dev, S, K, N, r):
     ref = base + d_a @ Ad
     bound = U * (ref.abs() + (ref - base).abs() + d_a.abs() @ Ad.abs()) + 1e-5 * ref.abs().max()
     assert bool(((gx.double() - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("S,K,N,r,p,gate", [
+    (129, 144, 136, 128, 0.3, "mixed"),     # one line past a block, a column tail in every product, the largest rank block
+    (65, 208, 72, 100, 0.05, "mixed"),      # ranks past 96 that are not a multiple of 32; 16-column tails
+    (1, 16, 8, 3, 0.5, None),               # a single row, the smallest columns (p = 1/2 scales exactly: h is not rounded,
+                                            # as the dA and dB bounds, which have no term for it, need at one row)
+    (700, 4096, 256, 33, 0.9375, "mixed"),  # nearly everything dropped (again an exact scale); more splits than line blocks
+    (260, 1168, 520, 130, 0.1, "mixed"),    # ranks in two launches, one of two ranks
+])
+def test_streaming_edges(dev, S, K, N, r, p, gate):
+    """The streaming products and the wide writes at the edges of their 128-line
+    blocks, 64-wide chunks and rank blocks."""
+    run_case(dev, S, K, N, r, p, gate=gate, seed=S + r)
+
+
+def test_unaligned_rows_take_the_library_products(dev):
+    """N = 4: lora_B's products and the up-projection cannot use 16-byte rows."""
+    run_case(dev, 70, 256, 4, 12, 0.1, seed=3)
