@@ -6,6 +6,7 @@ if it is missing every operation raises, naming the build command.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 import threading
 from pathlib import Path
@@ -119,13 +120,50 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+def raise_error(name: str, rc: int) -> None:
+    msg = load().mga_last_error().decode(errors="replace")
+    cls = CapacityError if rc == MGA_ERR_CAPACITY else MGAError
+    raise cls(name, rc, msg)
+
+
 def call(name: str, *args) -> None:
     fn = getattr(load(), name)
     rc = fn(*args)
     if rc != MGA_OK:
-        msg = load().mga_last_error().decode(errors="replace")
-        cls = CapacityError if rc == MGA_ERR_CAPACITY else MGAError
-        raise cls(name, rc, msg)
+        raise_error(name, rc)
+
+
+TORCH_MODULE_PATH = _HERE / "lib" / "_mga_torch.so"
+_torch_module = None
+
+
+def load_torch_module():
+    """The native forms of the per-layer calls (csrc/mga_torch.cpp), bound to
+    the loaded library; raise if the module has not been built."""
+    global _torch_module
+    if _torch_module is not None:
+        return _torch_module
+    lib = load()
+    with _lock:
+        if _torch_module is None:
+            if not TORCH_MODULE_PATH.exists():
+                raise RuntimeError(f"{TORCH_MODULE_PATH} is missing: build it with `python __graft_entry__.py` "
+                                   "(or mtp-glora_amd/build.py)")
+            spec = importlib.util.spec_from_file_location("_mga_torch", TORCH_MODULE_PATH)
+            module = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(module)
+            module.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in SIGNATURES},
+                        raise_error)
+            _torch_module = module
+    return _torch_module
+
+
+def native(name: str, t, *args):
+    """``name``(t, *args) of the native module for a GPU tensor t; None where
+    the call is not of the form it takes (the Python form then runs)."""
+    if not getattr(t, "is_cuda", False):
+        return None
+    return getattr(_torch_module or load_torch_module(), name)(t, *args)
 
 
 def version() -> int:

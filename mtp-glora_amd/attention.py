@@ -90,6 +90,12 @@ def mtp_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
     if k0 != v0:
         raise RuntimeError("key and value have different gradient starts")
     # the kernels read K/V from the full views; gradients go to k_src / v_src
+    r = _lib.native("attention", query, k_src, v_src, key, value,
+                    [mask.mtp_code, mask.kv_num_blocks, mask.kv_indices, mask.full_kv_num_blocks,
+                     mask.full_kv_indices, mask.q_num_blocks, mask.q_indices, mask.full_q_num_blocks,
+                     mask.full_q_indices], mask.prefix_len, float(scale), k0)
+    if r is not None:
+        return r
     return _MTPAttention.apply(query, k_src, v_src, key.detach(), value.detach(), mask,
                                float(scale), k0)
 

@@ -1,14 +1,17 @@
-"""Build recipe for libmtp_glora_amd.so (gfx950), in-tree.
+"""Build recipe for libmtp_glora_amd.so (gfx950) and the torch module, in-tree.
 
 ``python -m`` is not needed: ``build_library()`` runs hipcc on every
 ``csrc/*.hip`` file and links them into ``lib/libmtp_glora_amd.so`` next to
-this file. hipcc cross-compiles for gfx950 without a GPU present.
+this file; hipcc cross-compiles for gfx950 without a GPU present.
+``build_torch_module()`` compiles ``csrc/mga_torch.cpp`` (host code only)
+against the installed torch into ``lib/_mga_torch.so``.
 """
 from __future__ import annotations
 
 import os
 import shutil
 import subprocess
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -16,6 +19,7 @@ PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 LIB_DIR = PKG_DIR / "lib"
 LIB_NAME = "libmtp_glora_amd.so"
+TORCH_MODULE = "_mga_torch.so"
 ARCH = os.environ.get("MGA_OFFLOAD_ARCH", "gfx950")
 
 # Packed fp32 VALU ops are disabled for every device pass (hipcc's host pass
@@ -83,5 +87,28 @@ def build_library(verbose: bool = False, jobs: int = 4, src_dir=None, out_path=N
     return out
 
 
+def build_torch_module(verbose: bool = False) -> Path:
+    """Compile csrc/mga_torch.cpp into lib/_mga_torch.so."""
+    import torch
+    from torch.utils import cpp_extension
+    out = LIB_DIR / TORCH_MODULE
+    LIB_DIR.mkdir(parents=True, exist_ok=True)
+    tmp = out.with_suffix(".so.tmp")
+    include = [*cpp_extension.include_paths("cuda"), sysconfig.get_paths()["include"], "/opt/rocm/include"]
+    cmd = [shutil.which("g++") or "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+           *(f"-isystem{p}" for p in include), str(CSRC / "mga_torch.cpp"), "-o", str(tmp),
+           *(f"-L{p}" for p in cpp_extension.library_paths()), "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu",
+           "-ltorch_python"]
+    res = subprocess.run(cmd, capture_output=True, text=True, timeout=COMPILE_TIMEOUT_S)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed on mga_torch.cpp:\n{res.stderr}")
+    if verbose:
+        print(" ".join(cmd))
+    os.replace(tmp, out)
+    return out
+
+
 if __name__ == "__main__":
+    print(build_torch_module(verbose=True))
     print(build_library(verbose=True))

@@ -25,7 +25,7 @@ import os
 
 import torch
 
-from . import ops
+from . import _lib, ops
 
 DEFAULT_CAPACITY = int(os.environ.get("MGA_CACHE_CAPACITY", 131072 + 16384))
 
@@ -137,9 +137,15 @@ class StreamingKVCache:
         P = self.prefix_len
         S = key_states.shape[2]
         kb, vb = self._k[layer_idx], self._v[layer_idx]
-        in_place = self._in_place(key_states, kb, P), self._in_place(value_states, vb, P)
+        restage = getattr(key_states, "_mga_restage", None)
+        r = _lib.native("update_kv", key_states, value_states, kb, vb, P, restage is not None)
+        if r is not None:
+            kf, vf, staged = r
+            in_place = staged, staged
+        else:
+            kf = vf = None
+            in_place = self._in_place(key_states, kb, P), self._in_place(value_states, vb, P)
         if in_place == (True, True):
-            restage = getattr(key_states, "_mga_restage", None)
             if restage is None:
                 raise ValueError("key / value states sit in the cache rows without a way to re-stage their "
                                  "regular rows (stage them with rope.qk_norm_rope_stage)")
@@ -147,16 +153,18 @@ class StreamingKVCache:
         elif any(in_place):
             raise ValueError("only one of key / value states sits in the cache rows")
         else:
-            ops.kv_append(key_states, value_states, kb, vb, dst_offset=P)   # raises on capacity
+            if kf is None:
+                ops.kv_append(key_states, value_states, kb, vb, dst_offset=P)   # raises on capacity
             self._staged[layer_idx] = (key_states, value_states)
-        self._bump(layer_idx)
         self._len[layer_idx] = P + S
-        kf = kb[None, :, :P + S]
-        vf = vb[None, :, :P + S]
-        if key_states.requires_grad:
-            kf = _StageKV.apply(key_states, kf)
-        if value_states.requires_grad:
-            vf = _StageKV.apply(value_states, vf)
+        if kf is None:
+            self._bump(layer_idx)
+            kf = kb[None, :, :P + S]
+            vf = vb[None, :, :P + S]
+            if key_states.requires_grad:
+                kf = _StageKV.apply(key_states, kf)
+            if value_states.requires_grad:
+                vf = _StageKV.apply(value_states, vf)
         # read by the HIP attention to send dK/dV straight to the chunk's K/V
         kf._mga_stage = (key_states, P)
         vf._mga_stage = (value_states, P)

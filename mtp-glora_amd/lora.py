@@ -32,6 +32,7 @@ and Llama projections have none), base weights frozen.
 """
 from __future__ import annotations
 
+import ctypes
 import math
 import warnings
 from typing import List
@@ -159,7 +160,9 @@ def gated_lora_linear(x, weight, lora_a, lora_b, gate_mask, scaling: float, drop
         raise NotImplementedError("the base weight must be frozen (the fused layer computes no gradient for it)")
     if seed is None:
         seed = int(torch.randint(0, 2 ** 62, (), dtype=torch.int64).item()) if dropout_p > 0 else 0
-    return _GatedLoRA.apply(x, weight, lora_a, lora_b, gate_mask, float(scaling), float(dropout_p), int(seed))
+    args = (x, weight, lora_a, lora_b, gate_mask, float(scaling), float(dropout_p))
+    y = _lib.native("gated_lora", *args, ctypes.c_int64(int(seed)).value)   # the seed's 64 bits
+    return y if y is not None else _GatedLoRA.apply(*args, int(seed))
 
 
 class GatedLoRALinear(nn.Module):

@@ -78,6 +78,14 @@ def soft_ce_backward(student: torch.Tensor, teacher: torch.Tensor, stats: torch.
 class StableSoftCrossEntropy(torch.autograd.Function):
     """Drop-in for mtp_glora/core/loss.py:259-330 (called at core/mtp.py:126)."""
 
+    @classmethod
+    def apply(cls, *args):
+        if cls is StableSoftCrossEntropy and len(args) == 2:
+            r = _lib.native("soft_ce", *args)
+            if r is not None:
+                return r
+        return super().apply(*args)
+
     @staticmethod
     def forward(ctx, student_logits: torch.Tensor, teacher_logits: torch.Tensor):
         if student_logits.ndim != 3 or teacher_logits.ndim != 3:

@@ -237,8 +237,8 @@ def qk_norm_rope_stage(query_states, key_states, value_states, q_weight, k_weigh
         if cos.requires_grad or sin.requires_grad:
             raise NotImplementedError("cos / sin require grad; the fused rope computes no gradient for them")
     k_dst, v_dst = cache.stage_rows(layer_idx, key_states.transpose(1, 2))
-    qe, ke, ve = _QKNormRopeStage.apply(query_states, key_states, value_states, q_weight, k_weight, cos, sin,
-                                        eps, k_dst, v_dst)
+    args = (query_states, key_states, value_states, q_weight, k_weight, cos, sin, eps, k_dst, v_dst)
+    qe, ke, ve = _lib.native("norm_rope_stage", *args) or _QKNormRopeStage.apply(*args)
     ke._mga_restage = _Restage(key_states, value_states, k_weight, cos, sin, eps)
     return qe, ke, ve
 
