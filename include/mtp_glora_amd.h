@@ -91,6 +91,15 @@ int mga_regular_index(const int64_t *regular_mask, int64_t stride, int32_t n,
                       int32_t *idx, int32_t *count, void *stream);
 
 /*
+ * mga_regular_index together with the position check of collator.py:251-258,
+ * queued without a host wait: count_mismatch[0] = count, count_mismatch[1] = 1
+ * when positions[idx[j] * position_stride] != P + j for any j < count, else 0.
+ */
+int mga_regular_index_check(const int64_t *regular_mask, int64_t stride, int32_t n, int32_t *idx,
+                            const int64_t *positions, int64_t position_stride, int64_t P,
+                            int32_t *count_mismatch, void *stream);
+
+/*
  * MTP block mask of a chunk with S tokens against a P-token cached prefix:
  * writes the per-token codes and the eight BlockMask tensors that
  * create_block_mask(mask_mod, B=None, H=None, Q_LEN=S, KV_LEN=P+S) returns for

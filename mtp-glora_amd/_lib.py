@@ -39,6 +39,7 @@ SIGNATURES = {
     "mga_last_error": [],
     "mga_kv_append": [_P, _P, _I64, _I64, _I64, _P, _I32, _P, _P, _I64, _I64, _I64, _I64, _I32, _I32, _I32, _P],
     "mga_regular_index": [_P, _I64, _I32, _P, _P, _P],
+    "mga_regular_index_check": [_P, _I64, _I32, _P, _P, _I64, _I64, _P, _P],
     "mga_mtp_block_mask": [_P, _I64, _I32, _I64, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P],
     "mga_attn_fwd": [_P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64,
                      _P, _P, _P, _P, _P, _P,

@@ -173,8 +173,21 @@ int mga_regular_index(const int64_t *regular_mask, int64_t stride, int32_t n, in
                       int32_t *count, void *stream) {
   if (!regular_mask || !idx || !count) return fail(MGA_ERR_INVALID, "mga_regular_index: null pointer");
   if (n <= 0 || stride <= 0) return fail(MGA_ERR_INVALID, "mga_regular_index: bad size/stride (%d, %lld)", n, (long long)stride);
-  mga::launch_regular_index(regular_mask, stride, n, idx, count, (hipStream_t)stream);
+  mga::launch_regular_index(regular_mask, stride, n, idx, nullptr, 0, 0, count, (hipStream_t)stream);
   return check_launch("mga_regular_index");
+}
+
+int mga_regular_index_check(const int64_t *regular_mask, int64_t stride, int32_t n, int32_t *idx,
+                            const int64_t *positions, int64_t position_stride, int64_t P, int32_t *count_mismatch,
+                            void *stream) {
+  const char *fn = "mga_regular_index_check";
+  if (!regular_mask || !idx || !positions || !count_mismatch) return fail(MGA_ERR_INVALID, "%s: null pointer", fn);
+  if (n <= 0 || stride <= 0 || position_stride <= 0)
+    return fail(MGA_ERR_INVALID, "%s: bad size/strides (%d, %lld, %lld)", fn, n, (long long)stride,
+                (long long)position_stride);
+  mga::launch_regular_index(regular_mask, stride, n, idx, positions, position_stride, P, count_mismatch,
+                            (hipStream_t)stream);
+  return check_launch(fn);
 }
 
 int mga_mtp_block_mask(const int64_t *gate, int64_t gate_stride, int32_t S, int64_t P,

@@ -156,6 +156,50 @@ __device__ __forceinline__ int key_code(const int32_t *code, int key, int P, int
   return key < P ? kCodeX : (key < L ? code[key - P] : kCodePad);
 }
 
+// Scan of a chunk's tokens by one 1024-thread workgroup: wave w takes the
+// tokens [begin, end), a multiple of 64 of them, lane l every 64th, so that a
+// wave's loads are one contiguous run each and independent of each other (a
+// contiguous segment per thread reads 16 lines per wave and load). bits holds
+// the lane's first 64 flags, so that the caller's second walk over the tokens
+// does not wait for them again; sums is LDS for 16 counts. n > 0.
+struct WaveSpan {
+  int begin, end, before, total;   // before: flags in the earlier waves' tokens
+  uint64_t bits;
+};
+template <typename F>
+__device__ __forceinline__ WaveSpan scan_flags(int n, int *sums, F flag) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int per = (n + 1023) / 1024 * 64;
+  WaveSpan s;
+  s.begin = min(n, wave * per);
+  s.end = min(n, s.begin + per);
+  s.bits = 0;
+  int c = 0, k = 0;
+  for (int i0 = s.begin + lane; i0 < s.end; i0 += 512, k += 8) {
+    bool f[8];   // eight loads in flight, clamped instead of skipped past the end
+#pragma unroll
+    for (int u = 0; u < 8; ++u) f[u] = flag(min(i0 + 64 * u, n - 1)) && i0 + 64 * u < s.end;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      c += f[u];
+      if (k < 64) s.bits |= (uint64_t)f[u] << (k + u);
+    }
+  }
+  for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, 64);
+  if (lane == 0) sums[wave] = c;
+  __syncthreads();
+  s.before = s.total = 0;
+  for (int w = 0; w < 16; ++w) {
+    const int v = sums[w];
+    s.before += w < wave ? v : 0;
+    s.total += v;
+  }
+  return s;
+}
+
+// Lanes below this one.
+__device__ __forceinline__ uint64_t lanes_below() { return (uint64_t(1) << (threadIdx.x & 63)) - 1; }
+
 // WG id -> logical work index so that consecutive logical indices land on the
 // same XCD (the hardware deals WG ids round-robin over the 8 XCDs).
 __device__ __forceinline__ int xcd_swizzle(int b, int n) {

@@ -31,8 +31,8 @@ void launch_kv_copy_rows(const void *src_k, const void *src_v, int64_t src_sh_b,
                          int64_t dst_sh_b, int64_t dst_ss_b, int64_t dst_off, int32_t n_heads,
                          int32_t row_bytes, hipStream_t stream);
 
-void launch_regular_index(const int64_t *mask, int64_t stride, int32_t n, int32_t *idx,
-                          int32_t *count, hipStream_t stream);
+void launch_regular_index(const int64_t *mask, int64_t stride, int32_t n, int32_t *idx, const int64_t *pos,
+                          int64_t pos_stride, int64_t P, int32_t *out, hipStream_t stream);
 
 void launch_mtp_block_mask(const int64_t *gate, int64_t gate_stride, int32_t S, int64_t P,
                            int32_t *code, int8_t *cls, int32_t *kv_num, int32_t *kv_idx,

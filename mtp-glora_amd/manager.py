@@ -74,16 +74,20 @@ class StreamingKVCacheManager:
         self._pending = None
         reg = chunk_data.get("regular_token_mask")
         if isinstance(reg, torch.Tensor) and reg.is_cuda:
-            idx, cnt = ops.regular_index(reg[0])
             if self._host is None:
                 self._host = torch.empty(2, dtype=torch.int32, pin_memory=True)
             pos = chunk_data.get("position_ids") if self.sanity_check else None
             check = None
-            if isinstance(pos, torch.Tensor) and pos.is_cuda and pos.dim() == 2 and pos.shape[1] == idx.numel():
+            row = reg[0]
+            if isinstance(pos, torch.Tensor) and pos.is_cuda and pos.dim() == 2 and pos.shape[1] == row.numel():
                 check = (pos, pos._version, self.past_seen_tokens)
-                src = torch.cat([cnt, self._position_mismatch(pos[0], idx, cnt, self.past_seen_tokens)])
+                if pos.dtype == torch.int64 and pos.device == row.device and pos.stride(1) > 0 and row.dim() == 1:
+                    idx, src = ops.regular_index(row, pos[0], self.past_seen_tokens)
+                else:
+                    idx, cnt = ops.regular_index(row)
+                    src = torch.cat([cnt, self._position_mismatch(pos[0], idx, cnt, self.past_seen_tokens)])
             else:
-                src = cnt
+                idx, src = ops.regular_index(row)
             self._host[:src.numel()].copy_(src, non_blocking=True)
             event = torch.cuda.Event()
             event.record()

@@ -68,6 +68,8 @@ def kv_append(src_k: torch.Tensor, src_v: torch.Tensor, dst_k: torch.Tensor, dst
 
     src: [1, H, S, D] or [H, S, D] views; dst: [H, capacity, D] buffers.
     """
+    if _lib.native("kv_append", src_k, src_v, dst_k, dst_v, dst_offset, idx, n_rows):
+        return
     sk, ssh, sss = _rows("src_k", src_k)
     sv, vsh, vss = _rows("src_v", src_v)
     if (vsh, vss) != (ssh, sss) or sv.shape != sk.shape:
@@ -95,9 +97,11 @@ def kv_append(src_k: torch.Tensor, src_v: torch.Tensor, dst_k: torch.Tensor, dst
               int(dst_offset), cap, H, D, dtype_code(dst_k.dtype), _stream(dst_k))
 
 
-def regular_index(regular_mask: torch.Tensor):
+def regular_index(regular_mask: torch.Tensor, positions: torch.Tensor | None = None, P: int = 0):
     """int32 indices of the nonzero entries of a [1, S] (or [S]) int64 mask,
-    plus the device count. Returns (idx[S], count[1])."""
+    plus the device count. Returns (idx[S], count[1]); with ``positions``
+    ([S] int64) (idx[S], [count, mismatch]), mismatch 1 when the regular
+    tokens' positions are not P, P + 1, ..."""
     _dev("regular_token_mask", regular_mask)
     m = regular_mask.reshape(-1) if regular_mask.dim() == 2 and regular_mask.shape[0] == 1 else regular_mask
     if m.dim() != 1:
@@ -106,6 +110,14 @@ def regular_index(regular_mask: torch.Tensor):
         m = m.to(torch.int64)
     n = m.numel()
     idx = torch.empty(n, dtype=torch.int32, device=m.device)
+    if positions is not None:
+        _dev("positions", positions)
+        if positions.dtype != torch.int64 or tuple(positions.shape) != (n,):
+            raise TypeError(f"positions: expected [{n}] int64, got {tuple(positions.shape)} {positions.dtype}")
+        out = torch.empty(2, dtype=torch.int32, device=m.device)
+        _lib.call("mga_regular_index_check", m.data_ptr(), m.stride(0), n, idx.data_ptr(), positions.data_ptr(),
+                  positions.stride(0), int(P), out.data_ptr(), _stream(m))
+        return idx, out
     cnt = torch.empty(1, dtype=torch.int32, device=m.device)
     _lib.call("mga_regular_index", m.data_ptr(), m.stride(0), n, idx.data_ptr(), cnt.data_ptr(),
               _stream(m))

@@ -66,3 +66,27 @@ def test_block_mask_config_sizes(mga, dev, cfg):
     want = mo.block_mask_mtp(seq.gate, cfg["P"])
     for n in NAMES:
         assert np.array_equal(getattr(bm, n).cpu().numpy(), want[n]), n
+
+
+@pytest.mark.parametrize("S,P", [(1, 0), (64, 1), (65, 127), (128, 128), (129, 0), (200, 129), (513, 256), (1100, 300)])
+@pytest.mark.parametrize("kind", ["mixed", "masks", "regular", "pads_within"])
+def test_codes_and_lists_at_tile_edges(mga, dev, S, P, kind):
+    """Codes, classes and lists against the predicate written out densely, with the codes in any order."""
+    g = torch.Generator().manual_seed(S)
+    gate = {"mixed": torch.randint(0, 2, (S,), generator=g), "masks": torch.ones(S, dtype=torch.long),
+            "regular": torch.zeros(S, dtype=torch.long), "pads_within": torch.randint(-1, 2, (S,), generator=g)}[kind]
+    t = mga.ops.mtp_block_mask_tensors(gate.to(dev)[None], P)
+    code = torch.where(gate == -1, -1, torch.where(gate == 0, -2, P + (gate == 0).cumsum(0)))
+    assert torch.equal(t["code"].cpu().long(), code)
+    keys = torch.cat([torch.full((P,), -2), code])
+    allowed = (torch.arange(P + S)[None] <= torch.arange(P, P + S)[:, None]) & (code != -1)[:, None] \
+        & ((keys == -2)[None] | (keys[None] == code[:, None]))
+    nq, nk = -(-S // 128), -(-(P + S) // 128)
+    tiles = torch.zeros(nq * 128, nk * 128)
+    tiles[:S, :P + S] = allowed
+    n = tiles.view(nq, 128, nk, 128).sum((1, 3))
+    for want, pre in (((n > 0) & (n < 128 * 128), ""), (n == 128 * 128, "full_")):
+        for sel, name in ((want, "kv"), (want.T, "q")):
+            num, idx = t[f"{pre}{name}_num_blocks"][0, 0].cpu(), t[f"{pre}{name}_indices"][0, 0].cpu()
+            assert torch.equal(num.long(), sel.sum(1))
+            assert torch.equal(idx.long(), torch.argsort(sel.int(), dim=1, descending=True, stable=True))

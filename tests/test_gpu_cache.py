@@ -190,3 +190,26 @@ def test_take_over_dynamic_cache(mga, dev):
     assert isinstance(out, mga.StreamingKVCache) and out.prefix_len == len(idx)
     for i, (k, v) in enumerate(out):
         assert torch.equal(k, ks[i][:, :, idx]) and torch.equal(v, (ks[i] + 1)[:, :, idx])
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 511, 513, 1024, 1025, 5121, 65536, 66000])
+def test_regular_index_check(mga, dev, n):
+    """Index, count and position flag at the edges of the waves' spans and of the flags kept in registers."""
+    g = torch.Generator().manual_seed(n)
+    for keep in (0.0, 0.3, 1.0):
+        reg = (torch.rand(n, generator=g) < keep).long()
+        ref = reg.nonzero(as_tuple=True)[0]
+        pos = torch.randint(0, 50, (n, 2), generator=g)
+        pos[ref, 0] = 77 + torch.arange(ref.numel())
+        dmask = torch.stack([reg, 1 - reg], 1).to(dev)[:, 0]      # stride 2, as the positions
+        for wrong in (None, *ref[:1].tolist(), *ref[-1:].tolist()):
+            p = pos.clone()
+            if wrong is not None:
+                p[wrong, 0] += 1
+            idx, out = mga.ops.regular_index(dmask, p.to(dev)[:, 0], 77)
+            assert out.tolist() == [ref.numel(), int(wrong is not None)]
+            assert torch.equal(idx[:ref.numel()].cpu().long(), ref)
+        idx, cnt = mga.ops.regular_index(dmask)
+        assert cnt.item() == ref.numel() and torch.equal(idx[:ref.numel()].cpu().long(), ref)
+    with pytest.raises(TypeError):
+        mga.ops.regular_index(dmask, pos.to(dev)[:, 0].int(), 77)
