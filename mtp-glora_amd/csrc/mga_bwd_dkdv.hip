@@ -30,6 +30,7 @@
 // over the query heads of a kv head, :957-966), restricted to keys >=
 // grad_start; dS formed from the fp32 P and rounded only before the dK
 // product, as [torch]_inductor/kernel/flex/templates/flex_backwards.py.jinja:570-618.
+#include <algorithm>
 #include <type_traits>
 
 #include "mga_common.hpp"
@@ -60,15 +61,15 @@ __device__ __forceinline__ V rows16(const void *t, uint32_t ofs) {
 }
 typedef __attribute__((__vector_size__(16 * sizeof(uint32_t)))) uint32_t u32x16;
 
-// The group's walk over its (query tile, head) pairs gr, gr + 2, ...: four
+// The group's walk over its (query tile, head) pairs p, p + 2, ...: four
 // 32-row steps per pair, the step within the pair being the index of the
 // four-fold unrolled step loop. Advanced once per pair (no division).
 struct PairWalk {
   int k, hh, it;
-  __device__ __forceinline__ void init(int gr, int G) {
+  __device__ __forceinline__ void init(int p, int G) {
     k = 0;
-    it = gr / G;
-    hh = gr - it * G;
+    it = p / G;
+    hh = p - it * G;
   }
   __device__ __forceinline__ void next(int G) {
     ++k;
@@ -89,7 +90,7 @@ struct PairInfo {
 }  // namespace
 
 template <int HD, typename T>
-__global__ __launch_bounds__(kThreads, 1) void attn_bwd_dkdv_kernel(AttnArgs a, int kh0, int nkh) {
+__global__ __launch_bounds__(kThreads, 1) void attn_bwd_dkdv_kernel(AttnArgs a, int kh0, int nkh, int ns) {
   typedef typename MfmaElem<T>::type E;
   constexpr int KS = HD / 16;
   constexpr int DB = HD / 32;
@@ -120,10 +121,11 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_dkdv_kernel(AttnArgs a, 
   const int G = a.Hq / a.Hkv;
 
   // item: kv head major (its key tiles share an XCD), key tiles in order (the
-  // first ones have the longest query lists)
-  const int li = xcd_swizzle(blockIdx.x, a.Hkv * nkh);
-  const int g = li / nkh;
-  const int kh = kh0 + li % nkh;
+  // first ones have the longest query lists), the parts of a tile together
+  const int li = xcd_swizzle(blockIdx.x, a.Hkv * nkh * ns);
+  const int item = li / ns, part = li - item * ns;
+  const int g = item / nkh;
+  const int kh = kh0 + item % nkh;
   const int kt = (kh * kKeys) / kBlock;     // block-mask key tile
 
   const int key = kh * kKeys + half * 32 + l32;
@@ -149,8 +151,10 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_dkdv_kernel(AttnArgs a, 
 
   TileList tiles = tile_list(a.q_num, a.q_idx, a.fq_num, a.fq_idx, kt, a.nQ);
   const int npart = tiles.npart;
-  const int npairs = G * tiles.ntot;                   // (query tile, head) pairs
-  const int mine = (npairs - gr + 1) / 2;              // pairs gr, gr + 2, ...
+  const int nall = G * tiles.ntot;                     // (query tile, head) pairs
+  const int first = nall * part / ns;                  // this part's: first .. first + npairs - 1
+  const int npairs = nall * (part + 1) / ns - first;
+  const int mine = (npairs - gr + 1) / 2;              // pairs first + gr, first + gr + 2, ...
   const int nsteps_other = 4 * ((npairs - (1 - gr) + 1) / 2);
   const int niter = (max(4 * mine, nsteps_other) + 1 + 3) / 4 * 4;   // + 1: B's last dK step
 
@@ -259,7 +263,7 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_dkdv_kernel(AttnArgs a, 
   PairWalk wkb;   // B: the pair after qp
   PairBase qp, dp_;   // B: pairs of the Q loads (step j + 2) and of the dO and row-data loads (step j + 1)
   if (role == 1) {
-    wkb.init(gr, G);
+    wkb.init(first + gr, G);
     qp = pbase(pinfo(wkb));
     wkb.next(G);
     dp_ = qp;
@@ -282,7 +286,7 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_dkdv_kernel(AttnArgs a, 
   if (role == 0) {
     // ------------------------------------------------------------------ A
     PairWalk wk;
-    wk.init(gr, G);
+    wk.init(first + gr, G);
     PairInfo cur;
     auto stepA = [&](auto jsel) {
       constexpr int J = decltype(jsel)::value;
@@ -459,6 +463,17 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_dkdv_kernel(AttnArgs a, 
         const f32x4 v = *reinterpret_cast<const f32x4 *>(x + ((db * 4 + q) * 64 + lane) * 4);
         acc[db][4 * q] += v[0]; acc[db][4 * q + 1] += v[1]; acc[db][4 * q + 2] += v[2]; acc[db][4 * q + 3] += v[3];
       }
+    if (ns > 1) {   // the part's sums: attn_bwd_dkdv_merge_kernel adds them
+      float *po = a.ws + ((int64_t)li * 4 + half * 2 + role) * (HD * 32);
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const f32x4 v = {acc[db][4 * q], acc[db][4 * q + 1], acc[db][4 * q + 2], acc[db][4 * q + 3]};
+          *reinterpret_cast<f32x4 *>(po + ((db * 4 + q) * 64 + lane) * 4) = v;
+        }
+      return;
+    }
     // lane = key, registers = dims 8 (r / 4) + 4 hi + r % 4 of block db
     if (key >= a.grad_start && key < a.L) {
       const int64_t row = key - a.grad_start;
@@ -475,19 +490,112 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_dkdv_kernel(AttnArgs a, 
   }
 }
 
+// dK and dV of the items that ran in parts: the parts' fp32 sums added in the
+// order of the parts. Workgroup (item, 32-dim block db), wave (half, role) as in
+// the item's group 0: lane = key, registers = dims.
+template <int HD, typename T>
+__global__ __launch_bounds__(256) void attn_bwd_dkdv_merge_kernel(AttnArgs a, int kh0, int nkh, int ns) {
+  constexpr int DB = HD / 32;
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int hi = lane >> 5, half = wave >> 1, role = wave & 1;
+  const int item = blockIdx.x / DB, db = blockIdx.x % DB;
+  const int g = item / nkh;
+  const int key = (kh0 + item % nkh) * kKeys + half * 32 + (lane & 31);
+  if (key < a.grad_start || key >= a.L) return;
+  const float *p0 = a.ws + ((int64_t)item * ns * 4 + wave) * (HD * 32) + (db * 256 + lane) * 4;
+  f32x4 v[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) v[q] = *reinterpret_cast<const f32x4 *>(p0 + q * 256);
+#pragma unroll 2
+  for (int p = 1; p < ns; ++p) {
+    const float *pp = p0 + (int64_t)p * (4 * HD * 32);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const f32x4 t = *reinterpret_cast<const f32x4 *>(pp + q * 256);
+      v[q][0] += t[0]; v[q][1] += t[1]; v[q][2] += t[2]; v[q][3] += t[3];
+    }
+  }
+  const int64_t row = key - a.grad_start;
+  const float f = role == 0 ? 1.f : a.scale;
+  T *out = role == 0 ? reinterpret_cast<T *>(a.dv) + g * a.dv_sh + row * a.dv_ss
+                     : reinterpret_cast<T *>(a.dk) + g * a.dk_sh + row * a.dk_ss;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) store4(out + db * 32 + 8 * q + 4 * hi, v[q][0] * f, v[q][1] * f, v[q][2] * f, v[q][3] * f);
+}
+
 // explicit instantiations: clang otherwise drops some host launch stubs of
-// this template, leaving undefined symbols
-template __global__ void attn_bwd_dkdv_kernel<128, bf16_t>(AttnArgs, int, int);
-template __global__ void attn_bwd_dkdv_kernel<64, bf16_t>(AttnArgs, int, int);
-template __global__ void attn_bwd_dkdv_kernel<128, f16_t>(AttnArgs, int, int);
-template __global__ void attn_bwd_dkdv_kernel<64, f16_t>(AttnArgs, int, int);
+// these templates, leaving undefined symbols
+#define MGA_DKDV_INST(HD, T)                                                          \
+  template __global__ void attn_bwd_dkdv_kernel<HD, T>(AttnArgs, int, int, int);      \
+  template __global__ void attn_bwd_dkdv_merge_kernel<HD, T>(AttnArgs, int, int, int);
+MGA_DKDV_INST(128, bf16_t)
+MGA_DKDV_INST(64, bf16_t)
+MGA_DKDV_INST(128, f16_t)
+MGA_DKDV_INST(64, f16_t)
+#undef MGA_DKDV_INST
+
+namespace {
+
+struct DkdvGrid {
+  int kh0, nkh;
+};
+DkdvGrid dkdv_grid(const AttnArgs &a) {
+  const int kh0 = a.grad_start / kKeys;
+  return {kh0, (a.L + kKeys - 1) / kKeys - kh0};
+}
+
+// Parts of every item. Unsplit, the launch lasts at least as long as the first
+// key tile's walk over all query tiles and heads, however few the items are
+// (one workgroup a CU). Measured in steps of about 1.1 us (32 rows of two
+// pairs), an XCD's share of the items, the heaviest being the first, ends at
+// about the larger of its longest part and its total over its CUs; a part costs
+// kPartSteps beyond its walk (key operands, cleared LDS, the groups' exchange),
+// the combining launch kMergeSteps and the traffic of the parts. A part keeps at
+// least two pairs a group; the lists are taken as causal ones.
+constexpr float kPartSteps = 5.f, kMergeSteps = 5.f, kStepSeconds = 1.1e-6f, kPartBytesPerSecond = 4e12f;
+constexpr int kMaxDkdvParts = 8;
+int dkdv_parts(const AttnArgs &a, int head_dim) {
+  if (a.grad_start >= a.L) return 1;
+  const DkdvGrid f = dkdv_grid(a);
+  const int slots = std::max(device_cu_count() / 8, 1), G = a.Hq / a.Hkv;
+  const int64_t items = (int64_t)a.Hkv * f.nkh, share = (items + 7) / 8;
+  if (share > 4 * slots) return 1;   // rounds enough to even out by themselves
+  auto steps = [&](int64_t i) {   // of key tile kh0 + i
+    const int64_t first = std::max((f.kh0 + i) * kKeys - a.P, (int64_t)0) / kBlock;
+    return 2.f * G * (float)(a.nQ - first);
+  };
+  float total = 0.f;
+  for (int64_t i = 0; i < share; ++i) total += steps(i % f.nkh);
+  const float longest = steps(0), traffic = (float)items * (kKeys * 2 * 4 * 2) * head_dim;
+  int best = 1;
+  float best_cost = std::max(longest, total / slots) + kPartSteps;
+  for (int ns = 2; ns <= kMaxDkdvParts && longest >= 16.f * ns; ++ns) {
+    const float cost = std::max(longest / ns + kPartSteps, (total + (float)share * ns * kPartSteps) / slots) +
+                       kMergeSteps + ns * traffic / (kPartBytesPerSecond * kStepSeconds);
+    if (cost < best_cost) {
+      best = ns;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
+}  // namespace
+
+int64_t dkdv_ws_floats(const AttnArgs &a, int head_dim) {
+  const int ns = dkdv_parts(a, head_dim);
+  return ns > 1 ? (int64_t)a.Hkv * dkdv_grid(a).nkh * ns * (kKeys * 2) * head_dim : 0;
+}
 
 template <int HD, typename T>
 void dkdv_launch(const AttnArgs &a, hipStream_t st) {
   if (a.grad_start >= a.L) return;
-  const int kh0 = a.grad_start / kKeys;
-  const int nkh = (a.L - kh0 * kKeys + kKeys - 1) / kKeys;
-  hipLaunchKernelGGL((attn_bwd_dkdv_kernel<HD, T>), dim3(a.Hkv * nkh), dim3(kThreads), 0, st, a, kh0, nkh);
+  const DkdvGrid f = dkdv_grid(a);
+  const int ns = a.ws ? dkdv_parts(a, HD) : 1;
+  hipLaunchKernelGGL((attn_bwd_dkdv_kernel<HD, T>), dim3(a.Hkv * f.nkh * ns), dim3(kThreads), 0, st, a, f.kh0, f.nkh, ns);
+  if (ns > 1)
+    hipLaunchKernelGGL((attn_bwd_dkdv_merge_kernel<HD, T>), dim3(a.Hkv * f.nkh * (HD / 32)), dim3(256), 0, st, a, f.kh0,
+                       f.nkh, ns);
 }
 
 template <int HD, typename T>

@@ -448,7 +448,8 @@ int64_t attn_bwd_ws_floats(const AttnArgs &a, int head_dim, int dtype) {
   if (dtype == kDtF32) return attn_bwd_f32_ws_floats(a, head_dim);
   const KeySplit sp = dq_split(a);
   const DqGrid f = dq_grid(a);
-  return sp.ns > 1 ? (int64_t)8 * sp.r * sp.ns * f.nw * head_dim * 32 : 0;
+  const int64_t dq = sp.ns > 1 ? (int64_t)8 * sp.r * sp.ns * f.nw * head_dim * 32 : 0;
+  return std::max(dq, dkdv_ws_floats(a, head_dim));   // the passes run one after the other
 }
 
 template <int HD, typename T>

@@ -47,11 +47,12 @@ constexpr int kDtF16 = 2;
 
 // head_dim in {64, 128}; dtype one of kDt*.
 void launch_attn_fwd(const AttnArgs &a, int head_dim, int dtype, hipStream_t stream);
-// fp32 words of AttnArgs::ws that the forward / the dQ pass of this shape use
+// fp32 words of AttnArgs::ws that the forward / the backward's passes of this shape use
 // (S, L, P, nQ, nKV, Hq, Hkv and, for the backward, grad_start set), 0 where
 // they do not split their items.
 int64_t attn_fwd_ws_floats(const AttnArgs &a, int head_dim, int dtype);
 int64_t attn_bwd_ws_floats(const AttnArgs &a, int head_dim, int dtype);
+int64_t dkdv_ws_floats(const AttnArgs &a, int head_dim);   // of it, the 16-bit dK/dV pass
 // passes: kBwdDq (delta + dQ) and/or kBwdDkDv (dK/dV; reads the delta the dQ pass wrote).
 constexpr int kBwdDq = 1;
 constexpr int kBwdDkDv = 2;
