@@ -100,14 +100,11 @@ struct Vec {   // bf16 and fp16
 #pragma unroll
     for (int i = 0; i < W; ++i) v[i] = (float)a[i];
   }
-  __device__ __forceinline__ static void load(const T *p, float (&v)[W]) {
-    unpack(*reinterpret_cast<const i32x4 *>(p), v);
-  }
-  __device__ __forceinline__ static void store(T *p, const float (&v)[W]) {
+  __device__ __forceinline__ static void store_nt(T *p, const float (&v)[W]) {
     typename Elem<T>::v8 a;
 #pragma unroll
     for (int i = 0; i < W; ++i) a[i] = (T)v[i];
-    *reinterpret_cast<i32x4 *>(p) = __builtin_bit_cast(i32x4, a);
+    __builtin_nontemporal_store(__builtin_bit_cast(i32x4, a), reinterpret_cast<i32x4 *>(p));
   }
 };
 template <>
@@ -118,12 +115,9 @@ struct Vec<float> {
 #pragma unroll
     for (int i = 0; i < W; ++i) v[i] = a[i];
   }
-  __device__ __forceinline__ static void load(const float *p, float (&v)[W]) {
-    unpack(*reinterpret_cast<const i32x4 *>(p), v);
-  }
-  __device__ __forceinline__ static void store(float *p, const float (&v)[W]) {
+  __device__ __forceinline__ static void store_nt(float *p, const float (&v)[W]) {
     f32x4 a = {v[0], v[1], v[2], v[3]};
-    *reinterpret_cast<f32x4 *>(p) = a;
+    __builtin_nontemporal_store(a, reinterpret_cast<f32x4 *>(p));
   }
 };
 
@@ -262,6 +256,15 @@ __global__ __launch_bounds__(1024) void soft_ce_combine_kernel(const float *__re
   }
 }
 
+// Bound by the streams. The forward walks every row's columns upwards, all rows
+// side by side, so what the last-level cache (256 MB) still holds of x and t are
+// the last columns: this kernel starts at the end and walks down, and writes the
+// gradient past the cache (nontemporal), so that it does not push them out. The
+// next turn's loads are issued before this turn's arithmetic, as in the forward.
+// Loss + gradient, bf16 x 151 936: 1 024 rows 316 -> 274 us (303 without the
+// nontemporal stores), 300 rows 99 -> 86 us, 2 048 rows 604 -> 558 us; fp32, 512
+// rows 312 -> 273 us. 52 rows, which the cache holds whole, 22.2 -> 23.2 us of
+// kernels in a call that takes 54 us.
 template <typename T, bool VEC>
 __global__ __launch_bounds__(kThreads) void soft_ce_bwd_kernel(const T *__restrict__ x, int64_t xs,
                                                              const T *__restrict__ t, int64_t ts, int32_t V,
@@ -270,7 +273,8 @@ __global__ __launch_bounds__(kThreads) void soft_ce_bwd_kernel(const T *__restri
                                                              const float *__restrict__ stats,
                                                              T *__restrict__ g, int64_t gs) {
   const int tid = threadIdx.x;
-  const int row = blockIdx.x / nsplit, sp = blockIdx.x - row * nsplit;
+  const int b = gridDim.x - 1 - blockIdx.x;
+  const int row = b / nsplit, sp = b - row * nsplit;
   const int c0 = sp * chunk, c1 = min(V, c0 + chunk);
   const T *xr = x + (int64_t)row * xs;
   const T *tr = t + (int64_t)row * ts;
@@ -279,24 +283,40 @@ __global__ __launch_bounds__(kThreads) void soft_ce_bwd_kernel(const T *__restri
   const float mxl = stats[row] * kL2E, mtl = stats[2 * N + row] * kL2E;
   // saved values are clamped already; clamping again matches loss.py:203-205
   const float ax = go / fmaxf(stats[N + row], kClamp), at = go / fmaxf(stats[3 * N + row], kClamp);
-  int cs = c0;
+  constexpr int W = Vec<T>::W;
+  const int nvec = VEC ? (c1 - c0) / W : 0;
+  for (int c = c0 + nvec * W + tid; c < c1; c += kThreads) {
+    const float xv = (float)xr[c], tv = (float)tr[c];
+    gr[c] = (T)(ax * ex2(__builtin_fmaf(xv, kL2E, -mxl)) - at * ex2(__builtin_fmaf(tv, kL2E, -mtl)));
+  }
   if constexpr (VEC) {
-    constexpr int W = Vec<T>::W;
-    const int nvec = (c1 - c0) / W;
-    for (int i = tid; i < nvec; i += kThreads) {
+    const i32x4 *xp = reinterpret_cast<const i32x4 *>(xr + c0) + tid;
+    const i32x4 *tp = reinterpret_cast<const i32x4 *>(tr + c0) + tid;
+    T *gp = gr + c0 + tid * W;
+    auto put = [&](int i, const i32x4 &xa, const i32x4 &ta) {
       float xv[W], tv[W], gv[W];
-      Vec<T>::load(xr + c0 + i * W, xv);
-      Vec<T>::load(tr + c0 + i * W, tv);
+      Vec<T>::unpack(xa, xv);
+      Vec<T>::unpack(ta, tv);
 #pragma unroll
       for (int e = 0; e < W; ++e)
         gv[e] = ax * ex2(__builtin_fmaf(xv[e], kL2E, -mxl)) - at * ex2(__builtin_fmaf(tv[e], kL2E, -mtl));
-      Vec<T>::store(gr + c0 + i * W, gv);
+      Vec<T>::store_nt(gp + (int64_t)i * W, gv);
+    };
+    const int nturn = nvec / (2 * kThreads);
+    for (int i = nturn * 2 * kThreads; i + tid < nvec; i += kThreads) put(i, xp[i], tp[i]);
+    if (nturn > 0) {
+      int n = (nturn - 1) * 2 * kThreads;
+      i32x4 xa = xp[n], ta = tp[n], xb = xp[n + kThreads], tb = tp[n + kThreads];
+      while (n > 0) {
+        n -= 2 * kThreads;
+        const i32x4 xc = xp[n], tc = tp[n], xd = xp[n + kThreads], td = tp[n + kThreads];
+        put(n + 3 * kThreads, xb, tb);
+        put(n + 2 * kThreads, xa, ta);
+        xa = xc; ta = tc; xb = xd; tb = td;
+      }
+      put(kThreads, xb, tb);
+      put(0, xa, ta);
     }
-    cs = c0 + nvec * W;
-  }
-  for (int c = cs + tid; c < c1; c += kThreads) {
-    const float xv = (float)xr[c], tv = (float)tr[c];
-    gr[c] = (T)(ax * ex2(__builtin_fmaf(xv, kL2E, -mxl)) - at * ex2(__builtin_fmaf(tv, kL2E, -mtl)));
   }
 }
 

@@ -143,3 +143,23 @@ def test_splits_and_row_sum(mga, dev, rows, V, dtype):
     assert bool(((loss.double() - want).abs() <= 1e-5 * want.abs()).all())
     total = mga.StableSoftCrossEntropy.apply(x, t)
     assert total.shape == () and abs(float(total) - float(want.sum())) <= 1e-5 * float(want.sum())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,V,dtype", [(1, 4088, torch.bfloat16),      # vectors, no whole turn
+                                          (1030, 4096, torch.bfloat16),   # one turn
+                                          (1030, 8195, torch.bfloat16),   # rows not 16-byte aligned
+                                          (1030, 14384, torch.bfloat16),  # three turns and a part of one
+                                          (40, 9004, torch.float32),      # splits, a short last one
+                                          (1030, 6148, torch.float32)])   # three turns and one vector
+def test_gradient_turns(mga, dev, rows, V, dtype):
+    """The gradient at the edges of its column walk, against float64 on the
+    GPU: two fp32 probabilities p and q, each within 1e-5 (sums of V terms), and
+    the output's rounding, |g - g'| <= u |g'| + 1e-5 (p + q)."""
+    print(f"case {rows} {V} {dtype}", flush=True)
+    gen = torch.Generator(device=dev).manual_seed(V)
+    x, t = ((torch.randn(1, rows, V, generator=gen, device=dev) * 3).to(dtype) for _ in range(2))
+    _, grad = _run(mga, x, t)
+    p, q = x.double().softmax(-1), t.double().softmax(-1)
+    u = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0
+    assert bool(((grad.double() - (p - q)).abs() <= u * (p - q).abs() + 1e-5 * (p + q) + 1e-30).all())
