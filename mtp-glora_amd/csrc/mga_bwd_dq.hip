@@ -436,10 +436,18 @@ DqGrid dq_grid(const AttnArgs &a) {
   return f;
 }
 
+// items per XCD that the launch without a workspace runs whole
+int dq_whole(const AttnArgs &a, const DqGrid &f) {
+  return f.nw == 8 ? dq_split_point(f.items, a.L, device_cu_count()) : f.nmax;
+}
+
 KeySplit dq_split(const AttnArgs &a) {
   const DqGrid f = dq_grid(a);
-  return key_split_plan(f.nmax, f.slots, last_round_tiles(a.S, a.P, a.Hkv, f.nslice, f.rows, f.nmax % f.slots),
-                        kDqPartTiles, kDqMergeTiles, 4);
+  const KeySplit sp = key_split_plan(f.nmax, f.slots,
+                                     last_round_tiles(a.S, a.P, a.Hkv, f.nslice, f.rows, f.nmax % f.slots),
+                                     kDqPartTiles, kDqMergeTiles, 4);
+  const QShare share{a.S, a.P, f.nslice, f.rows, f.nmax, f.slots};
+  return sp.ns > 1 && split_ends_first(sp, share, dq_whole(a, f), kDqMergeTiles) ? sp : no_split(f.nmax);
 }
 
 }  // namespace
@@ -461,7 +469,7 @@ void dq_launch(const AttnArgs &a, hipStream_t st) {
     sp.ws = a.ws;
     grid = 8 * sp.groups();
   } else {
-    if (f.nw == 8) k1 = dq_split_point(f.items, a.L, device_cu_count());
+    k1 = dq_whole(a, f);
     grid = 8 * k1;
   }
   if (grid > 0) {

@@ -697,8 +697,12 @@ FwdGrid fwd_grid(const AttnArgs &a) {
 // The split of the last items over their keys, ns = 1 for none.
 static KeySplit fwd_split(const AttnArgs &a) {
   const FwdGrid f = fwd_grid(a);
-  return key_split_plan(f.nmax, f.slots, last_round_tiles(a.S, a.P, a.Hkv, f.nslice, f.rows, f.nmax % f.slots),
-                        kFwdPartTiles, kFwdMergeTiles, 4);
+  const KeySplit sp = key_split_plan(f.nmax, f.slots,
+                                     last_round_tiles(a.S, a.P, a.Hkv, f.nslice, f.rows, f.nmax % f.slots),
+                                     kFwdPartTiles, kFwdMergeTiles, 4);
+  const QShare share{a.S, a.P, f.nslice, f.rows, f.nmax, f.slots};
+  return sp.ns > 1 && split_ends_first(sp, share, fwd_split_point(f.items, a.L, f.slots), kFwdMergeTiles)
+             ? sp : no_split(f.nmax);
 }
 
 int64_t attn_fwd_ws_floats(const AttnArgs &a, int head_dim, int dtype) {

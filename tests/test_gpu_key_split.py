@@ -106,3 +106,15 @@ def test_workspace_plan(mga):
     base = [p, 128, 4096, p, 128 * 64, 128, p, 128 * 64, 128, p, 128, 4096, p, p, p, p, p, p]
     rc = lib.mga_attn_fwd_ws(*base, 508, 20999, 20491, 32, 8, 128, 0, 0.1, p, 64, None)
     assert rc == mga._lib.MGA_ERR_INVALID and b"workspace" in lib.mga_last_error()
+
+
+@pytest.mark.parametrize("S,P,D", [(872, 1500, 128), (872, 1500, 64), (872, 6000, 64), (1000, 2500, 128),
+                                   (3248, 1500, 128), (3624, 2500, 128), (3624, 5000, 128)])
+def test_whole_items_where_they_end_first(mga, S, P, D):
+    """Chunks whose own keys are a large share of their lists (32 / 8 heads): the
+    slots that end early level the whole items, and the split launches timed 3
+    to 15% slower, so neither the forward nor the dQ pass is split."""
+    lib = mga.load_library()
+    assert lib.mga_attn_workspace_bytes(S, P + S, 32, 8, D, 0, 0, 0) == 0
+    assert lib.mga_attn_workspace_bytes(S, P + S, 32, 8, D, 0, 1, P + S) == 0   # no key gradients: dQ alone
+    assert lib.mga_attn_workspace_bytes(508, 20491 + 508, 32, 8, D, 0, 0, 0) > 0
