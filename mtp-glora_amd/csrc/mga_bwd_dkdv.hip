@@ -38,6 +38,7 @@
 
 #include "mga_common.hpp"
 #include "mga_internal.hpp"
+#include "mga_key_split.hpp"
 
 namespace mga {
 
@@ -554,12 +555,15 @@ DkdvGrid dkdv_grid(const AttnArgs &a) {
 // about the larger of its longest part and its total over its CUs; a part costs
 // kPartSteps beyond its walk (key operands, cleared LDS, the groups' exchange),
 // the combining launch kMergeSteps and the traffic of the parts. A part keeps at
-// least two pairs a group; the lists are taken as causal ones.
+// least two pairs a group; the lists are taken as causal ones. The items'
+// unequal lists level the CUs where there are enough of them, so the count of
+// parts so found is taken only if the launch then also ends earlier workgroup
+// by workgroup (SlotClock): without that, 2 872 rows went from 187 to 195 us
+// and, with 16 / 8 heads, 2 186 rows from 78 to 86 us.
 // dK/dV pass alone (bf16, 32 / 8 heads of 128), unsplit -> split with its
 // combining: 508 rows 40.8 -> 32.5 us, 905 rows 68.4 -> 54.6, 1 506 rows 96.1 ->
-// 72.3, 2 528 rows 163.5 -> 160.3; from 4 029 rows on the totals bound it and it
-// stays whole. 28 / 4 heads, 1 506 rows 156 -> 103 us; 8 / 2 heads, 2 528 rows
-// 148 -> 93 us.
+// 72.3, 2 528 rows 163.5 -> 160.3; from about 2 600 rows on it stays whole.
+// 28 / 4 heads, 1 506 rows 156 -> 103 us; 8 / 2 heads, 2 528 rows 148 -> 93 us.
 constexpr float kPartSteps = 5.f, kMergeSteps = 5.f, kStepSeconds = 1.1e-6f, kPartBytesPerSecond = 4e12f;
 constexpr int kMaxDkdvParts = 8;
 int dkdv_parts(const AttnArgs &a, int head_dim) {
@@ -585,7 +589,15 @@ int dkdv_parts(const AttnArgs &a, int head_dim) {
       best_cost = cost;
     }
   }
-  return best;
+  if (best == 1) return 1;
+  SlotClock whole(slots), split(slots);
+  for (int64_t i = 0; i < share; ++i) {
+    const float all = steps(i % f.nkh);
+    whole.run(all + kPartSteps);
+    for (int p = 0; p < best; ++p) split.run(all / best + kPartSteps);
+  }
+  const float combine = kMergeSteps + best * traffic / (kPartBytesPerSecond * kStepSeconds);
+  return split.end() + combine < whole.end() ? best : 1;
 }
 
 }  // namespace
