@@ -2,14 +2,14 @@
 // logits t, one row per drafted position) for gfx950. HBM-bound: each kernel
 // streams its rows once.
 //
-// Forward, two launches:
+// Forward, two or three launches:
 //   soft_ce_partial_kernel  - grid (row, column split): one pass over a column
 //       range of x and t keeps the online statistics of both rows at once,
 //       (mx, dx) of x and (mt, dt, S = sum e^{t - mt} x) of t, and writes
 //       them per split;
-//   soft_ce_combine_kernel  - one workgroup merges the splits of each row in
-//       a fixed order, writes ce = -S / dt + mx + log dx and (mx, dx, mt, dt),
-//       and sums the row losses.
+//   soft_ce_combine_kernel  - merges the splits of each row in a fixed order,
+//       writes ce = -S / dt + mx + log dx and (mx, dx, mt, dt), and, at few
+//       rows, sums the row losses (soft_ce_sum_kernel at many).
 // The reference reads x twice (an x pass, then a fused t + x pass,
 // mtp_glora/core/loss.py:63-124); here both rows are read once.
 // Backward: grad_x = go * (e^{x - mx} / dx - e^{t - mt} / dt), written in the
@@ -207,23 +207,35 @@ __global__ __launch_bounds__(kThreads) void soft_ce_partial_kernel(const T *__re
   }
 }
 
-// One workgroup: tpr (a power of two) neighbouring lanes take a row's splits and
-// merge them in a fixed order, then the row losses are summed, in a fixed
-// order, into *sum (unless null). Latency-bound (at most a few hundred KB): the
-// splits' loads of a row run side by side, 10.8 us for one thread a row at 52
-// rows of 19 splits against 5.2 us, and the separate sum's launch is gone.
+// Sum of the workgroup's values, in a fixed order; on thread 0.
+__device__ __forceinline__ float block_sum(float v) {
+  const int tid = threadIdx.x;
+  for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
+  __shared__ float wsum[16];
+  if ((tid & 63) == 0) wsum[tid >> 6] = v;
+  __syncthreads();
+  v = tid < 16 ? wsum[tid] : 0.f;
+  for (int m = 8; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
+  return v;
+}
+
+// tpr (a power of two) neighbouring lanes take a row's splits and merge them in
+// a fixed order. With sum (one workgroup then) the row losses are summed too, in
+// a fixed order. Latency-bound (at most a few hundred KB): the splits' loads of
+// a row run side by side, 10.8 us for one thread a row at 52 rows of 19 splits
+// against 5.2 us, and the separate sum's launch is gone.
 __global__ __launch_bounds__(1024) void soft_ce_combine_kernel(const float *__restrict__ part, int32_t N,
                                                                int32_t nsplit, int32_t tpr,
                                                                float *__restrict__ loss, float *__restrict__ stats,
                                                                float *__restrict__ sum) {
-  const int tid = threadIdx.x, j = tid & (tpr - 1);
+  const int tid = threadIdx.x, j = tid & (tpr - 1), rows = 1024 / tpr;
   float total = 0.f;
-  for (int r0 = 0; r0 < N; r0 += 1024 / tpr) {
-    const int row = r0 + tid / tpr;
+  for (int64_t r0 = (int64_t)blockIdx.x * rows; r0 < N; r0 += (int64_t)gridDim.x * rows) {
+    const int64_t row = r0 + tid / tpr;
     Stats acc;
     if (row < N)
       for (int sp = j; sp < nsplit; sp += tpr) {
-        const float *p = part + ((int64_t)row * nsplit + sp) * 5;
+        const float *p = part + (row * nsplit + sp) * 5;
         Stats o;
         o.mx = p[0];
         o.dx = p[1];
@@ -240,20 +252,31 @@ __global__ __launch_bounds__(1024) void soft_ce_combine_kernel(const float *__re
       loss[row] = ce;
       stats[row] = acc.mx;
       stats[N + row] = dx;
-      stats[2 * N + row] = acc.mt;
-      stats[3 * N + row] = dt;
+      stats[2 * (int64_t)N + row] = acc.mt;
+      stats[3 * (int64_t)N + row] = dt;
     }
   }
   if (!sum) return;
-  for (int m = 32; m >= 1; m >>= 1) total += __shfl_xor(total, m, 64);
-  __shared__ float wsum[16];
-  if ((tid & 63) == 0) wsum[tid >> 6] = total;
-  __syncthreads();
-  if (tid < 64) {
-    float v = tid < 16 ? wsum[tid] : 0.f;
-    for (int m = 8; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
-    if (tid == 0) *sum = v;
+  total = block_sum(total);
+  if (tid == 0) *sum = total;
+}
+
+// *sum = the row losses added in a fixed order, eight loads in flight a thread.
+__global__ __launch_bounds__(1024) void soft_ce_sum_kernel(const float *__restrict__ loss, int32_t N,
+                                                           float *__restrict__ sum) {
+  float total = 0.f;
+  for (int64_t r0 = 0; r0 < N; r0 += 8 * 1024) {
+    float v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int64_t r = r0 + u * 1024 + threadIdx.x;
+      v[u] = r < N ? loss[r] : 0.f;
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) total += v[u];
   }
+  total = block_sum(total);
+  if (threadIdx.x == 0) *sum = total;
 }
 
 // Bound by the streams. The forward walks every row's columns upwards, all rows
@@ -339,6 +362,13 @@ int64_t soft_ce_workspace_floats(int32_t N, int32_t V) {
   return (int64_t)N * ns * 5;
 }
 
+// Passes over the rows up to which one workgroup combines and sums them; beyond,
+// every pass is a workgroup and the sum a launch of its own. Whole forward, bf16
+// x 1 024 columns (a pass is 1 024 rows), one workgroup / one a pass: 2 048 rows
+// 10.8 / 11.6 us, 3 072 rows 13.3 / 13.3, 4 096 rows 15.9 / 15.1, 16 384 rows 46.7 /
+// 36.6; 65 536 rows of 512 columns 152 / 105 us.
+constexpr int kOneGroupPasses = 3;
+
 template <typename T>
 static void fwd_typed(const void *x, int64_t xs, const void *t, int64_t ts, int32_t N, int32_t V, bool vec,
                       float *loss, float *stats, float *sum, float *ws, hipStream_t st) {
@@ -353,7 +383,11 @@ static void fwd_typed(const void *x, int64_t xs, const void *t, int64_t ts, int3
                        (const T *)t, ts, V, ch, ns, ws);
   int tpr = 1;
   while (tpr < ns && tpr < 64) tpr *= 2;
-  hipLaunchKernelGGL(soft_ce_combine_kernel, dim3(1), dim3(1024), 0, st, ws, N, ns, tpr, loss, stats, sum);
+  const int passes = (int)(((int64_t)N * tpr + 1023) / 1024);   // of one workgroup over the rows
+  const bool one = sum && passes <= kOneGroupPasses;
+  hipLaunchKernelGGL(soft_ce_combine_kernel, dim3(one ? 1 : passes), dim3(1024), 0, st, ws, N, ns, tpr, loss, stats,
+                     one ? sum : nullptr);
+  if (sum && !one) hipLaunchKernelGGL(soft_ce_sum_kernel, dim3(1), dim3(1024), 0, st, loss, N, sum);
 }
 
 template <typename T>

@@ -163,3 +163,26 @@ def test_gradient_turns(mga, dev, rows, V, dtype):
     p, q = x.double().softmax(-1), t.double().softmax(-1)
     u = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0
     assert bool(((grad.double() - (p - q)).abs() <= u * (p - q).abs() + 1e-5 * (p + q) + 1e-30).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,V", [(3072, 96), (3073, 96),      # the last size of one workgroup, one pass more
+                                    (9 * 1024 + 5, 33),          # the sum's second turn
+                                    (1000, 10240)])              # several lanes a row
+def test_many_rows(mga, dev, rows, V):
+    """Row losses and their sum where one workgroup ends and one a pass begins,
+    against float64 on the GPU (1e-5, sums of V terms); without a sum asked for
+    the rows are the same bit for bit."""
+    from importlib import import_module
+    lossmod = import_module("mtp-glora_amd.loss")
+    gen = torch.Generator(device=dev).manual_seed(rows)
+    x, t = (torch.randn(1, rows, V, generator=gen, device=dev) * 3 for _ in range(2))
+    want = -(torch.softmax(t.double(), -1) * torch.log_softmax(x.double(), -1)).sum(-1)[0]
+    loss, total, stats = lossmod._forward(x, t)
+    assert bool(((loss.double() - want).abs() <= 1e-5 * want.abs()).all())
+    assert abs(float(total) - float(want.sum())) <= 1e-5 * float(want.sum())
+    again, stats2 = torch.empty_like(loss), torch.empty_like(stats)
+    ws = torch.empty(int(mga.load_library().mga_soft_ce_workspace_floats(rows, V)), device=dev)
+    mga._lib.call("mga_soft_ce_fwd", x.data_ptr(), V, t.data_ptr(), V, rows, V, mga.ops.dtype_code(x.dtype),
+                  again.data_ptr(), stats2.data_ptr(), ws.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    assert torch.equal(again, loss) and torch.equal(stats2, stats)
