@@ -100,11 +100,11 @@ struct Vec {   // bf16 and fp16
 #pragma unroll
     for (int i = 0; i < W; ++i) v[i] = (float)a[i];
   }
-  __device__ __forceinline__ static void store_nt(T *p, const float (&v)[W]) {
+  __device__ __forceinline__ static i32x4 pack(const float (&v)[W]) {
     typename Elem<T>::v8 a;
 #pragma unroll
     for (int i = 0; i < W; ++i) a[i] = (T)v[i];
-    __builtin_nontemporal_store(__builtin_bit_cast(i32x4, a), reinterpret_cast<i32x4 *>(p));
+    return __builtin_bit_cast(i32x4, a);
   }
 };
 template <>
@@ -115,9 +115,8 @@ struct Vec<float> {
 #pragma unroll
     for (int i = 0; i < W; ++i) v[i] = a[i];
   }
-  __device__ __forceinline__ static void store_nt(float *p, const float (&v)[W]) {
-    f32x4 a = {v[0], v[1], v[2], v[3]};
-    __builtin_nontemporal_store(a, reinterpret_cast<f32x4 *>(p));
+  __device__ __forceinline__ static i32x4 pack(const float (&v)[W]) {
+    return __builtin_bit_cast(i32x4, f32x4{v[0], v[1], v[2], v[3]});
   }
 };
 
@@ -281,14 +280,13 @@ __global__ __launch_bounds__(1024) void soft_ce_sum_kernel(const float *__restri
 
 // Bound by the streams. The forward walks every row's columns upwards, all rows
 // side by side, so what the last-level cache (256 MB) still holds of x and t are
-// the last columns: this kernel starts at the end and walks down, and writes the
-// gradient past the cache (nontemporal), so that it does not push them out. The
-// next turn's loads are issued before this turn's arithmetic, as in the forward.
-// Loss + gradient, bf16 x 151 936: 1 024 rows 316 -> 274 us (303 without the
-// nontemporal stores), 300 rows 99 -> 86 us, 2 048 rows 604 -> 558 us; fp32, 512
-// rows 312 -> 273 us. 52 rows, which the cache holds whole, 22.2 -> 23.2 us of
-// kernels in a call that takes 54 us.
-template <typename T, bool VEC>
+// the last columns: this kernel starts at the end and walks down. NT: the
+// gradient is written past the cache, so that it does not push them out (the rule
+// is at kCachedBytes). The next turn's loads are issued before this turn's
+// arithmetic, as in the forward. Loss + gradient, bf16 x 151 936, upwards with
+// ordinary stores / downwards / downwards past the cache: 1 024 rows 318 / 287 /
+// 267 us, 400 rows 109 / 109 / 99 us, 200 rows 59 / 57 / 57 us.
+template <typename T, bool VEC, bool NT>
 __global__ __launch_bounds__(kThreads) void soft_ce_bwd_kernel(const T *__restrict__ x, int64_t xs,
                                                              const T *__restrict__ t, int64_t ts, int32_t V,
                                                              int32_t chunk, int32_t nsplit, int32_t N,
@@ -323,7 +321,9 @@ __global__ __launch_bounds__(kThreads) void soft_ce_bwd_kernel(const T *__restri
 #pragma unroll
       for (int e = 0; e < W; ++e)
         gv[e] = ax * ex2(__builtin_fmaf(xv[e], kL2E, -mxl)) - at * ex2(__builtin_fmaf(tv[e], kL2E, -mtl));
-      Vec<T>::store_nt(gp + (int64_t)i * W, gv);
+      i32x4 *out = reinterpret_cast<i32x4 *>(gp + (int64_t)i * W);
+      if constexpr (NT) __builtin_nontemporal_store(Vec<T>::pack(gv), out);
+      else *out = Vec<T>::pack(gv);
     };
     const int nturn = nvec / (2 * kThreads);
     for (int i = nturn * 2 * kThreads; i + tid < nvec; i += kThreads) put(i, xp[i], tp[i]);
@@ -390,18 +390,28 @@ static void fwd_typed(const void *x, int64_t xs, const void *t, int64_t ts, int3
   if (sum && !one) hipLaunchKernelGGL(soft_ce_sum_kernel, dim3(1), dim3(1024), 0, st, loss, N, sum);
 }
 
+// Bytes of x, t and their gradient up to which the last-level cache holds all
+// three: the gradient is then written into it, where the next operation (the
+// head's backward) finds it. Loss + gradient + a copy of the gradient, bf16 x
+// 151 936, ordinary / past the cache: 52 rows 30.4 / 31.6 us, 200 rows (182 MB)
+// 74.5 / 78.7, 250 rows (228 MB) 93.5 / 95.5, without the copy 66.7 / 66.6, with x
+// just written too 126 / 117; 300 rows 124 / 116 us.
+constexpr int64_t kCachedBytes = 200 << 20;
+
 template <typename T>
 static void bwd_typed(const void *x, int64_t xs, const void *t, int64_t ts, int32_t N, int32_t V, bool vec,
                       const float *go, const float *stats, void *g, int64_t gs, hipStream_t st) {
   int32_t ns, ch;
   soft_ce_plan(N, V, &ns, &ch);
   const dim3 grid((unsigned)((int64_t)N * ns));
-  if (vec)
-    hipLaunchKernelGGL((soft_ce_bwd_kernel<T, true>), grid, dim3(kThreads), 0, st, (const T *)x, xs, (const T *)t,
-                       ts, V, ch, ns, N, go, stats, (T *)g, gs);
-  else
-    hipLaunchKernelGGL((soft_ce_bwd_kernel<T, false>), grid, dim3(kThreads), 0, st, (const T *)x, xs,
-                       (const T *)t, ts, V, ch, ns, N, go, stats, (T *)g, gs);
+  const bool nt = 3 * (int64_t)N * V * (int64_t)sizeof(T) > kCachedBytes;
+  auto run = [&](auto k) {
+    hipLaunchKernelGGL(k, grid, dim3(kThreads), 0, st, (const T *)x, xs, (const T *)t, ts, V, ch, ns, N, go, stats,
+                       (T *)g, gs);
+  };
+  if (vec && nt) run(soft_ce_bwd_kernel<T, true, true>);
+  else if (vec) run(soft_ce_bwd_kernel<T, true, false>);
+  else run(soft_ce_bwd_kernel<T, false, false>);
 }
 
 void launch_soft_ce_fwd(const void *x, int64_t xs, const void *t, int64_t ts, int32_t N, int32_t V, int dtype,

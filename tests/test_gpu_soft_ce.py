@@ -186,3 +186,21 @@ def test_many_rows(mga, dev, rows, V):
     mga._lib.call("mga_soft_ce_fwd", x.data_ptr(), V, t.data_ptr(), V, rows, V, mga.ops.dtype_code(x.dtype),
                   again.data_ptr(), stats2.data_ptr(), ws.data_ptr(), torch.cuda.current_stream().cuda_stream)
     assert torch.equal(again, loss) and torch.equal(stats2, stats)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,V,dtype", [(9000, 4088, torch.bfloat16),    # vectors, no whole turn
+                                          (9000, 4096, torch.float16),     # one turn
+                                          (5000, 14384, torch.bfloat16),   # three turns and a part of one
+                                          (3000, 6148, torch.float32)])    # three turns and one vector
+def test_gradient_past_the_cache(mga, dev, rows, V, dtype):
+    """More bytes than the last-level cache holds: written past it, the gradient
+    of a row is what it is among fewer rows, bit for bit (one split either way)."""
+    print(f"case {rows} {V} {dtype}", flush=True)
+    gen = torch.Generator(device=dev).manual_seed(V)
+    x, t = ((torch.randn(1, rows, V, generator=gen, device=dev) * 3).to(dtype) for _ in range(2))
+    few = 1100
+    assert 3 * x.nbytes > 210 << 20 > 3 * x[:, :few].nbytes
+    _, grad = _run(mga, x, t)
+    for i in (0, rows - few):
+        assert torch.equal(grad[:, i:i + few], _run(mga, x[:, i:i + few], t[:, i:i + few])[1])
