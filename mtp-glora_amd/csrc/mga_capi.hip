@@ -460,8 +460,6 @@ int mga_qk_norm_rope_bwd(const void *q, int64_t q_ss, int64_t q_hs, const void *
 
 namespace {
 
-// the streaming kernels' 32-bit lane offsets over 64 rows (128 of lora_A)
-constexpr int64_t kMaxStreamStride = int64_t(1) << 23;
 constexpr int64_t kBlasWorkspace = int64_t(32) << 20;   // hipBLASLt workspace per call
 
 int64_t align256(int64_t b) { return (b + 255) & ~int64_t(255); }
@@ -506,8 +504,6 @@ int check_vec_rows(const char *fn, const char *name, const void *ptr, int64_t rs
   if (!aligned16(ptr)) return fail(MGA_ERR_INVALID, "%s: %s is not 16-byte aligned", fn, name);
   if (rs < cols || rs % 8) return fail(MGA_ERR_INVALID, "%s: %s row stride %lld must be >= %lld and a multiple of 8",
                                        fn, name, (long long)rs, (long long)cols);
-  if (rs >= kMaxStreamStride)
-    return fail(MGA_ERR_INVALID, "%s: %s row stride %lld is too large (limit 2^23)", fn, name, (long long)rs);
   return MGA_OK;
 }
 
@@ -720,7 +716,8 @@ int mga_gated_lora_bwd(const void *grad_y, int64_t gy_rs, const void *x, int64_t
   // dB = dY^T t: one streaming pass over dY each (ranks up to 128, 16-byte
   // rows), else hipBLASLt
   const bool skinny = rank <= 128 && N % 8 == 0 && rows16(grad_y, gy_rs) && rows16(lora_b, b_rs) && rows16(t, t_rs) &&
-                      gy_rs < kMaxStreamStride && b_rs < kMaxStreamStride && t_rs < kMaxStreamStride;
+                      gy_rs < mga::kMaxStreamStride && b_rs < mga::kMaxStreamStride &&
+                      t_rs < mga::kMaxStreamStride;
   if (skinny) {
     mga::LoraSkinnyArgs sk = {};
     sk.dy = grad_y; sk.dy_rs = gy_rs; sk.t = t; sk.t_rs = t_rs; sk.b = lora_b; sk.b_rs = b_rs;

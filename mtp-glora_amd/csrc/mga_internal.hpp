@@ -137,9 +137,12 @@ struct LoraSkinnyArgs {
   const void *b; int64_t b_rs;         // lora_B [N, rank] bf16
   int32_t S, N, rank;
 };
+// Row strides from which a streaming product reads by 64-bit addresses (32-bit
+// lane offsets over 64 rows, lora_A's over 128 ranks).
+constexpr int64_t kMaxStreamStride = int64_t(1) << 23;
 // One rank-r product that streams a wide operand (see lora_stream_body). Rows
-// 16-byte aligned, strides a multiple of 8 elements below 2^23 (32-bit lane
-// offsets over 64 rows; lora_A's over 128 ranks).
+// 16-byte aligned, strides a multiple of 8 elements (kU and kDb: below
+// kMaxStreamStride).
 struct LoraStream {
   const void *x; int64_t x_rs;         // [rows, cols] bf16
   const void *sm; int64_t sm_rs;       // the small matrix, bf16

@@ -345,9 +345,12 @@ __global__ __launch_bounds__(256) void lora_transpose_kernel(const bf16_t *A, in
 // end as other elements of X, which are zeroed in the operand where they are
 // reduced over and stay in lines that nothing reads otherwise. Rank columns
 // past the rank hold junk that the finishing kernels do not read.
+// FAR (kDa and kDown, row strides of 2^23 elements and more, which the loads'
+// 32-bit lane offsets over a tile's rows do not reach): the same granules by
+// 64-bit addresses through registers, rows and columns past the end as zeros.
 enum { kDb = 0, kU = 1, kDa = 2, kDown = 3 };
 
-template <int KIND, int RB, bool DROP, bool WRITE_H>
+template <int KIND, int RB, bool DROP, bool WRITE_H, bool FAR = false>
 __device__ __forceinline__ void lora_stream_body(const LoraStream &a, int blk, int split, bf16_t *lds) {
   constexpr bool kCols = KIND == kDb || KIND == kDa;   // lines are columns of X, rows are reduced
   constexpr int RP = 32 * RB;                 // ranks of a small tile
@@ -396,6 +399,26 @@ __device__ __forceinline__ void lora_stream_body(const LoraStream &a, int blk, i
   auto issue = [&](int c, bf16_t *st) {
     const int k0 = chunk_of(min(c, nch - 1)) * 64;   // past the share: its last chunk again
     const int r0 = kCols ? k0 : line0, n0 = kCols ? line0 : k0;
+    if constexpr (FAR) {
+      auto put = [&](bf16_t *dst, const bf16_t *base, int64_t rs, int r, int nr, int c, int nc) {
+        const bf16x8 v = r < nr && c < nc ? load8(base + r * rs + c) : zero8();
+        *reinterpret_cast<i32x4 *>(dst + lane * 8) = __builtin_bit_cast(i32x4, v);
+      };
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int r = 16 * kq + 8 * i + (lane >> 3);
+        put(st + half * YT + (16 * kq + 8 * i) * 64, x, a.x_rs, r0 + r, a.rows, n0 + 8 * ((lane & 7) ^ swz<64>(r)), a.cols);
+      }
+#pragma unroll
+      for (int i = 0; i < MIA; ++i)
+        if (i < MIB || w < 4) {
+          const int r = 8 * (w + 8 * i) + (lane >> 3), slot = 64 * (w + 8 * i) + lane;
+          bf16_t *dst = st + 2 * YT + 512 * (w + 8 * i);
+          if constexpr (KIND == kDown) put(dst, sm, a.sm_rs, r, a.rank, k0 + 8 * ((lane & 7) ^ swz<64>(r)), a.cols);
+          else put(dst, sm, a.sm_rs, k0 + slot / MG, kdim, min(8 * (slot % MG), mcols - 8), mcols);
+        }
+      return;
+    }
     // resource ranges end with the last element of the tile's last existing row
     const int64_t yb = (int64_t)(min(64, a.rows - r0) - 1) * a.x_rs + a.cols - n0;
     const i32x4 ry =
@@ -580,18 +603,18 @@ __global__ __launch_bounds__(512, 1) void lora_skinny_kernel(LoraStream u, LoraS
   else lora_stream_body<kDb, RB, false, false>(b, (i - nbu * u.ns) % nbb, (i - nbu * u.ns) / nbb, lds);
 }
 
-template <int RB>
+template <int RB, bool FAR>
 __global__ __launch_bounds__(512, 1) void lora_da_kernel(LoraStream a) {
   __shared__ __attribute__((aligned(16))) bf16_t lds[kStreamLds<RB>];
   const int nb = (a.cols + 127) / 128;
-  lora_stream_body<kDa, RB, true, false>(a, blockIdx.x % nb, blockIdx.x / nb, lds);
+  lora_stream_body<kDa, RB, true, false, FAR>(a, blockIdx.x % nb, blockIdx.x / nb, lds);
 }
 
-template <int RB, bool DROP, bool WRITE_H>
+template <int RB, bool DROP, bool WRITE_H, bool FAR>
 __global__ __launch_bounds__(512, 1) void lora_down_kernel(LoraStream a) {
   __shared__ __attribute__((aligned(16))) bf16_t lds[kStreamLds<RB>];
   const int nb = (a.rows + 127) / 128;
-  lora_stream_body<kDown, RB, DROP, WRITE_H>(a, blockIdx.x % nb, blockIdx.x / nb, lds);
+  lora_stream_body<kDown, RB, DROP, WRITE_H, FAR>(a, blockIdx.x % nb, blockIdx.x / nb, lds);
 }
 
 // t[s][r] = T(T(s * T(sum over the splits, in order)) * gate), 0 for rank <= r
@@ -861,13 +884,36 @@ void skinny_plan(int32_t S, int32_t N, bool with_b, int32_t *nsu, int32_t *nsb) 
   stream_plan(blocks128(S), chunks64(N), nsu, with_b ? blocks128(N) : 0, with_b ? chunks64(S) : 0, nsb);
 }
 
-template <int RB>
+template <int RB, bool FAR>
 void down_rb(const LoraStream &a, bool drop, hipStream_t st) {
   const dim3 grid((unsigned)(blocks128(a.rows) * a.ns)), blk(512);
-  if (drop && a.h) hipLaunchKernelGGL((lora_down_kernel<RB, true, true>), grid, blk, 0, st, a);
-  else if (drop) hipLaunchKernelGGL((lora_down_kernel<RB, true, false>), grid, blk, 0, st, a);
-  else hipLaunchKernelGGL((lora_down_kernel<RB, false, false>), grid, blk, 0, st, a);
+  if (drop && a.h) hipLaunchKernelGGL((lora_down_kernel<RB, true, true, FAR>), grid, blk, 0, st, a);
+  else if (drop) hipLaunchKernelGGL((lora_down_kernel<RB, true, false, FAR>), grid, blk, 0, st, a);
+  else hipLaunchKernelGGL((lora_down_kernel<RB, false, false, FAR>), grid, blk, 0, st, a);
 }
+
+template <bool FAR>
+void down_rank(const LoraStream &a, bool drop, hipStream_t st) {
+  switch ((a.rank + 31) / 32) {
+    case 1: down_rb<1, FAR>(a, drop, st); break;
+    case 2: down_rb<2, FAR>(a, drop, st); break;
+    case 3: down_rb<3, FAR>(a, drop, st); break;
+    default: down_rb<4, FAR>(a, drop, st); break;
+  }
+}
+
+template <bool FAR>
+void da_rank(const LoraStream &a, hipStream_t st) {
+  const dim3 grid((unsigned)(blocks128(a.cols) * a.ns)), blk(512);
+  switch ((a.rank + 31) / 32) {
+    case 1: hipLaunchKernelGGL((lora_da_kernel<1, FAR>), grid, blk, 0, st, a); break;
+    case 2: hipLaunchKernelGGL((lora_da_kernel<2, FAR>), grid, blk, 0, st, a); break;
+    case 3: hipLaunchKernelGGL((lora_da_kernel<3, FAR>), grid, blk, 0, st, a); break;
+    default: hipLaunchKernelGGL((lora_da_kernel<4, FAR>), grid, blk, 0, st, a); break;
+  }
+}
+
+bool far_rows(const LoraStream &a) { return a.x_rs >= kMaxStreamStride || a.sm_rs >= kMaxStreamStride; }
 
 }  // namespace
 
@@ -893,12 +939,8 @@ void launch_lora_down(const LoraDownArgs &d, hipStream_t st) {
     a.keep_scale = d.keep_scale; a.thr = d.thr; a.seed = d.seed;
     a.h = r0 == 0 ? d.h : nullptr; a.h_rs = d.h_rs;
     const int rb = (a.rank + 31) / 32;
-    switch (rb) {
-      case 1: down_rb<1>(a, d.thr > 0, st); break;
-      case 2: down_rb<2>(a, d.thr > 0, st); break;
-      case 3: down_rb<3>(a, d.thr > 0, st); break;
-      default: down_rb<4>(a, d.thr > 0, st); break;
-    }
+    if (far_rows(a)) down_rank<true>(a, d.thr > 0, st);
+    else down_rank<false>(a, d.thr > 0, st);
     const int64_t n = (int64_t)d.S * (8 * rb);
     hipLaunchKernelGGL(lora_down_finish_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, 32 * rb,
                        d.gate, d.scaling, reinterpret_cast<bf16_t *>(d.t) + r0, d.t_rs);
@@ -913,13 +955,8 @@ void launch_lora_da(const LoraDaArgs &d, hipStream_t st) {
     a.part = d.part; a.rank = std::min(d.rank - r0, 128); a.ns = stream_split(d.K, d.S);
     a.keep_scale = d.keep_scale; a.thr = d.thr; a.seed = d.seed;
     const int rb = (a.rank + 31) / 32;
-    const dim3 grid((unsigned)(blocks128(d.K) * a.ns)), blk(512);
-    switch (rb) {
-      case 1: hipLaunchKernelGGL((lora_da_kernel<1>), grid, blk, 0, st, a); break;
-      case 2: hipLaunchKernelGGL((lora_da_kernel<2>), grid, blk, 0, st, a); break;
-      case 3: hipLaunchKernelGGL((lora_da_kernel<3>), grid, blk, 0, st, a); break;
-      default: hipLaunchKernelGGL((lora_da_kernel<4>), grid, blk, 0, st, a); break;
-    }
+    if (far_rows(a)) da_rank<true>(a, st);
+    else da_rank<false>(a, st);
     const int64_t n = (int64_t)a.rank * (d.K / 4);
     hipLaunchKernelGGL(lora_da_finish_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, 32 * rb,
                        reinterpret_cast<bf16_t *>(d.dA) + (int64_t)r0 * d.dA_rs, d.dA_rs);

@@ -357,7 +357,7 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> norm_rope_stage(const Tensor &
 // a [rows, cols] view that 16-byte vectors can read
 bool rows2(const Tensor &t, int64_t cols) {
   return t.dim() == 2 && t.size(1) == cols && t.size(0) > 0 && t.stride(1) == 1 && t.stride(0) >= cols &&
-         t.stride(0) % 8 == 0 && t.stride(0) < (int64_t(1) << 23) && aligned16(t);
+         t.stride(0) % 8 == 0 && aligned16(t);
 }
 
 struct GatedLora : public Function<GatedLora> {

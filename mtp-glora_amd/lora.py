@@ -59,8 +59,7 @@ def _rows(name: str, t: torch.Tensor, cols: int, dtype: torch.dtype = torch.bflo
     if t.shape[-1] != cols:
         raise ValueError(f"{name}: last dimension {t.shape[-1]} != {cols}")
     v = t.reshape(-1, cols)
-    # 32-bit lane offsets over a tile's rows: wider strides are copied
-    if v.stride(1) != 1 or v.stride(0) % 8 or v.stride(0) >= 1 << 23 or v.data_ptr() % 16:
+    if v.stride(1) != 1 or v.stride(0) % 8 or v.data_ptr() % 16:
         v = v.contiguous()
     return v
 

@@ -309,3 +309,42 @@ def test_streaming_edges(dev, S, K, N, r, p, gate):
 def test_unaligned_rows_take_the_library_products(dev):
     """N = 4: lora_B's products and the up-projection cannot use 16-byte rows."""
     run_case(dev, 70, 256, 4, 12, 0.1, seed=3)
+
+
+@pytest.mark.parametrize("S,K,r,p,x_rs,a_rs", [
+    (100, 256, 33, 0.1, 1 << 23, 256),               # x: the first stride past the 32-bit lane offsets
+    (65, 144, 8, 0.5, (1 << 23) + 8, 144),           # dropout output written, a 16-column tail
+    (3, 128, 96, 0.1, (1 << 26) + 16, 128),
+    (200, 640, 64, 0.0, 640, 1 << 23),               # lora_A
+    (70, 384, 128, 0.2, (1 << 22) + 8, (1 << 23) + 64),
+    (40, 256, 130, 0.1, 1 << 23, 1 << 23),           # both, ranks in two launches
+])
+def test_wide_row_strides(dev, S, K, r, p, x_rs, a_rs):
+    """x and lora_A as rows of far wider buffers: the streaming products are
+    those of dense rows bit for bit; y and dX, which pass through the library's
+    base product, within its fp32 order (1e-5) and the roundings of two results."""
+    print(f"case S={S} K={K} r={r} p={p} strides {x_rs} {a_rs}", flush=True)
+    lm = lora_mod()
+    x, W, A, B, gt = make(S, K, 96, r, dev, seed=S)
+    dy = torch.randn(S, 96, generator=torch.Generator(device=dev).manual_seed(S + 7), device=dev).bfloat16()
+
+    def wide(t, rs):
+        if rs == t.shape[1]:
+            return t
+        w = torch.empty((t.shape[0] - 1) * rs + t.shape[1], dtype=t.dtype, device=dev).as_strided(t.shape, (rs, 1))
+        return w.copy_(t)
+
+    def layer(x, A):
+        y, t, h = lm.gated_lora_forward(x, W, A, B, gt, 2.0, p, 77)
+        gx, ga, gb = lm.gated_lora_backward(dy, x, h, t, W, A, B, gt, 2.0, p, 77, True, p > 0, True)
+        return (y, gx), (t, h, ga, gb)
+
+    xw = wide(x, x_rs)
+    y = lm.gated_lora_linear(xw, W, A, B, gt, 2.0, p, seed=77)   # the public call reads the rows where they are
+    rounded, exact = layer(x, A)
+    assert bool(((y.float() - rounded[0].float()).abs() <= 2 * U * y.float().abs() + 1e-5 * y.float().abs().max()).all())
+    rounded_wide, exact_wide = layer(xw, wide(A, a_rs))
+    for a, b in zip(exact, exact_wide):
+        assert (a is None and b is None) or torch.equal(a, b)
+    for a, b in zip(rounded, rounded_wide):
+        assert bool(((a.float() - b.float()).abs() <= 2 * U * a.float().abs() + 1e-5 * a.float().abs().max()).all())
