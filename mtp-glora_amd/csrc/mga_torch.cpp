@@ -216,7 +216,10 @@ struct Attention : public Function<Attention> {
     TORCH_CHECK(d.sizes() == o.sizes(), "grad_output shape ", d.sizes(), " != output shape ", o.sizes());
     if (d.scalar_type() != q.scalar_type()) d = d.to(q.scalar_type());
     const int64_t eb = d.element_size();
-    if (d.stride(3) != 1 || d.stride(1) * eb % 16 || d.stride(2) * eb % 16 || !aligned16(d)) d = d.contiguous();
+    // rows that the kernels do not read where they are: one row expanded, or rows too far apart
+    if (d.stride(3) != 1 || d.stride(1) * eb % 16 || d.stride(2) * eb % 16 || d.stride(1) <= 0 ||
+        d.stride(1) >= (int64_t(1) << 23) || !aligned16(d))
+      d = d.clone(at::MemoryFormat::Contiguous);
     const auto opt = q.options().requires_grad(false);
     Tensor dq = at::empty({1, S, Hq, D}, opt), dk, dv;
     if (Lg > 0) {

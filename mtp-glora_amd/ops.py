@@ -259,8 +259,9 @@ def attn_bwd(q, k, v, o, lse, dout, code, bm: dict, P: int, scale: float, grad_s
     if d3.dtype != qq.dtype:
         d3 = d3.to(qq.dtype)
     if d3.stride(2) != 1 or (d3.stride(0) * d3.element_size()) % 16 or (d3.stride(1) * d3.element_size()) % 16 \
-            or d3.data_ptr() % 16:
-        d3 = d3.contiguous()
+            or not 0 < d3.stride(0) < 1 << 23 or d3.data_ptr() % 16:
+        # copied: also one row expanded, or rows too far apart for the kernels
+        d3 = d3.clone(memory_format=torch.contiguous_format)
     b = buffers if buffers is not None else bwd_buffers(q, k, grad_start)
     dq, dk, dv, delta = b["dq"], b["dk"], b["dv"], b["delta"]
     if dq.shape != (1, S, Hq, D) or delta.numel() != _lib.BWD_WS_WORDS_PER_ROW * Hq * S:

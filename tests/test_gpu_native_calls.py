@@ -48,7 +48,8 @@ def grads(outs, ins, douts):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("form", ["staged", "keys", "query_only", "no_grad", "strided", "expanded_grad"])
+@pytest.mark.parametrize("form", ["staged", "keys", "query_only", "no_grad", "strided", "expanded_grad",
+                                  "one_row_grad", "far_rows_grad"])
 def test_attention_and_cache(mga, dev, monkeypatch, dtype, form):
     P, Hq, Hkv, D = 37, 4, 2, 64
     seq = chunk_layout(65, 5, 3, P, seed=1, pad=2)
@@ -74,7 +75,14 @@ def test_attention_and_cache(mga, dev, monkeypatch, dtype, form):
         if form == "no_grad":
             return out
         d = torch.ones((), device=dev, dtype=dtype).expand(o.shape) if form == "expanded_grad" else do
+        if form == "one_row_grad":    # as the gradient of o.sum(1)
+            d = do[:, :1].expand(o.shape)
+        if form == "far_rows_grad":
+            d = torch.empty(S << 23, device=dev, dtype=dtype).as_strided(o.shape, (S << 23, 1 << 23, D, 1)).copy_(do)
         ins = [t for t in (qq, kk, vv) if t.requires_grad]
+        if form.endswith("_grad"):
+            dense = torch.autograd.grad(o, ins, do.new_empty(o.shape).copy_(d), retain_graph=True)
+            assert all(torch.equal(a, b) for a, b in zip(dense, torch.autograd.grad(o, ins, d, retain_graph=True)))
         return [t.detach() if t.dim() else t for t in out] + grads(o, ins, d) + list(grads(kf, [kk], kf.detach())
                                                                                       if kf.requires_grad else [])
 
