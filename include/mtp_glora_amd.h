@@ -59,6 +59,11 @@ extern "C" {
 /* Library version (major * 10000 + minor * 100 + patch). */
 int mga_version(void);
 
+/* Hash of the header that the library was built from (0: a build that did not
+ * define MGA_HEADER_HASH): modules with the C ABI compiled in compare it with
+ * their own before they call anything else. */
+uint64_t mga_header_hash(void);
+
 /* Message of the last error raised on the calling thread ("" if none). */
 const char *mga_last_error(void);
 

@@ -36,6 +36,7 @@ _F64 = ctypes.c_double
 _U64 = ctypes.c_uint64
 SIGNATURES = {
     "mga_version": [],
+    "mga_header_hash": [],
     "mga_last_error": [],
     "mga_kv_append": [_P, _P, _I64, _I64, _I64, _P, _I32, _P, _P, _I64, _I64, _I64, _I64, _I32, _I32, _I32, _P],
     "mga_regular_index": [_P, _I64, _I32, _P, _P, _P],
@@ -82,7 +83,8 @@ SIGNATURES = {
     "mga_soft_ce_bwd": [_P, _I64, _P, _I64, _I32, _I32, _I32, _P, _P, _P, _I64, _P],
 }
 _RESTYPES = {"mga_last_error": ctypes.c_char_p, "mga_soft_ce_workspace_floats": ctypes.c_int64,
-             "mga_gated_lora_workspace_bytes": ctypes.c_int64, "mga_attn_workspace_bytes": ctypes.c_int64}
+             "mga_gated_lora_workspace_bytes": ctypes.c_int64, "mga_attn_workspace_bytes": ctypes.c_int64,
+             "mga_header_hash": ctypes.c_uint64}
 
 
 class MGAError(RuntimeError):

@@ -8,6 +8,7 @@ against the installed torch into ``lib/_mga_torch.so``.
 """
 from __future__ import annotations
 
+import hashlib
 import os
 import shutil
 import subprocess
@@ -17,6 +18,7 @@ from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
+HEADER = PKG_DIR.parent / "include" / "mtp_glora_amd.h"
 LIB_DIR = PKG_DIR / "lib"
 LIB_NAME = "libmtp_glora_amd.so"
 TORCH_MODULE = "_mga_torch.so"
@@ -37,6 +39,11 @@ def hipcc() -> str:
 
 
 COMPILE_TIMEOUT_S = 900
+
+
+def header_flag() -> str:
+    """The C ABI's header as a number, compiled into the library and the torch module."""
+    return f"-DMGA_HEADER_HASH=0x{hashlib.sha256(HEADER.read_bytes()).hexdigest()[:16]}ull"
 
 
 def lib_path() -> Path:
@@ -60,7 +67,7 @@ def build_library(verbose: bool = False, jobs: int = 4, src_dir=None, out_path=N
 
     def compile_one(src: Path) -> Path:
         obj = objdir / (src.stem + ".o")
-        cmd = [cc, *COMMON_FLAGS, *DEVICE_FLAGS, "-c", str(src), "-o", str(obj)]
+        cmd = [cc, *COMMON_FLAGS, *DEVICE_FLAGS, header_flag(), "-c", str(src), "-o", str(obj)]
         try:
             # a compiler that loops (it has, on some unrolled kernels) fails
             # the build instead of holding it forever
@@ -96,7 +103,7 @@ def build_torch_module(verbose: bool = False) -> Path:
     tmp = out.with_suffix(".so.tmp")
     include = [*cpp_extension.include_paths("cuda"), sysconfig.get_paths()["include"], "/opt/rocm/include"]
     cmd = [shutil.which("g++") or "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1",
-           "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+           "-DUSE_ROCM=1", header_flag(), f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
            *(f"-isystem{p}" for p in include), str(CSRC / "mga_torch.cpp"), "-o", str(tmp),
            *(f"-L{p}" for p in cpp_extension.library_paths()), "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu",
            "-ltorch_python"]

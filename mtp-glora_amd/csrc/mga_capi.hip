@@ -133,6 +133,11 @@ extern "C" {
 
 int mga_version(void) { return 100; }
 
+#ifndef MGA_HEADER_HASH
+#define MGA_HEADER_HASH 0
+#endif
+uint64_t mga_header_hash(void) { return MGA_HEADER_HASH; }
+
 const char *mga_last_error(void) { return g_err; }
 
 int mga_kv_append(const void *src_k, const void *src_v, int64_t src_stride_h, int64_t src_stride_s,

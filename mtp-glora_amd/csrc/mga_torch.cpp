@@ -34,7 +34,7 @@ using torch::autograd::Function;
 using torch::autograd::variable_list;
 
 #define MGA_API(X)                                                                                    \
-  X(mga_kv_append) X(mga_attn_workspace_bytes) X(mga_attn_fwd_ws) X(mga_attn_bwd_ws) \
+  X(mga_header_hash) X(mga_kv_append) X(mga_attn_workspace_bytes) X(mga_attn_fwd_ws) X(mga_attn_bwd_ws) \
   X(mga_qk_norm_rope_stage_fwd) X(mga_qk_norm_rope_bwd) X(mga_gated_lora_workspace_bytes)             \
   X(mga_gated_lora_fwd) X(mga_gated_lora_bwd) X(mga_soft_ce_workspace_floats) X(mga_soft_ce_loss)     \
   X(mga_soft_ce_bwd)
@@ -47,6 +47,11 @@ struct Api {
 PyObject *g_raise = nullptr;   // raise(function name, code): owned for the life of the process
 
 void bind_api(const std::map<std::string, int64_t> &addr, const py::object &raise) {
+  // argument lists are compiled in: a library of another header must not be called
+  const auto at = addr.find("mga_header_hash");
+  if (at == addr.end() || reinterpret_cast<decltype(&::mga_header_hash)>(at->second)() != MGA_HEADER_HASH)
+    throw std::runtime_error("_mga_torch.so and libmtp_glora_amd.so were built from different headers: build both "
+                             "with `python __graft_entry__.py`");
 #define X(f) g.f = reinterpret_cast<decltype(&::f)>(addr.at(#f));
   MGA_API(X)
 #undef X

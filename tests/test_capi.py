@@ -123,3 +123,18 @@ def test_stage_invalid_arguments(mga, kw):
     lib = mga.load_library()
     assert _stage(lib, **kw) == mga._lib.MGA_ERR_INVALID
     assert lib.mga_last_error() != b""
+
+
+def test_torch_module_refuses_a_library_of_another_header(mga):
+    """The argument lists are compiled into the module, so it binds only to a
+    library whose header was its own; the binding it has stays."""
+    module = mga._lib.load_torch_module()
+    lib = mga.load_library()
+    addr = {n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in mga._lib.SIGNATURES}
+    assert lib.mga_header_hash() != 0
+    other = ctypes.CFUNCTYPE(ctypes.c_uint64)(lambda: lib.mga_header_hash() ^ 1)
+    for wrong in (dict(addr, mga_header_hash=ctypes.cast(other, ctypes.c_void_p).value),
+                  {n: a for n, a in addr.items() if n != "mga_header_hash"}):
+        with pytest.raises(RuntimeError, match="__graft_entry__"):
+            module.bind(wrong, mga._lib.raise_error)
+    module.bind(addr, mga._lib.raise_error)
