@@ -36,6 +36,23 @@ def qkv(S, P, Hq, Hkv, D, dtype, dev, seed=0, std=0.5):
     return q, k, v, kp, vp, do
 
 
+def attn_fwd_unsplit(mga, q, k, v, mask, scale):
+    """ops.attn_fwd by the C entry point without a workspace: no item is split
+    over its keys into parts, a short last round runs as two-group workgroups."""
+    ops, bm = mga.ops, mask.kernel_tensors()
+    _, Hq, S, D = q.shape
+    L = k.shape[2]
+    o = torch.empty(1, S, Hq, D, dtype=q.dtype, device=q.device)
+    lse = torch.empty(1, Hq, S, dtype=torch.float32, device=q.device)
+    mga._lib.call("mga_attn_fwd", q.data_ptr(), q.stride(1), q.stride(2), k.data_ptr(), k.stride(1), k.stride(2),
+                  v.data_ptr(), v.stride(1), v.stride(2), o.data_ptr(), D, Hq * D, lse.data_ptr(),
+                  mask.mtp_code.data_ptr(), bm["kv_num_blocks"].data_ptr(), bm["kv_indices"].data_ptr(),
+                  bm["full_kv_num_blocks"].data_ptr(), bm["full_kv_indices"].data_ptr(),
+                  S, L, mask.prefix_len, Hq, k.shape[1], D, ops.dtype_code(q.dtype), scale,
+                  torch.cuda.current_stream().cuda_stream)
+    return o, lse
+
+
 def f64(t):
     return t.detach().double().cpu().numpy()
 

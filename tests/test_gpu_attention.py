@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 import torch
 
-from gpu_helpers import (MAX_ABS, MEAN_ABS, check, chunk_layout, f64, qkv, round_to,
+from gpu_helpers import (MAX_ABS, MEAN_ABS, attn_fwd_unsplit, check, chunk_layout, f64, qkv, round_to,
                          rounding_model_grad_errors, torch_dense_reference)
 from oracle import mtp_oracle as mo
 
@@ -20,7 +20,9 @@ pytestmark = pytest.mark.gpu
 
 
 def run_case(mga, dev, n_reg, n_anchor, draft, P, Hq, Hkv, D, dtype=torch.bfloat16, seed=0,
-             pad=0, tail=False, every=None, use_cache=True, std=0.5):
+             pad=0, tail=False, every=None, use_cache=True, std=0.5, workspace=True):
+    """workspace=False: the C entry points without a workspace (gradients of
+    the chunk's rows), which never run an item in parts."""
     print(f"case n_reg={n_reg} anchors={n_anchor} draft={draft} P={P} Hq={Hq} Hkv={Hkv} D={D} "
           f"{dtype} pad={pad} tail={tail} cache={use_cache} std={std}", flush=True)
     seq = chunk_layout(n_reg, n_anchor, draft, P, seed=seed, pad=pad, tail=tail, every=every)
@@ -30,6 +32,13 @@ def run_case(mga, dev, n_reg, n_anchor, draft, P, Hq, Hkv, D, dtype=torch.bfloat
     k.requires_grad_()
     v.requires_grad_()
     bm = mga.build_mtp_block_mask(torch.tensor(seq.gate, device=dev)[None], P)
+    if not workspace:
+        kf, vf = torch.cat([kp, k.detach()], dim=2), torch.cat([vp, v.detach()], dim=2)
+        o, lse = attn_fwd_unsplit(mga, q.detach(), kf, vf, bm, D ** -0.5)
+        q.grad, k.grad, v.grad = mga.ops.attn_bwd(q.detach(), kf, vf, o, lse, do, bm.mtp_code, bm.kernel_tensors(), P,
+                                                  D ** -0.5, P)
+        torch.cuda.synchronize()
+        return seq, q, k, v, kp, vp, do, o, lse
     if use_cache:
         cache = mga.StreamingKVCache(capacity=P + S + 64, num_layers=1)
         if P:
@@ -105,10 +114,11 @@ def test_attention_small_fp16(mga, dev, c):
                    max_abs=F16_MAX_ABS, mean_abs=F16_MEAN_ABS, scaled=True)
 
 
-# Keys of at least 16 tiles and at most one round of items per XCD: the
-# forward and the dQ pass run every item as two-group workgroups (even and
-# odd tiles of the item's list, merged through LDS). Configs 2 and 4 run the
-# mixed launches (the last round two-group) in test_attention_full_config.
+# Keys of at least 16 tiles and at most half a round of items per XCD. Without
+# a workspace the forward and the dQ pass run every item as two-group workgroups
+# (even and odd tiles of the item's list, merged through LDS); the autograd call
+# has one and may run the items in parts. Config 2 without a workspace runs the
+# mixed launches (the last round two-group).
 SPLIT = [
     dict(n_reg=800, n_anchor=50, draft=4, P=1536, Hq=8, Hkv=2, D=128, pad=11),
     dict(n_reg=700, n_anchor=60, draft=4, P=1800, Hq=4, Hkv=1, D=64, tail=True),
@@ -117,10 +127,11 @@ SPLIT = [
 ]
 
 
+@pytest.mark.parametrize("workspace", [True, False])
 @pytest.mark.parametrize("c", SPLIT)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_attention_two_group_items(mga, dev, c, dtype):
-    seq, q, k, v, kp, vp, do, o, lse = run_case(mga, dev, dtype=dtype, seed=9, **c)
+def test_attention_two_group_items(mga, dev, c, dtype, workspace):
+    seq, q, k, v, kp, vp, do, o, lse = run_case(mga, dev, dtype=dtype, seed=9, workspace=workspace, **c)
     tol = dict(max_abs=F16_MAX_ABS, mean_abs=F16_MEAN_ABS, scaled=True) if dtype == torch.float16 else {}
     compare_oracle(seq, c["P"], q, k, v, kp, vp, do, o, lse, c["D"], grad_start=c["P"], **tol)
 
@@ -289,15 +300,22 @@ def test_attention_full_config(mga, dev, cfg):
     full_config_case(mga, dev, cfg, torch.bfloat16)
 
 
-# Config 2's chunk and prefix with other head geometries, each launching the
-# dQ pass as 8-wave pair items plus a two-group last round: G = 2 (two heads
-# per slice, 128 rows per item: 320 items), G = 8 (two slices of four heads:
-# 640 items) and D = 64.
+# Config 2's chunk and prefix with other head geometries: G = 2 (two heads per
+# slice, 128 rows per item: 320 items), G = 8 (two slices of four heads: 640
+# items) and D = 64. Without a workspace (below) the forward and the dQ pass run
+# them as 8-wave pair items plus a two-group last round.
 @pytest.mark.parametrize("heads", [dict(Hq=16, Hkv=8, D=128), dict(Hq=32, Hkv=4, D=128),
                                    dict(Hq=32, Hkv=8, D=64)],
                          ids=lambda h: f"hq{h['Hq']}_hkv{h['Hkv']}_d{h['D']}")
 def test_attention_config2_head_geometries(mga, dev, heads):
     full_config_case(mga, dev, dict(n_reg=4096, n_anchor=256, draft=4, P=8192, **heads), torch.bfloat16)
+
+
+@pytest.mark.parametrize("heads", [dict(), dict(Hq=16, Hkv=8, D=128), dict(Hq=32, Hkv=8, D=64)],
+                         ids=["hq32_hkv8_d128", "hq16_hkv8_d128", "hq32_hkv8_d64"])
+def test_attention_config2_without_workspace(mga, dev, heads):
+    full_config_case(mga, dev, dict(n_reg=4096, n_anchor=256, draft=4, P=8192, **heads), torch.bfloat16,
+                     workspace=False)
 
 
 def test_attention_full_config_fp16(mga, dev):
@@ -313,11 +331,11 @@ def test_attention_full_config_fp32(mga, dev):
                      max_abs=F32_MAX_ABS, mean_abs=F32_MEAN_ABS, grad_scaled=True)
 
 
-def full_config_case(mga, dev, cfg, dtype, max_abs=MAX_ABS, mean_abs=MEAN_ABS, grad_scaled=False):
+def full_config_case(mga, dev, cfg, dtype, max_abs=MAX_ABS, mean_abs=MEAN_ABS, grad_scaled=False, workspace=True):
     Hq, Hkv, D = cfg.get("Hq", 32), cfg.get("Hkv", 8), cfg.get("D", 128)
     seq, q, k, v, kp, vp, do, o, lse = run_case(
         mga, dev, cfg["n_reg"], cfg["n_anchor"], cfg["draft"], cfg["P"], Hq, Hkv, D, seed=2,
-        every=cfg.get("every"), dtype=dtype)
+        every=cfg.get("every"), dtype=dtype, workspace=workspace)
     P = cfg["P"]
     allowed = mo.mtp_mask_dense(seq.gate, P)
     kfull = torch.cat([kp, k.detach()], dim=2)

@@ -299,6 +299,8 @@ def test_long_reductions(dev, S, K, N, r):
                                             # as the dA and dB bounds, which have no term for it, need at one row)
     (700, 4096, 256, 33, 0.9375, "mixed"),  # nearly everything dropped (again an exact scale); more splits than line blocks
     (260, 1168, 520, 130, 0.1, "mixed"),    # ranks in two launches, one of two ranks
+    (320, 128, 32768, 128, 0.05, "mixed"),  # the wide write of y by ten waves a workgroup, the largest LDS of both forms
+    (320, 32768, 64, 128, 0.05, "mixed"),   # and of dX
 ])
 def test_streaming_edges(dev, S, K, N, r, p, gate):
     """The streaming products and the wide writes at the edges of their 128-line

@@ -8,8 +8,8 @@ Bounds, u the operand type's unit roundoff (2^-8 bf16, 2^-11 fp16: half a
 unit in the last place of a value at the bottom of its binade, so two
 roundings of nearly the same value lie up to 2 u apart):
 * o: the parts round their probabilities at another running offset, so each
-  of the two outputs is off by at most u sum p |v| <= u max|v| before its own
-  rounding: |o - o'| <= 2 u (max|v| + |o|);
+  of the two outputs is off by at most u sum p |v| before its own rounding (the
+  sum is the forward of |v|): |o - o'| <= 2 u (sum p |v| + |o|);
 * lse: fp32 sums in another order, |lse - lse'| <= 1e-5;
 * dQ: dS is formed from the same lse, so only the fp32 sum's order (bounded by
   1e-5 max|dq|) and the output's rounding differ:
@@ -22,7 +22,7 @@ Repeated calls are equal bit for bit."""
 import pytest
 import torch
 
-from gpu_helpers import chunk_layout, qkv
+from gpu_helpers import attn_fwd_unsplit, chunk_layout, qkv
 
 UNIT = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 0.0}
 
@@ -63,19 +63,14 @@ def test_split_equals_unsplit(mga, dev, c, dtype):
     assert lib.load().mga_attn_workspace_bytes(*size, 0, 0) > 0 and lib.load().mga_attn_workspace_bytes(*size, 1, P) > 0
 
     o, lse = ops.attn_fwd(q, kf, vf, code, bm, P, scale)
-    o1, lse1 = torch.empty_like(o), torch.empty_like(lse)
-    lib.call("mga_attn_fwd", q.data_ptr(), q.stride(1), q.stride(2), kf.data_ptr(), kf.stride(1), kf.stride(2),
-             vf.data_ptr(), vf.stride(1), vf.stride(2), o1.data_ptr(), D, c["Hq"] * D, lse1.data_ptr(),
-             code.data_ptr(), bm["kv_num_blocks"].data_ptr(), bm["kv_indices"].data_ptr(),
-             bm["full_kv_num_blocks"].data_ptr(), bm["full_kv_indices"].data_ptr(),
-             S, P + S, P, c["Hq"], c["Hkv"], D, ops.dtype_code(dtype), scale,
-             torch.cuda.current_stream().cuda_stream)
+    o1, lse1 = attn_fwd_unsplit(mga, q, kf, vf, mask, scale)
+    pv = attn_fwd_unsplit(mga, q, kf, vf.abs(), mask, scale)[0].float()
     assert torch.equal(torch.isneginf(lse), torch.isneginf(lse1))
     seen = torch.isfinite(lse1)
     assert float((lse - lse1)[seen].abs().max()) <= 1e-5
     d = (o.float() - o1.float()).abs()
     eps = 1e-5 * float(o1.float().abs().max()) if dtype == torch.float32 else 0.0
-    assert bool((d <= eps + 2 * u * (float(vf.abs().max()) + o1.float().abs())).all())
+    assert bool((d <= eps + 2 * u * (pv + o1.float().abs())).all())
 
     args = (q, kf, vf, o1, lse1, do, code, bm, P, scale, P)
     dq, dk, dv = ops.attn_bwd(*args, key_split=True)
@@ -92,16 +87,18 @@ def test_split_equals_unsplit(mga, dev, c, dtype):
 
 def test_workspace_plan(mga):
     """Whole rounds and short key lists need no workspace; the split ones stay
-    below 600 MB at the largest sizes; a smaller workspace is refused before
-    any device work."""
+    within four rounds of parts (a part: 8 waves of a 32-row O^T with its offsets
+    and sums) at the largest sizes; a smaller workspace is refused before any
+    device work."""
     lib = mga.load_library()
     assert lib.mga_attn_workspace_bytes(2048, 30720, 32, 8, 128, 0, 0, 0) == 0     # 32 items an XCD
     assert lib.mga_attn_workspace_bytes(320, 320, 32, 8, 128, 0, 0, 0) == 0        # three tiles of keys
     assert lib.mga_attn_workspace_bytes(508, 20999, 32, 8, 96, 0, 0, 0) == 0       # not a supported head_dim
+    most = 4 * 32 * 8 * 8 * (128 * 32 + 128) * 4   # rounds, slots an XCD, XCDs, waves, fp32 words of a wave
     for S in range(33, 6200, 97):
         for P in (0, 1000, 30000, 131072):
             for back in (0, 1):
-                assert 0 <= lib.mga_attn_workspace_bytes(S, P + S, 32, 8, 128, 0, back, P) < 600 << 20
+                assert 0 <= lib.mga_attn_workspace_bytes(S, P + S, 32, 8, 128, 0, back, P) <= most
     p = 16
     base = [p, 128, 4096, p, 128 * 64, 128, p, 128 * 64, 128, p, 128, 4096, p, p, p, p, p, p]
     rc = lib.mga_attn_fwd_ws(*base, 508, 20999, 20491, 32, 8, 128, 0, 0.1, p, 64, None)
@@ -120,7 +117,7 @@ def test_whole_items_where_they_end_first(mga, S, P, D):
     assert lib.mga_attn_workspace_bytes(508, 20491 + 508, 32, 8, D, 0, 0, 0) > 0
 
 
-@pytest.mark.parametrize("S,Hq,Hkv,D", [(2872, 32, 8, 128), (3062, 32, 8, 128), (2186, 16, 8, 128), (3248, 32, 8, 64)])
+@pytest.mark.parametrize("S,Hq,Hkv,D", [(2872, 32, 8, 128), (3062, 32, 8, 128), (3248, 32, 8, 64)])
 def test_key_tiles_whole_where_they_end_first(mga, S, Hq, Hkv, D):
     """Chunks whose key tiles level the CUs whole (the pass timed 2 to 10% slower
     in parts): the backward's workspace is the dQ pass's alone."""
@@ -129,3 +126,33 @@ def test_key_tiles_whole_where_they_end_first(mga, S, Hq, Hkv, D):
         dq = lib.mga_attn_workspace_bytes(S, P + S, Hq, Hkv, D, 0, 1, P + S)
         assert lib.mga_attn_workspace_bytes(S, P + S, Hq, Hkv, D, 0, 1, P) == dq
     assert lib.mga_attn_workspace_bytes(872, 872, 32, 8, D, 0, 1, 0) > 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("c", [dict(n_reg=520, n_anchor=18, P=200, Hq=32, Hkv=8, D=128, pad=8),
+                               dict(n_reg=500, n_anchor=25, P=500, Hq=28, Hkv=4, D=128, pad=0),
+                               dict(n_reg=401, n_anchor=24, P=199, Hq=12, Hkv=2, D=64, pad=3)])
+@pytest.mark.parametrize("from_first", [True, False])
+def test_prefix_keys_in_parts(mga, dev, c, dtype, from_first):
+    """dK and dV of prefix keys too (plain key tensors), all of them or from a row
+    inside a key tile on, with the pass's query lists in parts: the bound of
+    split and whole above, the combined rows of the first and the last tile among
+    them."""
+    ops, lib = mga.ops, mga._lib.load()
+    P, D, scale, u = c["P"], c["D"], c["D"] ** -0.5, UNIT[dtype]
+    start = 0 if from_first else 71
+    seq = chunk_layout(c["n_reg"], c["n_anchor"], 4, P, seed=6, pad=c["pad"])
+    S = len(seq.gate)
+    size = (S, P + S, c["Hq"], c["Hkv"], D, ops.dtype_code(dtype), 1)
+    print(f"case {c} {dtype} from {start}", flush=True)
+    assert lib.mga_attn_workspace_bytes(*size, start) > lib.mga_attn_workspace_bytes(*size, P + S)   # beyond dQ's
+    q, k, v, kp, vp, do = qkv(S, P, c["Hq"], c["Hkv"], D, dtype, dev, seed=6, std=1.0)
+    kf, vf = torch.cat([kp, k], 2), torch.cat([vp, v], 2)
+    mask = mga.build_mtp_block_mask(torch.tensor(seq.gate, device=dev)[None], P)
+    o, lse = attn_fwd_unsplit(mga, q, kf, vf, mask, scale)
+    args = (q, kf, vf, o, lse, do, mask.mtp_code, mask.kernel_tensors(), P, scale, start)
+    for a, b in zip(ops.attn_bwd(*args, key_split=True), ops.attn_bwd(*args)):
+        d = (a.float() - b.float()).abs()
+        assert a.shape[2] in (S, P + S - start)
+        assert bool((d <= 2 * u * b.float().abs() + 1e-5 * float(b.float().abs().max())).all())
