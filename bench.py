@@ -307,11 +307,11 @@ def gated_lora_phase(torch, timer, S: int, K: int, N: int, rank: int, p: float, 
         secs.append(time.perf_counter() - t0)
     cpu_s = sorted(secs[1:])[0]
     # HIP kernels' algorithmic bytes: the down-projection reads x and writes t
-    # (no dropout output is kept); the dX term is written once; grad_A reads x
-    # again (and d_a) to draw the mask
+    # (no dropout output is kept); the LoRA terms of y and dX are written once
+    # (lora_outer_kernel); grad_A reads x again (and d_a) to draw the mask
     rp = (rank + 31) // 32 * 32
     down_bytes = S * K * 2 + S * rp * 2
-    dx_bytes = S * K * 2 if p > 0 else 0
+    y_bytes, dx_bytes = S * rp * 2 + S * N * 2, S * rp * 2 + S * K * 2
     da_bytes = S * K * 2 + S * rp * 2 + rank * K * 2 if p > 0 else 0
     return {"S": S, "in": K, "out": N, "rank": rank, "dropout": p, "dtype": "bf16",
             "fwd_ms": round(t_f, 4), "bwd_ms": round(t_b, 4), "base_gemm_ms": round(t_gemm, 4),
@@ -319,7 +319,8 @@ def gated_lora_phase(torch, timer, S: int, K: int, N: int, rank: int, p: float, 
             "base_gemm_tflops": round(2.0 * S * K * N / (t_gemm * 1e-3) / 1e12, 1),
             "fwd_over_base_gemm": round(t_f / t_gemm, 3),
             "torch_eager_gpu_fwd_bwd_ms": round(t_ref, 4),
-            "kernel_bytes": {"lora_down_kernel": down_bytes, "lora_dx_kernel": dx_bytes, "lora_da_kernel": da_bytes},
+            "kernel_bytes": {"lora_down_kernel": down_bytes, "lora_outer_kernel (y)": y_bytes,
+                             "lora_outer_kernel (dX)": dx_bytes, "lora_da_kernel": da_bytes},
             "cpu_rows_per_s": round(cpu_rows / cpu_s, 1), "gpu_rows_per_s": round(S / ((t_f + t_b) * 1e-3), 1),
             "cpu_sample": f"the reference's ops as torch eager bf16 on the CPU, fwd + bwd, {cpu_rows} rows, "
                           f"best of 2 after a warm-up, {torch.get_num_threads()} threads"}
@@ -515,9 +516,9 @@ def layer_step_phase(torch, mga, syn, geo: dict, steps: int, warmup: int, seed: 
     n = max(steps, 5)
     t_fwd = timer(lambda: lib_ops.attn_fwd(qd, kf, vf, code, bmt, P, scale), n)
     t_dq = timer(lambda: lib_ops.attn_bwd(qd, kf, vf, o, lse, do, code, bmt, P, scale, P,
-                                          passes=libc.BWD_DQ, buffers=bufs), n)
+                                          passes=libc.BWD_DQ, buffers=bufs, key_split=True), n)
     t_dkdv = timer(lambda: lib_ops.attn_bwd(qd, kf, vf, o, lse, do, code, bmt, P, scale, P,
-                                            passes=libc.BWD_DKDV, buffers=bufs), n)
+                                            passes=libc.BWD_DKDV, buffers=bufs, key_split=True), n)
     passes = {}
     for name, t, f in (("fwd", t_fwd, 4 * (a_pre + a_cur)), ("bwd_dq_pass", t_dq, 6 * (a_pre + a_cur)),
                        ("bwd_dkdv_pass", t_dkdv, 4 * a_cur)):
@@ -553,7 +554,9 @@ def load_traffic(path: str, config: int):
         return None
     if t.get("config") != config:
         return None
-    return {k: v["traffic_bytes"] for k, v in t.get("kernels", {}).items()}
+    out = {k: v["traffic_bytes"] for k, v in t.get("kernels", {}).items()}
+    # an attention pass whose items run in parts: the launch that combines them too
+    return {k: v + out.get(k.replace("_kernel", "_merge_kernel"), 0) for k, v in out.items()}
 
 
 def pmc_pass(torch, mga, libc, q, k, v, do, kp, cache, chunk0, P, S, R, Hkv, D, scale) -> int:
@@ -577,8 +580,8 @@ def pmc_pass(torch, mga, libc, q, k, v, do, kp, cache, chunk0, P, S, R, Hkv, D, 
     qd = q.detach()
     o, lse = ops.attn_fwd(qd, kf, vf, code, bmt, P, scale)
     bufs = ops.bwd_buffers(qd, kf, P)
-    ops.attn_bwd(qd, kf, vf, o, lse, do, code, bmt, P, scale, P, passes=libc.BWD_DQ, buffers=bufs)
-    ops.attn_bwd(qd, kf, vf, o, lse, do, code, bmt, P, scale, P, passes=libc.BWD_DKDV, buffers=bufs)
+    ops.attn_bwd(qd, kf, vf, o, lse, do, code, bmt, P, scale, P, passes=libc.BWD_DQ, buffers=bufs, key_split=True)
+    ops.attn_bwd(qd, kf, vf, o, lse, do, code, bmt, P, scale, P, passes=libc.BWD_DKDV, buffers=bufs, key_split=True)
     idx, cnt = ops.regular_index(chunk0["regular_token_mask"])
     app_k = torch.empty(Hkv, R + 16, D, dtype=torch.bfloat16, device=dev)
     app_v = torch.empty_like(app_k)
@@ -873,9 +876,9 @@ def main() -> int:
     t_mask = timer(lambda: mga.build_mtp_block_mask(chunk0["gate_mask"], P), n)
     t_fwd = timer(lambda: lib_ops.attn_fwd(qd, kf, vf, code, bmt, P, scale), n)
     t_dq = timer(lambda: lib_ops.attn_bwd(qd, kf, vf, o, lse, do, code, bmt, P, scale, P,
-                                          passes=libc.BWD_DQ, buffers=bufs), n)
+                                          passes=libc.BWD_DQ, buffers=bufs, key_split=True), n)
     t_dkdv = timer(lambda: lib_ops.attn_bwd(qd, kf, vf, o, lse, do, code, bmt, P, scale, P,
-                                            passes=libc.BWD_DKDV, buffers=bufs), n)
+                                            passes=libc.BWD_DKDV, buffers=bufs, key_split=True), n)
     app_dst = torch.empty(Hkv, R + 16, D, dtype=torch.bfloat16, device=dev)
     app_dst_v = torch.empty_like(app_dst)
     t_commit = graph_time(torch, lambda: lib_ops.kv_append(k.detach(), v.detach(), app_dst, app_dst_v,
