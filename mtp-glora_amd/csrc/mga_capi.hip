@@ -602,7 +602,6 @@ int gated_lora_bwd_general(const char *fn, int dtype, const void *grad_y, int64_
 }  // namespace
 
 int64_t mga_gated_lora_workspace_bytes(int32_t S, int32_t K, int32_t N, int32_t rank) {
-  (void)N;
   if (S <= 0 || K <= 0 || rank <= 0) return 0;
   return lora_ws_bytes(S, K, N, rank);
 }

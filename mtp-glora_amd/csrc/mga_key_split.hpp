@@ -148,7 +148,7 @@ struct QShare {
 // their own. key_split_plan takes the last round's items as equally long and
 // the slots as free at the same time; where the chunk's own keys are a large
 // share of the lists, the slots that end early level the whole items by
-// themselves. So both launches are run through SlotClock (2 to 5 us of host
+// themselves. So both launches are run through SlotClock (up to 2.5 us of host
 // time), in key tiles: a whole item costs its list + 1; a part 1.05 of its
 // share + 2 (the parts of an item stream K and V apart from each other); two
 // groups half the longest list + 4, + 12 behind another launch, whose end they
