@@ -160,8 +160,8 @@ struct QShare {
 // 2 500, 265 -> 284 and 350 -> 369 us. With this rule one is left (3 361 rows on
 // 11 280, head_dim 64, dQ 571 -> 589 us), and nine that gained 3 to 17% run whole.
 inline bool split_ends_first(const KeySplit &sp, const QShare &f, int k1, float merge_cost) {
-  constexpr float kItem = 1.f, kPart = 2.f, kPartPace = 1.05f, kTwoGroups = 4.f, kTwoGroupsBehind = 12.f, kLonePace = 0.9f;
-  constexpr float kGain = 1.02f;
+  constexpr float kItem = 1.f, kPart = 2.f, kPartPace = 1.05f, kTwoGroups = 4.f, kTwoGroupsBehind = 12.f;
+  constexpr float kLonePace = 0.9f, kGain = 1.02f;
   constexpr int kRounds = 7;   // the rounds before the last that are looked at
   const int o0 = std::max(0, sp.k - kRounds * f.slots);
   const bool two_a_cu = f.slots > device_cu_count() / 8;
