@@ -561,8 +561,9 @@ DkdvGrid dkdv_grid(const AttnArgs &a) {
 // least two pairs a group; the lists are taken as causal ones. The items'
 // unequal lists level the CUs where there are enough of them, so the count of
 // parts so found is taken only if the launch then also ends earlier workgroup
-// by workgroup (SlotClock): without that, 2 872 rows went from 187 to 195 us
-// and, with 16 / 8 heads, 2 186 rows from 78 to 86 us.
+// by workgroup (SlotClock): without that, 2 872 rows went from 187 to 195 us and
+// with 16 / 8 heads 2 186 rows from 78 to 86 us, 1 190 rows behind a prefix from
+// 46.0 to 47.3 us and, of head_dim 64, 2 000 rows from 49.0 to 50.8 us.
 // dK/dV pass alone (bf16, 32 / 8 heads of 128), unsplit -> split with its
 // combining: 508 rows 40.8 -> 32.5 us, 905 rows 68.4 -> 54.6, 1 506 rows 96.1 ->
 // 72.3, 2 528 rows 163.5 -> 160.3; from about 2 600 rows on it stays whole.
@@ -593,14 +594,17 @@ int dkdv_parts(const AttnArgs &a, int head_dim) {
     }
   }
   if (best == 1) return 1;
+  // in us: a step by head_dim, a whole item's cost beyond its steps, a part's,
+  // the combining launch's and its bytes per us (fitted to 297 timed launches)
+  const float step = head_dim == 128 ? 1.1f : 0.8f;
+  constexpr float kItem = 5.5f, kPart = 7.f, kCombine = 5.5f, kBytes = 2.5e6f;
   SlotClock whole(slots), split(slots);
   for (int64_t i = 0; i < share; ++i) {
-    const float all = steps(i % f.nkh);
-    whole.run(all + kPartSteps);
-    for (int p = 0; p < best; ++p) split.run(all / best + kPartSteps);
+    const float all = steps(i % f.nkh) * step;
+    whole.run(all + kItem);
+    for (int p = 0; p < best; ++p) split.run(all / best + kPart);
   }
-  const float combine = kMergeSteps + best * traffic / (kPartBytesPerSecond * kStepSeconds);
-  return split.end() + combine < whole.end() ? best : 1;
+  return split.end() + kCombine + best * traffic / kBytes < whole.end() ? best : 1;
 }
 
 }  // namespace

@@ -117,7 +117,7 @@ def test_whole_items_where_they_end_first(mga, S, P, D):
     assert lib.mga_attn_workspace_bytes(508, 20491 + 508, 32, 8, D, 0, 0, 0) > 0
 
 
-@pytest.mark.parametrize("S,Hq,Hkv,D", [(2872, 32, 8, 128), (3062, 32, 8, 128), (3248, 32, 8, 64)])
+@pytest.mark.parametrize("S,Hq,Hkv,D", [(2872, 32, 8, 128), (3062, 32, 8, 128), (3248, 32, 8, 64), (2000, 16, 8, 64)])
 def test_key_tiles_whole_where_they_end_first(mga, S, Hq, Hkv, D):
     """Chunks whose key tiles level the CUs whole (the pass timed 2 to 10% slower
     in parts): the backward's workspace is the dQ pass's alone."""
