@@ -441,12 +441,12 @@ int dq_whole(const AttnArgs &a, const DqGrid &f) {
   return f.nw == 8 ? dq_split_point(f.items, a.L, device_cu_count()) : f.nmax;
 }
 
-KeySplit dq_split(const AttnArgs &a) {
+KeySplit dq_split(const AttnArgs &a, int head_dim) {
   const DqGrid f = dq_grid(a);
   const KeySplit sp = key_split_plan(f.nmax, f.slots,
                                      last_round_tiles(a.S, a.P, a.Hkv, f.nslice, f.rows, f.nmax % f.slots),
                                      kDqPartTiles, kDqMergeTiles, 4);
-  const QShare share{a.S, a.P, f.nslice, f.rows, f.nmax, f.slots};
+  const QShare share{a.S, a.P, f.nslice, f.rows, f.nmax, f.slots, head_dim};
   return sp.ns > 1 && split_ends_first(sp, share, dq_whole(a, f), kDqMergeTiles) ? sp : no_split(f.nmax);
 }
 
@@ -454,7 +454,7 @@ KeySplit dq_split(const AttnArgs &a) {
 
 int64_t attn_bwd_ws_floats(const AttnArgs &a, int head_dim, int dtype) {
   if (dtype == kDtF32) return attn_bwd_f32_ws_floats(a, head_dim);
-  const KeySplit sp = dq_split(a);
+  const KeySplit sp = dq_split(a, head_dim);
   const DqGrid f = dq_grid(a);
   const int64_t dq = sp.ns > 1 ? (int64_t)8 * sp.r * sp.ns * f.nw * head_dim * 32 : 0;
   return std::max(dq, dkdv_ws_floats(a, head_dim));   // the passes run one after the other
@@ -463,7 +463,7 @@ int64_t attn_bwd_ws_floats(const AttnArgs &a, int head_dim, int dtype) {
 template <int HD, typename T>
 void dq_launch(const AttnArgs &a, hipStream_t st) {
   const DqGrid f = dq_grid(a);
-  KeySplit sp = a.ws ? dq_split(a) : no_split(f.nmax);
+  KeySplit sp = a.ws ? dq_split(a, HD) : no_split(f.nmax);
   int k1 = f.nmax, grid;
   if (sp.ns > 1) {
     sp.ws = a.ws;

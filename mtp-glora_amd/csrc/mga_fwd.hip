@@ -695,19 +695,19 @@ FwdGrid fwd_grid(const AttnArgs &a) {
 }  // namespace
 
 // The split of the last items over their keys, ns = 1 for none.
-static KeySplit fwd_split(const AttnArgs &a) {
+static KeySplit fwd_split(const AttnArgs &a, int head_dim) {
   const FwdGrid f = fwd_grid(a);
   const KeySplit sp = key_split_plan(f.nmax, f.slots,
                                      last_round_tiles(a.S, a.P, a.Hkv, f.nslice, f.rows, f.nmax % f.slots),
                                      kFwdPartTiles, kFwdMergeTiles, 4);
-  const QShare share{a.S, a.P, f.nslice, f.rows, f.nmax, f.slots};
+  const QShare share{a.S, a.P, f.nslice, f.rows, f.nmax, f.slots, head_dim};
   return sp.ns > 1 && split_ends_first(sp, share, fwd_split_point(f.items, a.L, f.slots), kFwdMergeTiles)
              ? sp : no_split(f.nmax);
 }
 
 int64_t attn_fwd_ws_floats(const AttnArgs &a, int head_dim, int dtype) {
   if (dtype == kDtF32) return attn_fwd_f32_ws_floats(a, head_dim);
-  const KeySplit sp = fwd_split(a);
+  const KeySplit sp = fwd_split(a, head_dim);
   const FwdGrid f = fwd_grid(a);
   return sp.ns > 1 ? (int64_t)8 * sp.r * sp.ns * f.nw * part_floats(head_dim) : 0;
 }
@@ -715,7 +715,7 @@ int64_t attn_fwd_ws_floats(const AttnArgs &a, int head_dim, int dtype) {
 template <int HD, typename T>
 static void fwd_launch(const AttnArgs &a, hipStream_t st) {
   const FwdGrid f = fwd_grid(a);
-  KeySplit sp = a.ws ? fwd_split(a) : no_split(f.nmax);
+  KeySplit sp = a.ws ? fwd_split(a, HD) : no_split(f.nmax);
   int k1 = f.nmax, grid = 8 * f.nmax;
   if (sp.ns > 1) {
     sp.ws = a.ws;

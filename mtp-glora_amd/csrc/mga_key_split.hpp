@@ -136,7 +136,7 @@ class SlotClock {
 // The items of the first XCD's share, which holds the longest lists: rows row
 // blocks of a kv head's nslice head slices, last rows first.
 struct QShare {
-  int S, P, nslice, rows, nmax, slots;
+  int S, P, nslice, rows, nmax, slots, head_dim;
   int tiles(int o) const {   // key tiles of item o
     const int nqb = (S + rows - 1) / rows, qb = nqb - 1 - o % (nslice * nqb) / nslice;
     return (P + std::min((qb + 1) * rows, S) + kBlock - 1) / kBlock;
@@ -151,17 +151,19 @@ struct QShare {
 // themselves. So both launches are run through SlotClock (up to 2.5 us of host
 // time), in key tiles: a whole item costs its list + 1; a part 1.05 of its
 // share + 2 (the parts of an item stream K and V apart from each other); two
-// groups half the longest list + 4, + 12 behind another launch, whose end they
-// wait for; 4-wave workgroups, two slots a CU, run in 0.9 of the time where no
-// CU gets two. Of 412 16-bit launches timed with and without their plan (11
-// geometries, 124 to 5 900 rows, 0 to 20 000 prefix keys) 32 were slower split,
-// by up to 15%: 872 rows x 32 heads on 1 500 keys, forward 57.0 -> 60.6 us, dQ
-// 63.3 -> 68.7; 3 248 rows on 1 500, 191 -> 207 and 250 -> 265 us; 3 624 on
-// 2 500, 265 -> 284 and 350 -> 369 us. With this rule one is left (3 361 rows on
-// 11 280, head_dim 64, dQ 571 -> 589 us), and nine that gained 3 to 17% run whole.
+// groups half the longest list + 4 (head_dim 64: 2.5), + 12 behind another
+// launch, whose end they wait for; 4-wave workgroups, two slots a CU, run in 0.9
+// of the time where no CU gets two. Of 412 16-bit launches timed with and without
+// their plan (11 geometries, 124 to 5 900 rows, 0 to 20 000 prefix keys) 32 were
+// slower split, by up to 15%: 872 rows x 32 heads on 1 500 keys, forward 57.0 ->
+// 60.6 us, dQ 63.3 -> 68.7; 3 248 rows on 1 500, 191 -> 207 and 250 -> 265 us;
+// 3 624 on 2 500, 265 -> 284 and 350 -> 369 us. With this rule one is left (3 361
+// rows on 11 280, head_dim 64, dQ 571 -> 589 us), and ten that gained 3 to 17%
+// run whole.
 inline bool split_ends_first(const KeySplit &sp, const QShare &f, int k1, float merge_cost) {
-  constexpr float kItem = 1.f, kPart = 2.f, kPartPace = 1.05f, kTwoGroups = 4.f, kTwoGroupsBehind = 12.f;
+  constexpr float kItem = 1.f, kPart = 2.f, kPartPace = 1.05f, kTwoGroupsBehind = 12.f;
   constexpr float kLonePace = 0.9f, kGain = 1.02f;
+  const float two_groups = f.head_dim == 64 ? 2.5f : 4.f;
   constexpr int kRounds = 7;   // the rounds before the last that are looked at
   const int o0 = std::max(0, sp.k - kRounds * f.slots);
   const bool two_a_cu = f.slots > device_cu_count() / 8;
@@ -169,7 +171,7 @@ inline bool split_ends_first(const KeySplit &sp, const QShare &f, int k1, float 
   SlotClock whole(f.slots), split(f.slots);
   for (int o = o0; o < k1; ++o) whole.run(kItem + f.tiles(o));
   float unsplit = whole.end() * pace(k1 - o0);
-  if (k1 < f.nmax) unsplit += (k1 > 0 ? kTwoGroupsBehind : kTwoGroups) + 0.5f * f.tiles(k1);
+  if (k1 < f.nmax) unsplit += (k1 > 0 ? kTwoGroupsBehind : two_groups) + 0.5f * f.tiles(k1);
   for (int o = o0; o < sp.k; ++o) split.run(kItem + f.tiles(o));
   for (int o = sp.k; o < f.nmax; ++o) split.run(kPart + kPartPace * sp.begin(1, f.tiles(o)));
   for (int o = sp.k; o < f.nmax; ++o)

@@ -106,7 +106,7 @@ def test_workspace_plan(mga):
 
 
 @pytest.mark.parametrize("S,P,D", [(872, 1500, 128), (872, 1500, 64), (872, 6000, 64), (1000, 2500, 128),
-                                   (3248, 1500, 128), (3624, 2500, 128), (3624, 5000, 128)])
+                                   (3248, 1500, 128), (3624, 2500, 128), (3624, 5000, 128), (724, 2489, 64)])
 def test_whole_items_where_they_end_first(mga, S, P, D):
     """Chunks whose own keys are a large share of their lists (32 / 8 heads): the
     slots that end early level the whole items, and the split launches timed 3
