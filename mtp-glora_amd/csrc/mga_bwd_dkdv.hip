@@ -566,7 +566,7 @@ DkdvGrid dkdv_grid(const AttnArgs &a) {
 // 46.0 to 47.3 us and, of head_dim 64, 2 000 rows from 49.0 to 50.8 us.
 // dK/dV pass alone (bf16, 32 / 8 heads of 128), unsplit -> split with its
 // combining: 508 rows 40.8 -> 32.5 us, 905 rows 68.4 -> 54.6, 1 506 rows 96.1 ->
-// 72.3, 2 528 rows 163.5 -> 160.3; from about 2 600 rows on it stays whole.
+// 72.3, 2 000 rows 125 -> 104; from about 2 500 rows on it stays whole.
 // 28 / 4 heads, 1 506 rows 156 -> 103 us; 8 / 2 heads, 2 528 rows 148 -> 93 us.
 constexpr float kPartSteps = 5.f, kMergeSteps = 5.f, kStepSeconds = 1.1e-6f, kPartBytesPerSecond = 4e12f;
 constexpr int kMaxDkdvParts = 8;
